@@ -100,11 +100,41 @@ struct Boxes {
 };
 
 // ------------------------------------------------------------ bounding box
-constexpr int kRedBlocks = 1024;
+// min, max, min, max over a workgroup of NW waves, on every thread
+template <int NW>
+__device__ __forceinline__ void block_bounds(double* v, double (*sm)[4]) {
+#pragma unroll
+  for (int d = 32; d > 0; d >>= 1) {
+    v[0] = fmin(v[0], __shfl_xor(v[0], d, 64));
+    v[1] = fmax(v[1], __shfl_xor(v[1], d, 64));
+    v[2] = fmin(v[2], __shfl_xor(v[2], d, 64));
+    v[3] = fmax(v[3], __shfl_xor(v[3], d, 64));
+  }
+  const int w = threadIdx.x >> 6;
+  if ((threadIdx.x & 63) == 0)
+    for (int k = 0; k < 4; ++k) sm[w][k] = v[k];
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < NW; ++i) {
+    v[0] = fmin(v[0], sm[i][0]);
+    v[1] = fmax(v[1], sm[i][1]);
+    v[2] = fmin(v[2], sm[i][2]);
+    v[3] = fmax(v[3], sm[i][3]);
+  }
+}
 
-__global__ void k_bbox_partial(const double* __restrict__ src, int64_t ns,
-                               const double* __restrict__ trg, int64_t nt, double* part) {
-  __shared__ double sm[4][256];
+constexpr int kRedBlocks = 512;
+
+// Per-block bounds of all points into part[4 block ..]; also clears the words
+// that the key kernel and the sort count in.
+__global__ __launch_bounds__(256) void k_bbox_partial(const double* __restrict__ src, int64_t ns,
+                                                      const double* __restrict__ trg, int64_t nt,
+                                                      double* part, unsigned* words,
+                                                      int64_t nwords) {
+  __shared__ double sm[4][4];
+  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < nwords;
+       i += (int64_t)gridDim.x * 256)
+    words[i] = 0;
   double v[4] = {INFINITY, -INFINITY, INFINITY, -INFINITY};
   const int64_t n = ns + nt;
   for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) {
@@ -115,40 +145,34 @@ __global__ void k_bbox_partial(const double* __restrict__ src, int64_t ns,
     v[2] = fmin(v[2], y);
     v[3] = fmax(v[3], y);
   }
-  for (int k = 0; k < 4; ++k) sm[k][threadIdx.x] = v[k];
-  __syncthreads();
-  for (int s = 128; s > 0; s >>= 1) {
-    if ((int)threadIdx.x < s) {
-      sm[0][threadIdx.x] = fmin(sm[0][threadIdx.x], sm[0][threadIdx.x + s]);
-      sm[1][threadIdx.x] = fmax(sm[1][threadIdx.x], sm[1][threadIdx.x + s]);
-      sm[2][threadIdx.x] = fmin(sm[2][threadIdx.x], sm[2][threadIdx.x + s]);
-      sm[3][threadIdx.x] = fmax(sm[3][threadIdx.x], sm[3][threadIdx.x + s]);
-    }
-    __syncthreads();
-  }
-  if (threadIdx.x < 4) part[4 * blockIdx.x + threadIdx.x] = sm[threadIdx.x][0];
+  block_bounds<4>(v, sm);
+  if (threadIdx.x == 0)
+    for (int k = 0; k < 4; ++k) part[4 * blockIdx.x + k] = v[k];
 }
 
-__global__ void k_bbox_final(const double* part, int nb, double* out) {
-  __shared__ double sm[4][256];
-  double v[4] = {INFINITY, -INFINITY, INFINITY, -INFINITY};
-  for (int i = threadIdx.x; i < nb; i += 256) {
+// The bounds from the per-block ones, by every workgroup that needs them
+// (at most 16 KiB of L2 reads), into v on every thread.
+template <int NW>
+__device__ __forceinline__ void bounds_of_parts(const double* part, int nb, double* v,
+                                                double (*sm)[4]) {
+  v[0] = v[2] = INFINITY;
+  v[1] = v[3] = -INFINITY;
+  for (int i = threadIdx.x; i < nb; i += 64 * NW) {
     v[0] = fmin(v[0], part[4 * i]);
     v[1] = fmax(v[1], part[4 * i + 1]);
     v[2] = fmin(v[2], part[4 * i + 2]);
     v[3] = fmax(v[3], part[4 * i + 3]);
   }
-  for (int k = 0; k < 4; ++k) sm[k][threadIdx.x] = v[k];
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    for (int i = 1; i < 256; ++i) {
-      v[0] = fmin(v[0], sm[0][i]);
-      v[1] = fmax(v[1], sm[1][i]);
-      v[2] = fmin(v[2], sm[2][i]);
-      v[3] = fmax(v[3], sm[3][i]);
-    }
-    for (int k = 0; k < 4; ++k) out[k] = v[k];
-  }
+  block_bounds<NW>(v, sm);
+}
+
+// Bounding square (pts_tree2d.f:455-517) of the bounds
+FMM2D_HD void root_square(const double* bb, double* cx, double* cy, double* bs) {
+  *bs = bb[1] - bb[0];
+  const double sizey = bb[3] - bb[2];
+  if (sizey > *bs) *bs = sizey;
+  *cx = (bb[0] + bb[1]) / 2;
+  *cy = (bb[2] + bb[3]) / 2;
 }
 
 // ------------------------------------------------------------ point paths
@@ -166,34 +190,71 @@ __global__ void k_bbox_final(const double* part, int nb, double* out) {
 constexpr int kD1 = 20;
 constexpr int kD2Max = 31;
 
-__global__ void k_path_keys(int64_t n, const double* __restrict__ xy, double cx0, double cy0,
-                            const double* __restrict__ half, int d1, int d2,
-                            unsigned long long* key1, unsigned long long* key2, int* iota) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const double x = xy[2 * i], y = xy[2 * i + 1];
-  double cx = cx0, cy = cy0;
+// The path of (x, y) over `levels` levels from the box (cx, cy) of half size
+// 2 h on, which moves along (box sizes are halved exactly as the reference's
+// boxsize(l+1) = boxsize(l)/2).
+__device__ __forceinline__ unsigned long long path_key(double x, double y, double& cx, double& cy,
+                                                       double& h, int levels) {
   unsigned long long k = 0;
-  for (int l = 1; l <= d1; ++l) {
+  for (int l = 0; l < levels; ++l) {
     const int qx = (x < cx) ? 0 : 1, qy = (y < cy) ? 0 : 1;
     k = (k << 2) | (unsigned long long)(2 * qy + qx);
-    const double h = half[l];
+    h *= 0.5;
     cx += qx ? h : -h;
     cy += qy ? h : -h;
   }
-  key1[i] = k;
-  if (d2 > 0) {
-    k = 0;
-    for (int l = d1 + 1; l <= d1 + d2; ++l) {
-      const int qx = (x < cx) ? 0 : 1, qy = (y < cy) ? 0 : 1;
-      k = (k << 2) | (unsigned long long)(2 * qy + qx);
-      const double h = half[l];
-      cx += qx ? h : -h;
-      cy += qy ? h : -h;
+  return k;
+}
+
+// The keys of one set over d1 and (second word) d2 further levels
+__global__ void k_path_keys(int64_t n, const double* __restrict__ xy, double cx0, double cy0,
+                            double bs0, int d1, int d2, unsigned long long* key1,
+                            unsigned long long* key2) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  double cx = cx0, cy = cy0, h = 0.5 * bs0;
+  key1[i] = path_key(xy[2 * i], xy[2 * i + 1], cx, cy, h, d1);
+  key2[i] = path_key(xy[2 * i], xy[2 * i + 1], cx, cy, h, d2);
+}
+
+// The keys of d1 levels of both sets (blockIdx.y), from the per-block bounds,
+// with the digit counts of their sort (hist[set][pass][digit]); block 0
+// writes the bounds.
+__global__ __launch_bounds__(kRsCountThreads) void k_keys_count(const double* __restrict__ src, int64_t ns,
+                                                    const double* __restrict__ trg, int64_t nt,
+                                                    const double* part, int nb, int d1,
+                                                    int npass, unsigned long long* ksrc,
+                                                    unsigned long long* ktrg, unsigned* hist,
+                                                    double* bounds) {
+  constexpr int kP = (2 * kD1 + 7) / 8;
+  constexpr int NT = kRsCountThreads;
+  __shared__ double sm[NT / 64][4];
+  __shared__ unsigned h[kP][256];
+  double bb[4];
+  bounds_of_parts<NT / 64>(part, nb, bb, sm);
+  if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0)
+    for (int k = 0; k < 4; ++k) bounds[k] = bb[k];
+  for (int q = threadIdx.x; q < kP * 256; q += NT) (&h[0][0])[q] = 0;
+  __syncthreads();
+  const double* xy = blockIdx.y ? trg : src;
+  const int64_t n = blockIdx.y ? nt : ns;
+  unsigned long long* out = blockIdx.y ? ktrg : ksrc;
+  double cx0, cy0, bs0;
+  root_square(bb, &cx0, &cy0, &bs0);
+  for (int64_t i0 = (int64_t)blockIdx.x * NT; i0 < n; i0 += (int64_t)gridDim.x * NT) {
+    const int64_t i = i0 + threadIdx.x;
+    unsigned long long k = 0;
+    if (i < n) {
+      double cx = cx0, cy = cy0, hh = 0.5 * bs0;
+      k = path_key(xy[2 * i], xy[2 * i + 1], cx, cy, hh, d1);
+      out[i] = k;
     }
-    key2[i] = k;
+    rs_count<kP>(h, k, i < n, npass);
   }
-  if (iota) iota[i] = (int)i;
+  __syncthreads();
+  hist += (size_t)256 * npass * blockIdx.y;
+  for (int q = threadIdx.x; q < npass * 256; q += NT)
+    if ((&h[0][0])[q]) atomicAdd(&hist[q], (&h[0][0])[q]);
 }
 
 template <typename T>
@@ -675,11 +736,11 @@ __global__ void k_reorg_apply(int64_t n, const int* map, const double* c0, const
 // inside each leaf, which the reference keeps in input order: label every
 // point (in input order) with its leaf's first position, then stable-sort.
 __global__ void k_leaf_label(int64_t n, const int* nchild, const int* se, const int* perm,
-                             unsigned* label) {
+                             unsigned long long* label) {
   const int64_t b = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (b >= n || nchild[b] != 0) return;
   const int s = se[2 * b];
-  for (int i = s; i < se[2 * b + 1]; ++i) label[perm[i]] = (unsigned)s;
+  for (int i = s; i < se[2 * b + 1]; ++i) label[perm[i]] = (unsigned long long)s;
 }
 
 // The same order without the sort: inside each leaf (a contiguous range of
@@ -756,11 +817,6 @@ __global__ __launch_bounds__(kLeafSortWaves * 64) void k_leaf_sort(const int* bi
   }
 }
 
-__global__ void k_iota(int64_t n, int* v) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) v[i] = (int)i;
-}
-
 // ------------------------------------------------------------ host helpers
 // Points of one set (sources or targets) sorted by path key.
 struct PathKeys {
@@ -770,29 +826,28 @@ struct PathKeys {
   DBuf<int> perm;                   // sorted position -> input index
   Keys view() const { return Keys{k1.p, k2.p, d1, d2}; }
 
-  void build(const double* xy, int64_t np, double cx, double cy, const double* half, int dd1,
-             int dd2, hipStream_t st) {
+  void alloc(int64_t np, int dd1, int dd2, hipStream_t st) {
     n = np;
     d1 = dd1;
     d2 = dd2;
     perm.alloc(std::max<int64_t>(n, 1), st);
     k1.alloc(std::max<int64_t>(n, 1), st);
     k2.alloc(d2 > 0 ? std::max<int64_t>(n, 1) : 0, st);
+  }
+  // keys of both words (deep trees)
+  void build(const double* xy, int64_t np, double cx, double cy, double bs, int dd1, int dd2,
+             hipStream_t st) {
+    alloc(np, dd1, dd2, st);
     if (n == 0) return;
-    DBuf<unsigned long long> u1(n, st), u2(d2 > 0 ? n : 0, st);
-    DBuf<int> iota(n, st);
-    launch1d(k_path_keys, n, st, xy, cx, cy, half, d1, d2, u1.p, u2.p, iota.p);
-    if (d2 == 0) {
-      radix_sort(u1.p, k1.p, iota.p, perm.p, n, 2 * d1, st);
-    } else {
-      // lexicographic (key1, key2): stable LSD passes, key2 first
-      DBuf<unsigned long long> t2(n, st), t1(n, st);
-      DBuf<int> p1(n, st);
-      radix_sort(u2.p, t2.p, iota.p, p1.p, n, 2 * d2, st);
-      launch1d(k_gather_by<unsigned long long>, n, st, p1.p, u1.p, t1.p);
-      radix_sort(t1.p, k1.p, p1.p, perm.p, n, 2 * d1, st);
-      launch1d(k_gather_by<unsigned long long>, n, st, perm.p, u2.p, k2.p);
-    }
+    DBuf<unsigned long long> u1(n, st), u2(n, st);
+    launch1d(k_path_keys, n, st, xy, cx, cy, bs, d1, d2, u1.p, u2.p);
+    // lexicographic (key1, key2): stable LSD passes, key2 first
+    DBuf<unsigned long long> t2(n, st), t1(n, st);
+    DBuf<int> p1(n, st);
+    radix_sort(u2.p, t2.p, nullptr, p1.p, n, 2 * d2, st);
+    launch1d(k_gather_by<unsigned long long>, n, st, p1.p, u1.p, t1.p);
+    radix_sort(t1.p, k1.p, p1.p, perm.p, n, 2 * d1, st);
+    launch1d(k_gather_by<unsigned long long>, n, st, perm.p, u2.p, k2.p);
   }
 };
 
@@ -949,7 +1004,7 @@ struct TreePrep {
   std::vector<double> bsall;  // box size of every possible level
   double root[2] = {0.0, 0.0};
   bool walk_ok = false;
-  DBuf<double> dhalf;
+  DBuf<double> bounds;        // min x, max x, min y, max y on the device
   PathKeys pk[2];
 };
 
@@ -962,34 +1017,38 @@ void prepare_into(TreePrep& P, const double* src, int64_t ns, const double* trg,
   P.ns = ns;
   P.nt = nt;
   P.nlmax = nlmax;
-  // ---- bounding square (pts_tree2d.f:455-517)
-  double bb[4];
-  {
-    const int nb = (int)std::min<int64_t>(kRedBlocks, std::max<int64_t>(1, ceil_div(ns + nt, 256)));
-    DBuf<double> part(4 * nb, st), out(4, st);
-    hipLaunchKernelGGL(k_bbox_partial, dim3(nb), dim3(256), 0, st, src, ns, trg, nt, part.p);
-    hipLaunchKernelGGL(k_bbox_final, dim3(1), dim3(256), 0, st, part.p, nb, out.p);
-    readback(bb, out.p, sizeof(bb), st);
-  }
-  // box sizes of every possible level (boxsize(l+1) = boxsize(l)/2)
-  std::vector<double>& bsall = P.bsall;
-  bsall.assign(nlmax + 2, 0.0);
-  bsall[0] = bb[1] - bb[0];
-  const double sizey = bb[3] - bb[2];
-  if (sizey > bsall[0]) bsall[0] = sizey;
-  for (int l = 1; l < (int)bsall.size(); ++l) bsall[l] = bsall[l - 1] / 2;
-  P.root[0] = (bb[0] + bb[1]) / 2;
-  P.root[1] = (bb[2] + bb[3]) / 2;
-  P.walk_ok = std::max(std::fabs(P.root[0]), std::fabs(P.root[1])) <= std::ldexp(bsall[0], 20);
-
-  // ---- point paths, sorted (sources and targets separately)
-  std::vector<double> half(bsall.size());
-  for (size_t l = 0; l < half.size(); ++l) half[l] = 0.5 * bsall[l];
-  P.dhalf.alloc(half.size(), st);
-  upload_bytes(P.dhalf.p, half.data(), sizeof(double) * half.size(), st);
   const int d1 = std::min(kD1, nlmax);
-  P.pk[0].build(src, ns, P.root[0], P.root[1], P.dhalf.p, d1, 0, st);
-  P.pk[1].build(trg, nt, P.root[0], P.root[1], P.dhalf.p, d1, 0, st);
+  P.pk[0].alloc(ns, d1, 0, st);
+  P.pk[1].alloc(nt, d1, 0, st);
+  P.bounds.alloc(4, st);
+  // bounds, keys with their digit counts, one launch per digit
+  const int nb = (int)std::min<int64_t>(kRedBlocks, std::max<int64_t>(1, ceil_div(ns + nt, 256)));
+  DBuf<double> part(4 * nb, st);
+  DBuf<unsigned long long> u0(ns, st), u1(nt, st);
+  RsPlan rs;
+  rs.init(ns, nt, 2 * d1, st);
+  hipLaunchKernelGGL(k_bbox_partial, dim3(nb), dim3(256), 0, st, src, ns, trg, nt, part.p,
+                     rs.words.p, (int64_t)rs.words.n);
+  const int64_t m = std::max(ns, nt);
+  hipLaunchKernelGGL(k_keys_count,
+                     dim3(rs_count_grid(m), nt > 0 ? 2 : 1), dim3(kRsCountThreads), 0, st, src, ns, trg, nt, (const double*)part.p, nb, d1, rs.npass,
+                     u0.p, u1.p, rs.hist(0), P.bounds.p);
+  hip_throw(hipGetLastError(), "path keys");
+  const unsigned long long* ki[2] = {u0.p, u1.p};
+  unsigned long long* ko[2] = {P.pk[0].k1.p, P.pk[1].k1.p};
+  int* vo[2] = {P.pk[0].perm.p, P.pk[1].perm.p};
+  rs.sort(ki, ko, nullptr, vo, st);
+}
+
+// the host's share of a preparation, from the bounds
+void prepare_host(TreePrep& P, const double* bb) {
+  double bs0;
+  root_square(bb, &P.root[0], &P.root[1], &bs0);
+  // box sizes of every possible level (boxsize(l+1) = boxsize(l)/2)
+  P.bsall.assign(P.nlmax + 2, 0.0);
+  P.bsall[0] = bs0;
+  for (int l = 1; l < (int)P.bsall.size(); ++l) P.bsall[l] = P.bsall[l - 1] / 2;
+  P.walk_ok = std::max(std::fabs(P.root[0]), std::fabs(P.root[1])) <= std::ldexp(bs0, 20);
 }
 }  // namespace
 
@@ -997,6 +1056,9 @@ TreePrep* tree_prepare(const double* src, int64_t ns, const double* trg, int64_t
                        hipStream_t st) {
   std::unique_ptr<TreePrep> P(new TreePrep());
   prepare_into(*P, src, ns, trg, nt, nlmax, st);
+  double bb[4];
+  readback(bb, P->bounds.p, sizeof(bb), st);
+  prepare_host(*P, bb);
   return P.release();
 }
 
@@ -1019,12 +1081,14 @@ void build_tree(const double* src, int64_t ns, const double* trg, int64_t nt, in
   const TreePrep* P = prep;
   if (!tree_prepare_matches(prep, src, ns, trg, nt, nlmax)) {
     prepare_into(own, src, ns, trg, nt, nlmax, st);
+    double bb[4];
+    readback(bb, own.bounds.p, sizeof(bb), st);
+    prepare_host(own, bb);
     P = &own;
   }
   const std::vector<double>& bsall = P->bsall;
   const double* root = P->root;
   bld.walk_ok = P->walk_ok;
-  const double* dhalf_p = P->dhalf.p;
   const int d1 = std::min(kD1, nlmax);
   // the keys in use: the prepared ones, or deeper ones made below (points
   // closer than 2^-21 of the domain)
@@ -1081,8 +1145,8 @@ void build_tree(const double* src, int64_t ns, const double* trg, int64_t nt, in
         // for points closer than 2^-21 of the domain)
         if (bld.scan(n) > 0) {
           const int d2 = std::min(kD2Max, std::min(62, nlmax) - d1);
-          pkx[0].build(src, ns, root[0], root[1], dhalf_p, d1, d2, st);
-          pkx[1].build(trg, nt, root[0], root[1], dhalf_p, d1, d2, st);
+          pkx[0].build(src, ns, root[0], root[1], bsall[0], d1, d2, st);
+          pkx[1].build(trg, nt, root[0], root[1], bsall[0], d1, d2, st);
           pk[0] = &pkx[0];
           pk[1] = &pkx[1];
           bld.ks = pk[0]->view();
@@ -1244,14 +1308,12 @@ void build_tree(const double* src, int64_t ns, const double* trg, int64_t nt, in
   for (int k = 0; k < 2; ++k) {
     if (npts[k] == 0 || !hbig[k]) continue;
     // a leaf too large for k_leaf_sort: stable sort of all points by leaf
-    DBuf<unsigned> label(npts[k], st), lsorted(npts[k], st);
-    DBuf<int> iota(npts[k], st);
+    DBuf<unsigned long long> label(npts[k], st), lsorted(npts[k], st);
     launch1d(k_leaf_label, nb, st, bld.B.nchild.p, se[k], pk[k]->perm.p, label.p);
     int bits = 1;
     while ((int64_t(1) << bits) <= npts[k]) ++bits;
     // values: input indices 0..n-1 in input order
-    launch1d(k_iota, npts[k], st, iota.p);
-    radix_sort(label.p, lsorted.p, iota.p, perm[k]->p, npts[k], bits, st);
+    radix_sort(label.p, lsorted.p, nullptr, perm[k]->p, npts[k], bits, st);
   }
   t.isrcse = std::move(bld.B.ses);
   t.itargse = std::move(bld.B.set);
@@ -1451,36 +1513,29 @@ void hist_from_keys(const unsigned long long* ks, int64_t ns, const unsigned lon
 void key_leaf_histogram(const double* src, int64_t ns, const double* trg, int64_t nt, int ndiv,
                         int nbins, double* hist, double* boxsize0, hipStream_t st) {
   if (nbins < 1 || nbins > kLeafHistMax) throw HipError{hipErrorInvalidValue, "histogram bins"};
-  double bb[4];
-  {
-    const int nb = (int)std::min<int64_t>(kRedBlocks, std::max<int64_t>(1, ceil_div(ns + nt, 256)));
-    DBuf<double> part(4 * nb, st), out(4, st);
-    hipLaunchKernelGGL(k_bbox_partial, dim3(nb), dim3(256), 0, st, src, ns, trg, nt, part.p);
-    hipLaunchKernelGGL(k_bbox_final, dim3(1), dim3(256), 0, st, part.p, nb, out.p);
-    readback(bb, out.p, sizeof(bb), st);
-  }
-  const double bs = std::max(bb[1] - bb[0], bb[3] - bb[2]);
-  if (boxsize0) *boxsize0 = bs;
   // levels up to nbins - 1 tell every bin apart (the last bin takes the leaf
   // levels from nbins - 1 on): shorter keys, fewer sort passes
   const int d1 = std::max(1, std::min(kD1, nbins - 1));
-  // half[l] = boxsize(l) / 2 with boxsize(l + 1) = boxsize(l) / 2, as in build_tree
-  std::vector<double> half(d1 + 2);
-  double bsl = bs;
-  for (int l = 0; l < (int)half.size(); ++l) {
-    half[l] = 0.5 * bsl;
-    bsl = bsl / 2;
-  }
-  DBuf<double> dhalf(half.size(), st);
-  upload_bytes(dhalf.p, half.data(), sizeof(double) * half.size(), st);
-  const double cx = (bb[0] + bb[1]) / 2, cy = (bb[2] + bb[3]) / 2;
+  const int nb = (int)std::min<int64_t>(kRedBlocks, std::max<int64_t>(1, ceil_div(ns + nt, 256)));
+  DBuf<double> part(4 * nb, st), bounds(4, st);
   DBuf<unsigned long long> k0(ns, st), ks(ns, st), kt(std::max<int64_t>(nt, 1), st);
-  launch1d(k_path_keys, ns, st, src, cx, cy, (const double*)dhalf.p, d1, 0, k0.p,
-           (unsigned long long*)nullptr, (int*)nullptr);
-  if (nt > 0)
-    launch1d(k_path_keys, nt, st, trg, cx, cy, (const double*)dhalf.p, d1, 0, kt.p,
-             (unsigned long long*)nullptr, (int*)nullptr);
-  radix_sort(k0.p, ks.p, (const int*)nullptr, (int*)nullptr, ns, 2 * d1, st);
+  RsPlan rs;  // the targets' keys are used unsorted
+  rs.init(ns, 0, 2 * d1, st);
+  hipLaunchKernelGGL(k_bbox_partial, dim3(nb), dim3(256), 0, st, src, ns, trg, nt, part.p,
+                     rs.words.p, (int64_t)rs.words.n);
+  hipLaunchKernelGGL(k_keys_count,
+                     dim3(rs_count_grid(std::max(ns, nt)), nt > 0 ? 2 : 1),
+                     dim3(kRsCountThreads), 0, st, src, ns, trg, nt, (const double*)part.p, nb, d1, rs.npass,
+                     k0.p, kt.p, rs.hist(0), bounds.p);
+  hip_throw(hipGetLastError(), "path keys");
+  const unsigned long long* ki[2] = {k0.p, nullptr};
+  unsigned long long* ko[2] = {ks.p, nullptr};
+  rs.sort(ki, ko, nullptr, nullptr, st);
+  if (boxsize0) {
+    double bb[4], cx, cy;
+    readback(bb, bounds.p, sizeof(bb), st);
+    root_square(bb, &cx, &cy, boxsize0);
+  }
   hist_from_keys(ks.p, ns, kt.p, nt, d1, ndiv, nbins, hist, st);
 }
 

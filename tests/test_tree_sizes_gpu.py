@@ -1,6 +1,6 @@
 """The GPU quadtree against the C oracle's (oracle/oracle.c), array for array, at the sizes where the
-build changes its ways: one workgroup's scan (16384 elements: 131072 sort keys, or that many boxes), tiles
-of 4096, and trees from a single leaf to tens of thousands of boxes."""
+build changes its ways: the sort's tiles (512, 1024, 2048 keys, by size), one workgroup's scan (16384
+boxes) and scan tiles of 4096, and trees from a single leaf to tens of thousands of boxes."""
 import numpy as np
 import pytest
 
@@ -33,7 +33,7 @@ def rows(lists, count):
 @pytest.mark.parametrize("kind,n,nt,ndiv", [
     ("uniform", 1, 0, 15), ("uniform", 15, 0, 15), ("uniform", 16, 3, 15), ("uniform", 300, 1, 1),
     ("clusters", 1000, 0, 15), ("clusters", 4095, 4097, 15), ("curve", 8192, 1000, 20), ("clusters", 8193, 70, 3),
-    ("curve", 30011, 20003, 20), ("clusters", 131072, 0, 40), ("uniform", 131073, 0, 15), ("clusters", 135169, 5, 8),
+    ("uniform", 16384, 513, 15), ("clusters", 16385, 512, 15), ("curve", 30011, 20003, 20), ("clusters", 262145, 1, 60), ("clusters", 131072, 0, 40), ("uniform", 131073, 0, 15), ("clusters", 135169, 5, 8),
 ])
 def test_tree_sizes(kind, n, nt, ndiv):
     from fmm2d_amd.tree import build_tree
