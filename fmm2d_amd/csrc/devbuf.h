@@ -30,6 +30,9 @@ inline void hip_throw(hipError_t e, const char* what) {
 constexpr size_t kReadbackMax = 4096;
 constexpr size_t kUploadInline = 1024;
 void readback(void* dst, const void* src, size_t bytes, hipStream_t st);
+// two pieces in one round trip
+void readback2(void* dst, const void* src, size_t bytes, void* dst2, const void* src2,
+               size_t bytes2, hipStream_t st);
 void upload_bytes(void* dst, const void* src, size_t bytes, hipStream_t st);
 
 // Workspace cache (ws.cpp).  ws_alloc returns at least `bytes` bytes usable

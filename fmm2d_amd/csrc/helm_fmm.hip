@@ -1431,9 +1431,6 @@ int helmholtz_fmm(const HelmArgs& a, hipStream_t st) {
       launch1d(k_gather_dens, ns, st, nd, t.isrc.p, a.dipstr, dps.p);
       launch1d(k_gather_dipvec, ns, st, nd, t.isrc.p, a.dipvec, dvs.p);
     }
-    DBuf<int> leaf_s(ns, st), leaf_t(std::max<int64_t>(nt, 1), st);
-    launch1d(k_leaf_of, nb, st, t.nchild.p, t.isrcse.p, leaf_s.p);
-    if (nt > 0) launch1d(k_leaf_of, nb, st, t.nchild.p, t.itargse.p, leaf_t.p);
     DBuf<cplx> mp(ncoef, st), loc(ncoef, st);
     mp.zero();
     loc.zero();
@@ -1450,12 +1447,12 @@ int helmholtz_fmm(const HelmArgs& a, hipStream_t st) {
     // ---- step 1: P2M (rows of the sources, then their sums per leaf)
     {
       DBuf<int64_t> roff(ns, st), rtot(1, st);
-      launch1d(k_hp2m_rowlen, ns, st, d_lev.p, leaf_s.p, t.ilevel.p, roff.p);
+      launch1d(k_hp2m_rowlen, ns, st, d_lev.p, t.leaf_s.p, t.ilevel.p, roff.p);
       exclusive_scan(roff.p, roff.p, ns, rtot.p, st);
       int64_t nrow = 0;
       readback(&nrow, rtot.p, sizeof(int64_t), st);
       DBuf<cplx> gJ(std::max<int64_t>(nrow, 1), st), uJ(ns, st);
-      launch1d(k_hp2m_rows, ns, st, zk, d_lev.p, leaf_s.p, t.ilevel.p, t.centers.p, xs.p,
+      launch1d(k_hp2m_rows, ns, st, zk, d_lev.p, t.leaf_s.p, t.ilevel.p, t.centers.p, xs.p,
                (const int64_t*)roff.p, gJ.p, uJ.p);
 #define FMM2D_P2M(C, D)                                                                       \
   hipLaunchKernelGGL((k_hp2m_g<C, D>), dim3(nb), dim3(kW), 0, st, nd, zk, d_lev.p, t.ilevel.p, \
@@ -1507,8 +1504,8 @@ int helmholtz_fmm(const HelmArgs& a, hipStream_t st) {
         launch_heval<2>(n, st, nd, zk, d_lev.p, xy, lf, t, L, mp.p, loc.p, P_, G_, H_);
       else launch_heval<3>(n, st, nd, zk, d_lev.p, xy, lf, t, L, mp.p, loc.p, P_, G_, H_);
     };
-    if (pg > 0) eval(pg, ns, xs.p, leaf_s.p, ps.p, gs.p, hs.p);
-    if (pgt > 0) eval(pgt, nt, xt.p, leaf_t.p, pt.p, gt.p, ht.p);
+    if (pg > 0) eval(pg, ns, xs.p, t.leaf_s.p, ps.p, gs.p, hs.p);
+    if (pgt > 0) eval(pgt, nt, xt.p, t.leaf_t.p, pt.p, gt.p, ht.p);
     tm.mark(6);
     // ---- step 8: near field, thresh = |zk| boxsize(0) 2^-51 (hfmm2d.f:1527)
     const int ifnear = o ? o->ifnear : 1;
@@ -1517,10 +1514,10 @@ int helmholtz_fmm(const HelmArgs& a, hipStream_t st) {
       DBuf<int2> seg((size_t)kSegRow * t.nboxes, st);
       launch1d(k_near_segs, t.nboxes, st, L.n1.p, L.l1.p, sse, seg.p);
       if (pg > 0)
-        launch_hnear(pg, a.ifcharge, a.ifdipole, ns, st, nd, zk, xs.p, leaf_s.p, seg.p, xs.p,
+        launch_hnear(pg, a.ifcharge, a.ifdipole, ns, st, nd, zk, xs.p, t.leaf_s.p, seg.p, xs.p,
                      chs.p, dps.p, dvs.p, thresh, ps.p, gs.p, hs.p, mixed);
       if (pgt > 0)
-        launch_hnear(pgt, a.ifcharge, a.ifdipole, nt, st, nd, zk, xt.p, leaf_t.p, seg.p, xs.p,
+        launch_hnear(pgt, a.ifcharge, a.ifdipole, nt, st, nd, zk, xt.p, t.leaf_t.p, seg.p, xs.p,
                      chs.p, dps.p, dvs.p, thresh, pt.p, gt.p, ht.p, mixed);
     }
     tm.mark(7);
@@ -1665,8 +1662,6 @@ int helmholtz_mps(const HelmMpsArgs& a, hipStream_t st) {
     DBuf<HLev> d_lev = upload(lev, st);
     DBuf<MpsExp> ex(n, st);
     launch1d(k_mps_gather, n, st, t.isrc.p, a.centers, a.rscale, a.mterms, a.impole, ex.p);
-    DBuf<int> leaf(n, st);
-    launch1d(k_leaf_of, nb, st, t.nchild.p, t.isrcse.p, leaf.p);
     DBuf<cplx> mp(ncoef, st), loc(ncoef, st);
     mp.zero();
     loc.zero();
@@ -1687,7 +1682,7 @@ int helmholtz_mps(const HelmMpsArgs& a, hipStream_t st) {
     helm_box_passes(t, L, lev, sl, nterms, nd, zk, 1, 0, mp.p, loc.p, tm, st);
     // ---- steps 6-7: list-3 multipoles and the leaf's local at every centre
     hipLaunchKernelGGL(k_mps_far, dim3((unsigned)n), dim3(kMpsW), lds, st, n, nd, zk, d_lev.p,
-                       nl, leaf.p, t.ilevel.p, L.n3.p, L.l3.p, t.centers.p, ex.p, mp.p, loc.p,
+                       nl, t.leaf_s.p, t.ilevel.p, L.n3.p, L.l3.p, t.centers.p, ex.p, mp.p, loc.p,
                        a.local);
     hip_throw(hipGetLastError(), "mps far");
     tm.mark(6);
@@ -1696,7 +1691,7 @@ int helmholtz_mps(const HelmMpsArgs& a, hipStream_t st) {
     if (ifnear) {
       const double thresh = std::hypot(zk.re, zk.im) * t.boxsize[0] * std::ldexp(1.0, -51);
       hipLaunchKernelGGL(k_mps_near, dim3((unsigned)n), dim3(kMpsW), lds, st, n, nd, zk, thresh,
-                         leaf.p, L.n1.p, L.l1.p, se, ex.p, a.mpole, a.local);
+                         t.leaf_s.p, L.n1.p, L.l1.p, se, ex.p, a.mpole, a.local);
       hip_throw(hipGetLastError(), "mps near");
     }
     tm.mark(7);

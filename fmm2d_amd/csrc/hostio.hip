@@ -27,9 +27,11 @@ namespace {
 
 constexpr int kBoxHead = 16;  // words before the data (the sequence number is word 0)
 
-__global__ void k_readback(const unsigned* __restrict__ src, int nw, unsigned* box,
+__global__ void k_readback(const unsigned* __restrict__ src, int nw,
+                           const unsigned* __restrict__ src2, int nw2, unsigned* box,
                            unsigned seq) {
   for (int i = threadIdx.x; i < nw; i += blockDim.x) box[kBoxHead + i] = src[i];
+  for (int i = threadIdx.x; i < nw2; i += blockDim.x) box[kBoxHead + nw + i] = src2[i];
   __threadfence_system();
   __syncthreads();
   if (threadIdx.x == 0) __hip_atomic_store(box, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
@@ -77,9 +79,15 @@ void box_release(Box* b) {
 }  // namespace
 
 void readback(void* dst, const void* src, size_t bytes, hipStream_t st) {
-  if (bytes == 0) return;
-  if (bytes > kReadbackMax || bytes % 4 != 0) {
-    hip_throw(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, st), "copy");
+  readback2(dst, src, bytes, nullptr, nullptr, 0, st);
+}
+
+void readback2(void* dst, const void* src, size_t bytes, void* dst2, const void* src2,
+               size_t bytes2, hipStream_t st) {
+  if (bytes + bytes2 == 0) return;
+  if (bytes + bytes2 > kReadbackMax || bytes % 4 != 0 || bytes2 % 4 != 0) {
+    if (bytes) hip_throw(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, st), "copy");
+    if (bytes2) hip_throw(hipMemcpyAsync(dst2, src2, bytes2, hipMemcpyDeviceToHost, st), "copy");
     hip_throw(hipStreamSynchronize(st), "sync");
     return;
   }
@@ -91,7 +99,8 @@ void readback(void* dst, const void* src, size_t bytes, hipStream_t st) {
   if (++b->seq == 0) b->seq = 1;  // 0 is the initial word
   const unsigned seq = b->seq;
   hipLaunchKernelGGL(k_readback, dim3(1), dim3(256), 0, st, static_cast<const unsigned*>(src),
-                     (int)(bytes / 4), b->h, seq);
+                     (int)(bytes / 4), static_cast<const unsigned*>(src2), (int)(bytes2 / 4),
+                     b->h, seq);
   hip_throw(hipGetLastError(), "readback launch");
   // poll for up to 200 microseconds, then block on the stream (which also
   // reports a failure of the work queued before)
@@ -106,7 +115,8 @@ void readback(void* dst, const void* src, size_t bytes, hipStream_t st) {
       break;
     }
   }
-  std::memcpy(dst, b->h + kBoxHead, bytes);
+  if (bytes) std::memcpy(dst, b->h + kBoxHead, bytes);
+  if (bytes2) std::memcpy(dst2, b->h + kBoxHead + bytes / 4, bytes2);
 }
 
 void upload_bytes(void* dst, const void* src, size_t bytes, hipStream_t st) {

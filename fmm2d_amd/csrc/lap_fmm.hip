@@ -1522,9 +1522,6 @@ int laplace_fmm(int kind, const CauchyArgs& a, hipStream_t st) {
                a.ifdipole ? a.dipstr : nullptr, a.dipvec, chs.p, dps.p, a.src, xs.p,
                a.ifpgh > 0 ? invs.p : nullptr);
     }
-    DBuf<int> leaf_s(ns, st), leaf_t(std::max<int64_t>(nt, 1), st);
-    launch1d(k_leaf_of, nb, st, t.nchild.p, t.isrcse.p, leaf_s.p);
-    if (nt > 0) launch1d(k_leaf_of, nb, st, t.nchild.p, t.itargse.p, leaf_t.p);
     const int64_t nexp = (int64_t)nb * nd * P;
     DBuf<cplx> mp(nexp, st), loc(nexp, st);
     mp.zero();
@@ -1699,10 +1696,10 @@ int laplace_fmm(int kind, const CauchyArgs& a, hipStream_t st) {
       launch1d(k_to_f32, 2 * nexp, st, reinterpret_cast<const double*>(loc.p), loc32.p);
     }
     if (pg > 0)
-      launch_eval(pg, ns, st, nd, P, xs.p, leaf_s.p, t, d_nterms.p, d_rsc.p, L, mp.p, loc.p,
+      launch_eval(pg, ns, st, nd, P, xs.p, t.leaf_s.p, t, d_nterms.p, d_rsc.p, L, mp.p, loc.p,
                   mp32.p, loc32.p, ps.p, gs.p, hs.p);
     if (pgt > 0)
-      launch_eval(pgt, nt, st, nd, P, xt.p, leaf_t.p, t, d_nterms.p, d_rsc.p, L, mp.p, loc.p,
+      launch_eval(pgt, nt, st, nd, P, xt.p, t.leaf_t.p, t, d_nterms.p, d_rsc.p, L, mp.p, loc.p,
                   mp32.p, loc32.p, pt.p, gt.p, ht.p);
     tm.mark(6);
     // ---- step 8: near field, thresh = boxsize(0) 2^-51 (cfmm2d.f:1276)
@@ -1730,11 +1727,11 @@ int laplace_fmm(int kind, const CauchyArgs& a, hipStream_t st) {
       tm.mark(15);  // FP32 strength copies, segment rows; [7] the near-field kernels alone
       if (pg > 0)
         launch_near(mixed, re, pg, a.ifcharge, a.ifdipole, ns, st,
-                    NearArgs{nd, xs.p, leaf_s.p, seg.p, 1, slow.p, nslow.p, xs.p, chs.p, dps.p,
+                    NearArgs{nd, xs.p, t.leaf_s.p, seg.p, 1, slow.p, nslow.p, xs.p, chs.p, dps.p,
                              ch32.p, dp32.p, thresh, ps.p, gs.p, hs.p});
       if (pgt > 0)
         launch_near(mixed, re, pgt, a.ifcharge, a.ifdipole, nt, st,
-                    NearArgs{nd, xt.p, leaf_t.p, seg.p, 0, slow.p, nslow.p, xs.p, chs.p, dps.p,
+                    NearArgs{nd, xt.p, t.leaf_t.p, seg.p, 0, slow.p, nslow.p, xs.p, chs.p, dps.p,
                              ch32.p, dp32.p, thresh, pt.p, gt.p, ht.p});
     }
     tm.mark(7);

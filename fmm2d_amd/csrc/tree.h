@@ -24,6 +24,7 @@ struct Tree {
   DBuf<int> ilevel, iparent, nchild, ichild /*4*/, ncoll, coll /*9*/;
   DBuf<int> isrcse, itargse;  // [start, end) per box, 2 per box
   DBuf<int> isrc, itarg;      // sorted position -> original point index
+  DBuf<int> leaf_s, leaf_t;   // sorted position -> leaf box
 };
 
 // M2L offset slots.  A box in child position q of its parent (0..3 for

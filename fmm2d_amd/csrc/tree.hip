@@ -320,91 +320,38 @@ __global__ void k_total(int n, const int* flag, const int* offs, int* total) {
 }
 
 // Refinement of several levels between host synchronisations: dlev[2 l],
-// dlev[2 l + 1] hold the first box and the box count of level l, written by
-// k_level_next on the device; the launches cover an upper bound `ub` of the
-// level's size and read the count from dlev.
-__global__ void k_refine_flags_lv(int64_t ub, const int* dlev, int l, const int* ses,
-                                  const int* set, int idivflag, int ndiv, int* flag) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= ub) return;
+// dlev[2 l + 1] hold the first box and the box count of level l, the launches
+// cover an upper bound of the level's size and read the count from dlev.  Two
+// launches a level: the full boxes of every 256 (part), then their children,
+// each workgroup adding the counts of those before it; the last one of the
+// level writes the next level's range.
+constexpr int kRefTile = 256;
+
+__device__ __forceinline__ bool box_full(int b, const int* ses, const int* set, int idivflag,
+                                         int ndiv) {
+  const int cs = ses[2 * b + 1] - ses[2 * b], ct = set[2 * b + 1] - set[2 * b];
+  int nn = cs;
+  if (idivflag == 1) nn = ct;
+  if (idivflag == 2) nn = max(cs, ct);
+  return nn > ndiv;
+}
+
+__global__ __launch_bounds__(kRefTile) void k_lv_count(const int* dlev, int l, const int* ses,
+                                                       const int* set, int idivflag, int ndiv,
+                                                       int* part) {
   const int lo = dlev[2 * l], n = dlev[2 * l + 1];
-  int f = 0;
-  if (i < n) {
-    const int b = lo + (int)i;
-    const int cs = ses[2 * b + 1] - ses[2 * b], ct = set[2 * b + 1] - set[2 * b];
-    int nn = cs;
-    if (idivflag == 1) nn = ct;
-    if (idivflag == 2) nn = max(cs, ct);
-    f = nn > ndiv ? 1 : 0;
-  }
-  flag[i] = f;
+  const int64_t i = (int64_t)blockIdx.x * kRefTile + threadIdx.x;
+  if ((int64_t)blockIdx.x * kRefTile >= n) return;
+  const int c = __syncthreads_count(i < n && box_full(lo + (int)i, ses, set, idivflag, ndiv));
+  if (threadIdx.x == 0) part[blockIdx.x] = c;
 }
 
-// level l+1 = the children of level l's flagged boxes, numbered from *dnb
-__global__ void k_level_next(int64_t ub, const int* flag, const int* offs, int* dlev, int l,
-                             int* dnb) {
-  const int nref = offs[ub - 1] + flag[ub - 1];
-  dlev[2 * (l + 1)] = *dnb;
-  dlev[2 * (l + 1) + 1] = 4 * nref;
-  *dnb += 4 * nref;
-}
-
-// box 1 (index 0): the root, holding every point
-__global__ void k_init_root(double cx, double cy, int ns, int nt, double* centers, int* ilevel,
-                            int* iparent, int* nchild, int* ichild, int* ses, int* set,
-                            int* iflag) {
-  centers[0] = cx;
-  centers[1] = cy;
-  ilevel[0] = 0;
-  iparent[0] = -1;
-  nchild[0] = 0;
-  for (int q = 0; q < 4; ++q) ichild[q] = -1;
-  ses[0] = 0;
-  ses[1] = ns;
-  set[0] = 0;
-  set[1] = nt;
-  iflag[0] = 0;
-}
-
-// cum[k] = exclusive-scan value at segment start cut[k]; cut[K] = n, the
-// scanned length, gives the grand total
-// Box ranges refined together with one scan (Builder::refine_segments),
-// passed by value: segment j covers flag positions [pos[j], pos[j+1]) and
-// boxes lo[j] ..; its children are at level lev[j] with half box size half[j].
-constexpr int kRefSeg = 64;
-struct RefSegs {
-  int k;
-  int pos[kRefSeg + 1];
-  int lo[kRefSeg];
-  int lev[kRefSeg];
-  double half[kRefSeg];
-};
-
-// the segment of flag position i: the last j with pos[j] <= i (skips empty ones)
-__device__ __forceinline__ int seg_of(const RefSegs& R, int64_t i) {
-  int a = 0, b = R.k - 1;
-  while (a < b) {
-    const int m = (a + b + 1) >> 1;
-    if (R.pos[m] <= i) a = m;
-    else b = m - 1;
-  }
-  return a;
-}
-
-__global__ void k_iflag_segs(int64_t n, RefSegs R, const int* iflag, int* flag) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const int j = seg_of(R, i);
-  flag[i] = iflag[R.lo[j] + (int)(i - R.pos[j])] > 0 ? 1 : 0;
-}
-
-// cum[k] = flagged boxes before segment k (k = 0..K)
-__global__ void k_seg_totals(RefSegs R, const int* flag, const int* offs, int* cum) {
-  const int n = R.pos[R.k];
-  for (int k = threadIdx.x; k <= R.k; k += blockDim.x) {
-    const int c = R.pos[k];
-    cum[k] = (c < n) ? offs[c] : (n > 0 ? offs[n - 1] + flag[n - 1] : 0);
-  }
+// the sum of part[0 .. m), on every thread of a workgroup of 256
+__device__ __forceinline__ int sum_parts(const int* part, int m, int* lds) {
+  int s = 0, tot;
+  for (int k = threadIdx.x; k < m; k += kRefTile) s += part[k];
+  block_exclusive_scan(s, lds, &tot);
+  return tot;
 }
 
 // Children of the flagged boxes lo..lo+n-1 are numbered base + 4*offs + q, q =
@@ -457,25 +404,34 @@ __global__ void k_make_children(int64_t n, int lo, const int* flag, const int* o
                    ichild, ses, set, iflag, mode, ks, kt);
 }
 
-__global__ void k_make_children_segs(int64_t n, RefSegs R, const int* flag, const int* offs,
-                                     int base, double* centers, int* ilevel, int* iparent,
-                                     int* nchild, int* ichild, int* ses, int* set, int* iflag,
-                                     Keys ks, Keys kt) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n || !flag[i]) return;
-  const int j = seg_of(R, i);
-  make_children_of(R.lo[j] + (int)(i - R.pos[j]), base + 4 * offs[i], R.half[j], R.lev[j],
-                   centers, ilevel, iparent, nchild, ichild, ses, set, iflag, 1, ks, kt);
-}
-
-__global__ void k_make_children_lv(int64_t ub, const int* dlev, int l, const int* flag,
-                                   const int* offs, double half, double* centers, int* ilevel,
-                                   int* iparent, int* nchild, int* ichild, int* ses, int* set,
-                                   int* iflag, Keys ks, Keys kt) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= ub || i >= dlev[2 * l + 1] || !flag[i]) return;
-  make_children_of(dlev[2 * l] + (int)i, dlev[2 * (l + 1)] + 4 * offs[i], half, l + 1, centers,
-                   ilevel, iparent, nchild, ichild, ses, set, iflag, 0, ks, kt);
+__global__ __launch_bounds__(kRefTile) void k_lv_children(int* dlev, int l, const int* part,
+                                                          int idivflag, int ndiv, double half,
+                                                          double* centers, int* ilevel,
+                                                          int* iparent, int* nchild, int* ichild,
+                                                          int* ses, int* set, int* iflag, Keys ks,
+                                                          Keys kt) {
+  __shared__ int lds[kScanWaves + 1];
+  const int lo = dlev[2 * l], n = dlev[2 * l + 1];
+  const int64_t i0 = (int64_t)blockIdx.x * kRefTile, i = i0 + threadIdx.x;
+  const int nb = lo + n;  // the level's boxes are the last ones made
+  if (i0 >= n) {
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+      dlev[2 * (l + 1)] = nb;
+      dlev[2 * (l + 1) + 1] = 0;
+    }
+    return;
+  }
+  const int carry = sum_parts(part, blockIdx.x, lds);
+  const bool f = i < n && box_full(lo + (int)i, ses, set, idivflag, ndiv);
+  int own;
+  const int ex = block_exclusive_scan(f ? 1 : 0, lds, &own);
+  if (i0 + kRefTile >= n && threadIdx.x == 0) {
+    dlev[2 * (l + 1)] = nb;
+    dlev[2 * (l + 1) + 1] = 4 * (carry + own);
+  }
+  if (f)
+    make_children_of(lo + (int)i, nb + 4 * (carry + ex), half, l + 1, centers, ilevel, iparent,
+                     nchild, ichild, ses, set, iflag, 0, ks, kt);
 }
 
 // ------------------------------------------------------------ colleagues
@@ -514,29 +470,6 @@ __global__ void k_coll(int64_t n, int lo, double bs, const int* iparent, const i
 // interleaved code of (iy, ix), iy bit above ix bit, coarsest level first.
 constexpr int kWalkLevels = 29;
 
-// (ix, iy) of every box, walking up to the root: the child centre is the
-// parent centre +- half the child size, so the comparisons are exact.
-__global__ void k_box_ij(int64_t nb, const int* iparent, const int* ilevel,
-                         const double* centers, unsigned* ij) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= nb) return;
-  int cur = (int)i;
-  const int lev = ilevel[cur];
-  double cx = centers[2 * cur], cy = centers[2 * cur + 1];
-  unsigned ix = 0, iy = 0;
-  for (int t = 0; t < lev; ++t) {
-    const int par = iparent[cur];
-    const double px = centers[2 * par], py = centers[2 * par + 1];
-    ix |= (cx > px ? 1u : 0u) << t;
-    iy |= (cy > py ? 1u : 0u) << t;
-    cur = par;
-    cx = px;
-    cy = py;
-  }
-  ij[2 * i] = ix;
-  ij[2 * i + 1] = iy;
-}
-
 // spread the 29 bits of v to the even bit positions
 __device__ __forceinline__ unsigned long long spread_bits(unsigned v) {
   unsigned long long x = v;
@@ -553,20 +486,41 @@ __device__ __forceinline__ unsigned long long path_code(unsigned ix, unsigned iy
   return spread_bits(ix) | (spread_bits(iy) << 1);
 }
 
-// Colleagues of every box in one pass.  The neighbour (jx, jy) of box b
-// (level lev, coordinates (ix, iy)) shares b's ancestors down to level
+// Colleagues of every box in one pass.  A box's coordinates (ix, iy) come from
+// walking up to the root: the child centre is the parent centre +- half the
+// child size, so the comparisons are exact.  The neighbour (jx, jy) of box b
+// (level lev) shares b's ancestors down to level
 // m = lev - max(bitlength(ix ^ jx), bitlength(iy ^ jy)); it is found by going
 // up lev - m parents and down lev - m child slots, slot 2 qy + qx taken from
 // the bits of (jx, jy) (the reference's child order (-,-), (+,-), (-,+),
-// (+,+)); a missing child ends the search.
+// (+,+)); a missing child ends the search.  Sets *big (if given) where a leaf
+// holds more than big_max sources or targets.
 __global__ void k_coll_walk(int64_t nb, const int* ilevel, const int* iparent, const int* ichild,
-                            const unsigned* ij, int* ncoll, int* coll) {
+                            const double* centers, int* ncoll, int* coll, const int* nchild,
+                            const int* ses, const int* set, int big_max, int* big) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= nb) return;
   const int b = (int)i;
   const int lev = ilevel[b];
+  if (big && nchild[b] == 0) {
+    const int m = max(ses[2 * i + 1] - ses[2 * i], set[2 * i + 1] - set[2 * i]);
+    if (m > big_max) *big = 1;
+  }
   const long long side = 1ll << lev;
-  const unsigned ix = ij[2 * i], iy = ij[2 * i + 1];
+  unsigned ix = 0, iy = 0;
+  {
+    int cur = b;
+    double cx = centers[2 * cur], cy = centers[2 * cur + 1];
+    for (int t = 0; t < lev; ++t) {
+      const int par = iparent[cur];
+      const double px = centers[2 * par], py = centers[2 * par + 1];
+      ix |= (cx > px ? 1u : 0u) << t;
+      iy |= (cy > py ? 1u : 0u) << t;
+      cur = par;
+      cx = px;
+      cy = py;
+    }
+  }
   int id[kMaxColl];
   unsigned long long code[kMaxColl];
   int cnt = 0;
@@ -601,6 +555,15 @@ __global__ void k_coll_walk(int64_t nb, const int* ilevel, const int* iparent, c
     }
   ncoll[i] = cnt;
   for (int k = 0; k < kMaxColl; ++k) coll[9 * i + k] = k < cnt ? id[k] : -1;
+}
+
+// *big = 1 if a leaf holds more than big_max sources or targets
+__global__ void k_big_leaves(int64_t nb, const int* nchild, const int* ses, const int* set,
+                             int big_max, int* big) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= nb || nchild[i] != 0) return;
+  const int m = max(ses[2 * i + 1] - ses[2 * i], set[2 * i + 1] - set[2 * i]);
+  if (m > big_max) *big = 1;
 }
 
 __global__ void k_root_coll(int* ncoll, int* coll) {
@@ -658,37 +621,6 @@ __global__ void k_flag2(int64_t n, int lo, double distest, const int* iparent, c
   }
 }
 
-// updateflags (tree_routs2d.f:217-326) over boxes lo1 .. lo1+n1-1, then
-// lo2 .. lo2+(n-n1)-1
-__global__ void k_updateflags(int64_t n, int n1, int lo1, int lo2, double distest,
-                              const int* ncoll, const int* coll, const int* ichild,
-                              const int* nchild, const double* centers, int* iflag) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const int b = i < n1 ? lo1 + (int)i : lo2 + (int)(i - n1);
-  if (iflag[b] != 3) return;
-  int f = 0;
-  const double bx = centers[2 * b], by = centers[2 * b + 1];
-  for (int k = 0; k < ncoll[b] && !f; ++k) {
-    const int j = coll[9 * b + k];
-    for (int q = 0; q < 4; ++q) {
-      const int kb = ichild[4 * j + q];
-      if (kb >= 0 && nchild[kb] > 0 && fabs(centers[2 * kb] - bx) <= distest &&
-          fabs(centers[2 * kb + 1] - by) <= distest) {
-        f = 1;
-        break;
-      }
-    }
-  }
-  iflag[b] = f;
-}
-
-__global__ void k_keep3(int64_t n, int* iflag) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  if (iflag[i] != 3) iflag[i] = 0;
-}
-
 // ------------------------------------------------------------ reorganisation
 // The new number of every box: the boxes are covered by segments (a level's
 // original boxes, a level's tail boxes), sorted by first box; segment k moves
@@ -722,13 +654,424 @@ __global__ void k_reorg_apply(int64_t n, const int* map, const double* c0, const
   c1[2 * m + 1] = c0[2 * i + 1];
   lev1[m] = lev0[i];
   nch1[m] = nch0[i];
-  fl1[m] = fl0[i];
+  fl1[m] = fl0[i] == 3 ? 3 : 0;  // the updateflags sweep starts from the flag-3 boxes
   s1[2 * m] = s0[2 * i];
   s1[2 * m + 1] = s0[2 * i + 1];
   t1[2 * m] = t0[2 * i];
   t1[2 * m + 1] = t0[2 * i + 1];
   par1[m] = par0[i] < 0 ? -1 : map[par0[i]];
   for (int q = 0; q < 4; ++q) ich1[4 * m + q] = ich0[4 * i + q] < 0 ? -1 : map[ich0[4 * i + q]];
+}
+
+// ------------------------------------------------------------ one-workgroup builds
+// The refinement of trees and levels of a few thousand boxes is a chain of
+// small dependent steps: as separate launches (flags, scan, next level,
+// children; flags per level) each step costs a launch of ~2.4 us and the
+// chain a host round trip of ~10 us per level, whatever its size.  One
+// workgroup of 1024 threads runs the whole chain instead, with barriers
+// between the steps.  Limits: kWgLevel boxes of a level in refinement (four
+// per thread; beyond it the per-level launches spread over the CUs win) and
+// kWgBoxes boxes in all in the flag passes (1765 boxes 5 us, 50000 250 us, where
+// the launches take 60).
+constexpr int kWgThreads = 1024;
+constexpr int kWgWaves = kWgThreads / 64;
+constexpr int kWgLevel = 4 * kWgThreads;
+constexpr int kWgBoxes = 8192;
+
+struct BoxPtrs {
+  double* centers;
+  int *ilevel, *iparent, *nchild, *ichild, *ncoll, *coll, *ses, *set, *iflag;
+};
+
+// State words of the kernels below: status, level, boxes, big-leaf flag
+// (k_coll_walk), then two words per level.
+constexpr int kStStatus = 0, kStLevel = 1, kStBoxes = 2, kStBig = 3, kStLev = 4;
+constexpr int kStWords = kStLev + 2 * (kMaxLevels + 2);
+
+// Level ranges and box sizes, by value
+struct LevelTab {
+  int ls[kMaxLevels + 1], le[kMaxLevels + 1];
+  double bs[kMaxLevels + 1];
+};
+
+// digit_bounds3 by a whole wavefront: 21 probes per bound and round (a box of
+// 1e6 points takes 5 rounds of dependent loads, not 20).
+__device__ void digit_bounds3_wave(const Keys& K, int64_t lo0, int64_t hi0, int lev, int* b) {
+  constexpr int kP = 21;
+  const int lane = threadIdx.x & 63;
+  const int q = min(lane / kP, 2), j = lane - q * kP;
+  const bool in = lane < 3 * kP;
+  int64_t lo = lo0, hi = hi0;
+  while (__ballot(hi > lo)) {
+    const int64_t w = hi - lo;
+    const bool last = w <= kP;
+    const int64_t pos = last ? lo + j : lo + (w * (j + 1)) / (kP + 1);
+    const bool use = in && (last ? j < w : true) && w > 0;
+    const bool below = use && digit_at(K, use ? pos : lo0, lev) < q + 1;
+    const unsigned long long m = (__ballot(below) >> (q * kP)) & ((1ull << kP) - 1ull);
+    const int c = __popcll(m);
+    if (w > 0) {
+      if (last) {
+        lo = hi = lo + c;
+      } else {
+        const int64_t l1 = c > 0 ? lo + (w * c) / (kP + 1) + 1 : lo;
+        const int64_t h1 = c < kP ? lo + (w * (c + 1)) / (kP + 1) : hi;
+        lo = l1;
+        hi = h1;
+      }
+    }
+  }
+  for (int k = 0; k < 3; ++k) b[k] = (int)__shfl(lo, k * kP, 64);
+}
+
+// the four children of box b by a whole wavefront (make_children_of, mode 0)
+__device__ void make_children_wave(int b, int c0, double half, int lev, const BoxPtrs& B,
+                                   const Keys& ks, const Keys& kt) {
+  const int lane = threadIdx.x & 63;
+  const int s0 = B.ses[2 * b], s1 = B.ses[2 * b + 1], t0 = B.set[2 * b], t1 = B.set[2 * b + 1];
+  int bs[3], bt[3];
+  digit_bounds3_wave(ks, s0, s1, lev, bs);
+  digit_bounds3_wave(kt, t0, t1, lev, bt);
+  if (lane < 4) {
+    const int q = lane, c = c0 + q;
+    B.centers[2 * c] = B.centers[2 * b] + ((q & 1) ? half : -half);
+    B.centers[2 * c + 1] = B.centers[2 * b + 1] + ((q & 2) ? half : -half);
+    B.iparent[c] = b;
+    B.nchild[c] = 0;
+    for (int k = 0; k < 4; ++k) B.ichild[4 * c + k] = -1;
+    B.ichild[4 * b + q] = c;
+    B.ilevel[c] = lev;
+    B.ses[2 * c] = q == 0 ? s0 : q == 1 ? bs[0] : q == 2 ? bs[1] : bs[2];
+    B.ses[2 * c + 1] = q == 0 ? bs[0] : q == 1 ? bs[1] : q == 2 ? bs[2] : s1;
+    B.set[2 * c] = q == 0 ? t0 : q == 1 ? bt[0] : q == 2 ? bt[1] : bt[2];
+    B.set[2 * c + 1] = q == 0 ? bt[0] : q == 1 ? bt[1] : q == 2 ? bt[2] : t1;
+    B.iflag[c] = 0;
+    if (q == 0) B.nchild[b] = 4;
+  }
+}
+
+// Refinement (pts_tree2d.f:551-631) from level l0 on (0: from the root, made
+// here) while levels hold at most kWgLevel boxes, keys reach (depth levels) and
+// the boxes fit cap.  State: status 1 done (level = nlevels), 0 stopped before
+// refining `level` (too many boxes, or keys too short), 2 the same for want of
+// capacity; first box and count of every level made.
+__global__ __launch_bounds__(kWgThreads) void k_refine_wg(const double* bounds, int ns, int nt,
+                                                          int idivflag, int ndiv, int nlmax,
+                                                          int depth, int cap, BoxPtrs B, Keys ks,
+                                                          Keys kt, int l0, int* st) {
+  __shared__ int list[kWgLevel];
+  __shared__ int lds[kWgWaves + 1];
+  const int tid = threadIdx.x, wave = tid >> 6;
+  double cx0, cy0, bs0;
+  root_square(bounds, &cx0, &cy0, &bs0);
+  double h = 0.5 * bs0;
+  for (int l = 0; l < l0; ++l) h *= 0.5;
+  int lo = 0, n = 1, nb = 1;
+  if (l0 == 0) {
+    if (tid == 0) {
+      B.centers[0] = cx0;
+      B.centers[1] = cy0;
+      B.ilevel[0] = 0;
+      B.iparent[0] = -1;
+      B.nchild[0] = 0;
+      for (int q = 0; q < 4; ++q) B.ichild[q] = -1;
+      B.ses[0] = 0;
+      B.ses[1] = ns;
+      B.set[0] = 0;
+      B.set[1] = nt;
+      B.iflag[0] = 0;
+      st[kStBig] = 0;
+      st[kStLev] = 0;
+      st[kStLev + 1] = 1;
+    }
+  } else {
+    nb = st[kStBoxes];
+    lo = st[kStLev + 2 * l0];
+    n = st[kStLev + 2 * l0 + 1];
+  }
+  __syncthreads();
+  int l = l0, status = 0;
+  for (;;) {
+    if (l >= nlmax) {
+      status = 1;
+      break;
+    }
+    if (n > kWgLevel || l + 1 > depth) break;
+    bool f[4];
+    int c = 0;
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int i = 4 * tid + u;
+      f[u] = i < n && box_full(lo + i, B.ses, B.set, idivflag, ndiv);
+      c += f[u] ? 1 : 0;
+    }
+    int nref;
+    int ex = block_exclusive_scan_w<kWgWaves>(c, lds, &nref);
+    if (nref == 0) {
+      status = 1;
+      break;
+    }
+    if (nb + 4 * nref > cap) {
+      status = 2;
+      break;
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      if (f[u]) list[ex++] = lo + 4 * tid + u;
+    __syncthreads();
+    h *= 0.5;
+    if (nref <= 4 * kWgWaves) {
+      for (int k = wave; k < nref; k += kWgWaves)
+        make_children_wave(list[k], nb + 4 * k, h, l + 1, B, ks, kt);
+    } else {
+      for (int k = tid; k < nref; k += kWgThreads)
+        make_children_of(list[k], nb + 4 * k, h, l + 1, B.centers, B.ilevel, B.iparent, B.nchild,
+                         B.ichild, B.ses, B.set, B.iflag, 0, ks, kt);
+    }
+    __syncthreads();
+    ++l;
+    lo = nb;
+    n = 4 * nref;
+    nb += n;
+    if (tid == 0) {
+      st[kStLev + 2 * l] = lo;
+      st[kStLev + 2 * l + 1] = n;
+    }
+  }
+  if (tid == 0) {
+    st[kStStatus] = status;
+    st[kStLevel] = l;
+    st[kStBoxes] = nb;
+  }
+}
+
+// The flag+ passes (k_flag2, finest level first) and the refinement of every
+// flagged box of levels 1 .. nl-2 (refine_segments over the levels in order).
+// cap holds 5 nb boxes.  State: boxes; per level the first and last of its new
+// boxes.
+__global__ __launch_bounds__(kWgThreads) void k_flags_wg(LevelTab T, int nl, int nb, BoxPtrs B,
+                                                         Keys ks, Keys kt, int* st) {
+  __shared__ int list[kWgLevel];
+  __shared__ int lds[kWgWaves + 1];
+  __shared__ int cnt, per[kMaxLevels + 2];
+  const int tid = threadIdx.x;
+  for (int k = tid; k < kMaxLevels + 2; k += kWgThreads) per[k] = 0;
+  for (int l = nl; l >= 1; --l) {
+    const double distest = 1.05 * (T.bs[l] + T.bs[l - 1]) / 2.0;
+    const int lo = T.ls[l], n = T.le[l] - lo;
+    for (int r0 = 0; r0 < n; r0 += kWgLevel) {
+      if (tid == 0) cnt = 0;
+      __syncthreads();
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int i = r0 + u * kWgThreads + tid;
+        const int f = i < n ? B.iflag[lo + i] : 0;
+        if (f == 1 || f == 2) list[atomicAdd(&cnt, 1)] = lo + i;
+      }
+      __syncthreads();
+      const int m = cnt;
+      for (int t = tid; t < 16 * m; t += kWgThreads) {
+        const int b = list[t >> 4], k = t & 15;
+        const int dad = B.iparent[b];
+        if (k >= B.ncoll[dad]) continue;
+        const int j = B.coll[9 * dad + k];
+        if (B.nchild[j] == 0 && B.iflag[j] == 0 &&
+            fabs(B.centers[2 * j] - B.centers[2 * b]) <= distest &&
+            fabs(B.centers[2 * j + 1] - B.centers[2 * b + 1]) <= distest)
+          B.iflag[j] = 2;
+      }
+      __syncthreads();
+    }
+  }
+  const int nb0 = nb;
+  if (nl >= 3) {
+    const int lo = T.ls[1], n = T.le[nl - 2] - lo;
+    for (int r0 = 0; r0 < n; r0 += kWgLevel) {
+      bool f[4];
+      int c = 0;
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int i = r0 + 4 * tid + u;
+        f[u] = i < n && B.iflag[lo + i] > 0;
+        c += f[u] ? 1 : 0;
+      }
+      int nref;
+      int ex = block_exclusive_scan_w<kWgWaves>(c, lds, &nref);
+      if (nref == 0) continue;  // uniform
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+        if (f[u]) list[ex++] = lo + r0 + 4 * tid + u;
+      __syncthreads();
+      for (int k = tid; k < nref; k += kWgThreads) {
+        const int b = list[k], lev = B.ilevel[b] + 1;
+        atomicAdd(&per[lev], 1);
+        make_children_of(b, nb + 4 * k, 0.5 * T.bs[lev], lev, B.centers, B.ilevel, B.iparent,
+                         B.nchild, B.ichild, B.ses, B.set, B.iflag, 1, ks, kt);
+      }
+      nb += 4 * nref;
+      __syncthreads();
+    }
+  }
+  __syncthreads();
+  if (tid == 0) {
+    int at = nb0;
+    for (int l = 0; l <= nl; ++l) {
+      st[kStLev + 2 * l] = at;
+      at += 4 * per[l];
+      st[kStLev + 2 * l + 1] = at;
+    }
+    st[kStBoxes] = nb;
+  }
+}
+
+// ------------------------------------------------------------ restriction sweeps
+// A sweep's boxes: n1 boxes from lo1 on, then the tail boxes [ts, te) of the
+// state words.  kLrTile boxes a workgroup of 256 threads, 16 lanes a box where
+// a box looks at its (parent's) colleagues.  Capacity and launch bounds are
+// guesses (cap, tail_ub); a sweep that would pass them sets the status word and
+// makes nothing, and the caller builds again with more room.
+constexpr int kLrTile = 64;
+
+struct LrSeq {
+  int n1, lo1, ts, te;
+  __device__ int n() const { return n1 + (te - ts); }
+  __device__ int box(int i) const { return i < n1 ? lo1 + i : ts + (i - n1); }
+};
+
+// flagged boxes (iflag > 0) of every kLrTile of the n boxes from lo on
+__global__ __launch_bounds__(256) void k_flag_count(int n, int lo, const int* iflag, int* part) {
+  const int i0 = blockIdx.x * 256;
+  const int i = i0 + threadIdx.x;
+  const unsigned long long m = __ballot(i < n && iflag[lo + i] > 0);
+  if ((threadIdx.x & 63) == 0 && i < n) part[i / kLrTile] = __popcll(m);
+}
+
+// Children of the flagged boxes of a sweep, numbered in sweep order from nb on
+// (make_children_of, mode 1).  SWEEP: level l of the updateflags sweep, nb = te
+// of that level, the new range is level l+1's; else the levels 1 .. nl-2 at
+// once, and st counts the refined boxes by child level.
+template <int SWEEP>
+__global__ __launch_bounds__(256) void k_flag_children(int n1, int lo1, int l, int nb,
+                                                       const int* part, LevelTab T, int cap,
+                                                       BoxPtrs B, Keys ks, Keys kt, int* st) {
+  __shared__ int lds[kScanWaves + 1];
+  __shared__ int per[kMaxLevels + 2];
+  LrSeq q{n1, lo1, 0, 0};
+  if (SWEEP) {
+    q.ts = st[kStLev + 2 * l];
+    q.te = nb = st[kStLev + 2 * l + 1];
+  }
+  const int n = q.n(), i0 = blockIdx.x * 256, i = i0 + threadIdx.x;
+  if (i0 >= n && blockIdx.x > 0) return;
+  for (int k = threadIdx.x; !SWEEP && k < kMaxLevels + 2; k += 256) per[k] = 0;
+  const int b = i < n ? q.box(i) : 0;
+  const bool f = i < n && B.iflag[b] > 0;
+  const int carry = sum_parts(part, min(i0, n) / kLrTile, lds);
+  int own;
+  const int ex = block_exclusive_scan(f ? 1 : 0, lds, &own);
+  const bool fits = nb + 4 * (int64_t)(carry + own) <= cap;
+  if (!fits && threadIdx.x == 0) st[kStStatus] = 1;
+  if (SWEEP && i0 + 256 >= n && threadIdx.x == 0) {
+    st[kStLev + 2 * (l + 1)] = nb;
+    st[kStLev + 2 * (l + 1) + 1] = fits ? nb + 4 * (carry + own) : nb;
+  }
+  if (f && fits) {
+    const int lev = SWEEP ? l + 1 : B.ilevel[b] + 1;
+    make_children_of(b, nb + 4 * (carry + ex), 0.5 * T.bs[lev], lev, B.centers, B.ilevel,
+                     B.iparent, B.nchild, B.ichild, B.ses, B.set, B.iflag, 1, ks, kt);
+    if (!SWEEP) atomicAdd(&per[lev], 1);
+  }
+  if (!SWEEP) {
+    __syncthreads();
+    for (int k = threadIdx.x; k < kMaxLevels + 2; k += 256)
+      if (per[k]) atomicAdd(&st[kStLev + 2 * k], per[k]);
+  }
+}
+
+// Level l of the updateflags sweep (tree_routs2d.f:217-326, pts_tree2d.f:
+// 940-1010): the tail boxes get their colleagues (k_coll's entries, in
+// (parent's colleague, child slot) order), then the flag-3 boxes keep their
+// flag, as 1, where a child of a colleague is refined and touches them.
+__global__ __launch_bounds__(256) void k_sweep_flags(int n1, int lo1, int l, int tail_ub,
+                                                     double lim, double distest, BoxPtrs B,
+                                                     int* part, int* st) {
+  __shared__ int list[kLrTile], hit[kLrTile];
+  __shared__ int cnt;
+  const LrSeq q{n1, lo1, st[kStLev + 2 * l], st[kStLev + 2 * l + 1]};
+  const int n = q.n(), i0 = blockIdx.x * kLrTile;
+  if (i0 >= n) return;
+  const int tid = threadIdx.x, lane = tid & 63;
+  if (blockIdx.x == 0 && tid == 0 && q.te - q.ts > tail_ub) st[kStStatus] = 1;
+  if (i0 + kLrTile > n1) {
+    for (int r = 0; r < kLrTile; r += 16) {
+      const int i = i0 + r + (tid >> 4), k = lane & 15;
+      const bool act = i >= n1 && i < n;
+      const int b = act ? q.box(i) : 0;
+      const int dad = act ? B.iparent[b] : 0;
+      const double bx = B.centers[2 * b], by = B.centers[2 * b + 1];
+      int id[4] = {-1, -1, -1, -1};
+      if (act && k < B.ncoll[dad]) {
+        const int j = B.coll[9 * dad + k];
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+          const int kb = B.ichild[4 * j + c];
+          if (kb >= 0 && fabs(B.centers[2 * kb] - bx) <= lim &&
+              fabs(B.centers[2 * kb + 1] - by) <= lim)
+            id[c] = kb;
+        }
+      }
+      const unsigned long long seg = 0xffffull << (lane & 48), lt = (1ull << lane) - 1ull;
+      int at = 0, tot = 0;
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        const unsigned long long m = __ballot(id[c] >= 0) & seg;
+        at += __popcll(m & lt);
+        tot += __popcll(m);
+      }
+#pragma unroll
+      for (int c = 0; c < 4; ++c)
+        if (id[c] >= 0) {
+          if (at < kMaxColl) B.coll[9 * b + at] = id[c];
+          ++at;
+        }
+      tot = min(tot, kMaxColl);
+      if (act && k == 0) B.ncoll[b] = tot;
+      if (act && k >= tot && k < kMaxColl) B.coll[9 * b + k] = -1;
+    }
+  }
+  if (tid < kLrTile) {  // the first wavefront
+    const int i = i0 + tid;
+    const int b = i < n ? q.box(i) : 0;
+    const bool f = i < n && B.iflag[b] == 3;
+    const unsigned long long m = __ballot(f);
+    const int at = __popcll(m & ((1ull << tid) - 1ull));
+    if (f) list[at] = b;
+    hit[tid] = 0;
+    if (tid == 0) cnt = __popcll(m);
+  }
+  __syncthreads();  // (the colleagues above are visible to the workgroup too)
+  const int m = cnt;
+  for (int t = tid; t < 16 * m; t += 256) {
+    const int b = list[t >> 4], k = t & 15;
+    if (k >= B.ncoll[b]) continue;
+    const int j = B.coll[9 * b + k];
+    const double bx = B.centers[2 * b], by = B.centers[2 * b + 1];
+    bool any = false;
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      const int kb = B.ichild[4 * j + c];
+      any = any || (kb >= 0 && B.nchild[kb] > 0 && fabs(B.centers[2 * kb] - bx) <= distest &&
+                    fabs(B.centers[2 * kb + 1] - by) <= distest);
+    }
+    if (any) hit[t >> 4] = 1;
+  }
+  __syncthreads();
+  if (tid < kLrTile) {
+    const bool h = tid < m && hit[tid] != 0;
+    if (tid < m) B.iflag[list[tid]] = h ? 1 : 0;
+    const unsigned long long k = __ballot(h);
+    if (tid == 0) part[blockIdx.x] = __popcll(k);
+  }
 }
 
 // ------------------------------------------------------------ final point order
@@ -744,76 +1087,56 @@ __global__ void k_leaf_label(int64_t n, const int* nchild, const int* se, const 
 }
 
 // The same order without the sort: inside each leaf (a contiguous range of
-// the path order) the input indices in increasing order, placed by rank.
-// Leaves of up to kLeafSmall points: one thread each, ranks over a register
-// copy; larger leaves are appended to `bigl` (in any order: each leaf is
-// independent) for k_leaf_sort.
-constexpr int kLeafSmall = 32;
-constexpr int kLeafSortMax = 2048;
-constexpr int kLeafSortWaves = 4;
+// the path order) the input indices in increasing order, placed by rank, one
+// thread per point (leaves of up to kLeafRankMax points).  blockIdx.y: sources,
+// targets.
+constexpr int kLeafRankMax = 2048;
 
-__global__ void k_leaf_sort_small(int64_t nb, const int* nchild, const int* se, const int* perm,
-                                  int* out, int* bigl, int* nbig) {
+struct LeafOrder {
+  int64_t n[2];
+  const int* leaf[2];
+  const int* se[2];
+  const int* perm[2];
+  int* out[2];
+};
+
+__global__ __launch_bounds__(256) void k_leaf_rank(LeafOrder a) {
+  const int y = blockIdx.y;
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= nb || nchild[i] != 0) return;
-  const int s = se[2 * i], m = se[2 * i + 1] - s;
-  if (m <= 0) return;
-  if (m > kLeafSmall) {
-    bigl[atomicAdd(nbig, 1)] = (int)i;
-    return;
+  if (i >= a.n[y]) return;
+  const int b = a.leaf[y][i];
+  const int s = a.se[y][2 * (int64_t)b], e = a.se[y][2 * (int64_t)b + 1];
+  const int* p = a.perm[y];
+  const int v = p[i];
+  int rank = 0;
+  int j = s;
+  for (; j + 4 <= e; j += 4) {
+    const int q0 = p[j], q1 = p[j + 1], q2 = p[j + 2], q3 = p[j + 3];
+    rank += (q0 < v) + (q1 < v) + (q2 < v) + (q3 < v);
   }
-  int v[kLeafSmall];
-#pragma unroll
-  for (int k = 0; k < kLeafSmall; ++k) v[k] = k < m ? perm[s + k] : 0x7fffffff;
-#pragma unroll
-  for (int k = 0; k < kLeafSmall; ++k) {
-    int rank = 0;
-#pragma unroll
-    for (int q = 0; q < kLeafSmall; ++q) rank += (v[q] < v[k]) ? 1 : 0;
-    if (k < m) out[s + rank] = v[k];
-  }
+  for (; j < e; ++j) rank += p[j] < v ? 1 : 0;
+  a.out[y][s + rank] = v;
 }
 
-// The leaves of `bigl`: one wavefront each in a grid-stride loop (4 per
-// block, each with its own LDS); up to 64 points rank through lane shuffles,
-// up to kLeafSortMax through LDS; a larger leaf sets *big and the caller falls
-// back to the labelled sort.
-__global__ __launch_bounds__(kLeafSortWaves * 64) void k_leaf_sort(const int* bigl,
-                                                                   const int* nbig,
-                                                                   const int* se, const int* perm,
-                                                                   int* out, int* big) {
-  __shared__ int shall[kLeafSortWaves][kLeafSortMax];
-  const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  int* sh = shall[wv];
-  const int nl = *nbig;
-  for (int li = blockIdx.x * kLeafSortWaves + wv; li < nl; li += gridDim.x * kLeafSortWaves) {
-    const int b = bigl[li];
-    const int s = se[2 * b], m = se[2 * b + 1] - s;
-    if (m > kLeafSortMax) {
-      if (lane == 0) *big = 1;
-      continue;
-    }
-    if (m <= 64) {
-      const int v = lane < m ? perm[s + lane] : 0x7fffffff;
-      int rank = 0;
-      // j is uniform: read lane j through the scalar unit (v_readlane)
-      for (int j = 0; j < m; ++j) rank += (__builtin_amdgcn_readlane(v, j) < v) ? 1 : 0;
-      if (lane < m) out[s + rank] = v;
-      continue;
-    }
-    for (int i = lane; i < m; i += 64) sh[i] = perm[s + i];
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    for (int i = lane; i < m; i += 64) {
-      const int v = sh[i];
-      int rank = 0;
-      for (int j = 0; j < m; ++j) rank += (sh[j] < v) ? 1 : 0;
-      out[s + rank] = v;
-    }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+// leaf[i] = the leaf holding sorted point i, for sources and targets
+// (blockIdx.y).  A wavefront takes 64 boxes and writes their point ranges one
+// box after the other with all 64 lanes (consecutive lanes on consecutive
+// points).
+__global__ void k_leaf_of(int64_t n, const int* nchild, const int* ses, const int* set,
+                          int* leaf_s, int* leaf_t) {
+  const int* se = blockIdx.y ? set : ses;
+  int* leaf = blockIdx.y ? leaf_t : leaf_s;
+  const int lane = threadIdx.x & 63;
+  const int64_t b0 = (int64_t)blockIdx.x * blockDim.x + (threadIdx.x & ~63);
+  const int64_t b = b0 + lane;
+  int s = 0, e = 0;
+  if (b < n && nchild[b] == 0) {
+    s = se[2 * b];
+    e = se[2 * b + 1];
+  }
+  for (int k = 0; k < 64; ++k) {
+    const int sk = __builtin_amdgcn_readlane(s, k), ek = __builtin_amdgcn_readlane(e, k);
+    for (int i = sk + lane; i < ek; i += 64) leaf[i] = (int)(b0 + k);
   }
 }
 
@@ -851,13 +1174,18 @@ struct PathKeys {
   }
 };
 
+inline BoxPtrs ptrs(const Boxes& b) {
+  return BoxPtrs{b.centers.p, b.ilevel.p, b.iparent.p, b.nchild.p, b.ichild.p,
+                 b.ncoll.p,   b.coll.p,   b.ses.p,     b.set.p,    b.iflag.p};
+}
+
 struct Builder {
   hipStream_t st;
   Boxes B;
   int nboxes = 0;
   DBuf<int> flag, offs, total;
   Keys ks{}, kt{};
-  // the centre comparisons of k_box_ij are exact when the domain is not far
+  // the centre comparisons of k_coll_walk are exact when the domain is not far
   // from the origin relative to its size
   bool walk_ok = false;
 
@@ -872,48 +1200,6 @@ struct Builder {
     int h = 0;
     readback(&h, total.p, sizeof(int), st);
     return h;
-  }
-  // Refine several box ranges with one scan: segment k covers boxes
-  // lo[k] .. lo[k]+n[k]-1 (flags from iflag > 0), children at level lev[k]
-  // with box size bsc[k].  Children are numbered in segment order, exactly as
-  // refining the segments one after the other.  first[k], last[k]: range of
-  // the children of segment k.
-  void refine_segments(const std::vector<int>& lo, const std::vector<int>& n,
-                       const std::vector<int>& lev, const std::vector<double>& bsc,
-                       std::vector<int>& first, std::vector<int>& last) {
-    const size_t K = lo.size();
-    if (K > (size_t)kRefSeg) throw HipError{hipErrorInvalidValue, "refinement segments"};
-    RefSegs R{};
-    R.k = (int)K;
-    R.pos[0] = 0;
-    for (size_t k = 0; k < K; ++k) {
-      R.pos[k + 1] = R.pos[k] + n[k];
-      R.lo[k] = lo[k];
-      R.lev[k] = lev[k];
-      R.half[k] = 0.5 * bsc[k];
-    }
-    first.assign(K, nboxes);
-    last.assign(K, nboxes);
-    const int ntot = R.pos[K];
-    if (ntot == 0) return;
-    ensure_flag(ntot);
-    launch1d(k_iflag_segs, ntot, st, R, B.iflag.p, flag.p);
-    scan_only(ntot);
-    if (total.n < K + 1) total.alloc(K + 1, st);
-    hipLaunchKernelGGL(k_seg_totals, dim3(1), dim3(64), 0, st, R, flag.p, offs.p, total.p);
-    std::vector<int> cum(K + 1, 0);
-    readback(cum.data(), total.p, sizeof(int) * (K + 1), st);
-    const int nref = cum[K];
-    if (nref == 0) return;
-    B.grow(nboxes + 4 * (size_t)nref, nboxes);
-    for (size_t k = 0; k < K; ++k) {
-      first[k] = nboxes + 4 * cum[k];
-      last[k] = nboxes + 4 * cum[k + 1];
-    }
-    launch1d(k_make_children_segs, ntot, st, R, flag.p, offs.p, nboxes, B.centers.p,
-             B.ilevel.p, B.iparent.p, B.nchild.p, B.ichild.p, B.ses.p, B.set.p, B.iflag.p, ks,
-             kt);
-    nboxes += 4 * nref;
   }
   void ensure_flag(int n) {
     if ((size_t)n > flag.n) {
@@ -933,16 +1219,16 @@ struct Builder {
     return nref;
   }
   void computecoll(const std::vector<int>& ls, const std::vector<int>& le,
-                   const std::vector<double>& bs, int nlevels) {
+                   const std::vector<double>& bs, int nlevels, int* big = nullptr) {
     // all levels at once by walking the tree from every box (integer
     // coordinates exact: at most kWalkLevels levels, domain near the origin)
     if (nlevels <= kWalkLevels && walk_ok) {
-      DBuf<unsigned> ij(2 * (int64_t)nboxes, st);
-      launch1d(k_box_ij, nboxes, st, B.iparent.p, B.ilevel.p, B.centers.p, ij.p);
-      launch1d(k_coll_walk, nboxes, st, B.ilevel.p, B.iparent.p, B.ichild.p, ij.p, B.ncoll.p,
-               B.coll.p);
+      launch1d(k_coll_walk, nboxes, st, B.ilevel.p, B.iparent.p, B.ichild.p, B.centers.p,
+               B.ncoll.p, B.coll.p, B.nchild.p, B.ses.p, B.set.p, kLeafRankMax, big);
       return;
     }
+    if (big)
+      launch1d(k_big_leaves, nboxes, st, B.nchild.p, B.ses.p, B.set.p, kLeafRankMax, big);
     hipLaunchKernelGGL(k_root_coll, dim3(1), dim3(1), 0, st, B.ncoll.p, B.coll.p);
     for (int l = 1; l <= nlevels; ++l)
       launch1d(k_coll, le[l] - ls[l], st, ls[l], bs[l], B.iparent.p, B.ichild.p, B.centers.p,
@@ -1070,25 +1356,14 @@ bool tree_prepare_matches(const TreePrep* p, const double* src, int64_t ns, cons
          p->nlmax == nlmax;
 }
 
-void build_tree(const double* src, int64_t ns, const double* trg, int64_t nt, int ndiv,
-                int idivflag, int nlmax, Tree& t, hipStream_t st, const TreePrep* prep) {
-  if (nlmax > kMaxLevels) throw HipError{hipErrorInvalidValue, "nlmax beyond 51"};
+// One build with capacity for `room` boxes for each one of the refinement
+// (false: the level restriction needs more).
+static bool build_try(const TreePrep* P, TreePrep* own, const double* src, int64_t ns,
+                      const double* trg, int64_t nt, int ndiv, int idivflag, int nlmax, Tree& t,
+                      hipStream_t st, int room) {
   Builder bld(st);
   t.ns = ns;
   t.nt = nt;
-  // bounding square, box sizes and sorted path keys: the caller's, or made here
-  TreePrep own;
-  const TreePrep* P = prep;
-  if (!tree_prepare_matches(prep, src, ns, trg, nt, nlmax)) {
-    prepare_into(own, src, ns, trg, nt, nlmax, st);
-    double bb[4];
-    readback(bb, own.bounds.p, sizeof(bb), st);
-    prepare_host(own, bb);
-    P = &own;
-  }
-  const std::vector<double>& bsall = P->bsall;
-  const double* root = P->root;
-  bld.walk_ok = P->walk_ok;
   const int d1 = std::min(kD1, nlmax);
   // the keys in use: the prepared ones, or deeper ones made below (points
   // closer than 2^-21 of the domain)
@@ -1097,28 +1372,75 @@ void build_tree(const double* src, int64_t ns, const double* trg, int64_t nt, in
   bld.ks = pk[0]->view();
   bld.kt = pk[1]->view();
 
-  size_t cap0 = std::max<size_t>(1024, (size_t)(8 * (ns + nt) / std::max(ndiv, 1)));
+  // room for the level restriction's bound (5 boxes for each one of the
+  // refinement, which makes 2 to 3 for every ndiv points) in small trees
+  size_t cap0 = std::max<size_t>(4096, (size_t)(16 * (ns + nt) / std::max(ndiv, 1)));
+  if (cap0 > 5 * (size_t)kWgBoxes) cap0 /= 2;
   bld.B.alloc(cap0, st);
-  bld.nboxes = 1;
-  hipLaunchKernelGGL(k_init_root, dim3(1), dim3(1), 0, st, root[0], root[1], (int)ns, (int)nt,
-                     bld.B.centers.p, bld.B.ilevel.p, bld.B.iparent.p, bld.B.nchild.p,
-                     bld.B.ichild.p, bld.B.ses.p, bld.B.set.p, bld.B.iflag.p);
+  DBuf<int> state(kStWords, st);
+  std::vector<int> hs(kStWords, 0);
 
-  // ---- level-by-level refinement (pts_tree2d.f:551-631).  While the
-  // bound on a level's size is moderate, kBatch levels run between host
-  // synchronisations (level ranges kept on the device); a refined box holds
-  // more than ndiv points, so a level has at most 4 (ns + nt) / (ndiv + 1)
-  // boxes.  Otherwise, and for the key-extension check at level d1, one level
-  // at a time with its exact count.
+  // ---- level-by-level refinement (pts_tree2d.f:551-631): by one workgroup
+  // while the levels are small, else in batches.  While the bound on a level's
+  // size is moderate, kBatch levels run between host synchronisations (level
+  // ranges kept on the device); a refined box holds more than ndiv points, so
+  // a level has at most 4 (ns + nt) / (ndiv + 1) boxes.  Otherwise, and for the
+  // key-extension check at level d1, one level at a time with its exact count.
+  auto refine_wg = [&](int l0) {
+    hipLaunchKernelGGL(k_refine_wg, dim3(1), dim3(kWgThreads), 0, st,
+                       (const double*)P->bounds.p, (int)ns, (int)nt, idivflag, ndiv, nlmax,
+                       pk[0]->d1 + pk[0]->d2, (int)std::min<size_t>(bld.B.cap, INT32_MAX),
+                       ptrs(bld.B), bld.ks, bld.kt, l0, state.p);
+    hip_throw(hipGetLastError(), "refine");
+  };
+  refine_wg(0);
+  if (own && own->bsall.empty()) {
+    // the bounds with the state, in one round trip
+    double bb[4];
+    readback2(hs.data(), state.p, sizeof(int) * kStWords, bb, own->bounds.p, sizeof(bb), st);
+    prepare_host(*own, bb);
+  } else {
+    readback(hs.data(), state.p, sizeof(int) * kStWords, st);
+  }
+  const std::vector<double>& bsall = P->bsall;
+  const double* root = P->root;
+  bld.walk_ok = P->walk_ok;
   std::vector<int> ls{0}, le{1};
   std::vector<double> bs{bsall[0]};
   int nlevels = nlmax;
   const int64_t lev_cap = 4 * ((ns + nt) / (std::max(ndiv, 0) + 1) + 1);
-  DBuf<int> dlev(2 * (nlmax + 2), st), dnb(1, st);
+  DBuf<int> dlev(2 * (nlmax + 2), st);
   int l = 0;
   bool done = false;
+  // the levels that a one-workgroup run added
+  auto take_wg = [&]() {
+    bld.nboxes = hs[kStBoxes];
+    for (int k = l + 1; k <= hs[kStLevel]; ++k) {
+      bs.push_back(bsall[k]);
+      ls.push_back(hs[kStLev + 2 * k]);
+      le.push_back(hs[kStLev + 2 * k] + hs[kStLev + 2 * k + 1]);
+    }
+    l = hs[kStLevel];
+    if (hs[kStStatus] == 1) {
+      nlevels = l;
+      done = true;
+    } else if (hs[kStStatus] == 2) {
+      bld.B.grow(2 * bld.B.cap + 4 * (size_t)kWgLevel, bld.nboxes);
+    }
+  };
+  take_wg();
   while (!done && l < nlmax) {
     const int lo = ls[l], n = le[l] - ls[l];
+    if (n <= kWgLevel && l + 1 <= pk[0]->d1 + pk[0]->d2) {
+      hs[kStBoxes] = bld.nboxes;
+      hs[kStLev + 2 * l] = lo;
+      hs[kStLev + 2 * l + 1] = n;
+      upload_bytes(state.p, hs.data(), sizeof(int) * kStWords, st);
+      refine_wg(l);
+      readback(hs.data(), state.p, sizeof(int) * kStWords, st);
+      take_wg();
+      continue;
+    }
     // the batch: levels l .. l+K-1 refined, sizes bounded by ub[k]
     int K = std::min(kBatch, nlmax - l);
     if (pk[0]->d2 == 0 && l < d1) K = std::min(K, d1 - l);
@@ -1169,28 +1491,25 @@ void build_tree(const double* src, int64_t ns, const double* trg, int64_t nt, in
     bld.B.grow(bld.nboxes + (size_t)reserve, bld.nboxes);
     int64_t ubmax = 1;
     for (int k = 0; k < K; ++k) ubmax = std::max(ubmax, ub[k]);
-    bld.ensure_flag((int)ubmax);
+    DBuf<int> part(ceil_div(ubmax, kRefTile), st);
     {
-      const int h[3] = {lo, n, bld.nboxes};
-      upload_bytes(dlev.p + 2 * l, h, 2 * sizeof(int), st);
-      upload_bytes(dnb.p, h + 2, sizeof(int), st);
+      const int h[2] = {lo, n};
+      upload_bytes(dlev.p + 2 * l, h, sizeof(h), st);
       for (int k = 0; k < K; ++k) {
         const int L = l + k;
-        launch1d(k_refine_flags_lv, ub[k], st, dlev.p, L, bld.B.ses.p, bld.B.set.p, idivflag,
-                 ndiv, bld.flag.p);
-        bld.scan_only((int)ub[k]);
-        hipLaunchKernelGGL(k_level_next, dim3(1), dim3(1), 0, st, ub[k], bld.flag.p, bld.offs.p,
-                           dlev.p, L, dnb.p);
-        launch1d(k_make_children_lv, ub[k], st, dlev.p, L, bld.flag.p, bld.offs.p,
-                 0.5 * bsall[L + 1], bld.B.centers.p, bld.B.ilevel.p, bld.B.iparent.p,
-                 bld.B.nchild.p, bld.B.ichild.p, bld.B.ses.p, bld.B.set.p, bld.B.iflag.p, bld.ks,
-                 bld.kt);
+        const dim3 grid(ceil_div(ub[k], kRefTile));
+        hipLaunchKernelGGL(k_lv_count, grid, dim3(kRefTile), 0, st, (const int*)dlev.p, L,
+                           bld.B.ses.p, bld.B.set.p, idivflag, ndiv, part.p);
+        hipLaunchKernelGGL(k_lv_children, grid, dim3(kRefTile), 0, st, dlev.p, L,
+                           (const int*)part.p, idivflag, ndiv, 0.5 * bsall[L + 1],
+                           bld.B.centers.p, bld.B.ilevel.p, bld.B.iparent.p, bld.B.nchild.p,
+                           bld.B.ichild.p, bld.B.ses.p, bld.B.set.p, bld.B.iflag.p, bld.ks,
+                           bld.kt);
+        hip_throw(hipGetLastError(), "refine");
       }
       std::vector<int> hl(2 * (K + 1));
-      int hnb = 0;
       readback(hl.data(), dlev.p + 2 * l, sizeof(int) * 2 * (K + 1), st);
-      readback(&hnb, dnb.p, sizeof(int), st);
-      bld.nboxes = hnb;
+      bld.nboxes = hl[2 * K] + hl[2 * K + 1];
       for (int k = 1; k <= K; ++k) {
         if (hl[2 * k + 1] == 0) {
           nlevels = l + k - 1;
@@ -1207,72 +1526,124 @@ void build_tree(const double* src, int64_t ns, const double* trg, int64_t nt, in
   ls.resize(nlevels + 1);
   le.resize(nlevels + 1);
   bs.resize(nlevels + 1);
-  bld.computecoll(ls, le, bs, nlevels);
+  bld.computecoll(ls, le, bs, nlevels, state.p + kStBig);
 
-  // ---- level restriction (pts_tree_fix_lr, pts_tree2d.f:758-1061)
-  std::vector<int> ts1(nlevels + 1, 0), te1(nlevels + 1, 0);
-  int added1 = 0;
+  // ---- level restriction (pts_tree_fix_lr, pts_tree2d.f:758-1061); every
+  // box's iflag is 0 here
+  LevelTab T{};
+  auto level_tab = [&]() {
+    for (int k = 0; k <= nlevels; ++k) {
+      T.ls[k] = ls[k];
+      T.le[k] = le[k];
+      T.bs[k] = bs[k];
+    }
+  };
+  level_tab();
+  std::vector<int> ts(nlevels + 2, 0), te(nlevels + 2, 0);
+  int added = 0;
+  DBuf<int> part;
   if (nlevels >= 2) {
-    int* iflag = bld.B.iflag.p;
-    hip_throw(hipMemsetAsync(iflag, 0, sizeof(int) * bld.nboxes, st), "memset");
+    const int64_t nb0 = bld.nboxes;
+    // (large trees, of mostly regular regions, start with less)
+    const int64_t fac = nb0 <= 262144 ? room : std::max(3, room / 3);
+    bld.B.grow((size_t)std::min<int64_t>(fac * nb0 + 4096, INT32_MAX), nb0);
+    const int cap = (int)std::min<size_t>(bld.B.cap, INT32_MAX);
+    part.alloc(bld.B.cap / kLrTile + 1, st);
     {
       LevelReals dist{};
       for (int l = 2; l <= nlevels; ++l) dist.v[l] = 1.05 * (bs[l - 1] + bs[l - 2]) / 2.0;
       launch1d(k_flag1, le[nlevels] - ls[2], st, ls[2], dist, bld.B.ilevel.p, bld.B.iparent.p,
-               bld.B.ncoll.p, bld.B.coll.p, bld.B.nchild.p, bld.B.centers.p, iflag);
+               bld.B.ncoll.p, bld.B.coll.p, bld.B.nchild.p, bld.B.centers.p, bld.B.iflag.p);
     }
-    for (int l = nlevels; l >= 1; --l) {
-      const double distest = 1.05 * (bs[l] + bs[l - 1]) / 2.0;
-      launch1d(k_flag2, le[l] - ls[l], st, ls[l], distest, bld.B.iparent.p, bld.B.ncoll.p,
-               bld.B.coll.p, bld.B.nchild.p, bld.B.centers.p, iflag);
-    }
-    {
-      // the flags are fixed before this pass, so all levels refine in one scan
-      std::vector<int> lo, n, lev, first, last;
-      std::vector<double> bsc;
-      for (int l = 1; l <= nlevels - 2; ++l) {
-        lo.push_back(ls[l]);
-        n.push_back(le[l] - ls[l]);
-        lev.push_back(l + 1);
-        bsc.push_back(bs[l + 1]);
+    if (nb0 <= kWgBoxes && cap >= 5 * nb0) {  // (each box is refined at most once)
+      hipLaunchKernelGGL(k_flags_wg, dim3(1), dim3(kWgThreads), 0, st, T, nlevels, bld.nboxes,
+                         ptrs(bld.B), bld.ks, bld.kt, state.p);
+      hip_throw(hipGetLastError(), "level restriction");
+    } else {
+      for (int k = 0; k < kStWords; ++k)
+        if (k != kStBig) hs[k] = 0;
+      upload_bytes(state.p, hs.data(), sizeof(int) * kStBig, st);
+      upload_bytes(state.p + kStLev, hs.data() + kStLev, sizeof(int) * (kStWords - kStLev), st);
+      for (int l = nlevels; l >= 1; --l) {
+        const double distest = 1.05 * (bs[l] + bs[l - 1]) / 2.0;
+        launch1d(k_flag2, le[l] - ls[l], st, ls[l], distest, bld.B.iparent.p, bld.B.ncoll.p,
+                 bld.B.coll.p, bld.B.nchild.p, bld.B.centers.p, bld.B.iflag.p);
       }
-      bld.refine_segments(lo, n, lev, bsc, first, last);
-      for (int l = 1; l <= nlevels - 2; ++l) {
-        ts1[l + 1] = first[l - 1];
-        te1[l + 1] = last[l - 1];
-        added1 += last[l - 1] - first[l - 1];
+      // the flags are fixed now: all levels refine together
+      const int n = nlevels >= 3 ? le[nlevels - 2] - ls[1] : 0;
+      launch1d(k_flag_count, n, st, ls[1], (const int*)bld.B.iflag.p, part.p);
+      if (n > 0) {
+        hipLaunchKernelGGL(k_flag_children<0>, dim3(ceil_div(n, 256)), dim3(256), 0, st, n, ls[1],
+                           0, bld.nboxes, (const int*)part.p, T, cap, ptrs(bld.B), bld.ks, bld.kt,
+                           state.p);
+        hip_throw(hipGetLastError(), "level restriction");
       }
     }
+    readback(hs.data(), state.p, sizeof(int) * kStWords, st);
+    if (nb0 <= kWgBoxes && cap >= 5 * nb0) {
+      for (int l = 2; l <= nlevels - 1; ++l) {
+        ts[l] = hs[kStLev + 2 * l];
+        te[l] = hs[kStLev + 2 * l + 1];
+      }
+    } else {
+      if (hs[kStStatus] != 0) return false;  // out of room
+      int at = bld.nboxes;
+      for (int l = 2; l <= nlevels - 1; ++l) {
+        ts[l] = at;
+        te[l] = at += 4 * hs[kStLev + 2 * l];
+      }
+    }
+    for (int l = 2; l <= nlevels - 1; ++l) added += te[l] - ts[l];
+    bld.nboxes += added;
+  } else {
+    readback(hs.data(), state.p, sizeof(int) * kStLev, st);
   }
+  const bool big = hs[kStBig] != 0;
   // With no box added by the flagged refinement no box carries flag 3, the
   // updateflags sweep below refines nothing and both reorganisations are the
   // identity: the tree is already level-restricted.
-  if (nlevels >= 2 && added1 > 0) {
-    bld.reorg(ls, le, ts1, te1, nlevels);
+  if (added > 0) {
+    bld.reorg(ls, le, ts, te, nlevels);
     bld.computecoll(ls, le, bs, nlevels);
-    launch1d(k_keep3, bld.nboxes, st, bld.B.iflag.p);
-    std::vector<int> ts(nlevels + 1, 0), te(nlevels + 1, 0);
-    int added2 = 0;
+    level_tab();
+    // the sweep over the levels, the new boxes' ranges kept on the device:
+    // two launches a level and one round trip in all
+    const int cap = (int)std::min<size_t>(bld.B.cap, INT32_MAX);
+    for (int k = 0; k < kStWords; ++k) hs[k] = 0;
+    hs[kStLev + 2 * 2] = hs[kStLev + 2 * 2 + 1] = bld.nboxes;
+    upload_bytes(state.p, hs.data(), sizeof(int) * kStWords, st);
+    int64_t tail_ub = 0;
     for (int l = 2; l <= nlevels - 2; ++l) {
+      const int n1 = le[l] - ls[l];
       const double distest = 1.05 * (bs[l] + bs[l + 1]) / 2.0;
-      // the original then the tail boxes of level l (their flags are independent)
-      launch1d(k_updateflags, (le[l] - ls[l]) + (te[l] - ts[l]), st, le[l] - ls[l], ls[l], ts[l],
-               distest, bld.B.ncoll.p, bld.B.coll.p, bld.B.ichild.p, bld.B.nchild.p,
-               bld.B.centers.p, bld.B.iflag.p);
-      {
-        // the original then the tail boxes of level l, in one scan
-        std::vector<int> first, last;
-        bld.refine_segments({ls[l], ts[l]}, {le[l] - ls[l], te[l] - ts[l]}, {l + 1, l + 1},
-                            {bs[l + 1], bs[l + 1]}, first, last);
-        ts[l + 1] = first[0];
-        te[l + 1] = last[1];
-        added2 += te[l + 1] - ts[l + 1];
+      const unsigned n = (unsigned)(n1 + tail_ub);
+      if (n > 0) {
+        hipLaunchKernelGGL(k_sweep_flags, dim3(ceil_div(n, kLrTile)), dim3(256), 0, st, n1, ls[l],
+                           l, (int)tail_ub, kColl * bs[l], distest, ptrs(bld.B), part.p, state.p);
+        hipLaunchKernelGGL(k_flag_children<1>, dim3(ceil_div(n, 256)), dim3(256), 0, st, n1,
+                           ls[l], l, 0, (const int*)part.p, T, cap, ptrs(bld.B), bld.ks, bld.kt,
+                           state.p);
+        hip_throw(hipGetLastError(), "level restriction");
       }
-      launch1d(k_coll, te[l + 1] - ts[l + 1], st, ts[l + 1], bs[l + 1], bld.B.iparent.p,
-               bld.B.ichild.p, bld.B.centers.p, bld.B.ncoll.p, bld.B.coll.p);
+      tail_ub = std::min<int64_t>(
+          std::min<int64_t>(4 * (int64_t)n, (int64_t)cap - bld.nboxes), (int64_t)32768 * room);
     }
-    // (with nothing added the second reorganisation is the identity and the
-    // colleagues are those computed above)
+    std::fill(ts.begin(), ts.end(), 0);
+    std::fill(te.begin(), te.end(), 0);
+    int added2 = 0;
+    if (nlevels >= 4) {
+      readback(hs.data(), state.p, sizeof(int) * kStWords, st);
+      if (hs[kStStatus] != 0) return false;  // out of room
+      for (int l = 3; l <= nlevels - 1; ++l) {
+        ts[l] = hs[kStLev + 2 * l];
+        te[l] = hs[kStLev + 2 * l + 1];
+        added2 += te[l] - ts[l];
+      }
+      bld.nboxes += added2;
+    }
+    // the last level's tail has no colleagues yet; with nothing added the
+    // second reorganisation is the identity and the colleagues are those
+    // computed above
     if (added2 > 0) {
       bld.reorg(ls, le, ts, te, nlevels);
       bld.computecoll(ls, le, bs, nlevels);
@@ -1288,26 +1659,30 @@ void build_tree(const double* src, int64_t ns, const double* trg, int64_t nt, in
   t.boxsize = bs;
   t.isrc.alloc(std::max<int64_t>(ns, 1), st);
   t.itarg.alloc(std::max<int64_t>(nt, 1), st);
+  t.leaf_s.alloc(std::max<int64_t>(ns, 1), st);
+  t.leaf_t.alloc(std::max<int64_t>(nt, 1), st);
   DBuf<int>* perm[2] = {&t.isrc, &t.itarg};
   const int* se[2] = {bld.B.ses.p, bld.B.set.p};
   const int64_t npts[2] = {ns, nt};
-  DBuf<int> big(4, st), bigl(nb, st);
-  big.zero();
-  for (int k = 0; k < 2; ++k) {
-    if (npts[k] == 0) continue;
-    // big[k]: a leaf beyond kLeafSortMax; big[2 + k]: leaves beyond kLeafSmall
-    launch1d(k_leaf_sort_small, nb, st, bld.B.nchild.p, se[k], pk[k]->perm.p, perm[k]->p, bigl.p,
-             big.p + 2 + k);
-    const unsigned grid = (unsigned)std::min<int64_t>(4096, ceil_div(nb, kLeafSortWaves));
-    hipLaunchKernelGGL(k_leaf_sort, dim3(grid), dim3(kLeafSortWaves * 64), 0, st, bigl.p,
-                       big.p + 2 + k, se[k], pk[k]->perm.p, perm[k]->p, big.p + k);
-    hip_throw(hipGetLastError(), "kernel launch");
+  hipLaunchKernelGGL(k_leaf_of, dim3(ceil_div(nb, 256), nt > 0 ? 2 : 1), dim3(256), 0, st,
+                     (int64_t)nb, bld.B.nchild.p, se[0], se[1], t.leaf_s.p, t.leaf_t.p);
+  if (!big) {
+    LeafOrder a;
+    const int* leaf[2] = {t.leaf_s.p, t.leaf_t.p};
+    for (int k = 0; k < 2; ++k) {
+      a.n[k] = npts[k];
+      a.leaf[k] = leaf[k];
+      a.se[k] = se[k];
+      a.perm[k] = pk[k]->perm.p;
+      a.out[k] = perm[k]->p;
+    }
+    hipLaunchKernelGGL(k_leaf_rank, dim3(ceil_div(std::max(ns, nt), 256), nt > 0 ? 2 : 1),
+                       dim3(256), 0, st, a);
   }
-  int hbig[2] = {0, 0};
-  readback(hbig, big.p, sizeof(hbig), st);
-  for (int k = 0; k < 2; ++k) {
-    if (npts[k] == 0 || !hbig[k]) continue;
-    // a leaf too large for k_leaf_sort: stable sort of all points by leaf
+  hip_throw(hipGetLastError(), "point order");
+  for (int k = 0; k < 2 && big; ++k) {
+    if (npts[k] == 0) continue;
+    // some leaf is too large to rank: stable sort of all points by leaf
     DBuf<unsigned long long> label(npts[k], st), lsorted(npts[k], st);
     launch1d(k_leaf_label, nb, st, bld.B.nchild.p, se[k], pk[k]->perm.p, label.p);
     int bits = 1;
@@ -1324,6 +1699,24 @@ void build_tree(const double* src, int64_t ns, const double* trg, int64_t nt, in
   t.ichild = std::move(bld.B.ichild);
   t.ncoll = std::move(bld.B.ncoll);
   t.coll = std::move(bld.B.coll);
+  return true;
+}
+
+void build_tree(const double* src, int64_t ns, const double* trg, int64_t nt, int ndiv,
+                int idivflag, int nlmax, Tree& t, hipStream_t st, const TreePrep* prep) {
+  if (nlmax > kMaxLevels) throw HipError{hipErrorInvalidValue, "nlmax beyond 51"};
+  // bounding square, box sizes and sorted path keys: the caller's, or made here
+  TreePrep own;
+  const bool mine = !tree_prepare_matches(prep, src, ns, trg, nt, nlmax);
+  if (mine) prepare_into(own, src, ns, trg, nt, nlmax, st);
+  // The restriction adds about as many boxes as there are on curves and
+  // clusters, up to six times as many around isolated tight clusters.
+  for (int room = 8;; room *= 4) {
+    if (build_try(mine ? &own : prep, mine ? &own : nullptr, src, ns, trg, nt, ndiv, idivflag,
+                  nlmax, t, st, room))
+      return;
+    if (room > 1 << 20) throw HipError{hipErrorOutOfMemory, "tree boxes"};
+  }
 }
 
 // Points (sources + targets) held by the leaves of each level, levels beyond
