@@ -41,6 +41,7 @@
 #include "hankel32.h"
 #include "helm_ops.h"
 #include "lap_ops.h"
+#include "m2l.h"
 #include "p2p_math.h"
 #include "scan.h"
 #include "translate.h"
@@ -830,7 +831,8 @@ struct OpDesc {
   int g;        // index of G[0] in the table
   int w1, w2;   // first power of each power table
   int sa, sb, sc;
-  int pad;
+  int orbit;    // 1: fragments of m2l.h (pin = pout), 0: of translate.h
+  int ksc, rtc;
 };
 
 __global__ void k_to_f32(int64_t n, const double* in, float* out) {
@@ -842,13 +844,19 @@ __global__ void k_build_ops(const OpDesc* ops, const cplx* gt, const double* wt,
   const OpDesc o = ops[blockIdx.y];
   const int Pin = 2 * o.pin + 1, Pout = 2 * o.pout + 1;
   const int RTT = (2 * Pout + 15) / 16, KS = (2 * Pin + 3) / 4;
-  const int64_t total = (int64_t)RTT * KS * 64;
+  const int ksc = o.orbit ? o.ksc : 0, rtc = o.orbit ? o.rtc : 0;
+  const int64_t total = o.orbit ? (int64_t)16 * ksc * rtc * 64 : (int64_t)RTT * KS * 64;
   for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < total;
        e += (int64_t)gridDim.x * blockDim.x) {
     const int lane = (int)(e & 63);
     const int64_t rest = e >> 6;
     const int ks = (int)(rest % KS), rt = (int)(rest / KS);
-    const int row = 16 * rt + (lane & 15), col = 4 * ks + (lane >> 4);
+    int row = 16 * rt + (lane & 15), col = 4 * ks + (lane >> 4);
+    if (o.orbit) {
+      const M2LEntry m = m2l_entry((int)e, ksc, rtc, -1);
+      row = 2 * m.n + m.rpart;
+      col = 2 * m.j + m.cpart;
+    }
     double v = 0.0;
     if (row < 2 * Pout && col < 2 * Pin) {
       const int i = row / 2 - o.pout, j = col / 2 - o.pin;
@@ -898,7 +906,8 @@ int push_powers(OpTables& T, long double base, int emax) {
   return w0;
 }
 
-void add_op(OpTables& T, int pin, int pout, int g, int w1, int w2, int sa, int sb, int sc) {
+void add_op(OpTables& T, int pin, int pout, int g, int w1, int w2, int sa, int sb, int sc,
+            bool orbit = false) {
   OpDesc o{};
   o.af = T.af_total;
   o.pin = pin;
@@ -909,8 +918,11 @@ void add_op(OpTables& T, int pin, int pout, int g, int w1, int w2, int sa, int s
   o.sa = sa;
   o.sb = sb;
   o.sc = sc;
+  o.orbit = orbit ? 1 : 0;
+  o.ksc = m2l_ksc(2 * pin + 1);
+  o.rtc = m2l_rtc(2 * pin + 1);
   T.desc.push_back(o);
-  T.af_total += afrag_stride(2 * pin + 1, 2 * pout + 1);
+  T.af_total += orbit ? m2l_stride(2 * pin + 1) : afrag_stride(2 * pin + 1, 2 * pout + 1);
 }
 
 // scaled H_m(z) s^m, m = 0..mmax, long double upward recurrence from H0, H1
@@ -1210,19 +1222,26 @@ void helm_box_passes(const Tree& t, const Lists& L, const std::vector<HLev>& lev
       const int w1 = push_powers(T, sl[l], 2 * p);
       const int w2 = push_powers(T, 1.0L, p);
       std::vector<std::vector<lc>> hr(19);
-      for (int dx = -3; dx <= 3; ++dx)
-        for (int dy = -3; dy <= 3; ++dy) {
-          const int r2 = dx * dx + dy * dy;
-          if (std::abs(dx) <= 1 && std::abs(dy) <= 1) {
-            add_op(T, p, p, 0, w1, w2, 0, 0, 0);  // never referenced: zero table slot
-            T.desc.back().g = -1;
-            continue;
+      auto offset = [&](int dx, int dy, bool orbit) {
+        const int r2 = dx * dx + dy * dy;
+        if (hr[r2].empty())
+          hr[r2] = host_scaled_h(k * (bs * std::sqrt((long double)r2)), sl[l], 2 * p);
+        const int g = push_table(T, hr[r2], 2 * p, std::atan2((long double)dy, (long double)dx));
+        add_op(T, p, p, g, w1, w2, -1, 1, 1, orbit);
+      };
+      if (2 * p + 1 <= kM2LMaxP) {
+        for (int o = 0; o < kM2LOrbits; ++o) offset(kM2LBase[o][0], kM2LBase[o][1], true);
+      } else {
+        for (int dx = -3; dx <= 3; ++dx)
+          for (int dy = -3; dy <= 3; ++dy) {
+            if (std::abs(dx) <= 1 && std::abs(dy) <= 1) {
+              add_op(T, p, p, 0, w1, w2, 0, 0, 0);  // never referenced: zero table slot
+              T.desc.back().g = -1;
+              continue;
+            }
+            offset(dx, dy, false);
           }
-          if (hr[r2].empty())
-            hr[r2] = host_scaled_h(k * (bs * std::sqrt((long double)r2)), sl[l], 2 * p);
-          const int g = push_table(T, hr[r2], 2 * p, std::atan2((long double)dy, (long double)dx));
-          add_op(T, p, p, g, w1, w2, -1, 1, 1);
-        }
+      }
     }
     if (l <= nl - 1 && lev[l].on) {
       // M2M into level l from children at l + 1 (h2dmpmp, helmrouts2d.f:967-1090) and
@@ -1267,7 +1286,8 @@ void helm_box_passes(const Tree& t, const Lists& L, const std::vector<HLev>& lev
     for (const OpDesc& od : T.desc)
       if (od.g >= 0) {
         build.push_back(od);
-        maxaf = std::max(maxaf, afrag_stride(2 * od.pin + 1, 2 * od.pout + 1));
+        maxaf = std::max(maxaf, od.orbit ? m2l_stride(2 * od.pin + 1)
+                                         : afrag_stride(2 * od.pin + 1, 2 * od.pout + 1));
       }
     if (!build.empty()) {
       DBuf<OpDesc> d_desc = upload(build, st);
@@ -1304,7 +1324,7 @@ void helm_box_passes(const Tree& t, const Lists& L, const std::vector<HLev>& lev
     M2LPlan m2l;
     plan_m2l(t, L, pg, pgt, m2l, st);
     if (m2l.ntg > 0) {
-      DBuf<int> d_soff = upload(m2l_slot_offsets(), st);
+      DBuf<int> d_soff;  // offset slots of the levels that k_translate takes
       // FP32 copy of every level's multipoles (mixed precision)
       const int64_t ncoef = lev[nl].off + (int64_t)(t.nboxes - t.lstart[nl]) * nd *
                                               (2 * lev[nl].p + 1);
@@ -1313,10 +1333,24 @@ void helm_box_passes(const Tree& t, const Lists& L, const std::vector<HLev>& lev
       tm.mark(3);  // planning
       for (int l = 2; l <= nl; ++l) {
         if (op_m2l[l] < 0) continue;
+        const HLev& V = lev[l];
+        const int Pl = 2 * V.p + 1;
+        if (Pl <= kM2LMaxP) {
+          M2LSeg seg;
+          for (int q = 0; q < 4; ++q) seg.s0[q] = m2l.lev(q, l, nl);
+          seg.n = m2l.lev(0, l + 1, nl) - seg.s0[0];
+          const int64_t af = T.desc[op_m2l[l]].af;
+          launch_m2l<-1, 0>(nd, Pl, seg, m2l.tlist.p, L.s2.p,
+                            mixed ? (const void*)(af32.p + af) : (const void*)(d_af.p + af),
+                            V.box0, V.box0, t.ilevel.p, nullptr, nullptr,
+                            mixed ? (const void*)(mp32.p + 2 * V.off) : (const void*)(mpp + V.off),
+                            locp + V.off, mixed, st);
+          continue;
+        }
+        if (!d_soff.p) d_soff = upload(m2l_slot_offsets(), st);
         std::vector<TrGroup> groups;
         for (int q = 0; q < 4; ++q)
           groups.push_back(TrGroup{m2l.lev(q, l, nl), m2l.lev(q, l + 1, nl), 0, q});
-        const HLev& V = lev[l];
         if (mixed)
           launch_translate(0, 0, nd,
                            TrBufs{mp32.p + 2 * V.off, V.box0, 2 * V.p + 1, locp + V.off,

@@ -30,6 +30,7 @@
 #include "devbuf.h"
 #include "fmm_common.h"
 #include "lap_ops.h"
+#include "m2l.h"
 #include "p2p_math.h"
 #include "scan.h"
 #include "translate.h"
@@ -1292,15 +1293,24 @@ void make_matrices(int P, std::vector<cplx>& A, std::vector<cplx>& B, std::vecto
     }
 }
 
-// Translation operators of one expansion length P as MFMA fragments: the 49
-// M2L offsets, 4 M2M and 4 L2L quadrants in FP64, and the M2L offsets in FP32
-// for mixed precision.  They depend on P alone (the Laplace operators are
-// level independent), so each (device, P) builds them once; they stay for
-// the life of the process.
+// Translation operators of one expansion length P as MFMA fragments: the 4
+// M2M and 4 L2L quadrants (FP64), and the M2L operators in FP64 and, for mixed
+// precision, FP32: the 10 orbits of m2l.h up to kM2LMaxP coefficients, the 49
+// offsets for k_translate beyond.  They depend on P alone (the Laplace
+// operators are level independent), so each (device, P) builds them once;
+// they stay for the life of the process.
 struct LapOps {
-  double* af = nullptr;
-  float* af32 = nullptr;
+  double* af = nullptr;  // M2M, L2L
+  double* m2l = nullptr;
+  float* m2l32 = nullptr;
 };
+
+template <typename T> T* to_device(const std::vector<T>& v) {
+  T* p = nullptr;
+  hip_throw(hipMalloc(&p, v.size() * sizeof(T)), "alloc");
+  hip_throw(hipMemcpy(p, v.data(), v.size() * sizeof(T), hipMemcpyHostToDevice), "copy");
+  return p;
+}
 
 const LapOps& lap_ops(int P) {
   static std::mutex mu;
@@ -1312,18 +1322,22 @@ const LapOps& lap_ops(int P) {
   if (it != cache.end()) return it->second;
   std::vector<cplx> A, B, T;
   make_matrices(P, A, B, T);
-  std::vector<cplx> ops(T);
-  ops.insert(ops.end(), A.begin(), A.end());
+  std::vector<cplx> ops(A);
   ops.insert(ops.end(), B.begin(), B.end());
-  const std::vector<double> f64 = swizzle_ops(P, ops, kOff * kOff + 8);
-  const std::vector<float> f32 = swizzle_ops<float>(P, T, kOff * kOff);
   LapOps o;
-  hip_throw(hipMalloc(&o.af, f64.size() * sizeof(double)), "alloc");
-  hip_throw(hipMalloc(&o.af32, f32.size() * sizeof(float)), "alloc");
-  hip_throw(hipMemcpy(o.af, f64.data(), f64.size() * sizeof(double), hipMemcpyHostToDevice),
-            "copy");
-  hip_throw(hipMemcpy(o.af32, f32.data(), f32.size() * sizeof(float), hipMemcpyHostToDevice),
-            "copy");
+  o.af = to_device(swizzle_ops(P, ops, 8));
+  if (P <= kM2LMaxP) {
+    std::vector<std::vector<cplx>> orb;
+    for (int k = 0; k < kM2LOrbits; ++k) {
+      const size_t f = (size_t)((kM2LBase[k][0] + 3) * kOff + kM2LBase[k][1] + 3) * P * P;
+      orb.emplace_back(T.begin() + f, T.begin() + f + (size_t)P * P);
+    }
+    o.m2l = to_device(m2l_swizzle<double>(P, orb, 1));
+    o.m2l32 = to_device(m2l_swizzle<float>(P, orb, 1));
+  } else {
+    o.m2l = to_device(swizzle_ops(P, T, kOff * kOff));
+    o.m2l32 = to_device(swizzle_ops<float>(P, T, kOff * kOff));
+  }
   return cache.emplace(std::make_pair(dev, P), o).first->second;
 }
 
@@ -1636,8 +1650,8 @@ int laplace_fmm(int kind, const CauchyArgs& a, hipStream_t st) {
 #undef FMM2D_P2L_W
 #undef FMM2D_P2L_W32
     tm.mark(1);
-    // ---- translation operators as MFMA fragments: 49 M2L offsets, 4 M2M, 4 L2L
-    const int opM2M = kOff * kOff, opL2L = opM2M + 4;
+    // ---- translation operators as MFMA fragments: 4 M2M, 4 L2L
+    const int opM2M = 0, opL2L = 4;
     const double* d_af = ops.af;
     std::vector<int2> band(nl + 1);
     for (int l = 0; l <= nl; ++l) band[l] = int2{0, 2 * (nterms[l] + 1)};
@@ -1663,24 +1677,24 @@ int laplace_fmm(int kind, const CauchyArgs& a, hipStream_t st) {
       M2LPlan m2l;
       plan_m2l(t, L, pg, pgt, m2l, st);
       if (m2l.ntg > 0) {
-        DBuf<int> d_soff = upload(m2l_slot_offsets(), st);
-        std::vector<TrGroup> groups;
-        for (int q = 0; q < 4; ++q)
-          groups.push_back(TrGroup{m2l.cls_seg[q], m2l.cls_seg[q + 1], 0, q});
-        if (mixed) {
-          // FP32 operators and the FP32 copy of the multipoles
-          tm.mark(3);  // planning
-          launch_translate(0, 1, nd, TrBufs{mp32.p, 0, P, loc.p, 0, P}, kSlots, groups,
-                           m2l.tlist.p, L.s2.p, d_soff.p, ops.af32, t.ilevel.p, d_band.p,
-                           d_logr.p, st, true, true, true);
-          tm.mark(13);  // the M2L kernel alone
+        const void* msrc = mixed ? (const void*)mp32.p : (const void*)mp.p;
+        const void* mops = mixed ? (const void*)ops.m2l32 : (const void*)ops.m2l;
+        tm.mark(3);  // planning
+        if (P <= kM2LMaxP) {
+          const M2LSeg seg{{m2l.cls_seg[0], m2l.cls_seg[1], m2l.cls_seg[2], m2l.cls_seg[3]},
+                           m2l.cls_seg[1] - m2l.cls_seg[0]};
+          launch_m2l<1, 1>(nd, P, seg, m2l.tlist.p, L.s2.p, mops, 0, 0, t.ilevel.p, d_band.p,
+                           d_logr.p, msrc, loc.p, mixed, st);
         } else {
-          tm.mark(3);  // planning
-          launch_translate(0, 1, nd, TrBufs{mp.p, 0, P, loc.p, 0, P}, kSlots, groups,
-                           m2l.tlist.p, L.s2.p, d_soff.p, d_af, t.ilevel.p, d_band.p,
-                           d_logr.p, st, false, true, true);
-          tm.mark(13);  // the M2L kernel alone
+          DBuf<int> d_soff = upload(m2l_slot_offsets(), st);
+          std::vector<TrGroup> groups;
+          for (int q = 0; q < 4; ++q)
+            groups.push_back(TrGroup{m2l.cls_seg[q], m2l.cls_seg[q + 1], 0, q});
+          launch_translate(0, 1, nd, TrBufs{msrc, 0, P, loc.p, 0, P}, kSlots, groups, m2l.tlist.p,
+                           L.s2.p, d_soff.p, mops, t.ilevel.p, d_band.p, d_logr.p, st, mixed, true,
+                           true);
         }
+        tm.mark(13);  // the M2L kernel alone
       }
     }
     tm.mark(3);
