@@ -1325,26 +1325,30 @@ void helm_box_passes(const Tree& t, const Lists& L, const std::vector<HLev>& lev
     plan_m2l(t, L, pg, pgt, m2l, st);
     if (m2l.ntg > 0) {
       DBuf<int> d_soff;  // offset slots of the levels that k_translate takes
-      // FP32 copy of every level's multipoles (mixed precision)
-      const int64_t ncoef = lev[nl].off + (int64_t)(t.nboxes - t.lstart[nl]) * nd *
-                                              (2 * lev[nl].p + 1);
-      DBuf<float> mp32(mixed ? 2 * std::max<int64_t>(ncoef, 1) : 0, st);
-      if (mixed) launch1d(k_to_f32, 2 * ncoef, st, (const double*)mpp, mp32.p);
+      // FP32 copy of the multipoles of the levels that k_translate takes, the
+      // coarse ones (mixed precision)
+      int64_t ncoef = 0;
+      for (int l = 2; l <= nl; ++l)
+        if (2 * lev[l].p + 1 > kM2LMaxP)
+          ncoef = lev[l].off + (int64_t)((l < nl ? t.lstart[l + 1] : t.nboxes) - t.lstart[l]) * nd *
+                                   (2 * lev[l].p + 1);
+      DBuf<float> mp32(mixed ? 2 * ncoef : 0, st);
+      if (mixed && ncoef > 0) launch1d(k_to_f32, 2 * ncoef, st, (const double*)mpp, mp32.p);
       tm.mark(3);  // planning
+      std::vector<M2LLev> orbit_levels;
       for (int l = 2; l <= nl; ++l) {
         if (op_m2l[l] < 0) continue;
         const HLev& V = lev[l];
         const int Pl = 2 * V.p + 1;
         if (Pl <= kM2LMaxP) {
-          M2LSeg seg;
-          for (int q = 0; q < 4; ++q) seg.s0[q] = m2l.lev(q, l, nl);
-          seg.n = m2l.lev(0, l + 1, nl) - seg.s0[0];
-          const int64_t af = T.desc[op_m2l[l]].af;
-          launch_m2l<-1, 0>(nd, Pl, seg, m2l.tlist.p, L.s2.p,
-                            mixed ? (const void*)(af32.p + af) : (const void*)(d_af.p + af),
-                            V.box0, V.box0, t.ilevel.p, nullptr, nullptr,
-                            mixed ? (const void*)(mp32.p + 2 * V.off) : (const void*)(mpp + V.off),
-                            locp + V.off, mixed, st);
+          M2LLev v{};
+          for (int q = 0; q < 4; ++q) v.s0[q] = m2l.lev(q, l, nl);
+          v.n = m2l.lev(0, l + 1, nl) - v.s0[0];
+          v.P = Pl;
+          v.box0 = V.box0;
+          v.off = V.off;
+          v.aoff = T.desc[op_m2l[l]].af;
+          orbit_levels.push_back(v);
           continue;
         }
         if (!d_soff.p) d_soff = upload(m2l_slot_offsets(), st);
@@ -1365,6 +1369,9 @@ void helm_box_passes(const Tree& t, const Lists& L, const std::vector<HLev>& lev
                            kSlots, groups, m2l.tlist.p, L.s2.p, d_soff.p, opptr(op_m2l[l]),
                            t.ilevel.p, nullptr, nullptr, st, false, true, true);
       }
+      launch_m2l<-1, 0>(nd, orbit_levels, m2l.tlist.p, L.s2.p,
+                        mixed ? (const void*)af32.p : (const void*)d_af.p, t.ilevel.p, nullptr,
+                        nullptr, mpp, locp, mixed, st);
       tm.mark(13);  // the M2L kernels alone
     }
   }

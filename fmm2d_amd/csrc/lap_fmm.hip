@@ -1666,10 +1666,11 @@ int laplace_fmm(int kind, const CauchyArgs& a, hipStream_t st) {
                        d_op4.p, d_af, t.ilevel.p, d_band.p, d_logr.p, st);
     tm.mark(2);
     // ---- step 4: M2L, targets grouped by child position (box order within a group)
-    // (mixed precision: FP32 copies of the multipoles, for the M2L and the
-    // list-3 evaluations, and of the locals after L2L, for L2P)
+    // (mixed precision: FP32 copies of the multipoles, for the list-3
+    // evaluations and the M2L of long expansions, and of the locals after L2L,
+    // for L2P)
     DBuf<float> mp32, loc32;
-    if (mixed) {
+    if (mixed && (nd == 1 || P > kM2LMaxP)) {
       mp32.alloc(2 * nexp, st);
       launch1d(k_to_f32, 2 * nexp, st, reinterpret_cast<const double*>(mp.p), mp32.p);
     }
@@ -1681,10 +1682,12 @@ int laplace_fmm(int kind, const CauchyArgs& a, hipStream_t st) {
         const void* mops = mixed ? (const void*)ops.m2l32 : (const void*)ops.m2l;
         tm.mark(3);  // planning
         if (P <= kM2LMaxP) {
-          const M2LSeg seg{{m2l.cls_seg[0], m2l.cls_seg[1], m2l.cls_seg[2], m2l.cls_seg[3]},
-                           m2l.cls_seg[1] - m2l.cls_seg[0]};
-          launch_m2l<1, 1>(nd, P, seg, m2l.tlist.p, L.s2.p, mops, 0, 0, t.ilevel.p, d_band.p,
-                           d_logr.p, msrc, loc.p, mixed, st);
+          M2LLev v{};
+          for (int q = 0; q < 4; ++q) v.s0[q] = m2l.cls_seg[q];
+          v.n = m2l.cls_seg[1] - m2l.cls_seg[0];
+          v.P = P;
+          launch_m2l<1, 1>(nd, {v}, m2l.tlist.p, L.s2.p, mops, t.ilevel.p, d_band.p, d_logr.p,
+                           mp.p, loc.p, mixed, st);
         } else {
           DBuf<int> d_soff = upload(m2l_slot_offsets(), st);
           std::vector<TrGroup> groups;

@@ -13,16 +13,27 @@
 // single), so a target takes 10 operators' worth of matrix work and not 27.
 //
 // A wavefront owns 16 (target, density) columns of one child position, a
-// workgroup 64 consecutive ones; per (orbit, b) chunk the operator's fragments
-// (v_mfma_*_16x16x4 A layout) are copied to LDS once for the four wavefronts,
-// two buffers deep, and every lane loads its component of the four sources'
-// coefficients one chunk ahead, into registers.  The products of class a
-// accumulate in their own tiles, so coefficients are padded to 8 RTC per
-// class.  (Per-wavefront operators read through L1 were the bound before: 15
-// KB a slot and wavefront, 50 GB over the 1.9e6 targets of lfmm2d N = 1e7.)
+// workgroup 16 NW consecutive ones.  Per orbit and group of HB classes the
+// wavefront loads its columns' source rows with consecutive lanes on
+// consecutive coefficients (one group ahead, into registers), forms the z_c of
+// each coefficient in the lane that holds its four sources, and keeps them in
+// LDS, from where every lane reads its B operand; the operator's fragments of
+// one class (v_mfma_*_16x16x4 A layout) are copied to LDS for the whole
+// workgroup, two buffers deep and loaded two classes ahead.  The products of
+// class a accumulate in their own tiles, so coefficients are padded to 8 RTC
+// per class.
 //
-// Neighbouring workgroups take the four child positions of the same parents,
-// whose sources are mostly the same boxes, on one XCD.
+// What bounded the simpler forms (lfmm2d N = 1e7, 1.9e6 targets of 19
+// coefficients): one operator per slot read through L1 by every wavefront,
+// 50 GB of operators, 6.2 ms; orbits with each lane gathering its own
+// components, 32 cache lines a load, 4.2 ms.  This form 3.8 ms: 40% of the
+// cycles in MFMA, 52% with the LDS active; LDS latency between the chunks'
+// barriers with two wavefronts per SIMD is what is left.
+//
+// All levels with the same tile shape go in one launch (the coarse levels of a
+// Helmholtz tree are a few workgroups of serial latency each).  Neighbouring
+// workgroups take the four child positions of the same parents, whose sources
+// are mostly the same boxes, on one XCD.
 #pragma once
 #include <vector>
 
@@ -100,42 +111,70 @@ inline std::vector<T> m2l_swizzle(int P, const std::vector<std::vector<cplx>>& o
   return out;
 }
 
-// Targets of one launch: child position q's are tlist[s0[q] .. s0[q] + n)
-struct M2LSeg {
-  int s0[4], n;
+// One level of a launch: child position q's targets are tlist[s0[q] .. s0[q] +
+// n); P coefficients; boxes from box0 on, expansions from off on (complex
+// values); operators from aoff on; first workgroup (of one child position) blk0.
+struct M2LLev {
+  int s0[4], n, P, box0, blk0;
+  int64_t off, aoff;
+};
+constexpr int kM2LMaxLev = 52;
+struct M2LTab {
+  int nlev, nblk;  // workgroups per child position
+  M2LLev lev[kM2LMaxLev];
 };
 
-template <typename T, int RTC, int KSC, int SGN, int LOGT>
-__global__ __launch_bounds__(256) void k_m2l(int nd, int P, int nblk, int per_xcd, M2LSeg seg,
-                                             const int* __restrict__ tlist,
-                                             const int* __restrict__ s2, M2LSlots orb,
-                                             const T* __restrict__ A, int sbox0, int dbox0,
-                                             const int* __restrict__ ilevel,
-                                             const int2* __restrict__ band,
-                                             const double* __restrict__ logr,
-                                             const T* __restrict__ src, cplx* dst) {
+static __device__ double m2l_zero[2];
+
+template <typename T> struct M2LPair {
+  T re, im;
+};
+
+template <typename T, int RTC, int KSC, int HB, int NW, int SGN, int LOGT>
+__global__ __launch_bounds__(64 * NW) void k_m2l(int nd, int per_xcd, M2LTab tab,
+                                                 const int* __restrict__ tlist,
+                                                 const int* __restrict__ s2, M2LSlots orb,
+                                                 const T* __restrict__ Aall,
+                                                 const int* __restrict__ ilevel,
+                                                 const int2* __restrict__ band,
+                                                 const double* __restrict__ logr,
+                                                 const cplx* __restrict__ srcall, cplx* dstall) {
   typedef typename Mfma<T>::acc_t acc_t;
+  typedef M2LPair<T> pair_t;
+  typedef M2LPair<double> dpair;
+  constexpr int NT = 64 * NW;
   constexpr int CH = KSC * 4 * RTC * 64;  // values of one (orbit, b) chunk
-  constexpr int NA = CH / 256;
+  constexpr int NA = (CH + NT - 1) / NT;
+  constexpr int CS = 2 * KSC;             // coefficients of a class, padded
+  constexpr int JH = HB * CS;             // coefficients of a group
+  constexpr int NIT = (16 * JH + 63) / 64;
+  constexpr int NG = 4 / HB;              // groups of an orbit
+  constexpr int ZS = JH + 1;              // z of a column, odd: reads without bank conflicts
   __shared__ T abuf[2][CH];
+  __shared__ pair_t zbuf[NW][4][16][ZS];
+  __shared__ int64_t offs[NW][2][16][4];
   __shared__ signed char slots[kM2LOrbits][4];
   const int64_t lblk = (int64_t)(blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
-  if (lblk >= 4 * (int64_t)nblk) return;
-  const int q = (int)(lblk & 3);
-  const int tid = threadIdx.x, lane = tid & 63, kr = lane >> 4;
+  if (lblk >= 4 * (int64_t)tab.nblk) return;
+  const int q = (int)(lblk & 3), pb = (int)(lblk >> 2);
+  int li = 0;
+  while (li + 1 < tab.nlev && pb >= tab.lev[li + 1].blk0) ++li;
+  const int P = tab.lev[li].P, box0 = tab.lev[li].box0;
+  const T* __restrict__ A = Aall + tab.lev[li].aoff;
+  const dpair* __restrict__ src = reinterpret_cast<const dpair*>(srcall) + tab.lev[li].off;
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, kr = lane >> 4, cl = lane & 15;
   if (tid < 4 * kM2LOrbits) (&slots[0][0])[tid] = (&orb.slot[q][0][0])[tid];
-  const int64_t col = (lblk >> 2) * 64 + (tid >> 6) * 16 + (lane & 15);
+  const int64_t col = (int64_t)(pb - tab.lev[li].blk0) * (16 * NW) + wv * 16 + cl;
   const int64_t tpos = col / nd;
   const int d = (int)(col - tpos * nd);
-  const int tb = tpos < seg.n ? tlist[seg.s0[q] + tpos] : -1;
+  const int tb = tpos < tab.lev[li].n ? tlist[tab.lev[li].s0[q] + tpos] : -1;
   const int comp = kr & 1, jp = kr >> 1;
-  const T sg = comp ? T(-1) : T(1);
   acc_t acc[4][RTC];
 #pragma unroll
   for (int a = 0; a < 4; ++a)
 #pragma unroll
     for (int r = 0; r < RTC; ++r) acc[a][r] = acc_t{0, 0, 0, 0};
-  // FP32: every orbit's sums are folded into FP64 ones (a long FP32 chain over
+  // FP32: z is formed in FP64 and rounded once, and every orbit's sums are folded into FP64 ones (a long FP32 chain over
   // the orbits doubled the error of hfmm2d, zk 30, eps 1e-6)
   constexpr bool FOLD = sizeof(T) == 4;
   d4v sum[FOLD ? 4 : 1][FOLD ? RTC : 1];
@@ -145,74 +184,124 @@ __global__ __launch_bounds__(256) void k_m2l(int nd, int P, int nblk, int per_xc
     for (int r = 0; r < (FOLD ? RTC : 1); ++r) sum[a][r] = d4v{0, 0, 0, 0};
   double m0 = 0;
   __syncthreads();
-  // the source of the orbit's kr-th rotation
-  auto my_source = [&](int o) {
-    const int sl = slots[o][kr];
-    return (tb >= 0 && sl >= 0) ? s2[(int64_t)kSlots * tb + sl] : -1;
+  // The source of the orbit's kr-th rotation, as the offset of its expansion (-1:
+  // none).  Loads are issued without branches, absent ones to a zero: a branch
+  // around each load made the wavefront wait for its address first.
+  int nextc = 0;
+  auto load_c = [&](int o) {
+    const int sl = o < kM2LOrbits ? slots[o][kr] : -1;
+    nextc = s2[tb >= 0 && sl >= 0 ? (int64_t)kSlots * tb + sl : 0];
   };
-  const T* px[4];
-  auto set_sources = [&](int myc) {
+  auto put_offs = [&](int o) {
+    const int sl = o < kM2LOrbits ? slots[o][kr] : -1;
+    offs[wv][o & 1][cl][kr] =
+        tb >= 0 && sl >= 0 && nextc >= 0 ? ((int64_t)(nextc - box0) * nd + d) * P : -1;
+  };
+  // task `it` of a lane: coefficient jl of column tc of the wavefront's group
+  dpair x[NIT][4];
+  auto load_x = [&](int ob, int g) {
+    int64_t of[NIT][4];
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      const int c = __shfl(myc, (lane & 15) + 16 * k, 64);
-      px[k] = c >= 0 ? src + ((int64_t)(c - sbox0) * nd + d) * 2 * P + comp : nullptr;
+    for (int it = 0; it < NIT; ++it) {
+      const int t = min(it * 64 + lane, 16 * JH - 1), tc = t / JH;
+#pragma unroll
+      for (int k = 0; k < 4; ++k) of[it][k] = offs[wv][ob][tc][k];
+    }
+#pragma unroll
+    for (int it = 0; it < NIT; ++it) {
+      const int t = min(it * 64 + lane, 16 * JH - 1), jl = t % JH;
+      const int j = g * HB + (jl & (HB - 1)) + 4 * (jl / HB);
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const dpair* p = of[it][k] >= 0 && j < P ? src + (of[it][k] + j)
+                                                 : reinterpret_cast<const dpair*>(m2l_zero);
+        x[it][k] = *p;
+      }
     }
   };
-  T v[2][KSC][4];
-  auto load_x = [&](int b, T (&w)[KSC][4]) {
+  auto store_z = [&]() {
 #pragma unroll
-    for (int ks = 0; ks < KSC; ++ks) {
-      const int j = b + 4 * (2 * ks + jp);
-#pragma unroll
-      for (int k = 0; k < 4; ++k) w[ks][k] = (px[k] && j < P) ? px[k][2 * j] : T(0);
+    for (int it = 0; it < NIT; ++it) {
+      const int t = it * 64 + lane, tc = t / JH, jl = t - tc * JH;
+      const int row = (jl & (HB - 1)) * CS + jl / HB;
+      if (16 * JH % 64 == 0 || t < 16 * JH) {
+        const dpair s02{x[it][0].re + x[it][2].re, x[it][0].im + x[it][2].im};
+        const dpair d02{x[it][0].re - x[it][2].re, x[it][0].im - x[it][2].im};
+        const dpair s13{x[it][1].re + x[it][3].re, x[it][1].im + x[it][3].im};
+        const dpair d13{x[it][1].re - x[it][3].re, x[it][1].im - x[it][3].im};
+        zbuf[wv][0][tc][row] = pair_t{(T)(s02.re + s13.re), (T)(s02.im + s13.im)};
+        zbuf[wv][1][tc][row] = pair_t{(T)(d02.re + d13.im), (T)(d02.im - d13.re)};  // - i d13
+        zbuf[wv][2][tc][row] = pair_t{(T)(s02.re - s13.re), (T)(s02.im - s13.im)};
+        zbuf[wv][3][tc][row] = pair_t{(T)(d02.re - d13.im), (T)(d02.im + d13.re)};
+      }
     }
   };
-  T ar[NA];
-  auto load_a = [&](int chunk) {
+  T ar[2][NA];
+  auto load_a = [&](int chunk, T (&r)[NA]) {
     const T* p = A + (int64_t)chunk * CH + tid;
 #pragma unroll
-    for (int i = 0; i < NA; ++i) ar[i] = p[256 * i];
+    for (int i = 0; i < NA; ++i)
+      if (CH % NT == 0 || NT * i + tid < CH) r[i] = p[NT * i];
   };
-  auto store_a = [&](int buf) {
+  auto store_a = [&](int buf, const T (&r)[NA]) {
 #pragma unroll
-    for (int i = 0; i < NA; ++i) abuf[buf][256 * i + tid] = ar[i];
+    for (int i = 0; i < NA; ++i)
+      if (CH % NT == 0 || NT * i + tid < CH) abuf[buf][NT * i + tid] = r[i];
   };
-  set_sources(my_source(0));
-  load_x(0, v[0]);
-  load_a(0);
-  store_a(0);
+  constexpr int NCH = 4 * kM2LOrbits;
+  load_a(0, ar[0]);
+  load_a(1, ar[1]);
+  load_c(0);
+  put_offs(0);
+  load_c(1);
+  wave_lds_fence();
+  load_x(0, 0);
+  store_a(0, ar[0]);
+  store_z();
   __syncthreads();
 #pragma unroll 1
   for (int o = 0; o < kM2LOrbits; ++o) {
-    const int nextc = o + 1 < kM2LOrbits ? my_source(o + 1) : -1;
+    const int ob = o & 1;
+    put_offs(o + 1);
+    wave_lds_fence();
+    load_c(o + 2);
 #pragma unroll
-    for (int b = 0; b < 4; ++b) {
-      constexpr int one = 1;
-      const int cur = b & one;
-      const bool more = b < 3 || o + 1 < kM2LOrbits;
-      if (more) {
-        load_a(4 * o + b + 1);
-        if (b == 3) set_sources(nextc);
-        load_x((b + 1) & 3, v[cur ^ 1]);
-      }
+    for (int g = 0; g < NG; ++g) {
 #pragma unroll
-      for (int ks = 0; ks < KSC; ++ks) {
-        const T s02 = v[cur][ks][0] + v[cur][ks][2], d02 = v[cur][ks][0] - v[cur][ks][2];
-        const T s13 = v[cur][ks][1] + v[cur][ks][3], d13 = v[cur][ks][1] - v[cur][ks][3];
-        const T o13 = sg * __shfl_xor(d13, 16, 64);  // the other component, for -+i d13
-        const T z[4] = {s02 + s13, d02 + o13, s02 - s13, d02 - o13};
-        if (LOGT && b == 0 && ks == 0) m0 += (double)z[0];
-#pragma unroll
-        for (int c = 0; c < 4; ++c) {
-          const int a = (c - SGN * b) & 3;
-#pragma unroll
-          for (int r = 0; r < RTC; ++r)
-            acc[a][r] =
-                Mfma<T>::step(abuf[cur][((ks * 4 + c) * RTC + r) * 64 + lane], z[c], acc[a][r]);
+      for (int u = 0; u < HB; ++u) {
+        constexpr int one = 1;
+        const int b = g * HB + u, cur = b & one, chunk = 4 * o + b;
+        if (chunk + 2 < NCH) load_a(chunk + 2, ar[cur]);
+        // the next group's rows (past the last orbit: none), after
+        // the operator's loads: loads return in order, and the rows come from
+        // farther away
+        if (u == 0) {
+          if (g + 1 < NG) load_x(ob, g + 1);
+          else load_x(ob ^ 1, 0);
         }
+#pragma unroll
+        for (int ks = 0; ks < KSC; ++ks) {
+          T z[4];
+#pragma unroll
+          for (int c = 0; c < 4; ++c) {
+            const pair_t* zp = &zbuf[wv][c][cl][u * CS + 2 * ks + jp];
+            z[c] = reinterpret_cast<const T*>(zp)[comp];
+          }
+          if (LOGT && b == 0 && ks == 0) m0 += (double)z[0];
+#pragma unroll
+          for (int c = 0; c < 4; ++c) {
+            const int a = (c - SGN * b) & 3;
+#pragma unroll
+            for (int r = 0; r < RTC; ++r)
+              acc[a][r] = Mfma<T>::step(abuf[cur][((ks * 4 + c) * RTC + r) * 64 + lane], z[c],
+                                        acc[a][r]);
+          }
+        }
+        if (chunk + 1 < NCH) store_a(cur ^ 1, ar[cur ^ 1]);
+        __syncthreads();
       }
-      if (more) store_a(cur ^ 1);
-      __syncthreads();
+      store_z();
+      wave_lds_fence();
     }
     if constexpr (FOLD) {
 #pragma unroll
@@ -228,7 +317,8 @@ __global__ __launch_bounds__(256) void k_m2l(int nd, int P, int nblk, int per_xc
   if (tb < 0) return;
   const int lev = ilevel[tb];
   const int2 bd = band ? band[lev] : int2{0, 2 * P};
-  double* L = reinterpret_cast<double*>(dst + ((int64_t)(tb - dbox0) * nd + d) * P);
+  double* L = reinterpret_cast<double*>(dstall + tab.lev[li].off +
+                                        ((int64_t)(tb - box0) * nd + d) * P);
   // the level-dependent part log(boxsize) M_0 of L_0: lanes 0..15 hold the
   // sources' sum of Re M_0, lanes 16..31 of Im M_0
   const double lm = (LOGT && lane < 32) ? logr[lev] * m0 : 0.0;
@@ -248,39 +338,52 @@ __global__ __launch_bounds__(256) void k_m2l(int nd, int P, int nblk, int per_xc
   if (LOGT && lane < 32) L[kr] += lm;
 }
 
-// One M2L launch.  fp32: operators and sources are float (an orbit's sums FP32).  P <= kM2LMaxP.
+// The M2L of the given levels (blk0 is set here), one launch per tile shape.
+// fp32: operators and z are float (an orbit's sums FP32).  Every P <= kM2LMaxP;
+// src and dst hold P values per (box, density) at the levels' off.
 template <int SGN, int LOGT>
-inline void launch_m2l(int nd, int P, const M2LSeg& seg, const int* tlist, const int* s2,
-                       const void* A, int sbox0, int dbox0, const int* ilevel, const int2* band,
-                       const double* logr, const void* src, cplx* dst, bool fp32,
-                       hipStream_t st) {
-  if (seg.n <= 0) return;
+inline void launch_m2l(int nd, const std::vector<M2LLev>& levels, const int* tlist, const int* s2,
+                       const void* A, const int* ilevel, const int2* band, const double* logr,
+                       const cplx* src, cplx* dst, bool fp32, hipStream_t st) {
   const M2LSlots orb = m2l_orbit_slots();
-  const int64_t nblk = ((int64_t)seg.n * nd + 63) / 64;
-  const int per_xcd = (int)((4 * nblk + 7) / 8);
-#define FMM2D_M2L(T, RTC, KSC)                                                                  \
-  hipLaunchKernelGGL((k_m2l<T, RTC, KSC, SGN, LOGT>), dim3((unsigned)(8 * per_xcd)), dim3(256), \
-                     0, st, nd, P, (int)nblk, per_xcd, seg, tlist, s2, orb,                     \
-                     static_cast<const T*>(A), sbox0, dbox0, ilevel, band, logr,                \
-                     static_cast<const T*>(src), dst)
-#define FMM2D_M2L_K(T)                \
-  switch (m2l_ksc(P)) {               \
-    case 2: FMM2D_M2L(T, 1, 2); break; \
-    case 3: FMM2D_M2L(T, 1, 3); break; \
-    case 4: FMM2D_M2L(T, 1, 4); break; \
-    case 5: FMM2D_M2L(T, 2, 5); break; \
-    case 6: FMM2D_M2L(T, 2, 6); break; \
-    case 7: FMM2D_M2L(T, 2, 7); break; \
-    default: FMM2D_M2L(T, 2, 8); break; \
+  for (int ksc = 2; ksc <= 8; ++ksc) {
+    const int nw = (!fp32 && ksc == 5) ? 8 : 4;
+    M2LTab tab{};
+    for (const M2LLev& v : levels) {
+      if (m2l_ksc(v.P) != ksc || v.n <= 0) continue;
+      if (tab.nlev == kM2LMaxLev) throw HipError{hipErrorInvalidValue, "m2l levels"};
+      M2LLev& t = tab.lev[tab.nlev++];
+      t = v;
+      t.blk0 = tab.nblk;
+      tab.nblk += (int)(((int64_t)v.n * nd + 16 * nw - 1) / (16 * nw));
+    }
+    if (tab.nlev == 0) continue;
+    const int per_xcd = (int)((4 * (int64_t)tab.nblk + 7) / 8);
+#define FMM2D_M2L(T, RTC, KSC, HB, NW)                                                         \
+  hipLaunchKernelGGL((k_m2l<T, RTC, KSC, HB, NW, SGN, LOGT>), dim3((unsigned)(8 * per_xcd)),   \
+                     dim3(64 * NW), 0, st, nd, per_xcd, tab, tlist, s2, orb,                   \
+                     static_cast<const T*>(A), ilevel, band, logr, src, dst)
+// 8 wavefronts share the operators where their z fits the LDS beside them and
+// 4 would leave one wavefront per SIMD (33 to 40 coefficients, FP64)
+#define FMM2D_M2L_K(T, NW5)                   \
+  switch (ksc) {                              \
+    case 2: FMM2D_M2L(T, 1, 2, 2, 4); break;  \
+    case 3: FMM2D_M2L(T, 1, 3, 2, 4); break;  \
+    case 4: FMM2D_M2L(T, 1, 4, 2, 4); break;  \
+    case 5: FMM2D_M2L(T, 2, 5, 1, NW5); break; \
+    case 6: FMM2D_M2L(T, 2, 6, 1, 4); break;  \
+    case 7: FMM2D_M2L(T, 2, 7, 1, 4); break;  \
+    default: FMM2D_M2L(T, 2, 8, 1, 4); break; \
   }
-  if (fp32) {
-    FMM2D_M2L_K(float)
-  } else {
-    FMM2D_M2L_K(double)
-  }
+    if (fp32) {
+      FMM2D_M2L_K(float, 4)
+    } else {
+      FMM2D_M2L_K(double, 8)
+    }
 #undef FMM2D_M2L_K
 #undef FMM2D_M2L
-  hip_throw(hipGetLastError(), "m2l");
+    hip_throw(hipGetLastError(), "m2l");
+  }
 }
 
 }  // namespace fmm2d
