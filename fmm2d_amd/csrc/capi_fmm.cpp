@@ -416,7 +416,7 @@ int fmm2d_tree_get(void* handle, int* laddr, int* ilevel, int* iparent, int* nch
     }
     if (nlist1) {
       if (!h->have_lists) {
-        build_lists(t, h->l, h->st);
+        build_lists(t, h->l, h->st, true);
         h->have_lists = true;
       }
       const int caps[4] = {kMaxList1, kMaxList2, kMaxList3, kMaxList4};

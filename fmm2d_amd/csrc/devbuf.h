@@ -28,11 +28,25 @@ inline void hip_throw(hipError_t e, const char* what) {
 // at once).  Sizes beyond the limits, or not a multiple of 4, copy and
 // synchronise.
 constexpr size_t kReadbackMax = 4096;
-constexpr size_t kUploadInline = 1024;
+constexpr size_t kUploadInline = 3072;
 void readback(void* dst, const void* src, size_t bytes, hipStream_t st);
 // two pieces in one round trip
 void readback2(void* dst, const void* src, size_t bytes, void* dst2, const void* src2,
                size_t bytes2, hipStream_t st);
+// A readback whose wait comes later: begin queues the store, finish waits for
+// it (the work queued in between keeps the device busy meanwhile).
+struct AsyncRead {
+  void* box = nullptr;
+  size_t n1 = 0, n2 = 0;
+  hipStream_t st = nullptr;
+  bool done = false;
+  AsyncRead() = default;
+  AsyncRead(const AsyncRead&) = delete;
+  AsyncRead& operator=(const AsyncRead&) = delete;
+  ~AsyncRead();
+  void begin(const void* src, size_t bytes, const void* src2, size_t bytes2, hipStream_t s);
+  void finish(void* dst, void* dst2);
+};
 void upload_bytes(void* dst, const void* src, size_t bytes, hipStream_t st);
 
 // Workspace cache (ws.cpp).  ws_alloc returns at least `bytes` bytes usable

@@ -7,6 +7,7 @@
 #pragma once
 
 #include <algorithm>
+#include <cstring>
 #include <vector>
 
 #include "devbuf.h"
@@ -47,23 +48,36 @@ __global__ void k_gather_xy(int64_t n, const int* perm, const double* xy, double
   out[2 * i + 1] = xy[2 * (int64_t)j + 1];
 }
 
-// cfmm2d: densities copied as they are.
-__global__ void k_gather_dens(int64_t n, int nd, const int* perm, const cplx* in, cplx* out) {
+// cfmm2d, hfmm2d: points and densities copied as they are (absent: null).
+__global__ void k_gather_dens(int64_t n, int nd, const int* perm, const double* xy, double* oxy,
+                              const cplx* ch, cplx* och, const cplx* ds, cplx* ods,
+                              const double* dv, double* odv) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
   const int64_t j = perm[i];
-  for (int d = 0; d < nd; ++d) out[i * nd + d] = in[j * nd + d];
+  oxy[2 * i] = xy[2 * j];
+  oxy[2 * i + 1] = xy[2 * j + 1];
+  for (int d = 0; d < nd; ++d) {
+    if (ch) och[i * nd + d] = ch[j * nd + d];
+    if (ds) ods[i * nd + d] = ds[j * nd + d];
+  }
+  if (dv)
+    for (int k = 0; k < 2 * nd; ++k) odv[i * 2 * nd + k] = dv[j * 2 * nd + k];
 }
 
-
-// out[perm[i]] = in[i] for m values per point
-__global__ void k_scatter(int64_t n, int m, const int* perm, const cplx* in, cplx* out) {
+// out[perm[i]] = in[i] for m values per point, potential, gradient and second
+// derivatives (absent: null)
+__global__ void k_scatter(int64_t n, const int* perm, int m0, const cplx* in0, cplx* out0, int m1,
+                          const cplx* in1, cplx* out1, int m2, const cplx* in2, cplx* out2) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
   const int64_t j = perm[i];
-  for (int k = 0; k < m; ++k) out[j * m + k] = in[i * m + k];
+  for (int k = 0; k < m0; ++k) out0[j * m0 + k] = in0[i * m0 + k];
+  if (out1)
+    for (int k = 0; k < m1; ++k) out1[j * m1 + k] = in1[i * m1 + k];
+  if (out2)
+    for (int k = 0; k < m2; ++k) out2[j * m2 + k] = in2[i * m2 + k];
 }
-
 
 // ---------------------------------------------------------- near-field segments
 // The sources a leaf interacts with directly (the boxes of its list 1,
@@ -146,78 +160,56 @@ __device__ __forceinline__ bool m2l_target(int b, const int* ilevel, const int* 
   return ilevel[b] >= 2 && n2[b] > 0 && npts_eval(b, sse, tse, ifpgh, ifpght) > 0;
 }
 
-// flag[p] = 1 if some child of box p is an M2L target
-__global__ void k_m2l_parent_flag(int64_t n, const int* ilevel, const int* nchild,
-                                  const int* ichild, const int* n2, const int* sse,
-                                  const int* tse, int ifpgh, int ifpght, int* flag) {
+// A tree has 1 + 4 np boxes, np of them with children, and the boxes of a level
+// l >= 1 are groups of four siblings: the k-th group of level l + 1 belongs to
+// a non-leaf box of level l, so the groups number the non-leaf boxes level by
+// level (pos[l] = groups of the levels up to l) and no list has to be made.
+constexpr int kPlanLevels = 54;
+struct PlanLevels {
+  int nl;
+  int lstart[kPlanLevels], pos[kPlanLevels];
+};
+
+// For the non-leaf box of group i: its id (list), the child slots of M2M (up: a
+// child without sources is skipped, laprouts2d.f via cfmm2d.f:962-983) and
+// L2L (down: all children when the parent has points to evaluate,
+// cfmm2d.f:1042-1076), and the child in position q if it is an M2L target
+// (tl[q np + i], else -1): siblings sit at the same position of the four
+// classes.  With p2l, also the boxes with list-4 work, in any order (their
+// number in *np2l, zero before).
+__global__ void k_plan(int64_t nb, int np, PlanLevels T, const int* iparent, const int* ilevel,
+                       const int* n2, const int* n4, const int* sse, const int* tse, int ifpgh,
+                       int ifpght, int* list, int* up, int* down, int* tl, int* p2l,
+                       int* np2l) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  int f = 0;
-  if (nchild[i] > 0)
+  if (i < np) {
+    int l = 0;
+    while (l + 1 < T.nl && T.pos[l + 1] <= i) ++l;
+    const int c0 = T.lstart[l + 1] + 4 * ((int)i - T.pos[l]);
+    const int b = iparent[c0];
+    const bool ev = npts_eval(b, sse, tse, ifpgh, ifpght) > 0;
+    list[i] = b;
+#pragma unroll
     for (int q = 0; q < 4; ++q) {
-      const int c = ichild[4 * i + q];
-      if (c >= 0 && m2l_target(c, ilevel, n2, sse, tse, ifpgh, ifpght)) f = 1;
+      const int c = c0 + q;
+      up[4 * i + q] = (sse[2 * c + 1] > sse[2 * c]) ? c : -1;
+      down[4 * i + q] = ev ? c : -1;
+      tl[(int64_t)q * np + i] = m2l_target(c, ilevel, n2, sse, tse, ifpgh, ifpght) ? c : -1;
     }
-  flag[i] = f;
-}
-
-// *total = flags set in flag[0..n), from its exclusive scan pos
-// out[pos[i]] = i for every flagged i (pos = exclusive scan of flag)
-__global__ void k_compact_flagged(int64_t n, const int* flag, const int* pos, int* out) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n && flag[i]) out[pos[i]] = (int)i;
-}
-
-// tlist[q * np + k] = child q of parent plist[k] if an M2L target, else -1
-__global__ void k_m2l_aligned(int64_t np, const int* plist, const int* ilevel, const int* ichild,
-                              const int* n2, const int* sse, const int* tse, int ifpgh,
-                              int ifpght, int* tlist) {
-  const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= np) return;
-  const int p = plist[k];
-  for (int q = 0; q < 4; ++q) {
-    const int c = ichild[4 * p + q];
-    tlist[q * np + k] =
-        (c >= 0 && m2l_target(c, ilevel, n2, sse, tse, ifpgh, ifpght)) ? c : -1;
+  }
+  if (p2l) {
+    const bool f = i < nb && ilevel[i] >= 2 && n4[i] > 0 &&
+                   npts_eval((int)i, sse, tse, ifpgh, ifpght) > 0;
+    const unsigned long long m = __ballot(f);
+    if (m) {
+      const int lane = threadIdx.x & 63, first = __ffsll((long long)m) - 1;
+      int at = 0;
+      if (lane == first) at = atomicAdd(np2l, __popcll(m));
+      at = __builtin_amdgcn_readlane(at, first);
+      if (f) p2l[at + __popcll(m & ((1ull << lane) - 1ull))] = (int)i;
+    }
   }
 }
-
-// Non-leaf boxes (in box order, hence level order) and their 4-child slots for
-// M2M (a child without sources is skipped, laprouts2d.f via cfmm2d.f:962-983)
-// and L2L (all children when the parent has points to evaluate, cfmm2d.f:1042-1076).
-__global__ void k_nonleaf_flag(int64_t n, const int* nchild, int* flag) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  flag[i] = nchild[i] > 0 ? 1 : 0;
-}
-
-__global__ void k_child_slots(int64_t n, const int* list, const int* ichild, const int* sse,
-                              const int* tse, int ifpgh, int ifpght, int* up, int* down) {
-  const int64_t pos = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (pos >= n) return;
-  const int b = list[pos];
-  const bool ev = npts_eval(b, sse, tse, ifpgh, ifpght) > 0;
-  for (int qq = 0; qq < 4; ++qq) {
-    const int c = ichild[4 * b + qq];
-    up[pos * 4 + qq] = (sse[2 * c + 1] > sse[2 * c]) ? c : -1;
-    down[pos * 4 + qq] = ev ? c : -1;
-  }
-}
-
-// out[l] = first position of list (sorted) at or beyond lstart[l], one thread
-// per l (launch >= nl + 2 threads)
-__global__ void k_level_bounds(const int* list, int n, const int* lstart, int nl, int* out) {
-  const int l = blockIdx.x * blockDim.x + threadIdx.x;
-  if (l > nl + 1) return;
-  int lo = 0, hi = n;
-  while (lo < hi) {
-    const int mid = (lo + hi) / 2;
-    if (list[mid] < lstart[l]) lo = mid + 1;
-    else hi = mid;
-  }
-  out[l] = lo;
-}
-
 
 // ---------------------------------------------------------- work counters
 // cnt[0] near pairs, [1] list-2 pairs, [2] M2M edges, [3] L2L edges,
@@ -283,7 +275,8 @@ struct Timer {
   void mark(int s) {
     if (!on) return;
     hipEvent_t e;
-    (void)hipEventCreate(&e);
+    // (without the system-scope fence of the default: 2.7 us a mark, not 4)
+    (void)hipEventCreateWithFlags(&e, hipEventDisableSystemFence);
     (void)hipEventRecord(e, st);
     ev.push_back(e);
     slot.push_back(s);
@@ -306,91 +299,57 @@ struct Timer {
 };
 
 
-// Non-leaf boxes level by level with their child slots: up[4 pos + q] is
-// child q if it holds sources (M2M input), down[4 pos + q] is child q if the
-// parent has points to evaluate (L2L output).  list[lev_pos[l] .. lev_pos[l+1])
-// are the non-leaf boxes of level l.
-struct ChildPlan {
-  DBuf<int> list, up, down;
+// The work lists of k_plan.  list[lev_pos[l] .. lev_pos[l+1]) are the non-leaf
+// boxes of level l; the M2L targets of level l in child position q are tl[q np
+// + lev_pos[l-1] .. q np + lev_pos[l]).
+struct BoxPlan {
+  DBuf<int> list, up, down, tl, p2l;
   std::vector<int> lev_pos;
-};
-
-void plan_children(const Tree& t, int pg, int pgt, ChildPlan& cp, hipStream_t st) {
-  const int nb = t.nboxes, nl = t.nlevels;
-  cp.list.alloc(nb, st);
-  cp.lev_pos.assign(nl + 2, 0);
-  DBuf<int> flag(nb, st), cnt(1, st), dlb(nl + 2, st);
-  launch1d(k_nonleaf_flag, nb, st, t.nchild.p, flag.p);
-  {
-    // stream compaction of the flagged box ids (exclusive scan, then scatter)
-    DBuf<int> pos(nb, st);
-    exclusive_scan(flag.p, pos.p, nb, cnt.p, st);
-    launch1d(k_compact_flagged, nb, st, (const int*)flag.p, (const int*)pos.p, cp.list.p);
-  }
-  int nnl = 0;
-  readback(&nnl, cnt.p, sizeof(int), st);
-  std::vector<int> lsx(t.lstart);
-  lsx.push_back(nb);
-  DBuf<int> d_lsx = upload(lsx, st);
-  if (nl + 2 > 64) throw HipError{hipErrorInvalidValue, "tree levels beyond 62"};
-  hipLaunchKernelGGL(k_level_bounds, dim3(1), dim3(64), 0, st, cp.list.p, nnl, d_lsx.p, nl,
-                     dlb.p);
-  cp.up.alloc(4 * (size_t)std::max(nnl, 1), st);
-  cp.down.alloc(4 * (size_t)std::max(nnl, 1), st);
-  launch1d(k_child_slots, nnl, st, cp.list.p, t.ichild.p, t.isrcse.p, t.itargse.p, pg, pgt,
-           cp.up.p, cp.down.p);
-  readback(cp.lev_pos.data(), dlb.p, sizeof(int) * (nl + 2), st);
-}
-
-// seg[q * (nl + 2) + l]: first position in tlist of class q at level >= l
-// M2L targets (level >= 2, non-empty list 2, points to evaluate) by child
-// position q (their sources per offset slot are Lists::s2).  The classes are
-// aligned by parent: entry k of class q is the q-th child of the k-th parent
-// with an M2L target among its children (parents in box order), or -1 when
-// that child is no target -- so sibling targets, whose list-2 sources are
-// mostly the same boxes, sit at the same position of the four classes (few
-// entries are -1: a refined box's children nearly always all hold points).
-// cls_seg[q] .. cls_seg[q+1] is class q, and lev_seg[q][l] .. lev_seg[q][l+1]
-// its part at level l.
-struct M2LPlan {
-  DBuf<int> tlist;
-  int cls_seg[5] = {0, 0, 0, 0, 0};
-  std::vector<int> lev_seg;  // 4 x (nl + 2)
-  int ntg = 0;
-  int lev(int q, int l, int nl) const { return lev_seg[(size_t)q * (nl + 2) + l]; }
-};
-
-void plan_m2l(const Tree& t, const Lists& L, int pg, int pgt, M2LPlan& mp, hipStream_t st) {
-  const int nb = t.nboxes, nl = t.nlevels;
-  DBuf<int> flag(nb, st), pos(nb + 1, st), cnt(1, st);
-  launch1d(k_m2l_parent_flag, nb, st, t.ilevel.p, t.nchild.p, t.ichild.p, L.n2.p, t.isrcse.p,
-           t.itargse.p, pg, pgt, flag.p);
-  exclusive_scan(flag.p, pos.p, nb, cnt.p, st);
   int np = 0;
-  readback(&np, cnt.p, sizeof(int), st);
-  DBuf<int> plist(std::max(np, 1), st);
-  launch1d(k_compact_flagged, nb, st, (const int*)flag.p, (const int*)pos.p, plist.p);
-  mp.tlist.alloc(4 * (size_t)std::max(np, 1), st);
-  launch1d(k_m2l_aligned, np, st, plist.p, t.ilevel.p, t.ichild.p, L.n2.p, t.isrcse.p,
-           t.itargse.p, pg, pgt, mp.tlist.p);
-  // targets of level l are children of parents of level l - 1: their rows
-  // start at the first parent at or beyond lstart[l - 1]
-  std::vector<int> lsx(nl + 2, 0);
-  for (int l = 1; l <= nl + 1; ++l) lsx[l] = (l - 1 <= nl) ? t.lstart[l - 1] : nb;
-  lsx[0] = 0;
-  DBuf<int> d_lsx = upload(lsx, st);
-  DBuf<int> dlb(nl + 2, st);
-  if (nl + 2 > 64) throw HipError{hipErrorInvalidValue, "tree levels beyond 62"};
-  hipLaunchKernelGGL(k_level_bounds, dim3(1), dim3(64), 0, st, plist.p, np, d_lsx.p, nl,
-                     dlb.p);
-  std::vector<int> lb(nl + 2, 0);
-  readback(lb.data(), dlb.p, sizeof(int) * lb.size(), st);
-  for (int q = 0; q <= 4; ++q) mp.cls_seg[q] = q * np;
-  mp.lev_seg.assign(4 * (size_t)(nl + 2), 0);
-  for (int q = 0; q < 4; ++q)
-    for (int l = 0; l <= nl + 1; ++l) mp.lev_seg[(size_t)q * (nl + 2) + l] = q * np + lb[l];
-  mp.ntg = 4 * np;
+};
+
+// np2l: a zeroed device counter, or null when the list-4 boxes are not needed
+void plan_boxes(const Tree& t, const Lists& L, int pg, int pgt, BoxPlan& bp, int* np2l,
+                hipStream_t st) {
+  const int nb = t.nboxes, nl = t.nlevels;
+  PlanLevels T{};
+  T.nl = nl;
+  if (nl + 2 > kPlanLevels) throw HipError{hipErrorInvalidValue, "tree levels"};
+  bp.lev_pos.assign(nl + 2, 0);
+  for (int l = 0; l <= nl; ++l) {
+    T.lstart[l] = t.lstart[l];
+    T.pos[l] = bp.lev_pos[l];
+    const int next = l < nl ? (l + 1 < nl ? t.lstart[l + 2] : nb) - t.lstart[l + 1] : 0;
+    bp.lev_pos[l + 1] = bp.lev_pos[l] + next / 4;
+  }
+  bp.np = bp.lev_pos[nl + 1];
+  const size_t np = (size_t)std::max(bp.np, 1);
+  bp.list.alloc(np, st);
+  bp.up.alloc(4 * np, st);
+  bp.down.alloc(4 * np, st);
+  bp.tl.alloc(4 * np, st);
+  if (np2l) bp.p2l.alloc(nb, st);
+  launch1d(k_plan, nb, st, bp.np, T, t.iparent.p, t.ilevel.p, L.n2.p, L.n4.p, t.isrcse.p,
+           t.itargse.p, pg, pgt, bp.list.p, bp.up.p, bp.down.p, bp.tl.p, bp.p2l.p, np2l);
 }
+
+// Several small host arrays in one upload.
+struct Blob {
+  std::vector<unsigned> w;
+  DBuf<unsigned> d;
+  template <typename T> size_t add(const std::vector<T>& v) {
+    static_assert(sizeof(T) % 4 == 0, "whole words");
+    const size_t at = (w.size() + 3) & ~size_t(3);
+    w.resize(at + v.size() * (sizeof(T) / 4), 0u);
+    if (!v.empty()) std::memcpy(w.data() + at, v.data(), v.size() * sizeof(T));
+    return at;
+  }
+  void upload(hipStream_t st) {
+    d.alloc(w.size(), st);
+    upload_bytes(d.p, w.data(), 4 * w.size(), st);
+  }
+  template <typename T> T* at(size_t off) const { return reinterpret_cast<T*>(d.p + off); }
+};
 
 // slot -> offset index (dx+3)*7 + (dy+3) for each child position q
 std::vector<int> m2l_slot_offsets() {

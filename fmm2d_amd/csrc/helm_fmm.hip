@@ -145,15 +145,6 @@ __device__ void scaled_h(cplx z, double s, int m, cplx* out) {
   }
 }
 
-// ---------------------------------------------------------- gathers
-__global__ void k_gather_dipvec(int64_t n, int nd, const int* perm, const double* in,
-                                double* out) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const int64_t j = perm[i];
-  for (int k = 0; k < 2 * nd; ++k) out[i * 2 * nd + k] = in[j * 2 * nd + k];
-}
-
 // ---------------------------------------------------------- P2M / P2L
 // The cylinder functions of each source (J/s^n about its leaf's centre for
 // P2M, H s^n about the target box's centre for P2L) are computed first, one
@@ -264,7 +255,7 @@ __global__ __launch_bounds__(kW) void k_hp2m_g(int nd, cplx zk, const HLev* lev,
 // a box b that takes list-4 work, 0 otherwise.
 __global__ void k_hp2l_count(int64_t nb, const HLev* lev, const int* ilevel, const int* n4,
                              const int* l4, const int* sse, const int* tse, int ifpgh,
-                             int ifpght, int* cnt) {
+                             int ifpght, int* cnt, int64_t* len) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= nb) return;
   const int b = (int)i;
@@ -276,14 +267,7 @@ __global__ void k_hp2l_count(int64_t nb, const HLev* lev, const int* ilevel, con
       s += sse[2 * c + 1] - sse[2 * c];
     }
   cnt[b] = s;
-}
-
-// Row storage of a box's pairs: cnt[b] rows of p+2 values of b's level.
-__global__ void k_hp2l_rowlen(int64_t nb, const HLev* lev, const int* ilevel, const int* cnt,
-                              int64_t* len) {
-  const int64_t b = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (b >= nb) return;
-  len[b] = (int64_t)cnt[b] * (lev[ilevel[b]].p + 2);
+  len[b] = (int64_t)s * (lev[l].p + 2);  // row storage of the box's pairs
 }
 
 // One thread per (box b, list-4 source j) pair t, pairs numbered box after
@@ -479,6 +463,7 @@ __device__ void eval_mpole(const Deriv& D, cplx z, double s, cplx w, cplx* res) 
 // One thread per evaluation point: local expansion of its leaf and
 // multipoles of the leaf's list-3 boxes (hfmm2d.f:1310-1520).
 template <int PG>
+// (the first to write the sorted outputs: they are assigned, the near field adds)
 __global__ __launch_bounds__(256) void k_heval(int64_t n, int nd, cplx zk, const HLev* lev, const double* xy,
                         const int* leaf, const int* ilevel, const double* centers, const int* n3,
                         const int* l3, const cplx* mp, const cplx* loc, cplx* pot, cplx* grad,
@@ -512,15 +497,15 @@ __global__ __launch_bounds__(256) void k_heval(int64_t n, int nd, cplx zk, const
       const Deriv D{hexp(mp, Lc, c, nd, d), Lc.p, 0.5 * zk, Lc.s, 1.0 / Lc.s, -1};
       eval_mpole<PG>(D, zk * r, Lc.s, w, res);
     }
-    pot[i * nd + d] += ik4 * res[0];
+    pot[i * nd + d] = ik4 * res[0];
     if (PG >= 2) {
-      grad[(2 * i) * nd + d] += ik4 * res[1];
-      grad[(2 * i + 1) * nd + d] += ik4 * res[2];
+      grad[(2 * i) * nd + d] = ik4 * res[1];
+      grad[(2 * i + 1) * nd + d] = ik4 * res[2];
     }
     if (PG >= 3) {
-      hess[(3 * i) * nd + d] += ik4 * res[3];
-      hess[(3 * i + 1) * nd + d] += ik4 * res[4];
-      hess[(3 * i + 2) * nd + d] += ik4 * res[5];
+      hess[(3 * i) * nd + d] = ik4 * res[3];
+      hess[(3 * i + 1) * nd + d] = ik4 * res[4];
+      hess[(3 * i + 2) * nd + d] = ik4 * res[5];
     }
   }
 }
@@ -614,15 +599,15 @@ __global__ __launch_bounds__(kHEvB) void k_heval_b(int64_t n, cplx zk, const HLe
     eval_local<PG>(D, zk * r, Lb.s, w, res);
   }
   const cplx ik4 = cplx{0.0, 0.25};
-  pot[i] += ik4 * res[0];
+  pot[i] = ik4 * res[0];
   if (PG >= 2) {
-    grad[2 * i] += ik4 * res[1];
-    grad[2 * i + 1] += ik4 * res[2];
+    grad[2 * i] = ik4 * res[1];
+    grad[2 * i + 1] = ik4 * res[2];
   }
   if (PG >= 3) {
-    hess[3 * i] += ik4 * res[3];
-    hess[3 * i + 1] += ik4 * res[4];
-    hess[3 * i + 2] += ik4 * res[5];
+    hess[3 * i] = ik4 * res[3];
+    hess[3 * i + 1] = ik4 * res[4];
+    hess[3 * i + 2] = ik4 * res[5];
   }
 }
 
@@ -1305,8 +1290,8 @@ void helm_box_passes(const Tree& t, const Lists& L, const std::vector<HLev>& lev
   if (mixed) launch1d(k_to_f32, T.af_total, st, (const double*)d_af.p, af32.p);
   tm.mark(12);
 
-  ChildPlan cp;
-  plan_children(t, pg, pgt, cp, st);
+  BoxPlan bp;
+  plan_boxes(t, L, pg, pgt, bp, nullptr, st);
   DBuf<int> d_op4 = upload(std::vector<int>{0, 1, 2, 3}, st);
   // ---- step 3: M2M, finest parents first (hfmm2d.f:1021-1100)
   for (int l = nl - 1; l >= 1; --l) {
@@ -1315,15 +1300,13 @@ void helm_box_passes(const Tree& t, const Lists& L, const std::vector<HLev>& lev
     launch_translate(0, 0, nd,
                      TrBufs{mpp + C.off, C.box0, 2 * C.p + 1, mpp + P.off, P.box0,
                             2 * P.p + 1},
-                     4, {TrGroup{cp.lev_pos[l], cp.lev_pos[l + 1], 0, 0}}, cp.list.p, cp.up.p,
+                     4, {TrGroup{bp.lev_pos[l], bp.lev_pos[l + 1], 0, 0}}, bp.list.p, bp.up.p,
                      d_op4.p, opptr(op_m2m[l]), t.ilevel.p, nullptr, nullptr, st);
   }
   tm.mark(2);
   // ---- step 4: M2L level by level, targets grouped by child position
   {
-    M2LPlan m2l;
-    plan_m2l(t, L, pg, pgt, m2l, st);
-    if (m2l.ntg > 0) {
+    if (bp.np > 0) {
       DBuf<int> d_soff;  // offset slots of the levels that k_translate takes
       // FP32 copy of the multipoles of the levels that k_translate takes, the
       // coarse ones (mixed precision)
@@ -1342,8 +1325,8 @@ void helm_box_passes(const Tree& t, const Lists& L, const std::vector<HLev>& lev
         const int Pl = 2 * V.p + 1;
         if (Pl <= kM2LMaxP) {
           M2LLev v{};
-          for (int q = 0; q < 4; ++q) v.s0[q] = m2l.lev(q, l, nl);
-          v.n = m2l.lev(0, l + 1, nl) - v.s0[0];
+          for (int q = 0; q < 4; ++q) v.s0[q] = q * bp.np + bp.lev_pos[l - 1];
+          v.n = bp.lev_pos[l] - bp.lev_pos[l - 1];
           v.P = Pl;
           v.box0 = V.box0;
           v.off = V.off;
@@ -1354,22 +1337,23 @@ void helm_box_passes(const Tree& t, const Lists& L, const std::vector<HLev>& lev
         if (!d_soff.p) d_soff = upload(m2l_slot_offsets(), st);
         std::vector<TrGroup> groups;
         for (int q = 0; q < 4; ++q)
-          groups.push_back(TrGroup{m2l.lev(q, l, nl), m2l.lev(q, l + 1, nl), 0, q});
+          groups.push_back(
+              TrGroup{q * bp.np + bp.lev_pos[l - 1], q * bp.np + bp.lev_pos[l], 0, q});
         if (mixed)
           launch_translate(0, 0, nd,
                            TrBufs{mp32.p + 2 * V.off, V.box0, 2 * V.p + 1, locp + V.off,
                                   V.box0, 2 * V.p + 1},
-                           kSlots, groups, m2l.tlist.p, L.s2.p, d_soff.p,
+                           kSlots, groups, bp.tl.p, L.s2.p, d_soff.p,
                            af32.p + T.desc[op_m2l[l]].af, t.ilevel.p, nullptr, nullptr, st,
                            true, true, true);
         else
           launch_translate(0, 0, nd,
                            TrBufs{mpp + V.off, V.box0, 2 * V.p + 1, locp + V.off, V.box0,
                                   2 * V.p + 1},
-                           kSlots, groups, m2l.tlist.p, L.s2.p, d_soff.p, opptr(op_m2l[l]),
+                           kSlots, groups, bp.tl.p, L.s2.p, d_soff.p, opptr(op_m2l[l]),
                            t.ilevel.p, nullptr, nullptr, st, false, true, true);
       }
-      launch_m2l<-1, 0>(nd, orbit_levels, m2l.tlist.p, L.s2.p,
+      launch_m2l<-1, 0>(nd, orbit_levels, bp.tl.p, L.s2.p,
                         mixed ? (const void*)af32.p : (const void*)d_af.p, t.ilevel.p, nullptr,
                         nullptr, mpp, locp, mixed, st);
       tm.mark(13);  // the M2L kernels alone
@@ -1383,8 +1367,8 @@ void helm_box_passes(const Tree& t, const Lists& L, const std::vector<HLev>& lev
     launch_translate(1, 0, nd,
                      TrBufs{locp + P.off, P.box0, 2 * P.p + 1, locp + C.off, C.box0,
                             2 * C.p + 1},
-                     4, {TrGroup{cp.lev_pos[l], cp.lev_pos[l + 1], 0, 0}}, cp.list.p,
-                     cp.down.p, d_op4.p, opptr(op_l2l[l]), t.ilevel.p, nullptr, nullptr, st);
+                     4, {TrGroup{bp.lev_pos[l], bp.lev_pos[l + 1], 0, 0}}, bp.list.p,
+                     bp.down.p, d_op4.p, opptr(op_l2l[l]), t.ilevel.p, nullptr, nullptr, st);
   }
   tm.mark(4);
 }
@@ -1459,44 +1443,52 @@ int helmholtz_fmm(const HelmArgs& a, hipStream_t st) {
       const int nbl = ((l < nl) ? t.lstart[l + 1] : nb) - t.lstart[l];
       ncoef += (int64_t)nbl * nd * (2 * nterms[l] + 1);
     }
-    DBuf<HLev> d_lev = upload(lev, st);
+    Blob blob;
+    const size_t b_lev = blob.add(lev);
+    blob.upload(st);
+    const HLev* d_lev = blob.at<HLev>(b_lev);
 
     // ---- sort and gather
     DBuf<double> xs(2 * ns, st), xt(2 * std::max<int64_t>(nt, 1), st);
     DBuf<cplx> chs(a.ifcharge ? ns * nd : 1, st), dps(a.ifdipole ? ns * nd : 1, st);
     DBuf<double> dvs(a.ifdipole ? 2 * ns * nd : 2, st);
-    launch1d(k_gather_xy, ns, st, t.isrc.p, a.src, xs.p);
+    launch1d(k_gather_dens, ns, st, nd, t.isrc.p, a.src, xs.p, a.ifcharge ? a.charge : nullptr, chs.p,
+             a.ifdipole ? a.dipstr : nullptr, dps.p, a.ifdipole ? a.dipvec : nullptr, dvs.p);
     if (nt > 0) launch1d(k_gather_xy, nt, st, t.itarg.p, a.targ, xt.p);
-    if (a.ifcharge) launch1d(k_gather_dens, ns, st, nd, t.isrc.p, a.charge, chs.p);
-    if (a.ifdipole) {
-      launch1d(k_gather_dens, ns, st, nd, t.isrc.p, a.dipstr, dps.p);
-      launch1d(k_gather_dipvec, ns, st, nd, t.isrc.p, a.dipvec, dvs.p);
-    }
-    DBuf<cplx> mp(ncoef, st), loc(ncoef, st);
-    mp.zero();
-    loc.zero();
+    DBuf<cplx> expan(2 * ncoef, st);  // multipoles, locals
+    expan.zero();
+    const struct {
+      cplx* p;
+    } mp{expan.p}, loc{expan.p + ncoef};
     const int pg = a.ifpgh, pgt = a.ifpghtarg;
     DBuf<cplx> ps(pg >= 1 ? ns * nd : 1, st), gs(pg >= 2 ? 2 * ns * nd : 1, st),
         hs(pg >= 3 ? 3 * ns * nd : 1, st);
     DBuf<cplx> pt(pgt >= 1 ? nt * nd : 1, st), gt(pgt >= 2 ? 2 * nt * nd : 1, st),
         ht(pgt >= 3 ? 3 * nt * nd : 1, st);
-    ps.zero(); gs.zero(); hs.zero(); pt.zero(); gt.zero(); ht.zero();
     tm.mark(9);
 
     const int* sse = t.isrcse.p;
     const int* tse = t.itargse.p;
+    // sizes of the rows of P2M and list 4, in one round trip
+    DBuf<int64_t> roff(ns, st), roff4(nb, st), rtot(2, st);
+    DBuf<int> cnt4(nb, st), off4(nb, st), tot4(1, st);
+    launch1d(k_hp2m_rowlen, ns, st, d_lev, t.leaf_s.p, t.ilevel.p, roff.p);
+    exclusive_scan(roff.p, roff.p, ns, rtot.p, st);
+    launch1d(k_hp2l_count, nb, st, d_lev, t.ilevel.p, L.n4.p, L.l4.p, sse, tse, pg, pgt, cnt4.p,
+             roff4.p);
+    exclusive_scan(cnt4.p, off4.p, nb, tot4.p, st);
+    exclusive_scan(roff4.p, roff4.p, nb, rtot.p + 1, st);
+    int64_t hrow[2] = {0, 0};
+    int np4 = 0;
+    readback2(hrow, rtot.p, sizeof(hrow), &np4, tot4.p, sizeof(int), st);
+    const int64_t nrow = hrow[0], nrow4 = hrow[1];
     // ---- step 1: P2M (rows of the sources, then their sums per leaf)
     {
-      DBuf<int64_t> roff(ns, st), rtot(1, st);
-      launch1d(k_hp2m_rowlen, ns, st, d_lev.p, t.leaf_s.p, t.ilevel.p, roff.p);
-      exclusive_scan(roff.p, roff.p, ns, rtot.p, st);
-      int64_t nrow = 0;
-      readback(&nrow, rtot.p, sizeof(int64_t), st);
       DBuf<cplx> gJ(std::max<int64_t>(nrow, 1), st), uJ(ns, st);
-      launch1d(k_hp2m_rows, ns, st, zk, d_lev.p, t.leaf_s.p, t.ilevel.p, t.centers.p, xs.p,
+      launch1d(k_hp2m_rows, ns, st, zk, d_lev, t.leaf_s.p, t.ilevel.p, t.centers.p, xs.p,
                (const int64_t*)roff.p, gJ.p, uJ.p);
 #define FMM2D_P2M(C, D)                                                                       \
-  hipLaunchKernelGGL((k_hp2m_g<C, D>), dim3(nb), dim3(kW), 0, st, nd, zk, d_lev.p, t.ilevel.p, \
+  hipLaunchKernelGGL((k_hp2m_g<C, D>), dim3(nb), dim3(kW), 0, st, nd, zk, d_lev, t.ilevel.p, \
                      t.nchild.p, sse, (const int64_t*)roff.p, gJ.p, uJ.p, chs.p, dps.p, dvs.p,  \
                      mp.p)
       if (a.ifcharge && !a.ifdipole) FMM2D_P2M(1, 0);
@@ -1508,23 +1500,12 @@ int helmholtz_fmm(const HelmArgs& a, hipStream_t st) {
     tm.mark(0);
     // ---- step 2: list 4 (pair counts, rows of the pairs, their sums per box)
     {
-      DBuf<int> cnt4(nb, st), off4(nb, st), tot4(1, st);
-      DBuf<int64_t> roff4(nb, st), rtot4(1, st);
-      launch1d(k_hp2l_count, nb, st, d_lev.p, t.ilevel.p, L.n4.p, L.l4.p, sse, tse, pg, pgt,
-               cnt4.p);
-      exclusive_scan(cnt4.p, off4.p, nb, tot4.p, st);
-      launch1d(k_hp2l_rowlen, nb, st, d_lev.p, t.ilevel.p, cnt4.p, roff4.p);
-      exclusive_scan(roff4.p, roff4.p, nb, rtot4.p, st);
-      int np4 = 0;
-      int64_t nrow4 = 0;
-      readback(&np4, tot4.p, sizeof(int), st);
-      readback(&nrow4, rtot4.p, sizeof(int64_t), st);
       if (np4 > 0) {
         DBuf<cplx> gH(std::max<int64_t>(nrow4, 1), st), uH(np4, st);
-        launch1d(k_hp2l_rows, np4, st, nb, zk, d_lev.p, t.ilevel.p, t.centers.p, L.l4.p, sse,
+        launch1d(k_hp2l_rows, np4, st, nb, zk, d_lev, t.ilevel.p, t.centers.p, L.l4.p, sse,
                  off4.p, xs.p, (const int64_t*)roff4.p, gH.p, uH.p);
 #define FMM2D_P2L(C, D)                                                                       \
-  hipLaunchKernelGGL((k_hp2l_g<C, D>), dim3(nb), dim3(kW), 0, st, nd, zk, d_lev.p, t.ilevel.p, \
+  hipLaunchKernelGGL((k_hp2l_g<C, D>), dim3(nb), dim3(kW), 0, st, nd, zk, d_lev, t.ilevel.p, \
                      L.n4.p, L.l4.p, sse, cnt4.p, off4.p, (const int64_t*)roff4.p, gH.p, uH.p, \
                      chs.p, dps.p, dvs.p, loc.p)
         if (a.ifcharge && !a.ifdipole) FMM2D_P2L(1, 0);
@@ -1540,10 +1521,10 @@ int helmholtz_fmm(const HelmArgs& a, hipStream_t st) {
     // ---- steps 6+7: list 3 and L2P
     auto eval = [&](int p_, int64_t n, const double* xy, const int* lf, cplx* P_, cplx* G_,
                     cplx* H_) {
-      if (p_ == 1) launch_heval<1>(n, st, nd, zk, d_lev.p, xy, lf, t, L, mp.p, loc.p, P_, G_, H_);
+      if (p_ == 1) launch_heval<1>(n, st, nd, zk, d_lev, xy, lf, t, L, mp.p, loc.p, P_, G_, H_);
       else if (p_ == 2)
-        launch_heval<2>(n, st, nd, zk, d_lev.p, xy, lf, t, L, mp.p, loc.p, P_, G_, H_);
-      else launch_heval<3>(n, st, nd, zk, d_lev.p, xy, lf, t, L, mp.p, loc.p, P_, G_, H_);
+        launch_heval<2>(n, st, nd, zk, d_lev, xy, lf, t, L, mp.p, loc.p, P_, G_, H_);
+      else launch_heval<3>(n, st, nd, zk, d_lev, xy, lf, t, L, mp.p, loc.p, P_, G_, H_);
     };
     if (pg > 0) eval(pg, ns, xs.p, t.leaf_s.p, ps.p, gs.p, hs.p);
     if (pgt > 0) eval(pgt, nt, xt.p, t.leaf_t.p, pt.p, gt.p, ht.p);
@@ -1563,12 +1544,12 @@ int helmholtz_fmm(const HelmArgs& a, hipStream_t st) {
     }
     tm.mark(7);
     // ---- unsort
-    if (pg >= 1) launch1d(k_scatter, ns, st, nd, t.isrc.p, ps.p, a.pot);
-    if (pg >= 2) launch1d(k_scatter, ns, st, 2 * nd, t.isrc.p, gs.p, a.grad);
-    if (pg >= 3) launch1d(k_scatter, ns, st, 3 * nd, t.isrc.p, hs.p, a.hess);
-    if (pgt >= 1) launch1d(k_scatter, nt, st, nd, t.itarg.p, pt.p, a.pottarg);
-    if (pgt >= 2) launch1d(k_scatter, nt, st, 2 * nd, t.itarg.p, gt.p, a.gradtarg);
-    if (pgt >= 3) launch1d(k_scatter, nt, st, 3 * nd, t.itarg.p, ht.p, a.hesstarg);
+    if (pg >= 1)
+      launch1d(k_scatter, ns, st, t.isrc.p, nd, ps.p, a.pot, 2 * nd, gs.p,
+               pg >= 2 ? a.grad : nullptr, 3 * nd, hs.p, pg >= 3 ? a.hess : nullptr);
+    if (pgt >= 1)
+      launch1d(k_scatter, nt, st, t.itarg.p, nd, pt.p, a.pottarg, 2 * nd, gt.p,
+               pgt >= 2 ? a.gradtarg : nullptr, 3 * nd, ht.p, pgt >= 3 ? a.hesstarg : nullptr);
     tm.mark(10);
     std::vector<unsigned long long> hc(6 * (nl + 1), 0ull);
     const bool counting = o && o->count_work;
@@ -1700,7 +1681,8 @@ int helmholtz_mps(const HelmMpsArgs& a, hipStream_t st) {
     const int nmax = 2 * std::max(pm[0], pbox);  // largest p1 + p2 of a translation
     const size_t lds = sizeof(cplx) * (2 * (size_t)nmax + 2);
     if (lds > kMpsLds) return FMM2D_ERR_UNSUPPORTED;
-    DBuf<HLev> d_lev = upload(lev, st);
+    DBuf<HLev> dlev_buf = upload(lev, st);
+    const HLev* d_lev = dlev_buf.p;
     DBuf<MpsExp> ex(n, st);
     launch1d(k_mps_gather, n, st, t.isrc.p, a.centers, a.rscale, a.mterms, a.impole, ex.p);
     DBuf<cplx> mp(ncoef, st), loc(ncoef, st);
@@ -1709,12 +1691,12 @@ int helmholtz_mps(const HelmMpsArgs& a, hipStream_t st) {
     tm.mark(9);
     const int* se = t.isrcse.p;
     // ---- step 1: expansions into their leaves' multipoles
-    hipLaunchKernelGGL(k_mps_p2m, dim3(nb), dim3(kMpsW), lds, st, nd, zk, d_lev.p, t.ilevel.p,
+    hipLaunchKernelGGL(k_mps_p2m, dim3(nb), dim3(kMpsW), lds, st, nd, zk, d_lev, t.ilevel.p,
                        t.nchild.p, se, t.centers.p, ex.p, a.mpole, mp.p);
     hip_throw(hipGetLastError(), "mps p2m");
     tm.mark(0);
     // ---- step 2: list-4 expansions into box locals
-    hipLaunchKernelGGL(k_mps_p2l, dim3(nb), dim3(kMpsW), lds, st, nd, zk, d_lev.p, t.ilevel.p,
+    hipLaunchKernelGGL(k_mps_p2l, dim3(nb), dim3(kMpsW), lds, st, nd, zk, d_lev, t.ilevel.p,
                        L.n4.p, L.l4.p, se, t.centers.p, ex.p, a.mpole, loc.p);
     hip_throw(hipGetLastError(), "mps p2l");
     tm.mark(1);
@@ -1722,7 +1704,7 @@ int helmholtz_mps(const HelmMpsArgs& a, hipStream_t st) {
     // expansion needs its local: pg = 1)
     helm_box_passes(t, L, lev, sl, nterms, nd, zk, 1, 0, mp.p, loc.p, tm, st);
     // ---- steps 6-7: list-3 multipoles and the leaf's local at every centre
-    hipLaunchKernelGGL(k_mps_far, dim3((unsigned)n), dim3(kMpsW), lds, st, n, nd, zk, d_lev.p,
+    hipLaunchKernelGGL(k_mps_far, dim3((unsigned)n), dim3(kMpsW), lds, st, n, nd, zk, d_lev,
                        nl, t.leaf_s.p, t.ilevel.p, L.n3.p, L.l3.p, t.centers.p, ex.p, mp.p, loc.p,
                        a.local);
     hip_throw(hipGetLastError(), "mps far");

@@ -37,12 +37,20 @@ __global__ void k_readback(const unsigned* __restrict__ src, int nw,
   if (threadIdx.x == 0) __hip_atomic_store(box, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
-struct InlineWords {
-  unsigned w[kUploadInline / 4];
+template <int N> struct InlineWords {
+  unsigned w[N];
 };
 
-__global__ void k_store_inline(unsigned* __restrict__ dst, int nw, InlineWords a) {
+template <int N>
+__global__ void k_store_inline(unsigned* __restrict__ dst, int nw, InlineWords<N> a) {
   for (int i = threadIdx.x; i < nw; i += blockDim.x) dst[i] = a.w[i];
+}
+
+template <int N> void store_inline(void* dst, const void* src, size_t bytes, hipStream_t st) {
+  InlineWords<N> a;
+  std::memcpy(a.w, src, bytes);
+  hipLaunchKernelGGL(k_store_inline<N>, dim3(1), dim3(256), 0, st, static_cast<unsigned*>(dst),
+                     (int)(bytes / 4), a);
 }
 
 struct Box {
@@ -91,32 +99,52 @@ void readback2(void* dst, const void* src, size_t bytes, void* dst2, const void*
     hip_throw(hipStreamSynchronize(st), "sync");
     return;
   }
+  AsyncRead r;
+  r.begin(src, bytes, src2, bytes2, st);
+  r.finish(dst, dst2);
+}
+
+AsyncRead::~AsyncRead() {
+  // an unfinished read (an error in between): its kernel may still write the box
+  if (!box) return;
+  if (!done && hipStreamSynchronize(st) != hipSuccess) return;
+  box_release(static_cast<Box*>(box));
+}
+
+void AsyncRead::begin(const void* src, size_t bytes, const void* src2, size_t bytes2,
+                      hipStream_t s) {
+  if (bytes + bytes2 > kReadbackMax || bytes % 4 != 0 || bytes2 % 4 != 0)
+    throw HipError{hipErrorInvalidValue, "readback size"};
   Box* b = box_acquire();
-  struct Release {
-    Box* b;
-    ~Release() { box_release(b); }
-  } rel{b};
+  box = b;
+  n1 = bytes;
+  n2 = bytes2;
+  st = s;
   if (++b->seq == 0) b->seq = 1;  // 0 is the initial word
-  const unsigned seq = b->seq;
   hipLaunchKernelGGL(k_readback, dim3(1), dim3(256), 0, st, static_cast<const unsigned*>(src),
                      (int)(bytes / 4), static_cast<const unsigned*>(src2), (int)(bytes2 / 4),
-                     b->h, seq);
+                     b->h, b->seq);
   hip_throw(hipGetLastError(), "readback launch");
+}
+
+void AsyncRead::finish(void* dst, void* dst2) {
+  Box* b = static_cast<Box*>(box);
   // poll for up to 200 microseconds, then block on the stream (which also
   // reports a failure of the work queued before)
   const auto t0 = std::chrono::steady_clock::now();
   for (unsigned it = 1;; ++it) {
-    if (__atomic_load_n(b->h, __ATOMIC_ACQUIRE) == seq) break;
+    if (__atomic_load_n(b->h, __ATOMIC_ACQUIRE) == b->seq) break;
     if ((it & 1023u) == 0 &&
         std::chrono::steady_clock::now() - t0 > std::chrono::microseconds(200)) {
       hip_throw(hipStreamSynchronize(st), "sync");
-      if (__atomic_load_n(b->h, __ATOMIC_ACQUIRE) != seq)
+      if (__atomic_load_n(b->h, __ATOMIC_ACQUIRE) != b->seq)
         throw HipError{hipErrorUnknown, "readback"};
       break;
     }
   }
-  if (bytes) std::memcpy(dst, b->h + kBoxHead, bytes);
-  if (bytes2) std::memcpy(dst2, b->h + kBoxHead + bytes / 4, bytes2);
+  done = true;
+  if (n1) std::memcpy(dst, b->h + kBoxHead, n1);
+  if (n2) std::memcpy(dst2, b->h + kBoxHead + n1 / 4, n2);
 }
 
 void upload_bytes(void* dst, const void* src, size_t bytes, hipStream_t st) {
@@ -126,10 +154,8 @@ void upload_bytes(void* dst, const void* src, size_t bytes, hipStream_t st) {
     hip_throw(hipStreamSynchronize(st), "sync");  // src may die after return
     return;
   }
-  InlineWords a;
-  std::memcpy(a.w, src, bytes);
-  hipLaunchKernelGGL(k_store_inline, dim3(1), dim3(256), 0, st, static_cast<unsigned*>(dst),
-                     (int)(bytes / 4), a);
+  if (bytes <= 1024) store_inline<256>(dst, src, bytes, st);
+  else store_inline<kUploadInline / 4>(dst, src, bytes, st);
   hip_throw(hipGetLastError(), "upload launch");
 }
 

@@ -98,11 +98,14 @@ __global__ void k_gather_split(int64_t n, int nd, int half, const int* perm, con
 
 // rfmm2d split (laplace/rfmm2d.f:65-84): real charge c -> Cauchy charge c,
 // real dipole (d, v) -> Cauchy dipole -(v1 + i v2) d.
-__global__ void k_gather_real(int64_t n, int nd, const int* perm, const double* ch,
-                              const double* ds, const double* dv, cplx* och, cplx* ods) {
+__global__ void k_gather_real(int64_t n, int nd, const int* perm, const double* xy, double* oxy,
+                              const double* ch, const double* ds, const double* dv, cplx* och,
+                              cplx* ods) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
   const int64_t j = perm[i];
+  oxy[2 * i] = xy[2 * j];
+  oxy[2 * i + 1] = xy[2 * j + 1];
   for (int d = 0; d < nd; ++d) {
     if (ch) och[i * nd + d] = mkc(ch[j * nd + d]);
     if (ds) {
@@ -334,24 +337,6 @@ __global__ __launch_bounds__(kW) void k_p2l(int nd, int P, const int* ilevel, co
     }
     __syncthreads();
   }
-}
-
-// Boxes with list-4 work (levels >= 2, a non-empty list 4, points to
-// evaluate): flag, then (after an exclusive scan of the flags) the list in
-// box order.
-__global__ void k_p2l_flag(int64_t nb, const int* ilevel, const int* n4, const int* sse,
-                           const int* tse, int ifpgh, int ifpght, int* flag) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= nb) return;
-  const int b = (int)i;
-  flag[b] = (ilevel[b] >= 2 && n4[b] > 0 && npts_eval(b, sse, tse, ifpgh, ifpght) > 0) ? 1 : 0;
-}
-
-__global__ void k_p2l_list(int64_t nb, const int* flag, const int* pos, int* list, int* cnt) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= nb) return;
-  if (flag[i]) list[pos[i]] = (int)i;
-  if (i == nb - 1) *cnt = pos[i] + flag[i];
 }
 
 // P2M (l2dformmp{c,d,cd}, laprouts2d.f:84-282) for expansions of at most PT
@@ -1348,7 +1333,7 @@ struct NearArgs {
   const int2* seg;   // near-field segment rows (k_near_segs)
   int self;          // the points are the sorted sources
   int* slow;         // FP32 path: points with pairs left to k_near_slow (n entries)
-  int* nslow;        // and their count
+  int* nslow;        // and their count (zero)
   const double* xs;
   const cplx* chs;
   const cplx* dps;
@@ -1366,7 +1351,7 @@ void launch_near_pg(int ifc, int ifd, int64_t n, hipStream_t st, int d0, const N
   const float lo = (float)(std::max(1e-20, 4.0 * q.thresh * q.thresh) * 1.001);
 #define FMM2D_NEAR_L(IFC, IFD)                                                                   \
   do {                                                                                           \
-    if (F32) hip_throw(hipMemsetAsync(q.nslow, 0, sizeof(int), st), "hipMemsetAsync");          \
+    if (F32 && d0 > 0) hip_throw(hipMemsetAsync(q.nslow, 0, sizeof(int), st), "hipMemsetAsync"); \
     launch1d_xcd(k_near<IFC, IFD, PG, NDT, F32, RE>, n, st, q.nd, d0, q.xy, q.leaf, q.seg,     \
                  q.self, q.xs, q.chs, q.dps, q.ch32, q.dp32, q.thresh, lo, q.slow, q.nslow,   \
                  q.p, q.g, q.h);                                                               \
@@ -1479,17 +1464,16 @@ int laplace_fmm(int kind, const CauchyArgs& a, hipStream_t st) {
     const int64_t ns = a.ns;
     const int64_t nt = (a.ifpghtarg > 0) ? a.nt : 0;
     // lfmm2d: 2 Cauchy densities per density, or 1 when all are real
-    int half = 0;
+    // (asked before the tree build, read after it)
+    AsyncRead imag;
+    DBuf<int> iflag;
     if (kind == 1) {
-      DBuf<int> flag(1, st);
-      flag.zero();
-      if (a.ifcharge) launch1d(k_any_imag, a.ns * a.nd, st, a.charge, flag.p);
-      if (a.ifdipole) launch1d(k_any_imag, a.ns * a.nd, st, a.dipstr, flag.p);
-      int h = 0;
-      readback(&h, flag.p, sizeof(int), st);
-      half = (h == 0) ? 1 : 0;
+      iflag.alloc(1, st);
+      iflag.zero();
+      if (a.ifcharge) launch1d(k_any_imag, a.ns * a.nd, st, a.charge, iflag.p);
+      if (a.ifdipole) launch1d(k_any_imag, a.ns * a.nd, st, a.dipstr, iflag.p);
+      imag.begin(iflag.p, sizeof(int), nullptr, 0, st);
     }
-    const int nd = (kind == 1 && !half) ? 2 * a.nd : a.nd;  // Cauchy densities
     int ndiv = lndiv2d(a.eps, ns, nt);
     int idivflag = 0;
     if (o && o->ndiv > 0) {
@@ -1503,6 +1487,13 @@ int laplace_fmm(int kind, const CauchyArgs& a, hipStream_t st) {
     Lists L;
     build_lists(t, L, st);
     tm.mark(8);
+    int half = 0;
+    if (kind == 1) {
+      int h = 0;
+      imag.finish(&h, nullptr);
+      half = (h == 0) ? 1 : 0;
+    }
+    const int nd = (kind == 1 && !half) ? 2 * a.nd : a.nd;  // Cauchy densities
     const int nl = t.nlevels, nb = t.nboxes;
     std::vector<int> nterms(nl + 1, l2dterms(a.eps));
     if (o && o->n_nterms > 0 && o->nterms)
@@ -1513,20 +1504,30 @@ int laplace_fmm(int kind, const CauchyArgs& a, hipStream_t st) {
     std::vector<double> rsc(t.boxsize), logr(nl + 1);
     for (int l = 0; l <= nl; ++l) logr[l] = std::log(rsc[l]);
     const LapOps& ops = lap_ops(P);
-    DBuf<int> d_nterms = upload(nterms, st);
-    DBuf<double> d_rsc = upload(rsc, st), d_logr = upload(logr, st);
+    std::vector<int2> band(nl + 1);
+    for (int l = 0; l <= nl; ++l) band[l] = int2{0, 2 * (nterms[l] + 1)};
+    Blob blob;
+    const size_t b_nterms = blob.add(nterms), b_rsc = blob.add(rsc), b_logr = blob.add(logr),
+                 b_band = blob.add(band), b_op4 = blob.add(std::vector<int>{0, 1, 2, 3}),
+                 b_cnt = blob.add(std::vector<int>{0, 0, 0});
+    blob.upload(st);
+    const int* d_nterms = blob.at<int>(b_nterms);
+    const double *d_rsc = blob.at<double>(b_rsc), *d_logr = blob.at<double>(b_logr);
+    const int2* d_band = blob.at<int2>(b_band);
+    const int* d_op4 = blob.at<int>(b_op4);
+    int* d_cnt = blob.at<int>(b_cnt);  // list-4 boxes; slow near-field points (sources, targets)
 
     // ---- sort and gather
     DBuf<double> xs(2 * ns, st), xt(2 * std::max<int64_t>(nt, 1), st);
     DBuf<cplx> chs(a.ifcharge ? ns * nd : 1, st), dps(a.ifdipole ? ns * nd : 1, st);
     DBuf<int> invs;  // lfmm2d: sorted position of each caller's source
-    if (kind != 1) launch1d(k_gather_xy, ns, st, t.isrc.p, a.src, xs.p);
     if (nt > 0) launch1d(k_gather_xy, nt, st, t.itarg.p, a.targ, xt.p);
     if (kind == 0) {
-      if (a.ifcharge) launch1d(k_gather_dens, ns, st, nd, t.isrc.p, a.charge, chs.p);
-      if (a.ifdipole) launch1d(k_gather_dens, ns, st, nd, t.isrc.p, a.dipstr, dps.p);
+      launch1d(k_gather_dens, ns, st, nd, t.isrc.p, a.src, xs.p, a.ifcharge ? a.charge : nullptr,
+               chs.p, a.ifdipole ? a.dipstr : nullptr, dps.p, (const double*)nullptr,
+               (double*)nullptr);
     } else if (kind == 2) {
-      launch1d(k_gather_real, ns, st, nd, t.isrc.p,
+      launch1d(k_gather_real, ns, st, nd, t.isrc.p, a.src, xs.p,
                a.ifcharge ? reinterpret_cast<const double*>(a.charge) : nullptr,
                a.ifdipole ? reinterpret_cast<const double*>(a.dipstr) : nullptr, a.dipvec,
                chs.p, dps.p);
@@ -1537,9 +1538,13 @@ int laplace_fmm(int kind, const CauchyArgs& a, hipStream_t st) {
                a.ifpgh > 0 ? invs.p : nullptr);
     }
     const int64_t nexp = (int64_t)nb * nd * P;
-    DBuf<cplx> mp(nexp, st), loc(nexp, st);
-    mp.zero();
-    loc.zero();
+    DBuf<cplx> expan(2 * nexp, st);  // multipoles, locals
+    expan.zero();
+    const struct {
+      cplx* p;
+    } mp{expan.p}, loc{expan.p + nexp};
+    BoxPlan bp;
+    plan_boxes(t, L, a.ifpgh, a.ifpghtarg, bp, P <= kW ? d_cnt : nullptr, st);
     const int pg = a.ifpgh, pgt = a.ifpghtarg;
     DBuf<cplx> ps(pg >= 1 ? ns * nd : 1, st), gs(pg >= 2 ? ns * nd : 1, st),
         hs(pg >= 3 ? ns * nd : 1, st);
@@ -1558,17 +1563,12 @@ int laplace_fmm(int kind, const CauchyArgs& a, hipStream_t st) {
     // ---- step 1: P2M, step 2: list 4 (wavefronts over compact box lists up
     // to 64 coefficients; the LDS forms above beyond)
     const bool re_ch = kind != 0;  // real Cauchy charges
-    DBuf<int> p2x_list(nb, st), p2x_cnt(1, st);
     // rows of P coefficients per wavefront: 32, or 16 beyond P = 32 (LDS
     // 4 x bat x P x 16 bytes <= 64 KiB)
     const int bat_x = P <= 32 ? 32 : 16;
     const size_t lds_p2x = (size_t)kP2lWaves * bat_x * P * sizeof(cplx);
     int p2x_grid = 0;
     if (P <= kW) {
-      DBuf<int> flag(nb, st), pos(nb, st);
-      launch1d(k_p2l_flag, nb, st, t.ilevel.p, L.n4.p, sse, tse, pg, pgt, flag.p);
-      exclusive_scan(flag.p, pos.p, nb, (int*)nullptr, st);
-      launch1d(k_p2l_list, nb, st, flag.p, pos.p, p2x_list.p, p2x_cnt.p);
       int dev = 0, ncu = 0, per_cu = 0;
       hip_throw(hipGetDevice(&dev), "device");
       hip_throw(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev), "cu");
@@ -1579,7 +1579,7 @@ int laplace_fmm(int kind, const CauchyArgs& a, hipStream_t st) {
     }
 #define FMM2D_P2L_W32(C, D, RE, F)                                                              \
   hipLaunchKernelGGL((k_p2l_w<C, D, RE, F>), dim3(p2x_grid), dim3(kP2lWaves * kW), lds_p2x,   \
-                     st, p2x_list.p, p2x_cnt.p, nd, P, t.ilevel.p, d_nterms.p, d_rsc.p,        \
+                     st, bp.p2l.p, d_cnt, nd, P, t.ilevel.p, d_nterms, d_rsc,        \
                      t.centers.p, L.n4.p, L.l4.p, sse, xs.p, chs.p, dps.p, bat_x, loc.p)
 #define FMM2D_P2L_W(C, D, RE)                  \
   do {                                         \
@@ -1587,8 +1587,8 @@ int laplace_fmm(int kind, const CauchyArgs& a, hipStream_t st) {
     else FMM2D_P2L_W32(C, D, RE, 0);           \
   } while (0)
 #define FMM2D_P2M_REG(PT, C, D, RE)                                                           \
-  launch1d_xcd(k_p2m_reg<PT, C, D, RE>, nbd, st, nd, P, t.ilevel.p, t.nchild.p, d_nterms.p,   \
-               d_rsc.p, t.centers.p, sse, xs.p, chs.p, dps.p, mp.p)
+  launch1d_xcd(k_p2m_reg<PT, C, D, RE>, nbd, st, nd, P, t.ilevel.p, t.nchild.p, d_nterms,   \
+               d_rsc, t.centers.p, sse, xs.p, chs.p, dps.p, mp.p)
 #define FMM2D_P2M_PT(C, D, RE)                  \
   if (P <= 16) FMM2D_P2M_REG(16, C, D, RE);     \
   else if (P <= 20) FMM2D_P2M_REG(20, C, D, RE); \
@@ -1621,27 +1621,27 @@ int laplace_fmm(int kind, const CauchyArgs& a, hipStream_t st) {
     } else {
       if (a.ifcharge && !a.ifdipole)
         hipLaunchKernelGGL((k_p2m<1, 0>), dim3(nb), dim3(kW), lds_p2m, st, nd, P, t.ilevel.p, t.nchild.p,
-                           d_nterms.p, d_rsc.p, t.centers.p, sse, xs.p, chs.p, dps.p, bat, mp.p);
+                           d_nterms, d_rsc, t.centers.p, sse, xs.p, chs.p, dps.p, bat, mp.p);
       else if (!a.ifcharge && a.ifdipole)
         hipLaunchKernelGGL((k_p2m<0, 1>), dim3(nb), dim3(kW), lds_p2m, st, nd, P, t.ilevel.p, t.nchild.p,
-                           d_nterms.p, d_rsc.p, t.centers.p, sse, xs.p, chs.p, dps.p, bat, mp.p);
+                           d_nterms, d_rsc, t.centers.p, sse, xs.p, chs.p, dps.p, bat, mp.p);
       else
         hipLaunchKernelGGL((k_p2m<1, 1>), dim3(nb), dim3(kW), lds_p2m, st, nd, P, t.ilevel.p, t.nchild.p,
-                           d_nterms.p, d_rsc.p, t.centers.p, sse, xs.p, chs.p, dps.p, bat, mp.p);
+                           d_nterms, d_rsc, t.centers.p, sse, xs.p, chs.p, dps.p, bat, mp.p);
       hip_throw(hipGetLastError(), "p2m");
       tm.mark(0);
       // ---- step 2: list 4
       if (a.ifcharge && !a.ifdipole)
-        hipLaunchKernelGGL((k_p2l<1, 0>), dim3(nb), dim3(kW), lds_p2l, st, nd, P, t.ilevel.p, d_nterms.p,
-                           d_rsc.p, t.centers.p, L.n4.p, L.l4.p, sse, tse, pg, pgt, xs.p, chs.p,
+        hipLaunchKernelGGL((k_p2l<1, 0>), dim3(nb), dim3(kW), lds_p2l, st, nd, P, t.ilevel.p, d_nterms,
+                           d_rsc, t.centers.p, L.n4.p, L.l4.p, sse, tse, pg, pgt, xs.p, chs.p,
                            dps.p, bat, loc.p);
       else if (!a.ifcharge && a.ifdipole)
-        hipLaunchKernelGGL((k_p2l<0, 1>), dim3(nb), dim3(kW), lds_p2l, st, nd, P, t.ilevel.p, d_nterms.p,
-                           d_rsc.p, t.centers.p, L.n4.p, L.l4.p, sse, tse, pg, pgt, xs.p, chs.p,
+        hipLaunchKernelGGL((k_p2l<0, 1>), dim3(nb), dim3(kW), lds_p2l, st, nd, P, t.ilevel.p, d_nterms,
+                           d_rsc, t.centers.p, L.n4.p, L.l4.p, sse, tse, pg, pgt, xs.p, chs.p,
                            dps.p, bat, loc.p);
       else
-        hipLaunchKernelGGL((k_p2l<1, 1>), dim3(nb), dim3(kW), lds_p2l, st, nd, P, t.ilevel.p, d_nterms.p,
-                           d_rsc.p, t.centers.p, L.n4.p, L.l4.p, sse, tse, pg, pgt, xs.p, chs.p,
+        hipLaunchKernelGGL((k_p2l<1, 1>), dim3(nb), dim3(kW), lds_p2l, st, nd, P, t.ilevel.p, d_nterms,
+                           d_rsc, t.centers.p, L.n4.p, L.l4.p, sse, tse, pg, pgt, xs.p, chs.p,
                            dps.p, bat, loc.p);
       hip_throw(hipGetLastError(), "p2l");
     }
@@ -1653,17 +1653,11 @@ int laplace_fmm(int kind, const CauchyArgs& a, hipStream_t st) {
     // ---- translation operators as MFMA fragments: 4 M2M, 4 L2L
     const int opM2M = 0, opL2L = 4;
     const double* d_af = ops.af;
-    std::vector<int2> band(nl + 1);
-    for (int l = 0; l <= nl; ++l) band[l] = int2{0, 2 * (nterms[l] + 1)};
-    DBuf<int2> d_band = upload(band, st);
-    ChildPlan cp;
-    plan_children(t, pg, pgt, cp, st);
-    DBuf<int> d_op4 = upload(std::vector<int>{0, 1, 2, 3}, st);
     // ---- step 3: M2M, finest parents first
     for (int l = nl - 1; l >= 1; --l)
       launch_translate(0, 0, nd, TrBufs{mp.p, 0, P, mp.p, 0, P}, 4,
-                       {TrGroup{cp.lev_pos[l], cp.lev_pos[l + 1], opM2M, 0}}, cp.list.p, cp.up.p,
-                       d_op4.p, d_af, t.ilevel.p, d_band.p, d_logr.p, st);
+                       {TrGroup{bp.lev_pos[l], bp.lev_pos[l + 1], opM2M, 0}}, bp.list.p, bp.up.p,
+                       d_op4, d_af, t.ilevel.p, d_band, d_logr, st);
     tm.mark(2);
     // ---- step 4: M2L, targets grouped by child position (box order within a group)
     // (mixed precision: FP32 copies of the multipoles, for the list-3
@@ -1675,26 +1669,24 @@ int laplace_fmm(int kind, const CauchyArgs& a, hipStream_t st) {
       launch1d(k_to_f32, 2 * nexp, st, reinterpret_cast<const double*>(mp.p), mp32.p);
     }
     {
-      M2LPlan m2l;
-      plan_m2l(t, L, pg, pgt, m2l, st);
-      if (m2l.ntg > 0) {
+      if (bp.np > 0) {
         const void* msrc = mixed ? (const void*)mp32.p : (const void*)mp.p;
         const void* mops = mixed ? (const void*)ops.m2l32 : (const void*)ops.m2l;
         tm.mark(3);  // planning
         if (P <= kM2LMaxP) {
           M2LLev v{};
-          for (int q = 0; q < 4; ++q) v.s0[q] = m2l.cls_seg[q];
-          v.n = m2l.cls_seg[1] - m2l.cls_seg[0];
+          for (int q = 0; q < 4; ++q) v.s0[q] = q * bp.np;
+          v.n = bp.np;
           v.P = P;
-          launch_m2l<1, 1>(nd, {v}, m2l.tlist.p, L.s2.p, mops, t.ilevel.p, d_band.p, d_logr.p,
+          launch_m2l<1, 1>(nd, {v}, bp.tl.p, L.s2.p, mops, t.ilevel.p, d_band, d_logr,
                            mp.p, loc.p, mixed, st);
         } else {
           DBuf<int> d_soff = upload(m2l_slot_offsets(), st);
           std::vector<TrGroup> groups;
           for (int q = 0; q < 4; ++q)
-            groups.push_back(TrGroup{m2l.cls_seg[q], m2l.cls_seg[q + 1], 0, q});
-          launch_translate(0, 1, nd, TrBufs{msrc, 0, P, loc.p, 0, P}, kSlots, groups, m2l.tlist.p,
-                           L.s2.p, d_soff.p, mops, t.ilevel.p, d_band.p, d_logr.p, st, mixed, true,
+            groups.push_back(TrGroup{q * bp.np, (q + 1) * bp.np, 0, q});
+          launch_translate(0, 1, nd, TrBufs{msrc, 0, P, loc.p, 0, P}, kSlots, groups, bp.tl.p,
+                           L.s2.p, d_soff.p, mops, t.ilevel.p, d_band, d_logr, st, mixed, true,
                            true);
         }
         tm.mark(13);  // the M2L kernel alone
@@ -1704,8 +1696,8 @@ int laplace_fmm(int kind, const CauchyArgs& a, hipStream_t st) {
     // ---- step 5: L2L, coarsest first
     for (int l = 1; l <= nl - 1; ++l)
       launch_translate(1, 0, nd, TrBufs{loc.p, 0, P, loc.p, 0, P}, 4,
-                       {TrGroup{cp.lev_pos[l], cp.lev_pos[l + 1], opL2L, 0}}, cp.list.p,
-                       cp.down.p, d_op4.p, d_af, t.ilevel.p, d_band.p, d_logr.p, st);
+                       {TrGroup{bp.lev_pos[l], bp.lev_pos[l + 1], opL2L, 0}}, bp.list.p,
+                       bp.down.p, d_op4, d_af, t.ilevel.p, d_band, d_logr, st);
     tm.mark(4);
     // ---- steps 6+7: list 3 and L2P
     if (mixed && nd == 1) {
@@ -1713,10 +1705,10 @@ int laplace_fmm(int kind, const CauchyArgs& a, hipStream_t st) {
       launch1d(k_to_f32, 2 * nexp, st, reinterpret_cast<const double*>(loc.p), loc32.p);
     }
     if (pg > 0)
-      launch_eval(pg, ns, st, nd, P, xs.p, t.leaf_s.p, t, d_nterms.p, d_rsc.p, L, mp.p, loc.p,
+      launch_eval(pg, ns, st, nd, P, xs.p, t.leaf_s.p, t, d_nterms, d_rsc, L, mp.p, loc.p,
                   mp32.p, loc32.p, ps.p, gs.p, hs.p);
     if (pgt > 0)
-      launch_eval(pgt, nt, st, nd, P, xt.p, t.leaf_t.p, t, d_nterms.p, d_rsc.p, L, mp.p, loc.p,
+      launch_eval(pgt, nt, st, nd, P, xt.p, t.leaf_t.p, t, d_nterms, d_rsc, L, mp.p, loc.p,
                   mp32.p, loc32.p, pt.p, gt.p, ht.p);
     tm.mark(6);
     // ---- step 8: near field, thresh = boxsize(0) 2^-51 (cfmm2d.f:1276)
@@ -1736,30 +1728,27 @@ int laplace_fmm(int kind, const CauchyArgs& a, hipStream_t st) {
       }
       DBuf<int2> seg((size_t)kSegRow * t.nboxes, st);
       launch1d(k_near_segs, t.nboxes, st, L.n1.p, L.l1.p, sse, seg.p);
-      DBuf<int> slow, nslow;
-      if (mixed) {
-        slow = DBuf<int>((size_t)std::max(ns, nt), st);
-        nslow = DBuf<int>(1, st);
-      }
+      DBuf<int> slow;
+      if (mixed) slow = DBuf<int>((size_t)std::max(ns, nt), st);
       tm.mark(15);  // FP32 strength copies, segment rows; [7] the near-field kernels alone
       if (pg > 0)
         launch_near(mixed, re, pg, a.ifcharge, a.ifdipole, ns, st,
-                    NearArgs{nd, xs.p, t.leaf_s.p, seg.p, 1, slow.p, nslow.p, xs.p, chs.p, dps.p,
+                    NearArgs{nd, xs.p, t.leaf_s.p, seg.p, 1, slow.p, d_cnt + 1, xs.p, chs.p, dps.p,
                              ch32.p, dp32.p, thresh, ps.p, gs.p, hs.p});
       if (pgt > 0)
         launch_near(mixed, re, pgt, a.ifcharge, a.ifdipole, nt, st,
-                    NearArgs{nd, xt.p, t.leaf_t.p, seg.p, 0, slow.p, nslow.p, xs.p, chs.p, dps.p,
+                    NearArgs{nd, xt.p, t.leaf_t.p, seg.p, 0, slow.p, d_cnt + 2, xs.p, chs.p, dps.p,
                              ch32.p, dp32.p, thresh, pt.p, gt.p, ht.p});
     }
     tm.mark(7);
     // ---- unsort
     if (kind == 0) {
-      if (pg >= 1) launch1d(k_scatter, ns, st, nd, t.isrc.p, ps.p, a.pot);
-      if (pg >= 2) launch1d(k_scatter, ns, st, nd, t.isrc.p, gs.p, a.grad);
-      if (pg >= 3) launch1d(k_scatter, ns, st, nd, t.isrc.p, hs.p, a.hess);
-      if (pgt >= 1) launch1d(k_scatter, nt, st, nd, t.itarg.p, pt.p, a.pottarg);
-      if (pgt >= 2) launch1d(k_scatter, nt, st, nd, t.itarg.p, gt.p, a.gradtarg);
-      if (pgt >= 3) launch1d(k_scatter, nt, st, nd, t.itarg.p, ht.p, a.hesstarg);
+      if (pg >= 1)
+        launch1d(k_scatter, ns, st, t.isrc.p, nd, ps.p, a.pot, nd, gs.p, pg >= 2 ? a.grad : nullptr,
+                 nd, hs.p, pg >= 3 ? a.hess : nullptr);
+      if (pgt >= 1)
+        launch1d(k_scatter, nt, st, t.itarg.p, nd, pt.p, a.pottarg, nd, gt.p,
+                 pgt >= 2 ? a.gradtarg : nullptr, nd, ht.p, pgt >= 3 ? a.hesstarg : nullptr);
     } else if (kind == 2) {
       if (pg >= 1)
         launch1d(k_scatter_real, ns, st, nd, pg, t.isrc.p, ps.p, gs.p, hs.p,

@@ -53,11 +53,20 @@ __device__ __forceinline__ int append2(bool p0, int e0, bool p1, int e1, int lan
   return cnt + __popcll(m0) + __popcll(m1);
 }
 
+// box size of every level, by value
+constexpr int kListLevels = 54;
+struct ListSizes {
+  double v[kListLevels];
+};
+
 __global__ __launch_bounds__(kListWaves * 64) void k_lists(
     int nb, const int* ilevel, const int* iparent, const int* nchild, const int* ichild,
-    const int* ncoll, const int* coll, const double* centers, const double* bsl, int* n1, int* l1,
+    const int* ncoll, const int* coll, const double* centers, ListSizes sz, int* n1, int* l1,
     int* n2, int* l2, int* n3, int* l3, int* n4, int* l4, int* s2) {
   __shared__ int slots[kListWaves][kBoxesPerWave][kSlots];
+  __shared__ double bsl[kListLevels];
+  for (int k = threadIdx.x; k < kListLevels; k += kListWaves * 64) bsl[k] = sz.v[k];
+  __syncthreads();
   const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int sb = lane / kBoxLanes;  // box of this lane in the wavefront (3: none)
   const int ll = lane - sb * kBoxLanes;
@@ -75,7 +84,7 @@ __global__ __launch_bounds__(kListWaves * 64) void k_lists(
     const int lev = ilevel[b];
     const double bx = centers[2 * b], by = centers[2 * b + 1];
     int* r1 = l1 + (int64_t)kMaxList1 * b;
-    int* r2 = l2 + (int64_t)kMaxList2 * b;
+    int* r2 = l2 ? l2 + (int64_t)kMaxList2 * b : nullptr;
     int* r3 = l3 + (int64_t)kMaxList3 * b;
     int* r4 = l4 + (int64_t)kMaxList4 * b;
     int c1 = 0, c2 = 0, c3 = 0, c4 = 0;
@@ -119,7 +128,8 @@ __global__ __launch_bounds__(kListWaves * 64) void k_lists(
         if (sl >= 0) ssh[sl] = kb1;
       }
     }
-    c2 = append2(far0, kb0, far1, kb1, lane, seg, c2, kMaxList2, r2);
+    // (the rows of list 2 are for callers that export them: the M2L reads s2)
+    c2 = append2(far0, kb0, far1, kb1, lane, seg, c2, l2 ? kMaxList2 : 0, r2);
     // entries contributed by coarser leaves (colleagues of the parent), one
     // lane per colleague (the even lanes)
     {
@@ -184,32 +194,32 @@ __global__ __launch_bounds__(kListWaves * 64) void k_lists(
 }
 }  // namespace
 
-void build_lists(const Tree& t, Lists& L, hipStream_t st) {
+void build_lists(const Tree& t, Lists& L, hipStream_t st, bool rows2) {
   const int nb = t.nboxes;
   L.n1.alloc(nb, st);
   L.n2.alloc(nb, st);
   L.n3.alloc(nb, st);
   L.n4.alloc(nb, st);
   L.l1.alloc((size_t)kMaxList1 * nb, st);
-  L.l2.alloc((size_t)kMaxList2 * nb, st);
+  if (rows2) L.l2.alloc((size_t)kMaxList2 * nb, st);
   L.l3.alloc((size_t)kMaxList3 * nb, st);
   L.l4.alloc((size_t)kMaxList4 * nb, st);
   L.s2.alloc((size_t)kSlots * nb, st);
   // boxsize per level, with one extra (finer) entry for the leaf test at the
   // deepest level, where computelists never reaches it (no non-leaf colleague)
-  std::vector<double> bsl(t.boxsize);
-  bsl.push_back(bsl.back() / 2);
-  DBuf<double> dbs(bsl.size(), st);
-  upload_bytes(dbs.p, bsl.data(), sizeof(double) * bsl.size(), st);
+  ListSizes sz{};
+  if (t.boxsize.size() + 1 > (size_t)kListLevels) throw HipError{hipErrorInvalidValue, "levels"};
+  for (size_t l = 0; l < t.boxsize.size(); ++l) sz.v[l] = t.boxsize[l];
+  sz.v[t.boxsize.size()] = t.boxsize.back() / 2;
   if (nb > 0) {
     const unsigned grid =
         (unsigned)std::min<int64_t>(8192, ceil_div(nb, kListWaves * kBoxesPerWave));
     hipLaunchKernelGGL(k_lists, dim3(grid), dim3(kListWaves * 64), 0, st, nb, t.ilevel.p,
                        t.iparent.p, t.nchild.p, t.ichild.p, t.ncoll.p, t.coll.p, t.centers.p,
-                       dbs.p, L.n1.p, L.l1.p, L.n2.p, L.l2.p, L.n3.p, L.l3.p, L.n4.p, L.l4.p,
+                       sz, L.n1.p, L.l1.p, L.n2.p, L.l2.p, L.n3.p, L.l3.p, L.n4.p, L.l4.p,
                        L.s2.p);
     hip_throw(hipGetLastError(), "kernel launch");
   }
-}  // dbs is released stream-ordered, after k_lists
+}
 
 }  // namespace fmm2d

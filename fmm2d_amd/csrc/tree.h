@@ -74,8 +74,9 @@ void build_tree(const double* src, int64_t ns, const double* trg, int64_t nt, in
                 int idivflag, int nlmax, Tree& t, hipStream_t st,
                 const TreePrep* prep = nullptr);
 
-// Lists 1-4 of computelists (common/tree_routs2d.f:486-710), as sets.
-void build_lists(const Tree& t, Lists& l, hipStream_t st);
+// Lists 1-4 of computelists (common/tree_routs2d.f:486-710), as sets.  The
+// rows of list 2 only with rows2 (its counts and offset slots always).
+void build_lists(const Tree& t, Lists& l, hipStream_t st, bool rows2 = false);
 
 // hist[l] (host, nbins <= kLeafHistMax values) = points, sources plus targets,
 // held by the leaves of level l; the last bin also takes every deeper level.
