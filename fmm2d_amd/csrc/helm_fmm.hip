@@ -42,6 +42,7 @@
 #include "helm_ops.h"
 #include "lap_ops.h"
 #include "m2l.h"
+#include "shift.h"
 #include "p2p_math.h"
 #include "scan.h"
 #include "translate.h"
@@ -810,13 +811,16 @@ __global__ void k_hnear32(int64_t n, int nd, int d0, cplx zk, const double* xy, 
 //   G[i - j] * w1[sa |i-j| + sb |j| + sc |i|] * w2[|i|]
 // with G the scaled cylinder-function table of the offset and w1, w2 powers
 // of the level scales, written straight into the swizzled MFMA A layout.
+// Operator layouts: fragments of translate.h, of m2l.h, rows of shift.h
+enum { kOpTranslate = 0, kOpOrbit = 1, kOpShift = 2 };
+
 struct OpDesc {
   int64_t af;   // first double of the swizzled operator
   int pin, pout;
   int g;        // index of G[0] in the table
   int w1, w2;   // first power of each power table
   int sa, sb, sc;
-  int orbit;    // 1: fragments of m2l.h (pin = pout), 0: of translate.h
+  int layout;   // kOpTranslate, kOpOrbit (pin = pout), kOpShift
   int ksc, rtc;
 };
 
@@ -829,18 +833,25 @@ __global__ void k_build_ops(const OpDesc* ops, const cplx* gt, const double* wt,
   const OpDesc o = ops[blockIdx.y];
   const int Pin = 2 * o.pin + 1, Pout = 2 * o.pout + 1;
   const int RTT = (2 * Pout + 15) / 16, KS = (2 * Pin + 3) / 4;
-  const int ksc = o.orbit ? o.ksc : 0, rtc = o.orbit ? o.rtc : 0;
-  const int64_t total = o.orbit ? (int64_t)16 * ksc * rtc * 64 : (int64_t)RTT * KS * 64;
+  const int ksc = o.ksc, rtc = o.rtc;
+  const int64_t total = o.layout == kOpOrbit   ? (int64_t)16 * ksc * rtc * 64
+                        : o.layout == kOpShift ? 2 * shift_stride(Pin, Pout)
+                                              : (int64_t)RTT * KS * 64;
   for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < total;
        e += (int64_t)gridDim.x * blockDim.x) {
     const int lane = (int)(e & 63);
     const int64_t rest = e >> 6;
     const int ks = (int)(rest % KS), rt = (int)(rest / KS);
     int row = 16 * rt + (lane & 15), col = 4 * ks + (lane >> 4);
-    if (o.orbit) {
+    if (o.layout == kOpOrbit) {
       const M2LEntry m = m2l_entry((int)e, ksc, rtc, -1);
       row = 2 * m.n + m.rpart;
       col = 2 * m.j + m.cpart;
+    } else if (o.layout == kOpShift) {  // re and im of the entry
+      int n, m;
+      shift_entry(e >> 1, Pout, o.pin - o.pout, &n, &m);
+      row = 2 * n + (int)(e & 1);
+      col = 2 * m;
     }
     double v = 0.0;
     if (row < 2 * Pout && col < 2 * Pin) {
@@ -891,8 +902,14 @@ int push_powers(OpTables& T, long double base, int emax) {
   return w0;
 }
 
+int64_t op_size(int layout, int pin, int pout) {
+  if (layout == kOpOrbit) return m2l_stride(2 * pin + 1);
+  if (layout == kOpShift) return 2 * shift_stride(2 * pin + 1, 2 * pout + 1);
+  return afrag_stride(2 * pin + 1);
+}
+
 void add_op(OpTables& T, int pin, int pout, int g, int w1, int w2, int sa, int sb, int sc,
-            bool orbit = false) {
+            int layout) {
   OpDesc o{};
   o.af = T.af_total;
   o.pin = pin;
@@ -903,11 +920,11 @@ void add_op(OpTables& T, int pin, int pout, int g, int w1, int w2, int sa, int s
   o.sa = sa;
   o.sb = sb;
   o.sc = sc;
-  o.orbit = orbit ? 1 : 0;
+  o.layout = layout;
   o.ksc = m2l_ksc(2 * pin + 1);
   o.rtc = m2l_rtc(2 * pin + 1);
   T.desc.push_back(o);
-  T.af_total += orbit ? m2l_stride(2 * pin + 1) : afrag_stride(2 * pin + 1, 2 * pout + 1);
+  T.af_total += op_size(layout, pin, pout);
 }
 
 // scaled H_m(z) s^m, m = 0..mmax, long double upward recurrence from H0, H1
@@ -1207,31 +1224,33 @@ void helm_box_passes(const Tree& t, const Lists& L, const std::vector<HLev>& lev
       const int w1 = push_powers(T, sl[l], 2 * p);
       const int w2 = push_powers(T, 1.0L, p);
       std::vector<std::vector<lc>> hr(19);
-      auto offset = [&](int dx, int dy, bool orbit) {
+      auto offset = [&](int dx, int dy, int layout) {
         const int r2 = dx * dx + dy * dy;
         if (hr[r2].empty())
           hr[r2] = host_scaled_h(k * (bs * std::sqrt((long double)r2)), sl[l], 2 * p);
         const int g = push_table(T, hr[r2], 2 * p, std::atan2((long double)dy, (long double)dx));
-        add_op(T, p, p, g, w1, w2, -1, 1, 1, orbit);
+        add_op(T, p, p, g, w1, w2, -1, 1, 1, layout);
       };
       if (2 * p + 1 <= kM2LMaxP) {
-        for (int o = 0; o < kM2LOrbits; ++o) offset(kM2LBase[o][0], kM2LBase[o][1], true);
+        for (int o = 0; o < kM2LOrbits; ++o) offset(kM2LBase[o][0], kM2LBase[o][1], kOpOrbit);
       } else {
         for (int dx = -3; dx <= 3; ++dx)
           for (int dy = -3; dy <= 3; ++dy) {
             if (std::abs(dx) <= 1 && std::abs(dy) <= 1) {
-              add_op(T, p, p, 0, w1, w2, 0, 0, 0);  // never referenced: zero table slot
+              add_op(T, p, p, 0, w1, w2, 0, 0, 0, kOpTranslate);  // never referenced: zero table slot
               T.desc.back().g = -1;
               continue;
             }
-            offset(dx, dy, false);
+            offset(dx, dy, kOpTranslate);
           }
       }
     }
-    if (l <= nl - 1 && lev[l].on) {
+    if (l >= 2 && l <= nl - 1 && lev[l].on) {
       // M2M into level l from children at l + 1 (h2dmpmp, helmrouts2d.f:967-1090) and
       // L2L from level l to its children (h2dlocloc, helmrouts2d.f:1096-1215);
-      // child - parent = (sx, sy) bs / 4
+      // child - parent = (1, 1) bs / 4, the other children's operators are this
+      // one's up to phases (levels 0 and 1 have neither M2L nor list-3 or
+      // list-4 boxes)
       const int pc = nterms[l + 1];
       const int mm = p + pc;
       const lc z = k * (bs * std::sqrt(2.0L) / 4.0L);
@@ -1241,25 +1260,19 @@ void helm_box_passes(const Tree& t, const Lists& L, const std::vector<HLev>& lev
         Jc[m] = J[m] / std::pow(sl[l + 1], (long double)m);
         Jp[m] = J[m] / std::pow(sl[l], (long double)m);
       }
+      const long double ang = std::atan2(1.0L, 1.0L);
       op_m2m[l] = (int)T.desc.size();
       {
         const int w1 = push_powers(T, sl[l + 1], 2 * std::max(p, pc));
         const int w2 = push_powers(T, sl[l + 1] / sl[l], p);
-        for (int q = 0; q < 4; ++q) {
-          const long double sx = (q & 1) ? 1.0L : -1.0L, sy = (q & 2) ? 1.0L : -1.0L;
-          const int g = push_table(T, Jc, mm, std::atan2(sy, sx));
-          add_op(T, pc, p, g, w1, w2, 1, 1, -1);
-        }
+        add_op(T, pc, p, push_table(T, Jc, mm, ang), w1, w2, 1, 1, -1, kOpShift);
       }
       op_l2l[l] = (int)T.desc.size();
       {
         const int w1 = push_powers(T, sl[l], 2 * std::max(p, pc));
         const int w2 = push_powers(T, sl[l + 1] / sl[l], pc);
-        for (int q = 0; q < 4; ++q) {
-          const long double sx = (q & 1) ? 1.0L : -1.0L, sy = (q & 2) ? 1.0L : -1.0L;
-          const int g = push_table(T, Jp, mm, std::atan2(-sy, -sx));
-          add_op(T, p, pc, g, w1, w2, 1, -1, 1);
-        }
+        add_op(T, p, pc, push_table(T, Jp, mm, std::atan2(-1.0L, -1.0L)), w1, w2, 1,
+               -1, 1, kOpShift);
       }
     }
   }
@@ -1271,8 +1284,7 @@ void helm_box_passes(const Tree& t, const Lists& L, const std::vector<HLev>& lev
     for (const OpDesc& od : T.desc)
       if (od.g >= 0) {
         build.push_back(od);
-        maxaf = std::max(maxaf, od.orbit ? m2l_stride(2 * od.pin + 1)
-                                         : afrag_stride(2 * od.pin + 1, 2 * od.pout + 1));
+        maxaf = std::max(maxaf, op_size(od.layout, od.pin, od.pout));
       }
     if (!build.empty()) {
       DBuf<OpDesc> d_desc = upload(build, st);
@@ -1292,16 +1304,17 @@ void helm_box_passes(const Tree& t, const Lists& L, const std::vector<HLev>& lev
 
   BoxPlan bp;
   plan_boxes(t, L, pg, pgt, bp, nullptr, st);
-  DBuf<int> d_op4 = upload(std::vector<int>{0, 1, 2, 3}, st);
+  auto shop = [&](int i) { return reinterpret_cast<const cplx*>(opptr(i)); };
+  auto side = [&](cplx* v, int l) {
+    const HLev& V = lev[l];
+    return ShiftSide{v + V.off, V.box0, 2 * V.p + 1, 2 * V.p + 1};
+  };
   // ---- step 3: M2M, finest parents first (hfmm2d.f:1021-1100)
-  for (int l = nl - 1; l >= 1; --l) {
+  for (int l = nl - 1; l >= 2; --l) {
     if (op_m2m[l] < 0) continue;
-    const HLev &P = lev[l], &C = lev[l + 1];
-    launch_translate(0, 0, nd,
-                     TrBufs{mpp + C.off, C.box0, 2 * C.p + 1, mpp + P.off, P.box0,
-                            2 * P.p + 1},
-                     4, {TrGroup{bp.lev_pos[l], bp.lev_pos[l + 1], 0, 0}}, bp.list.p, bp.up.p,
-                     d_op4.p, opptr(op_m2m[l]), t.ilevel.p, nullptr, nullptr, st);
+    launch_shift<1, -1>(nd, bp.lev_pos[l + 1] - bp.lev_pos[l], bp.list.p + bp.lev_pos[l],
+                        bp.up.p + 4 * (int64_t)bp.lev_pos[l], side(mpp, l + 1), side(mpp, l),
+                        lev[l + 1].p - lev[l].p, shop(op_m2m[l]), st);
   }
   tm.mark(2);
   // ---- step 4: M2L level by level, targets grouped by child position
@@ -1339,19 +1352,12 @@ void helm_box_passes(const Tree& t, const Lists& L, const std::vector<HLev>& lev
         for (int q = 0; q < 4; ++q)
           groups.push_back(
               TrGroup{q * bp.np + bp.lev_pos[l - 1], q * bp.np + bp.lev_pos[l], 0, q});
-        if (mixed)
-          launch_translate(0, 0, nd,
-                           TrBufs{mp32.p + 2 * V.off, V.box0, 2 * V.p + 1, locp + V.off,
-                                  V.box0, 2 * V.p + 1},
-                           kSlots, groups, bp.tl.p, L.s2.p, d_soff.p,
-                           af32.p + T.desc[op_m2l[l]].af, t.ilevel.p, nullptr, nullptr, st,
-                           true, true, true);
-        else
-          launch_translate(0, 0, nd,
-                           TrBufs{mpp + V.off, V.box0, 2 * V.p + 1, locp + V.off, V.box0,
-                                  2 * V.p + 1},
-                           kSlots, groups, bp.tl.p, L.s2.p, d_soff.p, opptr(op_m2l[l]),
-                           t.ilevel.p, nullptr, nullptr, st, false, true, true);
+        const void* msrc = mixed ? (const void*)(mp32.p + 2 * V.off) : (const void*)(mpp + V.off);
+        const int64_t af = T.desc[op_m2l[l]].af;
+        (mixed ? launch_translate<float, 0> : launch_translate<double, 0>)(
+            nd, Pl, msrc, locp + V.off, V.box0, kSlots, groups, bp.tl.p, L.s2.p, d_soff.p,
+            mixed ? (const void*)(af32.p + af) : (const void*)(d_af.p + af), t.ilevel.p, nullptr,
+            nullptr, st);
       }
       launch_m2l<-1, 0>(nd, orbit_levels, bp.tl.p, L.s2.p,
                         mixed ? (const void*)af32.p : (const void*)d_af.p, t.ilevel.p, nullptr,
@@ -1361,14 +1367,11 @@ void helm_box_passes(const Tree& t, const Lists& L, const std::vector<HLev>& lev
   }
   tm.mark(3);
   // ---- step 5: L2L, coarsest first (hfmm2d.f:1225-1300)
-  for (int l = 1; l <= nl - 1; ++l) {
+  for (int l = 2; l <= nl - 1; ++l) {
     if (op_l2l[l] < 0) continue;
-    const HLev &P = lev[l], &C = lev[l + 1];
-    launch_translate(1, 0, nd,
-                     TrBufs{locp + P.off, P.box0, 2 * P.p + 1, locp + C.off, C.box0,
-                            2 * C.p + 1},
-                     4, {TrGroup{bp.lev_pos[l], bp.lev_pos[l + 1], 0, 0}}, bp.list.p,
-                     bp.down.p, d_op4.p, opptr(op_l2l[l]), t.ilevel.p, nullptr, nullptr, st);
+    launch_shift<0, -1>(nd, bp.lev_pos[l + 1] - bp.lev_pos[l], bp.list.p + bp.lev_pos[l],
+                        bp.down.p + 4 * (int64_t)bp.lev_pos[l], side(locp, l), side(locp, l + 1),
+                        lev[l].p - lev[l + 1].p, shop(op_l2l[l]), st);
   }
   tm.mark(4);
 }

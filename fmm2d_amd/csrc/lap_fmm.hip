@@ -31,6 +31,7 @@
 #include "fmm_common.h"
 #include "lap_ops.h"
 #include "m2l.h"
+#include "shift.h"
 #include "p2p_math.h"
 #include "scan.h"
 #include "translate.h"
@@ -1235,31 +1236,30 @@ long double binom(int n, int k) {
 
 cplx tocplx(lcplx z) { return cplx{(double)z.real(), (double)z.imag()}; }
 
-// The fixed translation matrices (level independent for equal orders).
+// The fixed translation matrices (level independent for equal orders), entry
+// (input j, output n) at j P + n: M2M and L2L of the child up and right of the
+// parent's centre, M2L of the 49 offsets.
 void make_matrices(int P, std::vector<cplx>& A, std::vector<cplx>& B, std::vector<cplx>& T) {
-  A.assign(4 * (size_t)P * P, cplx{0, 0});
-  B.assign(4 * (size_t)P * P, cplx{0, 0});
+  A.assign((size_t)P * P, cplx{0, 0});
+  B.assign((size_t)P * P, cplx{0, 0});
   T.assign(kOff * kOff * (size_t)P * P, cplx{0, 0});
-  for (int q = 0; q < 4; ++q) {
-    const long double sx = (q & 1) ? 1.0L : -1.0L, sy = (q & 2) ? 1.0L : -1.0L;
-    // M2M: child - parent = (sx, sy) * r_child/2; r_parent = 2 r_child
-    const lcplx w = lcplx(sx, sy) / 2.0L, wh = w / 2.0L, wi = 1.0L / w;
-    for (int n = 0; n < P; ++n)
-      for (int j = 0; j <= n; ++j) {
-        lcplx v;
-        if (n == 0) v = 1.0L;
-        else if (j == 0) v = -std::pow(wh, n) / (long double)n;
-        else v = binom(n - 1, j - 1) * std::pow(wi, j) * std::pow(wh, n);
-        A[((size_t)q * P + j) * P + n] = tocplx(v);
-      }
-    // L2L: child - parent = (sx, sy) * r_parent/4; r_child = r_parent/2
-    const lcplx v4 = lcplx(sx, sy) / 4.0L;
-    for (int n = 0; n < P; ++n)
-      for (int j = n; j < P; ++j) {
-        const lcplx v = binom(j, n) * std::pow(v4, j - n) * std::pow(0.5L, n);
-        B[((size_t)q * P + j) * P + n] = tocplx(v);
-      }
-  }
+  // M2M: child - parent = (1, 1) * r_child/2; r_parent = 2 r_child
+  const lcplx w = lcplx(1.0L, 1.0L) / 2.0L, wh = w / 2.0L, wi = 1.0L / w;
+  for (int n = 0; n < P; ++n)
+    for (int j = 0; j <= n; ++j) {
+      lcplx v;
+      if (n == 0) v = 1.0L;
+      else if (j == 0) v = -std::pow(wh, n) / (long double)n;
+      else v = binom(n - 1, j - 1) * std::pow(wi, j) * std::pow(wh, n);
+      A[(size_t)j * P + n] = tocplx(v);
+    }
+  // L2L: child - parent = (1, 1) * r_parent/4; r_child = r_parent/2
+  const lcplx v4 = lcplx(1.0L, 1.0L) / 4.0L;
+  for (int n = 0; n < P; ++n)
+    for (int j = n; j < P; ++j) {
+      const lcplx v = binom(j, n) * std::pow(v4, j - n) * std::pow(0.5L, n);
+      B[(size_t)j * P + n] = tocplx(v);
+    }
   // M2L: source - target = u * r with u = dx + i dy, max(|dx|,|dy|) >= 2
   for (int dx = -3; dx <= 3; ++dx)
     for (int dy = -3; dy <= 3; ++dy) {
@@ -1278,14 +1278,14 @@ void make_matrices(int P, std::vector<cplx>& A, std::vector<cplx>& B, std::vecto
     }
 }
 
-// Translation operators of one expansion length P as MFMA fragments: the 4
-// M2M and 4 L2L quadrants (FP64), and the M2L operators in FP64 and, for mixed
-// precision, FP32: the 10 orbits of m2l.h up to kM2LMaxP coefficients, the 49
-// offsets for k_translate beyond.  They depend on P alone (the Laplace
+// Translation operators of one expansion length P: M2M and L2L in the layout of
+// shift.h (FP64), and the M2L operators as MFMA fragments in FP64 and, for
+// mixed precision, FP32: the 10 orbits of m2l.h up to kM2LMaxP coefficients,
+// the 49 offsets for k_translate beyond.  They depend on P alone (the Laplace
 // operators are level independent), so each (device, P) builds them once;
 // they stay for the life of the process.
 struct LapOps {
-  double* af = nullptr;  // M2M, L2L
+  cplx *m2m = nullptr, *l2l = nullptr;
   double* m2l = nullptr;
   float* m2l32 = nullptr;
 };
@@ -1295,6 +1295,17 @@ template <typename T> T* to_device(const std::vector<T>& v) {
   hip_throw(hipMalloc(&p, v.size() * sizeof(T)), "alloc");
   hip_throw(hipMemcpy(p, v.data(), v.size() * sizeof(T), hipMemcpyHostToDevice), "copy");
   return p;
+}
+
+// A P x P operator (input j, output n at j P + n) in the layout of shift.h
+std::vector<cplx> shift_layout(int P, const std::vector<cplx>& op) {
+  std::vector<cplx> out((size_t)shift_stride(P, P), cplx{0, 0});
+  for (size_t e = 0; e < out.size(); ++e) {
+    int n, m;
+    shift_entry((int64_t)e, P, 0, &n, &m);
+    if (m < P) out[e] = op[(size_t)m * P + n];
+  }
+  return out;
 }
 
 const LapOps& lap_ops(int P) {
@@ -1307,10 +1318,9 @@ const LapOps& lap_ops(int P) {
   if (it != cache.end()) return it->second;
   std::vector<cplx> A, B, T;
   make_matrices(P, A, B, T);
-  std::vector<cplx> ops(A);
-  ops.insert(ops.end(), B.begin(), B.end());
   LapOps o;
-  o.af = to_device(swizzle_ops(P, ops, 8));
+  o.m2m = to_device(shift_layout(P, A));
+  o.l2l = to_device(shift_layout(P, B));
   if (P <= kM2LMaxP) {
     std::vector<std::vector<cplx>> orb;
     for (int k = 0; k < kM2LOrbits; ++k) {
@@ -1508,13 +1518,12 @@ int laplace_fmm(int kind, const CauchyArgs& a, hipStream_t st) {
     for (int l = 0; l <= nl; ++l) band[l] = int2{0, 2 * (nterms[l] + 1)};
     Blob blob;
     const size_t b_nterms = blob.add(nterms), b_rsc = blob.add(rsc), b_logr = blob.add(logr),
-                 b_band = blob.add(band), b_op4 = blob.add(std::vector<int>{0, 1, 2, 3}),
+                 b_band = blob.add(band),
                  b_cnt = blob.add(std::vector<int>{0, 0, 0});
     blob.upload(st);
     const int* d_nterms = blob.at<int>(b_nterms);
     const double *d_rsc = blob.at<double>(b_rsc), *d_logr = blob.at<double>(b_logr);
     const int2* d_band = blob.at<int2>(b_band);
-    const int* d_op4 = blob.at<int>(b_op4);
     int* d_cnt = blob.at<int>(b_cnt);  // list-4 boxes; slow near-field points (sources, targets)
 
     // ---- sort and gather
@@ -1651,13 +1660,12 @@ int laplace_fmm(int kind, const CauchyArgs& a, hipStream_t st) {
 #undef FMM2D_P2L_W32
     tm.mark(1);
     // ---- translation operators as MFMA fragments: 4 M2M, 4 L2L
-    const int opM2M = 0, opL2L = 4;
-    const double* d_af = ops.af;
-    // ---- step 3: M2M, finest parents first
-    for (int l = nl - 1; l >= 1; --l)
-      launch_translate(0, 0, nd, TrBufs{mp.p, 0, P, mp.p, 0, P}, 4,
-                       {TrGroup{bp.lev_pos[l], bp.lev_pos[l + 1], opM2M, 0}}, bp.list.p, bp.up.p,
-                       d_op4, d_af, t.ilevel.p, d_band, d_logr, st);
+    // (levels 0 and 1 have neither M2L nor list-3 or list-4 boxes)
+    auto side = [&](cplx* v, int l) { return ShiftSide{v, 0, P, nterms[l] + 1}; };
+    for (int l = nl - 1; l >= 2; --l)
+      launch_shift<1, 1>(nd, bp.lev_pos[l + 1] - bp.lev_pos[l], bp.list.p + bp.lev_pos[l],
+                         bp.up.p + 4 * (int64_t)bp.lev_pos[l], side(mp.p, l + 1), side(mp.p, l), 0,
+                         ops.m2m, st);
     tm.mark(2);
     // ---- step 4: M2L, targets grouped by child position (box order within a group)
     // (mixed precision: FP32 copies of the multipoles, for the list-3
@@ -1685,19 +1693,19 @@ int laplace_fmm(int kind, const CauchyArgs& a, hipStream_t st) {
           std::vector<TrGroup> groups;
           for (int q = 0; q < 4; ++q)
             groups.push_back(TrGroup{q * bp.np, (q + 1) * bp.np, 0, q});
-          launch_translate(0, 1, nd, TrBufs{msrc, 0, P, loc.p, 0, P}, kSlots, groups, bp.tl.p,
-                           L.s2.p, d_soff.p, mops, t.ilevel.p, d_band, d_logr, st, mixed, true,
-                           true);
+          (mixed ? launch_translate<float, 1> : launch_translate<double, 1>)(
+              nd, P, msrc, loc.p, 0, kSlots, groups, bp.tl.p, L.s2.p, d_soff.p, mops, t.ilevel.p,
+              d_band, d_logr, st);
         }
         tm.mark(13);  // the M2L kernel alone
       }
     }
     tm.mark(3);
     // ---- step 5: L2L, coarsest first
-    for (int l = 1; l <= nl - 1; ++l)
-      launch_translate(1, 0, nd, TrBufs{loc.p, 0, P, loc.p, 0, P}, 4,
-                       {TrGroup{bp.lev_pos[l], bp.lev_pos[l + 1], opL2L, 0}}, bp.list.p,
-                       bp.down.p, d_op4, d_af, t.ilevel.p, d_band, d_logr, st);
+    for (int l = 2; l <= nl - 1; ++l)
+      launch_shift<0, -1>(nd, bp.lev_pos[l + 1] - bp.lev_pos[l], bp.list.p + bp.lev_pos[l],
+                          bp.down.p + 4 * (int64_t)bp.lev_pos[l], side(loc.p, l),
+                          side(loc.p, l + 1), 0, ops.l2l, st);
     tm.mark(4);
     // ---- steps 6+7: list 3 and L2P
     if (mixed && nd == 1) {
