@@ -45,8 +45,24 @@ struct AsyncRead {
   AsyncRead& operator=(const AsyncRead&) = delete;
   ~AsyncRead();
   void begin(const void* src, size_t bytes, const void* src2, size_t bytes2, hipStream_t s);
+  bool ready() const;  // finish would not wait
   void finish(void* dst, void* dst2);
 };
+// Pinned memory that a copy on st reads after the call that fills it has gone
+// on.  The destructor waits for st (idle at the end of an FMM call) and gives
+// the memory back to a pool of a few buffers, which fmm2d_release_workspace()
+// empties.
+struct Staging {
+  void* p = nullptr;
+  size_t cap = 0;
+  hipStream_t st = nullptr;
+  Staging() = default;
+  Staging(const Staging&) = delete;
+  Staging& operator=(const Staging&) = delete;
+  ~Staging();
+  void* get(size_t bytes, hipStream_t s);  // once
+};
+void staging_release();  // free the pooled buffers
 void upload_bytes(void* dst, const void* src, size_t bytes, hipStream_t st);
 
 // Workspace cache (ws.cpp).  ws_alloc returns at least `bytes` bytes usable

@@ -34,6 +34,7 @@
 #include <algorithm>
 #include <cmath>
 #include <complex>
+#include <cstring>
 #include <vector>
 
 #include "devbuf.h"
@@ -865,8 +866,6 @@ __global__ void k_build_ops(const OpDesc* ops, const cplx* gt, const double* wt,
   }
 }
 
-using lc = std::complex<long double>;
-
 struct OpTables {
   std::vector<OpDesc> desc;
   std::vector<cplx> g;
@@ -874,20 +873,32 @@ struct OpTables {
   int64_t af_total = 0;
 };
 
-cplx to_c(lc v) { return cplx{(double)v.real(), (double)v.imag()}; }
+cplx to_c(lx v) { return cplx{(double)v.re, (double)v.im}; }
+
+// e^{-i m a}, m = 0, 1, ..., as far as asked for
+struct Phases {
+  std::vector<lx> e;
+  lx u;
+  const std::vector<lx>& upto(int mmax, long double ang) {
+    if (e.empty()) {
+      u = lx{std::cos(ang), -std::sin(ang)};
+      e.push_back(lx{1, 0});
+    }
+    while ((int)e.size() <= mmax) e.push_back(e.back() * u);
+    return e;
+  }
+};
 
 // G[m] = F_|m| sign^m e^{-i m a} for m = -mmax..mmax from f[0..mmax]
-int push_table(OpTables& T, const std::vector<lc>& f, int mmax, long double ang) {
+int push_table(OpTables& T, const std::vector<lx>& f, int mmax, const std::vector<lx>& ph) {
   const int g0 = (int)T.g.size() + mmax;
   T.g.resize(T.g.size() + 2 * mmax + 1);
-  const lc u = std::polar(1.0L, -ang);
-  lc e = 1.0L;
   for (int m = 0; m <= mmax; ++m) {
-    const lc v = f[m] * e;                  // F_m e^{-i m a}
-    T.g[g0 + m] = to_c(v);
-    const lc vm = f[m] * std::conj(e);      // F_m e^{+i m a}
-    T.g[g0 - m] = to_c((m & 1) ? -vm : vm);
-    e *= u;
+    const lx x = f[m], e = ph[m];
+    const long double ac = x.re * e.re, bd = x.im * e.im, ad = x.re * e.im, bc = x.im * e.re;
+    T.g[g0 + m] = to_c(lx{ac - bd, ad + bc});          // F_m e^{-i m a}
+    const cplx v = to_c(lx{ac + bd, bc - ad});         // F_m e^{+i m a}
+    T.g[g0 - m] = (m & 1) ? -v : v;
   }
   return g0;
 }
@@ -928,14 +939,14 @@ void add_op(OpTables& T, int pin, int pout, int g, int w1, int w2, int sa, int s
 }
 
 // scaled H_m(z) s^m, m = 0..mmax, long double upward recurrence from H0, H1
-std::vector<lc> host_scaled_h(lc z, long double s, int mmax) {
-  std::vector<lc> h(mmax + 2);
+std::vector<lx> host_scaled_h(lx z, long double s, int mmax) {
+  std::vector<lx> h(mmax + 2);
   cplx h0, h1;
   hank01(to_c(z), &h0, &h1);
-  h[0] = lc(h0.re, h0.im);
-  h[1] = lc(h1.re, h1.im) * s;
-  for (int n = 1; n < mmax; ++n)
-    h[n + 1] = (2.0L * n * s / z) * h[n] - s * s * h[n - 1];
+  h[0] = lx{h0.re, h0.im};
+  h[1] = s * lx{h1.re, h1.im};
+  const lx r = to_lx((2.0L * s) / to_lc(z));
+  for (int n = 1; n < mmax; ++n) h[n + 1] = ((long double)n * r) * h[n] - (s * s) * h[n - 1];
   h.resize(mmax + 1);
   return h;
 }
@@ -1197,86 +1208,113 @@ __global__ __launch_bounds__(kMpsW) void k_mps_near(int64_t n, int nd, cplx zk, 
   }
 }
 
+// Host tables of the translation operators, level by level: next() makes one
+// level's, so that the caller can do so while the device is busy with
+// something else and look in between whether it has finished.
+struct HelmOps {
+  const Tree& t;
+  const std::vector<HLev>& lev;
+  const std::vector<long double>& sl;
+  const std::vector<int>& nterms;
+  lx k;
+  int nl, l = 1;
+  OpTables T;
+  std::vector<int> m2l, m2m, l2l;  // first operator of the level, or -1
+  std::vector<Phases> ph;          // of the 49 offsets, M2M and L2L
+
+  HelmOps(const Tree& t_, const std::vector<HLev>& lev_, const std::vector<long double>& sl_,
+          const std::vector<int>& nterms_, cplx zk)
+      : t(t_), lev(lev_), sl(sl_), nterms(nterms_), k{zk.re, zk.im}, nl(t_.nlevels),
+        m2l(nl + 1, -1), m2m(nl + 1, -1), l2l(nl + 1, -1), ph(51) {}
+  bool done() const { return l > nl; }
+  void next();
+};
+
+void HelmOps::next() {
+  const long double bs = t.boxsize[l];
+  const int p = nterms[l];
+  if (l >= 2 && lev[l].on) {
+    // M2L: source - target = (dx, dy) bs, max(|dx|,|dy|) >= 2 (h2dmploc,
+    // helmrouts2d.f:1221-1380)
+    m2l[l] = (int)T.desc.size();
+    const int w1 = push_powers(T, sl[l], 2 * p);
+    const int w2 = push_powers(T, 1.0L, p);
+    std::vector<std::vector<lx>> hr(19);
+    auto offset = [&](int dx, int dy, int layout) {
+      const int r2 = dx * dx + dy * dy;
+      if (hr[r2].empty())
+        hr[r2] = host_scaled_h((bs * std::sqrt((long double)r2)) * k, sl[l], 2 * p);
+      const auto& e = ph[(dx + 3) * 7 + dy + 3].upto(
+          2 * p, std::atan2((long double)dy, (long double)dx));
+      add_op(T, p, p, push_table(T, hr[r2], 2 * p, e), w1, w2, -1, 1, 1, layout);
+    };
+    if (2 * p + 1 <= kM2LMaxP) {
+      for (int o = 0; o < kM2LOrbits; ++o) offset(kM2LBase[o][0], kM2LBase[o][1], kOpOrbit);
+    } else {
+      for (int dx = -3; dx <= 3; ++dx)
+        for (int dy = -3; dy <= 3; ++dy) {
+          if (std::abs(dx) <= 1 && std::abs(dy) <= 1) {
+            add_op(T, p, p, 0, w1, w2, 0, 0, 0, kOpTranslate);  // never referenced: zero table slot
+            T.desc.back().g = -1;
+            continue;
+          }
+          offset(dx, dy, kOpTranslate);
+        }
+    }
+  }
+  if (l >= 2 && l <= nl - 1 && lev[l].on) {
+    // M2M into level l from children at l + 1 (h2dmpmp, helmrouts2d.f:967-1090) and
+    // L2L from level l to its children (h2dlocloc, helmrouts2d.f:1096-1215);
+    // child - parent = (1, 1) bs / 4, the other children's operators are this
+    // one's up to phases (levels 0 and 1 have neither M2L nor list-3 or
+    // list-4 boxes)
+    const int pc = nterms[l + 1];
+    const int mm = p + pc;
+    std::vector<lx> Jc = bessel_j((bs * std::sqrt(2.0L) / 4.0L) * k, std::max(mm, 1)), Jp(Jc);
+    // scaled by the child's / parent's s^-m
+    long double wc = 1.0L, wp = 1.0L;
+    for (int m = 0; m <= mm; ++m) {
+      Jc[m] = lx{Jc[m].re / wc, Jc[m].im / wc};
+      Jp[m] = lx{Jp[m].re / wp, Jp[m].im / wp};
+      wc *= sl[l + 1];
+      wp *= sl[l];
+    }
+    m2m[l] = (int)T.desc.size();
+    {
+      const int w1 = push_powers(T, sl[l + 1], 2 * std::max(p, pc));
+      const int w2 = push_powers(T, sl[l + 1] / sl[l], p);
+      const auto& e = ph[49].upto(mm, std::atan2(1.0L, 1.0L));
+      add_op(T, pc, p, push_table(T, Jc, mm, e), w1, w2, 1, 1, -1, kOpShift);
+    }
+    l2l[l] = (int)T.desc.size();
+    {
+      const int w1 = push_powers(T, sl[l], 2 * std::max(p, pc));
+      const int w2 = push_powers(T, sl[l + 1] / sl[l], pc);
+      const auto& e = ph[50].upto(mm, std::atan2(-1.0L, -1.0L));
+      add_op(T, p, pc, push_table(T, Jp, mm, e), w1, w2, 1, -1, 1, kOpShift);
+    }
+  }
+  ++l;
+}
+
 // Box-to-box passes shared by hfmm2d and hfmm2d_mps (hfmm2d.f:1021-1300,
 // hfmm2d_mps.f:520-760): translation operators for every level, then M2M
 // (finest parents first), M2L level by level and L2L (coarsest first), on the
 // per-level multipole and local blocks.  pg / pgt say which boxes hold
-// evaluation points (sources / targets), as the planners need.  mixed: the M2L
+// evaluation points (sources / targets), as the planners need.  stage: for the
+// operator tables, kept by the caller until st is done.  mixed: the M2L
 // runs on v_mfma_f32_16x16x4f32 with FP32 copies of the operators (the
 // swizzled A-fragment layout is the same for both element types) and of the
 // multipoles, accumulating in FP32 and adding into the FP64 locals.
-void helm_box_passes(const Tree& t, const Lists& L, const std::vector<HLev>& lev,
-                     const std::vector<long double>& sl, const std::vector<int>& nterms,
-                     int nd, cplx zk, int pg, int pgt, cplx* mpp, cplx* locp, Timer& tm,
-                     hipStream_t st, bool mixed = false) {
+void helm_box_passes(HelmOps& ops, const Lists& L, int nd, int pg, int pgt, cplx* mpp, cplx* locp,
+                     Staging& stage, Timer& tm, hipStream_t st, bool mixed = false) {
+  while (!ops.done()) ops.next();
+  const Tree& t = ops.t;
+  const std::vector<HLev>& lev = ops.lev;
+  const OpTables& T = ops.T;
+  const std::vector<int>&op_m2l = ops.m2l, &op_m2m = ops.m2m, &op_l2l = ops.l2l;
   const int nl = t.nlevels;
-  // ---- translation operators, level by level
-  OpTables T;
-  std::vector<int> op_m2l(nl + 1, -1), op_m2m(nl + 1, -1), op_l2l(nl + 1, -1);
-  const lc k(zk.re, zk.im);
-  for (int l = 1; l <= nl; ++l) {
-    const long double bs = t.boxsize[l];
-    const int p = nterms[l];
-    if (l >= 2 && lev[l].on) {
-      // M2L: source - target = (dx, dy) bs, max(|dx|,|dy|) >= 2 (h2dmploc,
-      // helmrouts2d.f:1221-1380)
-      op_m2l[l] = (int)T.desc.size();
-      const int w1 = push_powers(T, sl[l], 2 * p);
-      const int w2 = push_powers(T, 1.0L, p);
-      std::vector<std::vector<lc>> hr(19);
-      auto offset = [&](int dx, int dy, int layout) {
-        const int r2 = dx * dx + dy * dy;
-        if (hr[r2].empty())
-          hr[r2] = host_scaled_h(k * (bs * std::sqrt((long double)r2)), sl[l], 2 * p);
-        const int g = push_table(T, hr[r2], 2 * p, std::atan2((long double)dy, (long double)dx));
-        add_op(T, p, p, g, w1, w2, -1, 1, 1, layout);
-      };
-      if (2 * p + 1 <= kM2LMaxP) {
-        for (int o = 0; o < kM2LOrbits; ++o) offset(kM2LBase[o][0], kM2LBase[o][1], kOpOrbit);
-      } else {
-        for (int dx = -3; dx <= 3; ++dx)
-          for (int dy = -3; dy <= 3; ++dy) {
-            if (std::abs(dx) <= 1 && std::abs(dy) <= 1) {
-              add_op(T, p, p, 0, w1, w2, 0, 0, 0, kOpTranslate);  // never referenced: zero table slot
-              T.desc.back().g = -1;
-              continue;
-            }
-            offset(dx, dy, kOpTranslate);
-          }
-      }
-    }
-    if (l >= 2 && l <= nl - 1 && lev[l].on) {
-      // M2M into level l from children at l + 1 (h2dmpmp, helmrouts2d.f:967-1090) and
-      // L2L from level l to its children (h2dlocloc, helmrouts2d.f:1096-1215);
-      // child - parent = (1, 1) bs / 4, the other children's operators are this
-      // one's up to phases (levels 0 and 1 have neither M2L nor list-3 or
-      // list-4 boxes)
-      const int pc = nterms[l + 1];
-      const int mm = p + pc;
-      const lc z = k * (bs * std::sqrt(2.0L) / 4.0L);
-      std::vector<lc> J = bessel_j(z, std::max(mm, 1));
-      std::vector<lc> Jc(J), Jp(J);  // scaled by the child's / parent's s^-m
-      for (int m = 0; m <= mm; ++m) {
-        Jc[m] = J[m] / std::pow(sl[l + 1], (long double)m);
-        Jp[m] = J[m] / std::pow(sl[l], (long double)m);
-      }
-      const long double ang = std::atan2(1.0L, 1.0L);
-      op_m2m[l] = (int)T.desc.size();
-      {
-        const int w1 = push_powers(T, sl[l + 1], 2 * std::max(p, pc));
-        const int w2 = push_powers(T, sl[l + 1] / sl[l], p);
-        add_op(T, pc, p, push_table(T, Jc, mm, ang), w1, w2, 1, 1, -1, kOpShift);
-      }
-      op_l2l[l] = (int)T.desc.size();
-      {
-        const int w1 = push_powers(T, sl[l], 2 * std::max(p, pc));
-        const int w2 = push_powers(T, sl[l + 1] / sl[l], pc);
-        add_op(T, p, pc, push_table(T, Jp, mm, std::atan2(-1.0L, -1.0L)), w1, w2, 1,
-               -1, 1, kOpShift);
-      }
-    }
-  }
-  DBuf<double> d_af(std::max<int64_t>(T.af_total, 1), st);
+  DBuf<double> d_af(std::max<int64_t>(T.af_total, 1), st), tabs;
   {
     // drop the never-referenced slots from the build list
     std::vector<OpDesc> build;
@@ -1287,14 +1325,22 @@ void helm_box_passes(const Tree& t, const Lists& L, const std::vector<HLev>& lev
         maxaf = std::max(maxaf, op_size(od.layout, od.pin, od.pout));
       }
     if (!build.empty()) {
-      DBuf<OpDesc> d_desc = upload(build, st);
-      DBuf<cplx> d_g = upload(T.g, st);
-      DBuf<double> d_w = upload(T.w, st);
+      // tables in one pinned copy, which the host does not wait for
+      const size_t ng = sizeof(cplx) * T.g.size(), nw = sizeof(double) * T.w.size(),
+                   ndsc = sizeof(OpDesc) * build.size();
+      tabs.alloc((ng + nw + ndsc) / 8, st);
+      char* h = static_cast<char*>(stage.get(ng + nw + ndsc, st));
+      std::memcpy(h, T.g.data(), ng);
+      std::memcpy(h + ng, T.w.data(), nw);
+      std::memcpy(h + ng + nw, build.data(), ndsc);
+      hip_throw(hipMemcpyAsync(tabs.p, h, ng + nw + ndsc, hipMemcpyHostToDevice, st), "tables");
+      const char* d = reinterpret_cast<const char*>(tabs.p);
       const unsigned gx = (unsigned)std::min<int64_t>((maxaf + 255) / 256, 64);
       hipLaunchKernelGGL(k_build_ops, dim3(gx, (unsigned)build.size()), dim3(256), 0, st,
-                         d_desc.p, d_g.p, d_w.p, d_af.p);
+                         reinterpret_cast<const OpDesc*>(d + ng + nw),
+                         reinterpret_cast<const cplx*>(d),
+                         reinterpret_cast<const double*>(d + ng), d_af.p);
       hip_throw(hipGetLastError(), "build_ops");
-      hip_throw(hipStreamSynchronize(st), "sync");
     }
   }
   auto opptr = [&](int first) { return d_af.p + T.desc[first].af; };
@@ -1483,7 +1529,12 @@ int helmholtz_fmm(const HelmArgs& a, hipStream_t st) {
     exclusive_scan(roff4.p, roff4.p, nb, rtot.p + 1, st);
     int64_t hrow[2] = {0, 0};
     int np4 = 0;
-    readback2(hrow, rtot.p, sizeof(hrow), &np4, tot4.p, sizeof(int), st);
+    AsyncRead sizes;
+    sizes.begin(rtot.p, sizeof(hrow), tot4.p, sizeof(int), st);
+    Staging stage;
+    HelmOps ops(t, lev, sl, nterms, zk);
+    while (!ops.done() && !sizes.ready()) ops.next();
+    sizes.finish(hrow, &np4);
     const int64_t nrow = hrow[0], nrow4 = hrow[1];
     // ---- step 1: P2M (rows of the sources, then their sums per leaf)
     {
@@ -1520,7 +1571,7 @@ int helmholtz_fmm(const HelmArgs& a, hipStream_t st) {
     hip_throw(hipGetLastError(), "p2l");
     tm.mark(1);
 
-    helm_box_passes(t, L, lev, sl, nterms, nd, zk, pg, pgt, mp.p, loc.p, tm, st, mixed);
+    helm_box_passes(ops, L, nd, pg, pgt, mp.p, loc.p, stage, tm, st, mixed);
     // ---- steps 6+7: list 3 and L2P
     auto eval = [&](int p_, int64_t n, const double* xy, const int* lf, cplx* P_, cplx* G_,
                     cplx* H_) {
@@ -1705,7 +1756,9 @@ int helmholtz_mps(const HelmMpsArgs& a, hipStream_t st) {
     tm.mark(1);
     // ---- steps 3-5: M2M, M2L, L2L between boxes (every box holding an
     // expansion needs its local: pg = 1)
-    helm_box_passes(t, L, lev, sl, nterms, nd, zk, 1, 0, mp.p, loc.p, tm, st);
+    HelmOps ops(t, lev, sl, nterms, zk);
+    Staging stage;
+    helm_box_passes(ops, L, nd, 1, 0, mp.p, loc.p, stage, tm, st);
     // ---- steps 6-7: list-3 multipoles and the leaf's local at every centre
     hipLaunchKernelGGL(k_mps_far, dim3((unsigned)n), dim3(kMpsW), lds, st, n, nd, zk, d_lev,
                        nl, t.leaf_s.p, t.ilevel.p, L.n3.p, L.l3.p, t.centers.p, ex.p, mp.p, loc.p,

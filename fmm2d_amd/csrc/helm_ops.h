@@ -50,8 +50,24 @@ int helmholtz_mps(const HelmMpsArgs& a, hipStream_t st);
 // meets the criterion.
 int h2dterms(double bsize, cplx zk, double eps, int* ier);
 
+// Complex long double with plain products: std::complex's test every product
+// for NaN operands through a library call, ten times the time of the
+// recurrences below.
+struct lx {
+  long double re, im;
+};
+inline lx operator+(lx a, lx b) { return lx{a.re + b.re, a.im + b.im}; }
+inline lx operator-(lx a, lx b) { return lx{a.re - b.re, a.im - b.im}; }
+inline lx operator*(lx a, lx b) {
+  return lx{a.re * b.re - a.im * b.im, a.re * b.im + a.im * b.re};
+}
+inline lx operator*(long double s, lx a) { return lx{s * a.re, s * a.im}; }
+inline long double norm(lx a) { return a.re * a.re + a.im * a.im; }
+inline std::complex<long double> to_lc(lx a) { return {a.re, a.im}; }
+inline lx to_lx(std::complex<long double> a) { return lx{a.real(), a.imag()}; }
+
 // J_0(z) .. J_n(z) in long double (Miller's backward recurrence, normalised by
 // the Jacobi-Anger identity), n >= 1.
-std::vector<std::complex<long double>> bessel_j(std::complex<long double> z, int n);
+std::vector<lx> bessel_j(lx z, int n);
 
 }  // namespace fmm2d

@@ -13,6 +13,7 @@
 // runtime copies at launch, so no synchronisation keeps the host memory alive.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <atomic>
 #include <chrono>
 #include <cstring>
@@ -127,6 +128,11 @@ void AsyncRead::begin(const void* src, size_t bytes, const void* src2, size_t by
   hip_throw(hipGetLastError(), "readback launch");
 }
 
+bool AsyncRead::ready() const {
+  const Box* b = static_cast<const Box*>(box);
+  return __atomic_load_n(b->h, __ATOMIC_ACQUIRE) == b->seq;
+}
+
 void AsyncRead::finish(void* dst, void* dst2) {
   Box* b = static_cast<Box*>(box);
   // poll for up to 200 microseconds, then block on the stream (which also
@@ -145,6 +151,60 @@ void AsyncRead::finish(void* dst, void* dst2) {
   done = true;
   if (n1) std::memcpy(dst, b->h + kBoxHead, n1);
   if (n2) std::memcpy(dst2, b->h + kBoxHead + n1 / 4, n2);
+}
+
+namespace {
+
+// free staging buffers: at most kStagePool of at most kStageMax bytes
+constexpr size_t kStagePool = 8, kStageMax = size_t(4) << 20;
+struct StageBuf {
+  void* p;
+  size_t cap;
+};
+std::mutex g_stage_mu;
+std::vector<StageBuf> g_stage;
+
+}  // namespace
+
+void* Staging::get(size_t bytes, hipStream_t s) {
+  st = s;
+  {
+    std::lock_guard<std::mutex> g(g_stage_mu);
+    for (size_t k = 0; k < g_stage.size(); ++k)
+      if (g_stage[k].cap >= bytes) {
+        p = g_stage[k].p;
+        cap = g_stage[k].cap;
+        g_stage[k] = g_stage.back();
+        g_stage.pop_back();
+        return p;
+      }
+  }
+  const size_t want = std::max(size_t(1) << 18, (bytes + (size_t(1) << 16)) >> 16 << 16);
+  hip_throw(hipHostMalloc(&p, want, hipHostMallocDefault), "hipHostMalloc (staging)");
+  cap = want;
+  return p;
+}
+
+Staging::~Staging() {
+  if (!p) return;
+  if (hipStreamSynchronize(st) != hipSuccess) return;  // a copy may still read it
+  if (cap <= kStageMax) {
+    std::lock_guard<std::mutex> g(g_stage_mu);
+    if (g_stage.size() < kStagePool) {
+      g_stage.push_back(StageBuf{p, cap});
+      return;
+    }
+  }
+  (void)hipHostFree(p);
+}
+
+void staging_release() {
+  std::vector<StageBuf> all;
+  {
+    std::lock_guard<std::mutex> g(g_stage_mu);
+    all.swap(g_stage);
+  }
+  for (const StageBuf& b : all) (void)hipHostFree(b.p);
 }
 
 void upload_bytes(void* dst, const void* src, size_t bytes, hipStream_t st) {

@@ -24,7 +24,7 @@
 // latency.  A level took 8-10 us for 19 coefficients and 17-22 us for 61, of
 // which the memory traffic of the small ones is nothing and that of the
 // largest a third.  This form: lfmm2d N = 1e7 (13 levels, 19 coefficients,
-// 2.3e6 boxes) 1.52 -> 0.68 ms for both directions, hfmm2d at 2e6 points (16
+// 1.8e6 boxes) 1.52 -> 0.68 ms for both directions, hfmm2d at 2e6 points (16
 // levels, up to 201 coefficients) 2.64 -> 0.55 ms; a level of 470 parents 5 us; the
 // largest level moves its 320 MB at 3.7 TB/s.
 #pragma once

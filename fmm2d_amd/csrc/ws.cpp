@@ -101,6 +101,7 @@ void ws_free(void* p, hipStream_t st) {
 }
 
 int ws_release() {
+  staging_release();
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess) return FMM2D_ERR_HIP;
   std::lock_guard<std::mutex> lock(g_mu);
