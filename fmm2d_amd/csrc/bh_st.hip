@@ -102,7 +102,7 @@ __global__ __launch_bounds__(kBT) void k_bh_direct(
       if (IFC) {
         const cplx c1 = sm.c1[k], c2 = sm.c2[k];
         const cplx zr = z1c * z;  // zeta / conj(zeta)
-        v += (fast_log(rr)) * c1 + c2 * zr;
+        v += (2.0 * fast_hlog(rr)) * c1 + c2 * zr;
         if (PG >= 2) {
           g1 += c1 * z1;
           g2 += c2 * z1c;
@@ -188,7 +188,7 @@ __global__ __launch_bounds__(kBT) void k_st_direct(
       const double ri4 = ri2 * ri2;
       if (IFS) {
         const double a1 = sm.s1[k], a2 = sm.s2[k];
-        const double lg = 0.25 * fast_log(r2);
+        const double lg = 0.5 * fast_hlog(r2);
         const double rt = dx * dx - dy * dy;
         const double pl = dx * a1 + dy * a2, pl2 = dx * a2 + dy * a1;
         u1 += -a1 * lg + 0.5 * dx * pl * ri2;

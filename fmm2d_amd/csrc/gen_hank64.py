@@ -1,14 +1,16 @@
 """Generate hank64_tables.h: the FP64 coefficient tables of the real-argument
 Hankel pair (hankel.h, hank01_real).
 
-For x < X1: the ascending series (Abramowitz & Stegun 9.1.10, 9.1.11, 9.1.13)
-in q = x^2/4 with NSER terms (the first omitted term is below 1e-17 at x = 4):
+For x < X1: the sums of the ascending series (Abramowitz & Stegun 9.1.10, 9.1.11,
+9.1.13) in q = x^2/4 as their Chebyshev interpolants on [0, X1^2/4], NSER
+coefficients each (interpolation error below 1e-19; the series itself needs 17
+terms), computed with mpmath and rounded once to double:
   J0 = sum a_k q^k,            a_k = (-1)^k / (k!)^2
   J1 = (x/2) sum b_k q^k,      b_k = (-1)^k / (k! (k+1)!)
   Y0 = (2/pi) [(ln(x/2) + gamma) J0 + sum c_k q^k],  c_k = -H_k a_k
   Y1 = (2/pi) (ln(x/2) + gamma) J1 - 2/(pi x) - (x/(2 pi)) sum d_k q^k,
                                d_k = (2 H_k + 1/(k+1)) b_k
-(H_k the harmonic numbers; exact rationals rounded once to double).
+(H_k the harmonic numbers).
 
 For x >= X1:  H_nu(x) = sqrt(2/(pi x)) e^{i (x - nu pi/2 - pi/4)} (P_nu + i Q_nu)(s),
 s = X1/x in (0, 1].  The amplitude M_nu = P_nu + i Q_nu is smooth in s (it tends
@@ -28,8 +30,8 @@ import mpmath as mp
 import numpy as np
 
 X1 = 4
-NFIT = 20
-NSER = 17
+NFIT = 18
+NSER = 15
 mp.mp.dps = 40
 
 
@@ -37,15 +39,22 @@ def series():
     """Rows (a_k, b_k, c_k, d_k), k = 0..NSER-1, as doubles."""
     rows = []
     fk, H = Fraction(1), Fraction(0)
-    for k in range(NSER):
+    for k in range(45):
         if k > 0:
             fk *= k
             H += Fraction(1, k)
         ak = Fraction((-1) ** k) / (fk * fk)
         bk = Fraction((-1) ** k) / (fk * fk * (k + 1))
-        rows.append([float(ak), float(bk), float(-H * ak),
-                     float((2 * H + Fraction(1, k + 1)) * bk)])
-    return rows
+        rows.append([mp.mpf(v.numerator) / v.denominator
+                     for v in (ak, bk, -H * ak, (2 * H + Fraction(1, k + 1)) * bk)])
+    qmax = mp.mpf(X1) ** 2 / 4
+    cols = []
+    for j in range(4):
+        # in v = q / qmax on [0, 1]
+        c = cheb_interp_monomial(
+            lambda v: sum(r[j] * (v * qmax) ** k for k, r in enumerate(rows)), NSER - 1)
+        cols.append([float(p.real / qmax ** k) for k, p in enumerate(c)])
+    return [[cols[j][k] for j in range(4)] for k in range(NSER)]
 
 
 def amplitude(nu, x):
@@ -80,7 +89,7 @@ def cheb_interp_monomial(f, deg):
 def main():
     print("// Generated by gen_hank64.py -- FP64 coefficients of H0, H1 for real")
     print("// arguments.  FMM2D_H64_SER: rows (a_k, b_k, c_k, d_k) of the ascending")
-    print("// series in q = x^2/4, k = 0..NSER-1 (x < X1).  FMM2D_H64_AMP: rows")
+    print("// series' interpolants in q = x^2/4, k = 0..NSER-1 (x < X1).  FMM2D_H64_AMP: rows")
     print("// (P0, Q0, P1, Q1)_k of the amplitude polynomials in s = X1 / x, k = 0..NFIT")
     print("// (x >= X1).  Low order first.")
     print("#pragma once")

@@ -16,14 +16,14 @@
 //                      the terms fall below 1e-17 relative.
 //
 // Real positive z = x (every real wavenumber) takes its own path, hank01_real:
-//   x < 4              the ascending series as four polynomials of degree 16
-//                      in q = x^2/4 (Horner's rule; coefficients exact
-//                      rationals rounded once) and one logarithm;
+//   x < 4              the ascending series as four polynomials of degree 14
+//                      in q = x^2/4 (Chebyshev interpolants of its sums) and
+//                      one logarithm;
 //   x >= 4             H_nu(x) = sqrt(2/(pi x)) e^{i (x - nu pi/2 - pi/4)} M_nu(4/x),
-//                      the amplitude M_nu as polynomials of degree 20 in s = 4/x
+//                      the amplitude M_nu as polynomials of degree 18 in s = 4/x
 //                      (Chebyshev interpolants computed with mpmath; error about
 //                      one unit in the last place of |M| ~ 1), so a pair costs a
-//                      reciprocal, a square root, one sincos and 84 fused
+//                      reciprocal square root, one sincos and 72 fused
 //                      multiply-adds with no data-dependent loop.
 //                      Both tables: hank64_tables.h (gen_hank64.py).
 //
@@ -261,37 +261,37 @@ FMM2D_HD void hank01_real(double x, cplx* h0, cplx* h1) {
     double a = tab[4 * n], b = tab[4 * n + 1], c = tab[4 * n + 2], d = tab[4 * n + 3];
 #pragma unroll
     for (int k = n - 1; k >= 0; --k) {
-      a = fma(a, q, tab[4 * k]);
-      b = fma(b, q, tab[4 * k + 1]);
-      c = fma(c, q, tab[4 * k + 2]);
-      d = fma(d, q, tab[4 * k + 3]);
+      a = fma_k(a, q, tab[4 * k]);
+      b = fma_k(b, q, tab[4 * k + 1]);
+      c = fma_k(c, q, tab[4 * k + 2]);
+      d = fma_k(d, q, tab[4 * k + 3]);
     }
     const double xh = 0.5 * x;
     const double J1 = xh * b;
-    const double L = fast_log(xh) + kEuler;
+    const double L = fma_k(2.0, fast_hlog(xh), kEuler);
     const double Y0 = (2.0 / kPi) * fma(L, a, c);
     const double Y1 = (2.0 / kPi) * (L * J1) - (2.0 / kPi) * fast_rcp(x) - (1.0 / kPi) * (xh * d);
     *h0 = cplx{a, Y0};
     *h1 = cplx{J1, Y1};
     return;
   }
-  const double t = fast_rcp(x);
-  const double s = FMM2D_H64_X1 * t;
+  const double y = fast_rsqrt(x);
+  const double s = FMM2D_H64_X1 * (y * y);
   constexpr int o = 4 * FMM2D_H64_NSER, n = FMM2D_H64_NFIT;
   double p0 = tab[o + 4 * n], q0 = tab[o + 4 * n + 1], p1 = tab[o + 4 * n + 2],
          q1 = tab[o + 4 * n + 3];
 #pragma unroll
   for (int k = n - 1; k >= 0; --k) {
-    p0 = fma(p0, s, tab[o + 4 * k]);
-    q0 = fma(q0, s, tab[o + 4 * k + 1]);
-    p1 = fma(p1, s, tab[o + 4 * k + 2]);
-    q1 = fma(q1, s, tab[o + 4 * k + 3]);
+    p0 = fma_k(p0, s, tab[o + 4 * k]);
+    q0 = fma_k(q0, s, tab[o + 4 * k + 1]);
+    p1 = fma_k(p1, s, tab[o + 4 * k + 2]);
+    q1 = fma_k(q1, s, tab[o + 4 * k + 3]);
   }
   // sqrt(2/(pi x)) e^{i (x - pi/4)}: e^{i x} first, then the fixed rotation,
   // so the phase keeps the accuracy of sincos(x)
   double sn, cs;
-  sincos(x, &sn, &cs);
-  const double m = sqrt((2.0 / kPi) * t) * 0.70710678118654752440;
+  fast_sincos(x, &sn, &cs);
+  const double m = 0.56418958354775628695 * y;  // 1 / sqrt(pi x)
   const cplx e{m * (cs + sn), m * (sn - cs)};
   *h0 = e * cplx{p0, q0};
   const cplx m1 = e * cplx{p1, q1};

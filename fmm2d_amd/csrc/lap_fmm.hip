@@ -534,7 +534,7 @@ __global__ __launch_bounds__(kP2lWaves * kW) void k_p2l_w(
             const cplx u = r * zi;
             if (IFD) e = -(zi * dps[j * nd + d]);
             cplx t0 = e;
-            if (IFC) t0 += (0.5 * fast_log(rr)) * q;
+            if (IFC) t0 += fast_hlog(rr) * q;
             row[0] = t0;
             cplx v = mkc(1.0);  // u^m
             for (int m = 1; m <= p; ++m) {
@@ -622,7 +622,7 @@ __device__ __forceinline__ void mp_eval(double x, double y, int c, int nd, int d
   const cplx m0 = M[0];
   cplx g, g1, g2;
   horner<PG>(M, pc, true, u, g, g1, g2);
-  ap += (0.5 * fast_log(rr)) * m0 + g;
+  ap += fast_hlog(rr) * m0 + g;
   if (PG >= 2) {
     const cplx u2 = u * u;
     ag += (u * rci) * m0 - (u2 * rci) * g1;
@@ -863,7 +863,7 @@ __device__ __forceinline__ void pair_c64(double dx, double dy, double rr, const 
   const cplx zinv = cplx{dx * ri, -dy * ri};  // 1/z
   const cplx z2 = -(zinv * zinv);             // -1/z^2
   const cplx z3 = (-2.0) * (z2 * zinv);       // 2/z^3
-  const double lg = IFC ? 0.5 * fast_log(rr) : 0.0;
+  const double lg = IFC ? fast_hlog(rr) : 0.0;
 #pragma unroll
   for (int d = 0; d < NDT; ++d) {
     if (IFC) {

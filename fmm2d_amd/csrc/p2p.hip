@@ -77,9 +77,9 @@ __global__ __launch_bounds__(kTile) void direct_kernel(
     }
     __syncthreads();
     if (active) {
-      const int kb = w * TT, ke = min(nload, kb + TT);
-#pragma unroll(FAM == HELM ? 1 : 2)
-      for (int k = kb; k < ke; ++k) {
+      // (uniform: the same wave has the same w)
+      const int kb = __builtin_amdgcn_readfirstlane(w) * TT, ke = min(nload, kb + TT);
+      auto strengths = [&](int k) {
         SrcStr<NDT> s;
 #pragma unroll
         for (int d = 0; d < NDT; ++d) {
@@ -90,14 +90,19 @@ __global__ __launch_bounds__(kTile) void direct_kernel(
             s.dv[d][1] = sm.dv[(k * NDT + d) * 2 + 1];
           }
         }
+        return s;
+      };
+      auto pair = [&](int k) {
         const double dx = tx - sm.x[k], dy = ty - sm.y[k];
         if constexpr (FAM == CAUCHY)
-          pair_cauchy<IFC, IFD, PG, NDT>(dx, dy, s, thresh, thresh2, acc);
+          pair_cauchy<IFC, IFD, PG, NDT>(dx, dy, strengths(k), thresh, thresh2, acc);
         else if constexpr (FAM == LAPLACE)
-          pair_laplace<IFC, IFD, PG, NDT>(dx, dy, s, thresh, thresh2, acc);
+          pair_laplace<IFC, IFD, PG, NDT>(dx, dy, strengths(k), thresh, thresh2, acc);
         else
-          pair_helm<IFC, IFD, PG, NDT>(dx, dy, zk, s, thresh, acc);
-      }
+          pair_helm<IFC, IFD, PG, NDT>(dx, dy, zk, strengths(k), thresh, acc);
+      };
+#pragma unroll(FAM == HELM ? 1 : 2)
+      for (int k = kb; k < ke; ++k) pair(k);
     }
   }
   if constexpr (WS > 1) {

@@ -81,7 +81,7 @@ FMM2D_HD void pair_cauchy(double dx, double dy, const SrcStr<NDT>& s, double thr
   cplx z2 = -(zinv * zinv);                  // -1/z^2
   cplx z3 = (-2.0) * (z2 * zinv);             // 2/z^3
   double lg = 0.0;
-  if (IFC) lg = 0.5 * fast_log(rr);
+  if (IFC) lg = fast_hlog(rr);
 #pragma unroll
   for (int d = 0; d < NDT; ++d) {
     if (IFC) {
@@ -109,7 +109,7 @@ FMM2D_HD void pair_laplace(double dx, double dy, const SrcStr<NDT>& s, double th
   double px = dx * rinv, py = dy * rinv;  // charge gradient kernel
   double hxx = (rr - 2.0 * dx2) * rinv2, hxy = -2.0 * dx * dy * rinv2, hyy = (rr - 2.0 * dy2) * rinv2;
   double lg = 0.0;
-  if (IFC) lg = 0.5 * fast_log(rr);
+  if (IFC) lg = fast_hlog(rr);
   // dipole third-derivative kernel
   double rinv3 = rinv2 * rinv;
   double t1 = -2.0 * dx * (dx2 - 3.0 * dy2) * rinv3;
@@ -141,6 +141,51 @@ FMM2D_HD void pair_laplace(double dx, double dy, const SrcStr<NDT>& s, double th
 }
 
 // ---------------------------------------------------------------- Helmholtz
+// Potential and gradient of one pair for a real wavenumber, from H0 and H1 at
+// k r.  The same sums as in pair_helm with every factor that is real or
+// imaginary kept so, and with n = (dx, dy) / r and H2 = 2 H1 / x - H0 the
+// dipole's gradient as
+//   grad = -(i k^2 / 4) dipstr [n (n.v) H2 - v H1 / x]
+// (helmkernels2d.f:349-560): 55 instructions with charges and dipoles where
+// the complex form took 120.
+template <int IFC, int IFD, int PG, int NDT>
+FMM2D_HD void pair_helm_real(double dx, double dy, double k, double rinv, cplx h0, cplx h1,
+                             const SrcStr<NDT>& s, Acc<HELM, PG, NDT>& a) {
+  const double k4 = 0.25 * k;
+  if (IFC) {
+    const cplx p0{-0.25 * h0.im, 0.25 * h0.re};  // i/4 H0
+    const double w = k4 * rinv;
+    const cplx cdd{w * h1.im, -w * h1.re};  // -(i k/4) H1 / r
+#pragma unroll
+    for (int d = 0; d < NDT; ++d) {
+      const cplx c = s.charge[d];
+      a.pot[d] += p0 * c;
+      if (PG >= 2) {
+        const cplx cd = cdd * c;
+        a.grad[d][0] += cd * dx;
+        a.grad[d][1] += cd * dy;
+      }
+    }
+  }
+  if (IFD) {
+    const double ct = dx * rinv, st = dy * rinv;
+    const cplx c = (rinv * fast_rcp(k)) * h1;  // H1 / x
+    const cplx h2{fma(2.0, c.re, -h0.re), fma(2.0, c.im, -h0.im)};
+#pragma unroll
+    for (int d = 0; d < NDT; ++d) {
+      const double v1 = s.dv[d][0], v2 = s.dv[d][1];
+      const double vn = ct * v1 + st * v2;
+      const cplx e{-k4 * s.dipstr[d].im, k4 * s.dipstr[d].re};  // (i k/4) dipstr
+      a.pot[d] += (vn * h1) * e;
+      if (PG >= 2) {
+        const cplx A = vn * h2, f = -k * e;
+        a.grad[d][0] += (ct * A - v1 * c) * f;
+        a.grad[d][1] += (st * A - v2 * c) * f;
+      }
+    }
+  }
+}
+
 // OOL: evaluate the Hankel pair by a call to the general evaluator (for rarely
 // taken paths: their kernels then reserve neither registers nor scalar
 // registers for the table-driven real path).
@@ -148,21 +193,34 @@ template <int IFC, int IFD, int PG, int NDT, bool OOL = false>
 FMM2D_HD void pair_helm(double dx, double dy, cplx zk, const SrcStr<NDT>& s, double thresh,
                         Acc<HELM, PG, NDT>& a) {
   double rr = dx * dx + dy * dy;
-  double r = sqrt(rr);
+  // 1/r, then r with one correction (a point's own pair: r = 0)
+  const double rinv = fast_rsqrt(fmax(rr, 2.2250738585072014e-308));
+  double r = rr * rinv;
+  r = fma(fma(-r, r, rr), 0.5 * rinv, r);
   cplx z = zk * r;
   // |z| of a real wavenumber is |Re z| exactly (what hypot returns for it)
   const double absz = (zk.im == 0.0) ? fabs(z.re) : absc(z);
   if (skip_pair<HELM, IFC, IFD, PG>(rr, thresh, 0.0, absz)) return;
   cplx h0, h1;
-  if constexpr (OOL)
+  if constexpr (OOL) {
     hank01_complex(z, &h0, &h1);
-  else
-    hank01(z, &h0, &h1);
+  } else {
+    if constexpr (PG <= 2) {
+      // real wavenumber (the same for all pairs)
+      if (zk.im == 0.0 && zk.re > 0.0) {
+        hank01_real(z.re, &h0, &h1);
+        pair_helm_real<IFC, IFD, PG, NDT>(dx, dy, zk.re, rinv, h0, h1, s, a);
+        return;
+      }
+      hank01_complex(z, &h0, &h1);
+    } else {
+      hank01(z, &h0, &h1);
+    }
+  }
   const cplx ik4 = cplx{0.0, 0.25};
-  const double rinv = fast_rcp(r);
   const cplx kq = zk * ik4;  // i k / 4
   if (IFC) {
-    const cplx p0 = h0 * ik4;
+    const cplx p0{-0.25 * h0.im, 0.25 * h0.re};  // i/4 H0
     const cplx cdd = -(h1 * kq) * rinv;  // -(ik/4) H1 / r
     cplx hf1, hf2, hf3, cdd2;
     if (PG >= 3) {
