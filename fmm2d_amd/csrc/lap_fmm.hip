@@ -724,42 +724,23 @@ __device__ __forceinline__ void loc_eval32(double x, double y, int b, int P, con
   if (PG >= 3) ah = todbl(fscl((float)(2.0 * rinv * rinv), f2));
 }
 
-// Thread per point (any nd): local expansion, then the point's list-3 boxes.
-// The evaluation kernels are the first to write the sorted outputs: they
-// assign, and the near field adds after them.
-template <int PG>
-__global__ void k_eval(int64_t n, int nd, int P, const double* xy, const int* leaf,
-                       const int* ilevel, const int* nterms, const double* rsc,
-                       const double* centers, const int* n3, const int* l3, const cplx* mp,
-                       const cplx* loc, cplx* pot, cplx* grad, cplx* hess) {
-  const int64_t i = xcd_block() * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const int b = leaf[i];
-  const double x = xy[2 * i], y = xy[2 * i + 1];
-  const int c3 = n3[b];
-  for (int d = 0; d < nd; ++d) {
-    cplx ap, ag, ah;
-    loc_eval<PG>(x, y, b, nd, d, P, ilevel, nterms, rsc, centers, loc, ap, ag, ah);
-    for (int k3 = 0; k3 < c3; ++k3)
-      mp_eval<PG>(x, y, l3[(int64_t)kMaxList3 * b + k3], nd, d, P, ilevel, nterms, rsc, centers,
-                  mp, ap, ag, ah);
-    pot[i * nd + d] = ap;
-    if (PG >= 2) grad[i * nd + d] = ag;
-    if (PG >= 3) hess[i * nd + d] = ah;
-  }
-}
-
-// nd = 1: a block of kEvB consecutive points shares out their (point, list-3
-// box) pairs evenly -- in rounds of kEvB pairs, pair k to thread k mod kEvB,
-// its point found by binary search in the block's scan of list-3 counts --
-// so leaves with different list-3 lengths in one wavefront leave no lane
-// idle.  Each round's terms go to LDS, and each thread adds its own point's
-// terms from there in pair order (a fixed order: the sums do not depend on
-// scheduling).  Each thread then adds its own point's local expansion.
+// A block of kEvB consecutive points and one density (blockIdx.y) shares out
+// its (point, list-3 box) pairs evenly -- in rounds of kEvB pairs, pair k to
+// thread k mod kEvB, its point found by binary search in the block's scan of
+// list-3 counts -- so leaves with different list-3 lengths in one wavefront
+// leave no lane idle.  Each round's terms go to LDS, and each thread adds its
+// own point's terms from there in pair order (a fixed order: the sums do not
+// depend on scheduling).  Each thread then adds its own point's local
+// expansion.  The evaluation kernels are the first to write the sorted outputs:
+// they assign, and the near field adds after them.
+// Several densities: a thread per point that went through its densities in turn
+// was a chain of nd Horner loops in too few wavefronts: five densities at 1e5
+// points (Stokes) 404 -> 85 us, two with second derivatives at 5e4 359 -> 55 us.
 constexpr int kEvB = 256;
+constexpr int kEvMaxY = 32768;  // densities of one launch
 
 template <int PG, int F32>
-__global__ __launch_bounds__(kEvB) void k_eval_b(int64_t n, int P, const double* xy,
+__global__ __launch_bounds__(kEvB) void k_eval_b(int64_t n, int nd, int d0, int P, const double* xy,
                                                  const int* leaf, const int* ilevel,
                                                  const int* nterms, const double* rsc,
                                                  const double* centers, const int* n3,
@@ -773,7 +754,7 @@ __global__ __launch_bounds__(kEvB) void k_eval_b(int64_t n, int P, const double*
   __shared__ int sb[kEvB];
   __shared__ double sx[kEvB], sy[kEvB];
   __shared__ double part[2 * PG][kEvB];  // re, im of pot, grad, hess: one round's terms
-  const int tid = threadIdx.x;
+  const int tid = threadIdx.x, d = d0 + blockIdx.y;
   const int64_t i = xcd_block() * kEvB + tid;
   const bool live = i < n;
   const int b = live ? leaf[i] : 0;
@@ -804,7 +785,7 @@ __global__ __launch_bounds__(kEvB) void k_eval_b(int64_t n, int P, const double*
       if (F32)
         mp_eval32<PG>(sx[lo], sy[lo], c, P, ilevel, nterms, rsc, centers, mp32, ap, ag, ah);
       else
-        mp_eval<PG>(sx[lo], sy[lo], c, 1, 0, P, ilevel, nterms, rsc, centers, mp, ap, ag, ah);
+        mp_eval<PG>(sx[lo], sy[lo], c, nd, d, P, ilevel, nterms, rsc, centers, mp, ap, ag, ah);
       part[0][tid] = ap.re;
       part[1][tid] = ap.im;
       if (PG >= 2) {
@@ -828,10 +809,11 @@ __global__ __launch_bounds__(kEvB) void k_eval_b(int64_t n, int P, const double*
   if (!live) return;
   cplx ap, ag, ah;
   if (F32) loc_eval32<PG>(x, y, b, P, ilevel, nterms, rsc, centers, loc32, ap, ag, ah);
-  else loc_eval<PG>(x, y, b, 1, 0, P, ilevel, nterms, rsc, centers, loc, ap, ag, ah);
-  pot[i] = ap + cplx{my[0], my[1]};
-  if (PG >= 2) grad[i] = ag + cplx{my[2], my[3]};
-  if (PG >= 3) hess[i] = ah + cplx{my[4], my[5]};
+  else loc_eval<PG>(x, y, b, nd, d, P, ilevel, nterms, rsc, centers, loc, ap, ag, ah);
+  const int64_t at = i * nd + d;
+  pot[at] = ap + cplx{my[0], my[1]};
+  if (PG >= 2) grad[at] = ag + cplx{my[2], my[3]};
+  if (PG >= 3) hess[at] = ah + cplx{my[4], my[5]};
 }
 
 // ---------------------------------------------------------- near field
@@ -1426,18 +1408,20 @@ void launch_eval(int pg, int64_t n, hipStream_t st, int nd, int P, const double*
   const bool f32 = nd == 1 && mp32 && loc32;
 #define FMM2D_EVAL(PG)                                                                         \
   do {                                                                                         \
-    if (f32)                                                                                   \
-      launch1d_xcd(k_eval_b<PG, 1>, n, st, P, xy, leaf, t.ilevel.p, nterms, rsc, t.centers.p,  \
-                   L.n3.p, L.l3.p, mp, loc, mp32, loc32, p, g, h);                             \
-    else if (nd == 1)                                                                          \
-      launch1d_xcd(k_eval_b<PG, 0>, n, st, P, xy, leaf, t.ilevel.p, nterms, rsc, t.centers.p,  \
-                   L.n3.p, L.l3.p, mp, loc, (const float*)nullptr, (const float*)nullptr, p,   \
-                   g, h);                                                                      \
-    else                                                                                       \
-      launch1d_xcd(k_eval<PG>, n, st, nd, P, xy, leaf, t.ilevel.p, nterms, rsc, t.centers.p,   \
-                   L.n3.p, L.l3.p, mp, loc, p, g, h);                                          \
+    for (int d0 = 0; d0 < nd; d0 += kEvMaxY) {                                                 \
+      const dim3 grid(xcd_grid(ceil_div(n, kEvB)), (unsigned)std::min(nd - d0, kEvMaxY));      \
+      if (f32)                                                                                 \
+        hipLaunchKernelGGL((k_eval_b<PG, 1>), grid, dim3(kEvB), 0, st, n, nd, d0, P, xy, leaf, \
+                           t.ilevel.p, nterms, rsc, t.centers.p, L.n3.p, L.l3.p, mp, loc, mp32,\
+                           loc32, p, g, h);                                                    \
+      else                                                                                     \
+        hipLaunchKernelGGL((k_eval_b<PG, 0>), grid, dim3(kEvB), 0, st, n, nd, d0, P, xy, leaf, \
+                           t.ilevel.p, nterms, rsc, t.centers.p, L.n3.p, L.l3.p, mp, loc, mp32,\
+                           loc32, p, g, h);                                                    \
+      hip_throw(hipGetLastError(), "eval");                                                    \
+    }                                                                                          \
   } while (0)
-  static_assert(kEvB == 256, "launch1d_xcd launches blocks of 256 threads");
+  if (n <= 0) return;
   if (pg == 1) FMM2D_EVAL(1);
   else if (pg == 2) FMM2D_EVAL(2);
   else FMM2D_EVAL(3);
