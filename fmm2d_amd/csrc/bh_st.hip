@@ -32,6 +32,7 @@
 // gradient exactly as stokes/stfmm2d.f:184-300 does (including its constant
 // -sum(charge1) and the self term at the sources).
 #include "../../include/fmm2d_amd.h"
+#include <algorithm>
 #include "bh_st.h"
 #include "devbuf.h"
 #include "fastmath.h"
@@ -245,13 +246,13 @@ int64_t split_count(int64_t tblocks, int64_t ns) {
 // ---------------------------------------------------------------- bhfmm2d
 // the five Cauchy densities per biharmonic density (layout (5 nd, ns))
 __global__ void k_bh_densities(int64_t n, int nd, int ifc, int ifd, const double* src,
-                               double ox, double oy, const cplx* charge, const cplx* dip,
+                               const double* org, const cplx* charge, const cplx* dip,
                                cplx* cch, cplx* cdp) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;  // n = points x densities
   const int64_t j = i / nd;
   const int d = (int)(i - j * nd);
-  const cplx zj = cplx{src[2 * j] - ox, -(src[2 * j + 1] - oy)};  // conj(z~_j)
+  const cplx zj = cplx{src[2 * j] - org[0], -(src[2 * j + 1] - org[1])};  // conj(z~_j)
   const cplx c1 = ifc ? charge[(int64_t)nd * (2 * j) + d] : mkc(0.0);
   const cplx c2 = ifc ? charge[(int64_t)nd * (2 * j + 1) + d] : mkc(0.0);
   const cplx d1 = ifd ? dip[(int64_t)nd * (3 * j) + d] : mkc(0.0);
@@ -271,14 +272,14 @@ __global__ void k_bh_densities(int64_t n, int nd, int ifc, int ifd, const double
 }
 
 // the biharmonic outputs at n points from the Cauchy sums (5 nd densities)
-__global__ void k_bh_combine(int64_t n, int nd, int pg, const double* xy, double ox, double oy,
+__global__ void k_bh_combine(int64_t n, int nd, int pg, const double* xy, const double* org,
                              const cplx* P, const cplx* G, const cplx* H, cplx* vel,
                              cplx* grad) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;  // n = points x densities
   const int64_t j = i / nd;
   const int d = (int)(i - j * nd);
-  const cplx z = cplx{xy[2 * j] - ox, xy[2 * j + 1] - oy};
+  const cplx z = cplx{xy[2 * j] - org[0], xy[2 * j + 1] - org[1]};
   const int64_t b = 5 * i;
   const cplx C = P[b + 3] - G[b + 4];
   vel[i] = P[b + 0] + cj(P[b + 1] - G[b + 2]) + z * cj(C);
@@ -289,22 +290,12 @@ __global__ void k_bh_combine(int64_t n, int nd, int pg, const double* xy, double
   }
 }
 
-__global__ void k_bbox_centre(int64_t ns, const double* src, int64_t nt, const double* trg,
-                              double* out) {
-  // one block: min/max of x and y over sources and targets, then the centre
-  __shared__ double r[4][256];
-  double mn0 = 1e300, mx0 = -1e300, mn1 = 1e300, mx1 = -1e300;
-  for (int64_t i = threadIdx.x; i < ns + nt; i += blockDim.x) {
-    const double* p = i < ns ? src + 2 * i : trg + 2 * (i - ns);
-    mn0 = fmin(mn0, p[0]);
-    mx0 = fmax(mx0, p[0]);
-    mn1 = fmin(mn1, p[1]);
-    mx1 = fmax(mx1, p[1]);
-  }
-  r[0][threadIdx.x] = mn0;
-  r[1][threadIdx.x] = mx0;
-  r[2][threadIdx.x] = mn1;
-  r[3][threadIdx.x] = mx1;
+// Centre of the bounding box: every block's min and max of x and y over its
+// part of the sources and targets, then one block over the parts (a single
+// block over 1e5 points took 116 us, these two 8).
+constexpr int kCentreBlocks = 128;
+
+__device__ void block_minmax(double (&r)[4][256]) {
   __syncthreads();
   for (int s = 128; s > 0; s >>= 1) {
     if ((int)threadIdx.x < s) {
@@ -315,6 +306,34 @@ __global__ void k_bbox_centre(int64_t ns, const double* src, int64_t nt, const d
     }
     __syncthreads();
   }
+}
+
+__global__ __launch_bounds__(256) void k_bbox_part(int64_t ns, const double* src, int64_t nt,
+                                                   const double* trg, double* part) {
+  __shared__ double r[4][256];
+  double mn0 = 1e300, mx0 = -1e300, mn1 = 1e300, mx1 = -1e300;
+  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < ns + nt;
+       i += (int64_t)gridDim.x * 256) {
+    const double* p = i < ns ? src + 2 * i : trg + 2 * (i - ns);
+    mn0 = fmin(mn0, p[0]);
+    mx0 = fmax(mx0, p[0]);
+    mn1 = fmin(mn1, p[1]);
+    mx1 = fmax(mx1, p[1]);
+  }
+  r[0][threadIdx.x] = mn0;
+  r[1][threadIdx.x] = mx0;
+  r[2][threadIdx.x] = mn1;
+  r[3][threadIdx.x] = mx1;
+  block_minmax(r);
+  if (threadIdx.x < 4) part[4 * blockIdx.x + threadIdx.x] = r[threadIdx.x][0];
+}
+
+__global__ __launch_bounds__(256) void k_bbox_centre(int nparts, const double* part, double* out) {
+  __shared__ double r[4][256];
+  const int t = threadIdx.x;
+  for (int a = 0; a < 4; ++a)
+    r[a][t] = t < nparts ? part[4 * t + a] : ((a & 1) ? -1e300 : 1e300);
+  block_minmax(r);
   if (threadIdx.x == 0) {
     out[0] = 0.5 * (r[0][0] + r[1][0]);
     out[1] = 0.5 * (r[2][0] + r[3][0]);
@@ -350,13 +369,19 @@ __global__ void k_st_to_bh(int64_t n, int nd, int ifs, int ift, const double* st
   }
 }
 
-// zsum(d) = -sum_j charge1(d, j) (stfmm2d.f:186,198), one block per density
-__global__ void k_st_zsum(int64_t ns, int nd, const cplx* charge, cplx* zsum) {
+// zsum(d) = -sum_j charge1(d, j) (stfmm2d.f:186,198): the sums of kZsumBlocks
+// strided parts of the charges per density, then one block per density over
+// the parts in order (one block over 1e5 charges took 98 us, these two 8)
+constexpr int kZsumBlocks = 128;
+// stride, step: value j of density d is v[j stride + d step]
+__global__ __launch_bounds__(256) void k_st_zsum(int64_t ns, int64_t stride, int step, double sign,
+                                                 const cplx* v, cplx* zsum) {
   __shared__ double r[2][256];
   const int d = blockIdx.x;
   double sr = 0.0, si = 0.0;
-  for (int64_t j = threadIdx.x; j < ns; j += blockDim.x) {
-    const cplx c = charge[(int64_t)nd * (2 * j) + d];
+  for (int64_t j = (int64_t)blockIdx.y * 256 + threadIdx.x; j < ns;
+       j += (int64_t)gridDim.y * 256) {
+    const cplx c = v[j * stride + (int64_t)d * step];
     sr += c.re;
     si += c.im;
   }
@@ -370,7 +395,8 @@ __global__ void k_st_zsum(int64_t ns, int nd, const cplx* charge, cplx* zsum) {
     }
     __syncthreads();
   }
-  if (threadIdx.x == 0) zsum[d] = cplx{-r[0][0], -r[1][0]};
+  if (threadIdx.x == 0)
+    zsum[(int64_t)d * gridDim.y + blockIdx.y] = cplx{sign * r[0][0], sign * r[1][0]};
 }
 
 // stfmm2d.f:226-300: velocity, pressure and gradient from the biharmonic
@@ -403,12 +429,17 @@ int bh_fmm_impl(const BhArgs& a, hipStream_t st) {
   const int64_t ns = a.ns, nt = (a.ifpghtarg > 0) ? a.nt : 0;
   // origin: centre of the bounding box
   DBuf<double> dorg(2, st);
-  hipLaunchKernelGGL(k_bbox_centre, dim3(1), dim3(256), 0, st, ns, a.src, nt, a.targ, dorg.p);
-  double org[2];
-  readback(org, dorg.p, sizeof(org), st);
+  {
+    const int np = (int)std::max<int64_t>(1, std::min<int64_t>(kCentreBlocks, (ns + nt) / 256));
+    DBuf<double> part(4 * kCentreBlocks, st);
+    hipLaunchKernelGGL(k_bbox_part, dim3(np), dim3(256), 0, st, ns, a.src, nt, a.targ, part.p);
+    hipLaunchKernelGGL(k_bbox_centre, dim3(1), dim3(256), 0, st, np, (const double*)part.p,
+                       dorg.p);
+  }
+  const double* org = dorg.p;
   const int ndc = 5 * nd;
   DBuf<cplx> cch((size_t)ndc * ns, st), cdp((size_t)ndc * ns, st);
-  launch1d(k_bh_densities, ns * nd, st, nd, a.ifcharge, a.ifdipole, a.src, org[0], org[1],
+  launch1d(k_bh_densities, ns * nd, st, nd, a.ifcharge, a.ifdipole, a.src, org,
            a.charge, a.dip, cch.p, cdp.p);
   const int pg = a.ifpgh > 0 ? a.ifpgh + 1 : 0, pgt = (nt > 0) ? a.ifpghtarg + 1 : 0;
   DBuf<cplx> P((size_t)ndc * ns * (pg >= 1), st), G((size_t)ndc * ns * (pg >= 2), st),
@@ -439,10 +470,10 @@ int bh_fmm_impl(const BhArgs& a, hipStream_t st) {
   const int ier = laplace_fmm(0, c, st);
   if (ier != FMM2D_OK) return ier;
   if (a.ifpgh > 0)
-    launch1d(k_bh_combine, ns * nd, st, nd, a.ifpgh, a.src, org[0], org[1], P.p, G.p, H.p,
+    launch1d(k_bh_combine, ns * nd, st, nd, a.ifpgh, a.src, org, P.p, G.p, H.p,
              a.pot, a.grad);
   if (nt > 0)
-    launch1d(k_bh_combine, nt * nd, st, nd, a.ifpghtarg, a.targ, org[0], org[1], PT.p, GT.p,
+    launch1d(k_bh_combine, nt * nd, st, nd, a.ifpghtarg, a.targ, org, PT.p, GT.p,
              HT.p, a.pottarg, a.gradtarg);
   hip_throw(hipGetLastError(), "kernel launch");
   return FMM2D_OK;
@@ -584,7 +615,14 @@ int st_fmm(const StArgs& a, hipStream_t st) {
     dip.zero();
     launch1d(k_st_to_bh, ns * nd, st, nd, ifc, ifd, a.stoklet, a.strslet, a.strsvec, charge.p,
              dip.p);
-    hipLaunchKernelGGL(k_st_zsum, dim3(nd), dim3(256), 0, st, ns, nd, charge.p, zsum.p);
+    {
+      const unsigned nb = (unsigned)std::max<int64_t>(1, std::min<int64_t>(kZsumBlocks, ns / 256));
+      DBuf<cplx> part((size_t)nd * nb, st);
+      hipLaunchKernelGGL(k_st_zsum, dim3(nd, nb), dim3(256), 0, st, ns, (int64_t)2 * nd, 1, 1.0,
+                         (const cplx*)charge.p, part.p);
+      hipLaunchKernelGGL(k_st_zsum, dim3(nd), dim3(256), 0, st, (int64_t)nb, (int64_t)1,
+                         (int)nb, -1.0, (const cplx*)part.p, zsum.p);
+    }
     const int pg = a.ifppreg == 0 ? 0 : (a.ifppreg == 1 ? 1 : 2);
     const int pgt = a.ifppregtarg == 0 ? 0 : (a.ifppregtarg == 1 ? 1 : 2);
     DBuf<cplx> vel((size_t)nd * ns * (pg >= 1), st), grad((size_t)3 * nd * ns * (pg >= 2), st);
