@@ -343,7 +343,9 @@ __global__ __launch_bounds__(kW) void k_p2l(int nd, int P, const int* ilevel, co
 // P2M (l2dformmp{c,d,cd}, laprouts2d.f:84-282) for expansions of at most PT
 // coefficients: one thread per (box, density), for the leaves at levels >= 2,
 // runs over the leaf's sources with the running products w^n, w = (z - c)/r, accumulating
-// every coefficient in registers.  RE: real charges.
+// every coefficient in registers.  The first to write its expansion, it assigns
+// (adding to the cleared one, a chain of reads of whole cache lines for 16 bytes
+// each, took 903 us of lfmm2d N = 1e7 where this takes 389).  RE: real charges.
 template <int PT, int IFC, int IFD, int RE>
 __global__ __launch_bounds__(256) void k_p2m_reg(int64_t n, int nd, int P, const int* ilevel,
                                                  const int* nchild, const int* nterms,
@@ -417,7 +419,7 @@ __global__ __launch_bounds__(256) void k_p2m_reg(int64_t n, int nd, int P, const
   cplx* out = mp + ((int64_t)b * nd + d) * P;
 #pragma unroll
   for (int k = 0; k < PT; ++k)
-    if (k <= p) out[k] += acc[k];
+    if (k <= p) out[k] = acc[k];
 }
 
 // Orders one wavefront's LDS writes before its later LDS reads (the
