@@ -39,15 +39,12 @@ FMM2D_HD int m2l_slot(int q, int dx, int dy) {
   const int ix = dx - bx, iy = dy - by;
   if (ix < 0 || ix > 5 || iy < 0 || iy > 5) return -1;
   if (dx >= -1 && dx <= 1 && dy >= -1 && dy <= 1) return -1;
-  int s = 0;
-  for (int a = 0; a < 6; ++a)
-    for (int b = 0; b < 6; ++b) {
-      const int ex = bx + a, ey = by + b;
-      if (ex >= -1 && ex <= 1 && ey >= -1 && ey <= 1) continue;
-      if (a == ix && b == iy) return s;
-      ++s;
-    }
-  return -1;
+  // the cell's number in the 6 x 6 window, less the cells of the 3 x 3 block
+  // around the target (rows x0.., columns y0..) before it
+  const int x0 = -1 - bx, y0 = -1 - by;
+  const int rows = ix < x0 ? 0 : (ix > x0 + 2 ? 3 : ix - x0);
+  const int same = ix >= x0 && ix <= x0 + 2 && iy > y0 + 2 ? 3 : 0;
+  return 6 * ix + iy - 3 * rows - same;
 }
 
 struct Lists {
