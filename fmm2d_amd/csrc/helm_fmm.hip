@@ -1208,8 +1208,8 @@ __global__ __launch_bounds__(kMpsW) void k_mps_near(int64_t n, int nd, cplx zk, 
   }
 }
 
-// Host tables of the translation operators, level by level: next() makes one
-// level's, so that the caller can do so while the device is busy with
+// Host tables of the translation operators, level by level from the finest
+// (the cheapest) up: next() makes one level's, so that the caller can do so while the device is busy with
 // something else and look in between whether it has finished.
 struct HelmOps {
   const Tree& t;
@@ -1217,7 +1217,7 @@ struct HelmOps {
   const std::vector<long double>& sl;
   const std::vector<int>& nterms;
   lx k;
-  int nl, l = 1;
+  int nl, l;
   OpTables T;
   std::vector<int> m2l, m2m, l2l;  // first operator of the level, or -1
   std::vector<Phases> ph;          // of the 49 offsets, M2M and L2L
@@ -1225,8 +1225,8 @@ struct HelmOps {
   HelmOps(const Tree& t_, const std::vector<HLev>& lev_, const std::vector<long double>& sl_,
           const std::vector<int>& nterms_, cplx zk)
       : t(t_), lev(lev_), sl(sl_), nterms(nterms_), k{zk.re, zk.im}, nl(t_.nlevels),
-        m2l(nl + 1, -1), m2m(nl + 1, -1), l2l(nl + 1, -1), ph(51) {}
-  bool done() const { return l > nl; }
+        l(nl), m2l(nl + 1, -1), m2m(nl + 1, -1), l2l(nl + 1, -1), ph(51) {}
+  bool done() const { return l < 1; }
   void next();
 };
 
@@ -1294,7 +1294,7 @@ void HelmOps::next() {
       add_op(T, p, pc, push_table(T, Jp, mm, e), w1, w2, 1, -1, 1, kOpShift);
     }
   }
-  ++l;
+  --l;
 }
 
 // Box-to-box passes shared by hfmm2d and hfmm2d_mps (hfmm2d.f:1021-1300,
