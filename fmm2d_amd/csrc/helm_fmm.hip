@@ -151,56 +151,107 @@ __device__ void scaled_h(cplx z, double s, int m, cplx* out) {
 // The cylinder functions of each source (J/s^n about its leaf's centre for
 // P2M, H s^n about the target box's centre for P2L) are computed first, one
 // thread per source or (box, source) pair, into rows G; then one 64-lane
-// wavefront per box sums its rows, lane n adding to coefficients +-n:
+// wavefront per box sums its rows, a lane to every coefficient:
 //   charge  C_n += q G_n e^{-i n a},  C_{-n} += q (-1)^n G_n e^{i n a}
 //   dipole  C_n += q (k/2) [(v1 - i v2) g_{n-1} f_lo - (v1 + i v2) g_{n+1} f_hi]
 //           (g_j = G_|j| sign(j)^j e^{-i j a}; f_lo, f_hi powers of s from the
 //            scaling, swapped for negative n)
 // (h2dformmp{c,d,cd}, helmrouts2d.f:84-270 with ctompole/dtompole 1383-1490;
 //  h2dformta{c,d,cd}, helmrouts2d.f:517-705).
-template <int IFC, int IFD, int LOCAL>
-__device__ void accumulate_batch(int nd, int p, cplx zk, double s, const cplx* G, const cplx* U,
-                                 int nbat, int stride, int j0, const cplx* chs,
-                                 const cplx* dps, const double* dvs, cplx* out_p0) {
+//
+// A batch of up to 16 sources at a time: the wavefront forms W+_n = G_n e^{-i n
+// a} and W-_n = G_n e^{i n a} of the batch in LDS, a few lanes to a source, each
+// with one power by squaring and then products with e^{-i a}; then every lane
+// adds its coefficient's terms, which are single entries of W+ or W-.  With a
+// lane to every pair +-n and a power by squaring for each (lane, source), half
+// the lanes idled and the powers were most of the work: charges and dipoles of
+// 1e6 points (orders 20 to 27) P2M 460 -> 262 us, list 4 826 -> 355; charges on
+// the curve of 2e6 points 576 -> 565, 932 -> 624.  (4 KB a batch: 800 for 624;
+// four boxes a workgroup: 943.)
+constexpr int kHBatch = 16;
+constexpr int kHLds = 8192;  // bytes of a batch, unless one source needs more
+
+__host__ __device__ inline int hbatch_bytes(int p, int nb) {
+  return nb * (2 * (p + 2) + 3) * (int)sizeof(cplx);
+}
+
+// t-th row: G + t (p + 2), e^{-i a} U[t], source jof(t)
+template <int IFC, int IFD, int LOCAL, typename JOF>
+__device__ void accumulate_rows(int nd, int p, cplx zk, double s, const cplx* G, const cplx* U,
+                                int total, JOF jof, const cplx* chs, const cplx* dps,
+                                const double* dvs, cplx* sh, cplx* out_p0) {
   // LOCAL: (a_lo, a_hi) = (s, 1/s); multipole: (1/s, s)
   const double a_lo = LOCAL ? s : 1.0 / s, a_hi = LOCAL ? 1.0 / s : s;
   const cplx k2 = 0.5 * zk;
-  for (int n = threadIdx.x; n <= p; n += kW) {
-    const double sg = (n & 1) ? -1.0 : 1.0;
-    for (int d = 0; d < nd; ++d) {
-      cplx ap = mkc(0.0), am = mkc(0.0);
-      for (int jj = 0; jj < nbat; ++jj) {
-        const cplx* g = G + (int64_t)jj * stride;
-        const cplx u = U[jj];  // e^{-i a}
-        const cplx en = cpowi(u, n), ep = conjc(en);
-        const int64_t j = j0 + jj;
-        if (IFC) {
-          const cplx q = chs[j * nd + d];
-          const cplx t = q * g[n];
-          ap += t * en;
-          if (n > 0) am += sg * (t * ep);
-        }
-        if (IFD) {
-          const cplx q = k2 * dps[j * nd + d];
-          const double v1 = dvs[(2 * j) * nd + d], v2 = dvs[(2 * j + 1) * nd + d];
-          const cplx al = cplx{v1, -v2}, be = cplx{v1, v2};
-          const cplx ub = conjc(u);
-          if (n == 0) {
-            // g_{-1} = -G_1 e^{i a}, g_1 = G_1 e^{-i a}
-            ap += (q * a_hi) * (-(al * (g[1] * ub)) - be * (g[1] * u));
-          } else {
-            // +n: g_{n-1} = G_{n-1} e^{-i(n-1)a}, g_{n+1} = G_{n+1} e^{-i(n+1)a}
-            ap += q * ((a_lo * (al * (g[n - 1] * (en * ub)))) -
-                       (a_hi * (be * (g[n + 1] * (en * u)))));
-            // -n: g_{-n-1} = -sg G_{n+1} e^{i(n+1)a}, g_{-n+1} = -sg G_{n-1} e^{i(n-1)a}
-            am += q * ((a_hi * (al * ((-sg) * (g[n + 1] * (ep * ub))))) -
-                       (a_lo * (be * ((-sg) * (g[n - 1] * (ep * u))))));
+  const int lane = threadIdx.x, W = p + 2, nc = 2 * p + 1;
+  int nb = kHBatch;
+  while (nb > 1 && hbatch_bytes(p, nb) > kHLds) nb >>= 1;
+  const int ls = kW / nb, seg = (W + ls - 1) / ls;  // lanes a source, rows a lane
+  cplx* wp = sh;
+  cplx* wm = wp + nb * W;
+  cplx* sq = wm + nb * W;  // q, k/2 dipstr (v1 - i v2), k/2 dipstr (v1 + i v2) a source
+  for (int d = 0; d < nd; ++d) {
+    for (int m0 = 0; m0 < nc; m0 += 2 * kW) {
+      cplx acc[2] = {mkc(0.0), mkc(0.0)};
+      for (int t0 = 0; t0 < total; t0 += nb) {
+        const int cnt = min(nb, total - t0);
+        const int jj = lane / ls;
+        if (jj < cnt) {
+          const cplx u = U[t0 + jj];
+          const cplx* g = G + (int64_t)(t0 + jj) * W;
+          const int n0 = (lane - jj * ls) * seg, n1 = min(W, n0 + seg);
+          cplx e = cpowi(u, n0);
+          for (int n = n0; n < n1; ++n) {
+            const cplx v = g[n];
+            wp[jj * W + n] = v * e;
+            wm[jj * W + n] = v * conjc(e);
+            e = e * u;
           }
         }
+        if (lane < cnt) {
+          const int64_t j = jof(t0 + lane);
+          if (IFC) sq[3 * lane] = chs[j * nd + d];
+          if (IFD) {
+            const cplx q = k2 * dps[j * nd + d];
+            const double v1 = dvs[(2 * j) * nd + d], v2 = dvs[(2 * j + 1) * nd + d];
+            sq[3 * lane + 1] = q * cplx{v1, -v2};
+            sq[3 * lane + 2] = q * cplx{v1, v2};
+          }
+        }
+        wave_lds_fence();
+#pragma unroll
+        for (int a = 0; a < 2; ++a) {
+          const int m = m0 + lane + a * kW;
+          if (m >= nc) continue;
+          const bool neg = m < p;
+          const int n = neg ? p - m : m - p;
+          const cplx* w = (neg ? wm : wp) + n;
+          // the dipole's two terms: entries n -+ 1 of the same rows, at n = 0
+          // entry 1 of either
+          const cplx* w1 = n == 0 ? wm + 1 : neg ? w + 1 : w - 1;
+          const cplx* w2 = n == 0 ? wp + 1 : neg ? w - 1 : w + 1;
+          const double f1 = neg || n == 0 ? -a_hi : a_lo, f2 = neg ? a_lo : -a_hi;
+          cplx t = mkc(0.0), s1 = mkc(0.0), s2 = mkc(0.0);
+          for (int k = 0; k < cnt; ++k) {
+            if (IFC) t += sq[3 * k] * w[k * W];
+            if (IFD) {
+              s1 += sq[3 * k + 1] * w1[k * W];
+              s2 += sq[3 * k + 2] * w2[k * W];
+            }
+          }
+          if (IFD) t += f1 * s1 + f2 * s2;
+          acc[a] += t;
+        }
+        wave_lds_fence();  // the next batch overwrites the rows
       }
-      cplx* c = out_p0 + (int64_t)d * (2 * p + 1);
-      c[n] += ap;
-      if (n > 0) c[-n] += am;
+#pragma unroll
+      for (int a = 0; a < 2; ++a) {
+        const int m = m0 + lane + a * kW;
+        if (m < nc) {
+          const bool odd = m < p && ((p - m) & 1);
+          out_p0[(int64_t)d * nc + (m - p)] += odd ? -acc[a] : acc[a];
+        }
+      }
     }
   }
 }
@@ -220,19 +271,53 @@ __global__ void k_hp2m_rowlen(int64_t n, const HLev* lev, const int* leaf, const
   len[i] = (l >= 2 && lev[l].on) ? lev[l].p + 2 : 0;
 }
 
-__global__ void k_hp2m_rows(int64_t n, cplx zk, const HLev* lev, const int* leaf,
-                            const int* ilevel, const double* centers, const double* xs,
-                            const int64_t* roff, cplx* G, cplx* U) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const int b = leaf[i];
-  const int l = ilevel[b];
-  const HLev L = lev[l];
-  if (l < 2 || !L.on) return;
-  const double dx = xs[2 * i] - centers[2 * b], dy = xs[2 * i + 1] - centers[2 * b + 1];
-  const double r = hypot(dx, dy);
-  scaled_j(zk * r, L.s, L.p + 1, G + roff[i]);
-  U[i] = (r > 0.0) ? cplx{dx / r, -dy / r} : mkc(1.0);
+//
+// A wavefront's rows are formed in LDS (rowcap values a row at most, an odd
+// stride) and copied out row by row, consecutive lanes on consecutive values;
+// longer rows are formed in place.  In place, every step of the recurrence
+// wrote 16 bytes to each of 64 lines, and the lines left the L2 half written:
+// 1e6 points 634 -> 277 us.  (List 4's rows are written once as they are: in LDS
+// they took 924 us for 678.)
+constexpr int kRowCap = 31;  // 31 KB a wavefront: orders up to 29
+
+// The rows of the lanes with w > 0 values at sh + lane * stride to dst (lane's)
+__device__ __forceinline__ void copy_rows(const cplx* sh, int stride, int w, cplx* dst) {
+  wave_lds_fence();
+  for (unsigned long long m = __ballot(w > 0); m; m &= m - 1) {
+    const int r = __ffsll((long long)m) - 1;
+    const int n = __builtin_amdgcn_readlane(w, r);
+    const unsigned long long at = (unsigned long long)dst;
+    const unsigned lo = __builtin_amdgcn_readlane((int)(unsigned)at, r),
+                   hi = __builtin_amdgcn_readlane((int)(unsigned)(at >> 32), r);
+    cplx* o = (cplx*)(((unsigned long long)hi << 32) | lo);
+    const int lane = threadIdx.x;
+    if (lane < n) o[lane] = sh[r * stride + lane];
+  }
+}
+
+__global__ __launch_bounds__(kW) void k_hp2m_rows(int64_t n, cplx zk, const HLev* lev,
+                                                  const int* leaf, const int* ilevel,
+                                                  const double* centers, const double* xs,
+                                                  const int64_t* roff, cplx* G, cplx* U) {
+  __shared__ cplx sh[kW * kRowCap];
+  const int64_t i = (int64_t)blockIdx.x * kW + threadIdx.x;
+  int w = 0;
+  cplx* dst = G;
+  if (i < n) {
+    const int b = leaf[i];
+    const int l = ilevel[b];
+    const HLev L = lev[l];
+    if (l >= 2 && L.on) {
+      const double dx = xs[2 * i] - centers[2 * b], dy = xs[2 * i + 1] - centers[2 * b + 1];
+      const double r = hypot(dx, dy);
+      dst = G + roff[i];
+      const bool in = L.p + 2 <= kRowCap;
+      scaled_j(zk * r, L.s, L.p + 1, in ? sh + threadIdx.x * kRowCap : dst);
+      if (in) w = L.p + 2;
+      U[i] = (r > 0.0) ? cplx{dx / r, -dy / r} : mkc(1.0);
+    }
+  }
+  copy_rows(sh, kRowCap, w, dst);
 }
 
 // Then one wavefront per leaf sums its sources' rows into the multipole
@@ -249,8 +334,10 @@ __global__ __launch_bounds__(kW) void k_hp2m_g(int nd, cplx zk, const HLev* lev,
   if (l < 2 || !L.on || nchild[b] != 0) return;
   const int s0 = sse[2 * b], s1 = sse[2 * b + 1];
   if (s1 <= s0) return;
-  accumulate_batch<IFC, IFD, 0>(nd, L.p, zk, L.s, G + roff[s0], U + s0, s1 - s0, L.p + 2, s0,
-                                chs, dps, dvs, hexp(mp, L, b, nd, 0));
+  extern __shared__ cplx sh[];
+  accumulate_rows<IFC, IFD, 0>(
+      nd, L.p, zk, L.s, G + roff[s0], U + s0, s1 - s0, [=](int t) { return s0 + t; }, chs, dps,
+      dvs, sh, hexp(mp, L, b, nd, 0));
 }
 
 // List 4 in three steps, like P2M.  cnt[b] = sources of the list-4 boxes of
@@ -307,7 +394,7 @@ __global__ void k_hp2l_rows(int64_t np, int nb, cplx zk, const HLev* lev, const 
 }
 
 // One wavefront per box with list-4 work sums its pairs' rows into its local
-// expansion, list-4 box after list-4 box (their sources are contiguous).
+// expansion.
 template <int IFC, int IFD>
 __global__ __launch_bounds__(kW) void k_hp2l_g(int nd, cplx zk, const HLev* lev,
                                                const int* ilevel, const int* n4, const int* l4,
@@ -318,19 +405,25 @@ __global__ __launch_bounds__(kW) void k_hp2l_g(int nd, cplx zk, const HLev* lev,
   const int b = blockIdx.x;
   if (cnt[b] == 0) return;
   const HLev L = lev[ilevel[b]];
-  const int pstride = L.p + 2;
-  cplx* out = hexp(loc, L, b, nd, 0);
-  const int64_t pos0 = off[b];
-  int64_t pos = pos0;
-  const cplx* Gb = G + roff[b];  // row of pair pos at Gb + (pos - pos0) * pstride
-  for (int k = 0; k < n4[b]; ++k) {
-    const int c = l4[(int64_t)kMaxList4 * b + k];
-    const int c0 = sse[2 * c], c1 = sse[2 * c + 1];
-    if (c1 <= c0) continue;
-    accumulate_batch<IFC, IFD, 1>(nd, L.p, zk, L.s, Gb + (pos - pos0) * pstride, U + pos, c1 - c0,
-                                  pstride, c0, chs, dps, dvs, out);
-    pos += c1 - c0;
+  // list-4 box k's sources are rows pre[k] .. pre[k + 1]
+  int pre[kMaxList4 + 1], first[kMaxList4];
+  pre[0] = 0;
+#pragma unroll
+  for (int k = 0; k < kMaxList4; ++k) {
+    const int c = k < n4[b] ? l4[(int64_t)kMaxList4 * b + k] : -1;
+    first[k] = c >= 0 ? sse[2 * c] : 0;
+    pre[k + 1] = pre[k] + (c >= 0 ? sse[2 * c + 1] - sse[2 * c] : 0);
   }
+  auto jof = [&](int t) {
+    int j = first[0] + t;
+#pragma unroll
+    for (int k = 1; k < kMaxList4; ++k)
+      if (t >= pre[k]) j = first[k] + (t - pre[k]);
+    return j;
+  };
+  extern __shared__ cplx sh[];
+  accumulate_rows<IFC, IFD, 1>(nd, L.p, zk, L.s, G + roff[b], U + off[b], cnt[b], jof, chs, dps,
+                               dvs, sh, hexp(loc, L, b, nd, 0));
 }
 
 // ---------------------------------------------------------- evaluation
@@ -1536,13 +1629,16 @@ int helmholtz_fmm(const HelmArgs& a, hipStream_t st) {
     while (!ops.done() && !sizes.ready()) ops.next();
     sizes.finish(hrow, &np4);
     const int64_t nrow = hrow[0], nrow4 = hrow[1];
+    size_t hlds = kHLds;
+    for (int l = 2; l <= nl; ++l) hlds = std::max(hlds, (size_t)hbatch_bytes(nterms[l], 1));
     // ---- step 1: P2M (rows of the sources, then their sums per leaf)
     {
       DBuf<cplx> gJ(std::max<int64_t>(nrow, 1), st), uJ(ns, st);
-      launch1d(k_hp2m_rows, ns, st, zk, d_lev, t.leaf_s.p, t.ilevel.p, t.centers.p, xs.p,
-               (const int64_t*)roff.p, gJ.p, uJ.p);
+      hipLaunchKernelGGL(k_hp2m_rows, dim3(ceil_div(ns, kW)), dim3(kW), 0, st, ns, zk, d_lev,
+                         t.leaf_s.p, t.ilevel.p, t.centers.p, xs.p, (const int64_t*)roff.p, gJ.p,
+                         uJ.p);
 #define FMM2D_P2M(C, D)                                                                       \
-  hipLaunchKernelGGL((k_hp2m_g<C, D>), dim3(nb), dim3(kW), 0, st, nd, zk, d_lev, t.ilevel.p, \
+  hipLaunchKernelGGL((k_hp2m_g<C, D>), dim3(nb), dim3(kW), hlds, st, nd, zk, d_lev, t.ilevel.p,     \
                      t.nchild.p, sse, (const int64_t*)roff.p, gJ.p, uJ.p, chs.p, dps.p, dvs.p,  \
                      mp.p)
       if (a.ifcharge && !a.ifdipole) FMM2D_P2M(1, 0);
@@ -1559,7 +1655,7 @@ int helmholtz_fmm(const HelmArgs& a, hipStream_t st) {
         launch1d(k_hp2l_rows, np4, st, nb, zk, d_lev, t.ilevel.p, t.centers.p, L.l4.p, sse,
                  off4.p, xs.p, (const int64_t*)roff4.p, gH.p, uH.p);
 #define FMM2D_P2L(C, D)                                                                       \
-  hipLaunchKernelGGL((k_hp2l_g<C, D>), dim3(nb), dim3(kW), 0, st, nd, zk, d_lev, t.ilevel.p, \
+  hipLaunchKernelGGL((k_hp2l_g<C, D>), dim3(nb), dim3(kW), hlds, st, nd, zk, d_lev, t.ilevel.p,     \
                      L.n4.p, L.l4.p, sse, cnt4.p, off4.p, (const int64_t*)roff4.p, gH.p, uH.p, \
                      chs.p, dps.p, dvs.p, loc.p)
         if (a.ifcharge && !a.ifdipole) FMM2D_P2L(1, 0);
