@@ -174,8 +174,11 @@ __global__ __launch_bounds__(64 * NW) void k_m2l(int nd, int per_xcd, M2LTab tab
   for (int a = 0; a < 4; ++a)
 #pragma unroll
     for (int r = 0; r < RTC; ++r) acc[a][r] = acc_t{0, 0, 0, 0};
-  // FP32: z is formed in FP64 and rounded once, and every orbit's sums are folded into FP64 ones (a long FP32 chain over
-  // the orbits doubled the error of hfmm2d, zk 30, eps 1e-6)
+  // FP32: z is formed in FP64 and rounded once, and the sums are folded into
+  // FP64 ones after every second class of an orbit (hfmm2d N = 1e5, zk 30, eps
+  // 1e-6: error against direct sums 1.1e-7, the kernel 0.39 ms; a fold an orbit
+  // 1.5e-7, a little more than the one-source operators before it, and 0.29 ms; a
+  // fold a class 1.0e-7, 0.42 ms; one chain over all orbits 3e-7)
   constexpr bool FOLD = sizeof(T) == 4;
   d4v sum[FOLD ? 4 : 1][FOLD ? RTC : 1];
 #pragma unroll
@@ -297,21 +300,21 @@ __global__ __launch_bounds__(64 * NW) void k_m2l(int nd, int per_xcd, M2LTab tab
                                         acc[a][r]);
           }
         }
+        if (FOLD && (b & 1)) {
+#pragma unroll
+          for (int a = 0; a < 4; ++a)
+#pragma unroll
+            for (int r = 0; r < RTC; ++r) {
+#pragma unroll
+              for (int i = 0; i < 4; ++i) sum[FOLD ? a : 0][FOLD ? r : 0][i] += (double)acc[a][r][i];
+              acc[a][r] = acc_t{0, 0, 0, 0};
+            }
+        }
         if (chunk + 1 < NCH) store_a(cur ^ 1, ar[cur ^ 1]);
         __syncthreads();
       }
       store_z();
       wave_lds_fence();
-    }
-    if constexpr (FOLD) {
-#pragma unroll
-      for (int a = 0; a < 4; ++a)
-#pragma unroll
-        for (int r = 0; r < RTC; ++r) {
-#pragma unroll
-          for (int i = 0; i < 4; ++i) sum[a][r][i] += (double)acc[a][r][i];
-          acc[a][r] = acc_t{0, 0, 0, 0};
-        }
     }
   }
   if (tb < 0) return;
@@ -339,7 +342,7 @@ __global__ __launch_bounds__(64 * NW) void k_m2l(int nd, int per_xcd, M2LTab tab
 }
 
 // The M2L of the given levels (blk0 is set here), one launch per tile shape.
-// fp32: operators and z are float (an orbit's sums FP32).  Every P <= kM2LMaxP;
+// fp32: operators and z are float (sums of half an orbit FP32).  Every P <= kM2LMaxP;
 // src and dst hold P values per (box, density) at the levels' off.
 template <int SGN, int LOGT>
 inline void launch_m2l(int nd, const std::vector<M2LLev>& levels, const int* tlist, const int* s2,
