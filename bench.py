@@ -418,7 +418,7 @@ def main_hfmm2d(args):
                    "n": n, "nlevels": int(copts.nlevels), "nboxes": int(copts.nboxes)},
         "rel_l2_err": relerr,
         "stage_ms": {name: round(stage[k] * 1e3, 4) for k, name in STAGES.items()},
-        "roofline": {"bound": "mfma", "kernel": "k_translate (M2L, FP64 MFMA)",
+        "roofline": {"bound": "mfma", "kernel": "k_m2l (M2L, FP64 MFMA)",
                      "achieved": round(achieved, 3), "peak": PEAK["fp64_tflops"],
                      "unit": "TFLOP/s", "frac": round(achieved / PEAK["fp64_tflops"], 4),
                      "traffic": None, "launch_ms": round(t_m2l * 1e3, 4)},
@@ -878,7 +878,7 @@ def main():
     a_m2l = work[3] / t_m2l / 1e12 if t_m2l > 0 else 0.0
     a_near = work[7] / t_near / 1e12 if t_near > 0 else 0.0
     rl = {
-        "m2l": {"bound": "mfma", "kernel": "k_translate (M2L, %s MFMA)" % prec,
+        "m2l": {"bound": "mfma", "kernel": "k_m2l (M2L, %s MFMA)" % prec,
                 "achieved": round(a_m2l, 3), "peak": peak, "unit": "TFLOP/s",
                 "frac": round(a_m2l / peak, 4),
                 "traffic": read_traffic(TRAFFIC_KEYS[head][0]),
