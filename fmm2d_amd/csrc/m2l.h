@@ -323,8 +323,11 @@ __global__ __launch_bounds__(64 * NW) void k_m2l(int nd, int per_xcd, M2LTab tab
   double* L = reinterpret_cast<double*>(dstall + tab.lev[li].off +
                                         ((int64_t)(tb - box0) * nd + d) * P);
   // the level-dependent part log(boxsize) M_0 of L_0: lanes 0..15 hold the
-  // sources' sum of Re M_0, lanes 16..31 of Im M_0
+  // sources' sum of Re M_0, lanes 16..31 of Im M_0.  It is added by the lane that
+  // adds the row's sum (FP64: the same lanes; FP32: rows 0 and 1 are both of
+  // lanes 0..15), since nothing orders two lanes' updates of one value.
   const double lm = (LOGT && lane < 32) ? logr[lev] * m0 : 0.0;
+  const double lmi = (LOGT && FOLD) ? __shfl(lm, cl + 16, 64) : lm;
 #pragma unroll
   for (int a = 0; a < 4; ++a)
 #pragma unroll
@@ -334,11 +337,13 @@ __global__ __launch_bounds__(64 * NW) void k_m2l(int nd, int per_xcd, M2LTab tab
         const int row = 16 * r + Mfma<T>::row(kr, i);
         const int e = 2 * (a + 4 * (row >> 1)) + (row & 1);
         if (e < 2 * P && e >= bd.x && e < bd.y) {
-          if constexpr (FOLD) L[e] += sum[a][r][i];
-          else L[e] += acc[a][r][i];
+          double v = L[e];
+          if constexpr (FOLD) v += sum[a][r][i];
+          else v += acc[a][r][i];
+          if (LOGT && a == 0 && row < 2) v += row == 0 ? lm : lmi;
+          L[e] = v;
         }
       }
-  if (LOGT && lane < 32) L[kr] += lm;
 }
 
 // The M2L of the given levels (blk0 is set here), one launch per tile shape.

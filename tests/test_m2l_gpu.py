@@ -56,3 +56,24 @@ def test_helmholtz_orders(p, nd, prec):
     a = np.reshape(res["pot"], (nd, n))[:, :m]
     e = np.linalg.norm(a - ex) / np.linalg.norm(ex)
     assert e < bound(p, 1e-11 if prec == "fp64" else 4e-6), e
+
+
+@pytest.mark.parametrize("prec", ["fp64", "mixed"])
+@pytest.mark.parametrize("unit", [1.0, 1j])
+def test_log_term_of_either_part(prec, unit):
+    """Charges of one sign, all real or all imaginary: the M2L's log(boxsize) M_0 is most of that part of L_0, and
+    an update of it that gets lost (its row has the translation's own sum to add as well) leaves an error of order one."""
+    from fmm2d_amd.fmm2d import _fmm
+    rng = np.random.default_rng(7)
+    n, m, p = 3000, 80, 16
+    src = points(n, rng)
+    ch = unit * (1.0 + rng.random((2, n))) + 0j
+    opts = {"nterms": [p], "ndiv": 12, "precision": prec}
+    for nd in (1, 2):
+        c = (ch[0] if nd == 1 else ch) * (1.0 if nd == 1 else np.array([[1.0], [1j]]))
+        res, ier = _fmm("l", 1e-6, None, src, c, None, None, None, 1, 0, nd, opts)
+        assert ier == 0
+        ex = O.direct("l", nd, src, src[:, :m], np.reshape(c, (nd, n)), None, None, 1, 1e-16)["pottarg"]
+        a = np.reshape(res["pot"], (nd, n))[:, :m]
+        e = np.linalg.norm(a - ex) / np.linalg.norm(ex)
+        assert e < bound(p, 1e-12 if prec == "fp64" else 2e-6), e
