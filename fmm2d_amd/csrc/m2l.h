@@ -124,8 +124,6 @@ struct M2LTab {
   M2LLev lev[kM2LMaxLev];
 };
 
-static __device__ double m2l_zero[2];
-
 template <typename T> struct M2LPair {
   T re, im;
 };
@@ -217,7 +215,7 @@ __global__ __launch_bounds__(64 * NW) void k_m2l(int nd, int per_xcd, M2LTab tab
 #pragma unroll
       for (int k = 0; k < 4; ++k) {
         const dpair* p = of[it][k] >= 0 && j < P ? src + (of[it][k] + j)
-                                                 : reinterpret_cast<const dpair*>(m2l_zero);
+                                                 : reinterpret_cast<const dpair*>(tr_zero);
         x[it][k] = *p;
       }
     }

@@ -19,7 +19,17 @@
 // band[level] = [lo, hi) are the interleaved coefficient rows that level uses
 // (the rest stay zero); without one every row is used.  With LOGT the Laplace
 // M2L term log(boxsize) M_0 is added to L_0.
+//
+// The k loop is bound by the latency of its loads, operator fragments from L2
+// and one coefficient a lane: the fragments of all row tiles of a step and the
+// coefficient are in flight together, and the number of row tiles is a constant
+// of each copy of the loop, so that nothing in it is in a branch.  With the row
+// tiles under a test, each MFMA waited for its own load (and, where the test was
+// of a vector register, moved its accumulators to vector registers and back):
+// M2L of hfmm2d at eps 1e-12, 5e5 points (67 to 75 coefficients) 5.95 -> 3.2
+// ms, 3e5 points on a curve (67 to 185) 11.3 -> 5.7.
 #pragma once
+#include <type_traits>
 #include <vector>
 
 #include "common.h"
@@ -80,6 +90,8 @@ __device__ __forceinline__ void wave_lds_fence() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
+static __device__ double tr_zero[2];  // what an absent coefficient is loaded from
+
 // T is the arithmetic type of the operator (Afrag) and the source
 // expansions (src, 2 Pin values of T per box and density); the results are
 // added to the FP64 destination expansions.
@@ -96,7 +108,10 @@ __global__ __launch_bounds__(256) void k_translate(
   // contiguous range of targets, whose neighbouring source boxes then stay
   // in that XCD's L2.
   const int64_t lblk = (int64_t)(blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
-  const int64_t wv0 = lblk * 4 + (threadIdx.x >> 6);
+  // (the wavefront's number as a scalar: with the row tile's bound a vector
+  // condition every MFMA stood in a branch of its own, its accumulators moved to
+  // vector registers and back around it)
+  const int64_t wv0 = lblk * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   if (wv0 >= nwaves) return;
   const int lane = threadIdx.x & 63;
   // Split launches (few targets, long operators): wavefront wv0 also takes
@@ -132,6 +147,12 @@ __global__ __launch_bounds__(256) void k_translate(
   const int tb = tpos < tab.seg1[g] ? tlist[tpos] : -1;
   const bool valid = tb >= 0;
   const int kr = lane >> 4;
+  if (__ballot(valid) == 0) {
+    // no target in the tile
+    if (split && sk == 0 && rc == 0 && kr == 0)
+      dstoff[(int64_t)(tab.tile0[g] + tl) * 16 + (lane & 15)] = -1;
+    return;
+  }
   const int2 full = int2{0, 2 * P};
   const int ob = tab.opbase[g];
   const int sg = sk / ksplit, kg = sk - sg * ksplit;
@@ -143,26 +164,37 @@ __global__ __launch_bounds__(256) void k_translate(
 #pragma unroll
   for (int r = 0; r < RT; ++r) acc[r] = acc_t{0, 0, 0, 0};
   T m0 = 0;
-  for (int s = s_lo; s < s_hi; ++s) {
-    const int c = valid ? slots[(int64_t)tb * nslots + s] : -1;
-    const T* A = Afrag + (int64_t)(ob + slot_op[q * nslots + s]) * afs;
-    const T* M = nullptr;
-    int klo = 0, khi = 0;
-    if (c >= 0) {
-      M = src + ((int64_t)(c - box0) * nd + d) * 2 * P;
-      const int2 bd = band ? band[ilevel[c]] : full;
-      klo = bd.x;
-      khi = bd.y;
-    }
-    for (int ks = k_lo; ks < k_hi; ++ks) {
-      const int k = 4 * ks + kr;
-      const T b = (k >= klo && k < khi) ? M[k] : T(0);
-      if (LOGT && rc == 0 && ks == 0 && lane < 32) m0 += b;
+  auto products = [&](auto NRC) {
+    constexpr int NR = decltype(NRC)::value;  // row tiles of this chunk
+    for (int s = s_lo; s < s_hi; ++s) {
+      const int c = valid ? slots[(int64_t)tb * nslots + s] : -1;
+      const T* A = Afrag + (int64_t)(ob + slot_op[q * nslots + s]) * afs + lane;
+      const T* M = src + (c >= 0 ? ((int64_t)(c - box0) * nd + d) * 2 * P : 0);
+      int klo = 0, khi = 0;
+      if (c >= 0) {
+        const int2 bd = band ? band[ilevel[c]] : full;
+        klo = bd.x;
+        khi = bd.y;
+      }
+#pragma unroll 2
+      for (int ks = k_lo; ks < k_hi; ++ks) {
+        const int k = 4 * ks + kr;
+        T av[NR];
 #pragma unroll
-      for (int r = 0; r < RT; ++r)
-        if (rc + r < RTT)
-          acc[r] = Mfma<T>::step(A[((int64_t)(rc + r) * KS + ks) * 64 + lane], b, acc[r]);
+        for (int r = 0; r < NR; ++r) av[r] = A[((int64_t)(rc + r) * KS + ks) * 64];
+        // (absent coefficients are loaded from a zero: no load in a branch)
+        const T b = *((k >= klo && k < khi) ? M + k : reinterpret_cast<const T*>(tr_zero));
+        if (LOGT && rc == 0 && ks == 0 && lane < 32) m0 += b;
+#pragma unroll
+        for (int r = 0; r < NR; ++r) acc[r] = Mfma<T>::step(av[r], b, acc[r]);
+      }
     }
+  };
+  switch (min(RT, RTT - rc)) {
+    case 1: products(std::integral_constant<int, 1>{}); break;
+    case 2: products(std::integral_constant<int, 2>{}); break;
+    case 3: products(std::integral_constant<int, 3>{}); break;
+    default: products(std::integral_constant<int, RT>{}); break;
   }
   if (split) {
     const int64_t ncols = (int64_t)tab.tile0[tab.ng] * 16;

@@ -58,6 +58,28 @@ def test_helmholtz_orders(p, nd, prec):
     assert e < bound(p, 1e-11 if prec == "fp64" else 4e-6), e
 
 
+@pytest.mark.parametrize("kind,p,prec", [(k, p, prec) for k, ps in (("l", (71, 79, 87, 95)), ("h", (36, 40, 44, 47)))
+                                         for p in ps for prec in (("fp64", "mixed") if k == "l" else ("fp64",))])
+def test_last_row_tiles_of_long_operators(kind, p, prec):
+    """Operators of 65 coefficients and more (csrc/translate.h) with one to four row tiles in their last chunk (9 to
+    12 tiles in all), in one wavefront or split over slots and k steps, one density or two.  (Helmholtz operators of
+    these orders at this wavenumber are beyond FP32's range: 71! (1/2 pi)^72 > 3.4e38.)"""
+    from fmm2d_amd.fmm2d import _fmm
+    rng = np.random.default_rng(p)
+    n, m, zk = 2000, 60, 1.5
+    src = points(n, rng)
+    for nd in (1, 2):
+        ch = rng.standard_normal((nd, n)) + 1j * rng.standard_normal((nd, n))
+        opts = {"nterms": [p], "ndiv": 12, "precision": prec}
+        res, ier = _fmm(kind, 1e-6, zk if kind == "h" else None, src, ch[0] if nd == 1 else ch, None, None, None, 1, 0,
+                        nd, opts)
+        assert ier == 0
+        ex = O.direct(kind, nd, src, src[:, :m], ch, None, None, 1, 1e-16, **({"zk": zk} if kind == "h" else {}))
+        a = np.reshape(res["pot"], (nd, n))[:, :m]
+        e = np.linalg.norm(a - ex["pottarg"]) / np.linalg.norm(ex["pottarg"])
+        assert e < bound(p, {"fp64": 1e-11, "mixed": 4e-6}[prec]), e
+
+
 @pytest.mark.parametrize("prec", ["fp64", "mixed"])
 @pytest.mark.parametrize("unit", [1.0, 1j])
 def test_log_term_of_either_part(prec, unit):
