@@ -168,12 +168,18 @@ __device__ void scaled_h(cplx z, double s, int m, cplx* out) {
 // 1e6 points (orders 20 to 27) P2M 460 -> 262 us, list 4 826 -> 355; charges on
 // the curve of 2e6 points 576 -> 565, 932 -> 624.  (4 KB a batch: 800 for 624;
 // four boxes a workgroup: 943.)
+//
+// Up to 2 * 64 coefficients a lane takes coefficients -p + lane and -p + lane +
+// 64.  Longer expansions go in tiles of kHTile orders n with the lane's pair +-n,
+// each with the rows that it needs, so that a phase is formed once and a batch
+// takes no more LDS than a short expansion's (with the rows of all orders formed
+// again for every 128 coefficients, in LDS sized by the longest level: 312
+// charges a leaf of order 114, 170, 244 P2M 0.83, 1.81, 2.62 ms; a power for
+// every lane and source 0.68, 1.03, 1.39; now
+// 0.57, 0.85, 1.23).  (Densities still form the phases again.)
 constexpr int kHBatch = 16;
-constexpr int kHLds = 8192;  // bytes of a batch, unless one source needs more
-
-__host__ __device__ inline int hbatch_bytes(int p, int nb) {
-  return nb * (2 * (p + 2) + 3) * (int)sizeof(cplx);
-}
+constexpr int kHTile = 60;   // four sources of a tile in a batch
+constexpr int kHLds = 8192;  // bytes of a batch
 
 // t-th row: G + t (p + 2), e^{-i a} U[t], source jof(t)
 template <int IFC, int IFD, int LOCAL, typename JOF>
@@ -183,24 +189,34 @@ __device__ void accumulate_rows(int nd, int p, cplx zk, double s, const cplx* G,
   // LOCAL: (a_lo, a_hi) = (s, 1/s); multipole: (1/s, s)
   const double a_lo = LOCAL ? s : 1.0 / s, a_hi = LOCAL ? 1.0 / s : s;
   const cplx k2 = 0.5 * zk;
-  const int lane = threadIdx.x, W = p + 2, nc = 2 * p + 1;
-  int nb = kHBatch;
-  while (nb > 1 && hbatch_bytes(p, nb) > kHLds) nb >>= 1;
-  const int ls = kW / nb, seg = (W + ls - 1) / ls;  // lanes a source, rows a lane
-  cplx* wp = sh;
-  cplx* wm = wp + nb * W;
-  cplx* sq = wm + nb * W;  // q, k/2 dipstr (v1 - i v2), k/2 dipstr (v1 + i v2) a source
+  const int lane = threadIdx.x, nc = 2 * p + 1;
+  const bool wide = nc > 2 * kW;
   for (int d = 0; d < nd; ++d) {
-    for (int m0 = 0; m0 < nc; m0 += 2 * kW) {
+    for (int lo = 0; lo <= p; lo += kHTile) {  // (once if not wide)
+      // rows r0 .. r0 + W - 1
+      const int r0 = wide ? max(0, lo - 1) : 0;
+      const int W = (wide ? min(p, lo + kHTile - 1) : p) + 2 - r0;
+      int nb = kHBatch;
+      while (nb > 1 && nb * (2 * W + 3) * (int)sizeof(cplx) > kHLds) nb >>= 1;
+      const int ls = kW / nb, seg = (W + ls - 1) / ls;  // lanes a source, rows a lane
+      cplx* wp = sh;
+      cplx* wm = wp + nb * W;
+      cplx* sq = wm + nb * W;  // q, k/2 dipstr (v1 - i v2), k/2 dipstr (v1 + i v2) a source
+      // the order of the lane's a-th coefficient, beyond p if it has none
+      auto order = [&](int a) {
+        if (!wide) return lane + a * kW - p;
+        const int n = lo + lane;
+        return lane >= kHTile || n > p || (a == 1 && n == 0) ? p + 1 : a == 0 ? n : -n;
+      };
       cplx acc[2] = {mkc(0.0), mkc(0.0)};
       for (int t0 = 0; t0 < total; t0 += nb) {
         const int cnt = min(nb, total - t0);
         const int jj = lane / ls;
         if (jj < cnt) {
           const cplx u = U[t0 + jj];
-          const cplx* g = G + (int64_t)(t0 + jj) * W;
+          const cplx* g = G + (int64_t)(t0 + jj) * (p + 2) + r0;
           const int n0 = (lane - jj * ls) * seg, n1 = min(W, n0 + seg);
-          cplx e = cpowi(u, n0);
+          cplx e = cpowi(u, r0 + n0);
           for (int n = n0; n < n1; ++n) {
             const cplx v = g[n];
             wp[jj * W + n] = v * e;
@@ -221,11 +237,11 @@ __device__ void accumulate_rows(int nd, int p, cplx zk, double s, const cplx* G,
         wave_lds_fence();
 #pragma unroll
         for (int a = 0; a < 2; ++a) {
-          const int m = m0 + lane + a * kW;
-          if (m >= nc) continue;
-          const bool neg = m < p;
-          const int n = neg ? p - m : m - p;
-          const cplx* w = (neg ? wm : wp) + n;
+          const int m = order(a);
+          if (m > p) continue;
+          const bool neg = m < 0;
+          const int n = neg ? -m : m;
+          const cplx* w = (neg ? wm : wp) + (n - r0);
           // the dipole's two terms: entries n -+ 1 of the same rows, at n = 0
           // entry 1 of either
           const cplx* w1 = n == 0 ? wm + 1 : neg ? w + 1 : w - 1;
@@ -246,12 +262,10 @@ __device__ void accumulate_rows(int nd, int p, cplx zk, double s, const cplx* G,
       }
 #pragma unroll
       for (int a = 0; a < 2; ++a) {
-        const int m = m0 + lane + a * kW;
-        if (m < nc) {
-          const bool odd = m < p && ((p - m) & 1);
-          out_p0[(int64_t)d * nc + (m - p)] += odd ? -acc[a] : acc[a];
-        }
+        const int m = order(a);
+        if (m <= p) out_p0[(int64_t)d * nc + m] += m < 0 && (m & 1) ? -acc[a] : acc[a];
       }
+      if (!wide) break;
     }
   }
 }
@@ -271,13 +285,15 @@ __global__ void k_hp2m_rowlen(int64_t n, const HLev* lev, const int* leaf, const
   len[i] = (l >= 2 && lev[l].on) ? lev[l].p + 2 : 0;
 }
 
-//
-// A wavefront's rows are formed in LDS (rowcap values a row at most, an odd
+// A wavefront's rows are formed in LDS (kRowCap values a row at most, an odd
 // stride) and copied out row by row, consecutive lanes on consecutive values;
 // longer rows are formed in place.  In place, every step of the recurrence
 // wrote 16 bytes to each of 64 lines, and the lines left the L2 half written:
 // 1e6 points 634 -> 277 us.  (List 4's rows are written once as they are: in LDS
-// they took 924 us for 678.)
+// they took 924 us for 678.)  The rows formed in place, of orders from 30 on,
+// keep the limit of five wavefronts a CU that the LDS sets: with as many as fit,
+// more lines are half written at a time (P2M of 5e5 points at order 33 0.53 ->
+// 0.64 ms, of 2e5 at order 39 0.325 -> 0.341).
 constexpr int kRowCap = 31;  // 31 KB a wavefront: orders up to 29
 
 // The rows of the lanes with w > 0 values at sh + lane * stride to dst (lane's)
@@ -334,7 +350,7 @@ __global__ __launch_bounds__(kW) void k_hp2m_g(int nd, cplx zk, const HLev* lev,
   if (l < 2 || !L.on || nchild[b] != 0) return;
   const int s0 = sse[2 * b], s1 = sse[2 * b + 1];
   if (s1 <= s0) return;
-  extern __shared__ cplx sh[];
+  __shared__ cplx sh[kHLds / sizeof(cplx)];
   accumulate_rows<IFC, IFD, 0>(
       nd, L.p, zk, L.s, G + roff[s0], U + s0, s1 - s0, [=](int t) { return s0 + t; }, chs, dps,
       dvs, sh, hexp(mp, L, b, nd, 0));
@@ -421,7 +437,7 @@ __global__ __launch_bounds__(kW) void k_hp2l_g(int nd, cplx zk, const HLev* lev,
       if (t >= pre[k]) j = first[k] + (t - pre[k]);
     return j;
   };
-  extern __shared__ cplx sh[];
+  __shared__ cplx sh[kHLds / sizeof(cplx)];
   accumulate_rows<IFC, IFD, 1>(nd, L.p, zk, L.s, G + roff[b], U + off[b], cnt[b], jof, chs, dps,
                                dvs, sh, hexp(loc, L, b, nd, 0));
 }
@@ -1629,8 +1645,6 @@ int helmholtz_fmm(const HelmArgs& a, hipStream_t st) {
     while (!ops.done() && !sizes.ready()) ops.next();
     sizes.finish(hrow, &np4);
     const int64_t nrow = hrow[0], nrow4 = hrow[1];
-    size_t hlds = kHLds;
-    for (int l = 2; l <= nl; ++l) hlds = std::max(hlds, (size_t)hbatch_bytes(nterms[l], 1));
     // ---- step 1: P2M (rows of the sources, then their sums per leaf)
     {
       DBuf<cplx> gJ(std::max<int64_t>(nrow, 1), st), uJ(ns, st);
@@ -1638,7 +1652,7 @@ int helmholtz_fmm(const HelmArgs& a, hipStream_t st) {
                          t.leaf_s.p, t.ilevel.p, t.centers.p, xs.p, (const int64_t*)roff.p, gJ.p,
                          uJ.p);
 #define FMM2D_P2M(C, D)                                                                       \
-  hipLaunchKernelGGL((k_hp2m_g<C, D>), dim3(nb), dim3(kW), hlds, st, nd, zk, d_lev, t.ilevel.p,     \
+  hipLaunchKernelGGL((k_hp2m_g<C, D>), dim3(nb), dim3(kW), 0, st, nd, zk, d_lev, t.ilevel.p,     \
                      t.nchild.p, sse, (const int64_t*)roff.p, gJ.p, uJ.p, chs.p, dps.p, dvs.p,  \
                      mp.p)
       if (a.ifcharge && !a.ifdipole) FMM2D_P2M(1, 0);
@@ -1655,7 +1669,7 @@ int helmholtz_fmm(const HelmArgs& a, hipStream_t st) {
         launch1d(k_hp2l_rows, np4, st, nb, zk, d_lev, t.ilevel.p, t.centers.p, L.l4.p, sse,
                  off4.p, xs.p, (const int64_t*)roff4.p, gH.p, uH.p);
 #define FMM2D_P2L(C, D)                                                                       \
-  hipLaunchKernelGGL((k_hp2l_g<C, D>), dim3(nb), dim3(kW), hlds, st, nd, zk, d_lev, t.ilevel.p,     \
+  hipLaunchKernelGGL((k_hp2l_g<C, D>), dim3(nb), dim3(kW), 0, st, nd, zk, d_lev, t.ilevel.p,     \
                      L.n4.p, L.l4.p, sse, cnt4.p, off4.p, (const int64_t*)roff4.p, gH.p, uH.p, \
                      chs.p, dps.p, dvs.p, loc.p)
         if (a.ifcharge && !a.ifdipole) FMM2D_P2L(1, 0);
