@@ -50,8 +50,8 @@ struct AsyncRead {
 };
 // Pinned memory that a copy on st reads after the call that fills it has gone
 // on.  The destructor waits for st (idle at the end of an FMM call) and gives
-// the memory back to a pool of a few buffers, which fmm2d_release_workspace()
-// empties.
+// the memory back to a bounded pool (stage_pool.h), which
+// fmm2d_release_workspace() empties.
 struct Staging {
   void* p = nullptr;
   size_t cap = 0;

@@ -21,6 +21,7 @@
 #include <vector>
 
 #include "devbuf.h"
+#include "stage_pool.h"
 
 namespace fmm2d {
 
@@ -155,14 +156,8 @@ void AsyncRead::finish(void* dst, void* dst2) {
 
 namespace {
 
-// free staging buffers: at most kStagePool of at most kStageMax bytes
-constexpr size_t kStagePool = 8, kStageMax = size_t(4) << 20;
-struct StageBuf {
-  void* p;
-  size_t cap;
-};
 std::mutex g_stage_mu;
-std::vector<StageBuf> g_stage;
+StagePool g_stage;
 
 }  // namespace
 
@@ -170,17 +165,17 @@ void* Staging::get(size_t bytes, hipStream_t s) {
   st = s;
   {
     std::lock_guard<std::mutex> g(g_stage_mu);
-    for (size_t k = 0; k < g_stage.size(); ++k)
-      if (g_stage[k].cap >= bytes) {
-        p = g_stage[k].p;
-        cap = g_stage[k].cap;
-        g_stage[k] = g_stage.back();
-        g_stage.pop_back();
-        return p;
-      }
+    const StagePool::Buf b = g_stage.take(bytes);
+    if (b.p) {
+      p = b.p;
+      cap = b.cap;
+      return p;
+    }
   }
   const size_t want = std::max(size_t(1) << 18, (bytes + (size_t(1) << 16)) >> 16 << 16);
-  hip_throw(hipHostMalloc(&p, want, hipHostMallocDefault), "hipHostMalloc (staging)");
+  void* q = nullptr;
+  hip_throw(hipHostMalloc(&q, want, hipHostMallocDefault), "hipHostMalloc (staging)");
+  p = q;
   cap = want;
   return p;
 }
@@ -188,23 +183,25 @@ void* Staging::get(size_t bytes, hipStream_t s) {
 Staging::~Staging() {
   if (!p) return;
   if (hipStreamSynchronize(st) != hipSuccess) return;  // a copy may still read it
-  if (cap <= kStageMax) {
+  std::vector<StagePool::Buf> gone;
+  bool kept = false;
+  try {
     std::lock_guard<std::mutex> g(g_stage_mu);
-    if (g_stage.size() < kStagePool) {
-      g_stage.push_back(StageBuf{p, cap});
-      return;
-    }
+    gone = g_stage.give(StagePool::Buf{p, cap});
+    kept = true;
+  } catch (...) {  // no memory for the pool's list
   }
-  (void)hipHostFree(p);
+  if (!kept) (void)hipHostFree(p);
+  for (const StagePool::Buf& b : gone) (void)hipHostFree(b.p);
 }
 
 void staging_release() {
-  std::vector<StageBuf> all;
+  std::vector<StagePool::Buf> all;
   {
     std::lock_guard<std::mutex> g(g_stage_mu);
-    all.swap(g_stage);
+    all.swap(g_stage.free);
   }
-  for (const StageBuf& b : all) (void)hipHostFree(b.p);
+  for (const StagePool::Buf& b : all) (void)hipHostFree(b.p);
 }
 
 void upload_bytes(void* dst, const void* src, size_t bytes, hipStream_t st) {
