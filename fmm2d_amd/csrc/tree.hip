@@ -39,9 +39,9 @@ constexpr int64_t kBatchBoxes = 1 << 24;  // box capacity a batch may reserve
 
 // copy the first n[k] 4-byte words of src[k] to dst[k] for k = blockIdx.y
 struct WordCopies {
-  const unsigned* src[10];
-  unsigned* dst[10];
-  int64_t n[10];
+  const unsigned* src[8];
+  unsigned* dst[8];
+  int64_t n[8];
 };
 __global__ void k_copy_words(WordCopies c) {
   const int k = blockIdx.y;
@@ -50,9 +50,13 @@ __global__ void k_copy_words(WordCopies c) {
     c.dst[k][i] = c.src[k][i];
 }
 
+// The arrays that describe cap boxes.  The colleagues, 40 of a box's 104 bytes,
+// come with the first search for them and for the boxes there are then: the
+// refinement reserves more boxes than it makes.
 struct Boxes {
   DBuf<double> centers;
-  DBuf<int> ilevel, iparent, nchild, ichild, ncoll, coll, ses, set, iflag;
+  DBuf<int> ilevel, iparent, nchild, ichild, ses, set, iflag;
+  DBuf<int> ncoll, coll;
   size_t cap = 0;
   void alloc(size_t c, hipStream_t st) {
     cap = c;
@@ -61,18 +65,34 @@ struct Boxes {
     iparent.alloc(c, st);
     nchild.alloc(c, st);
     ichild.alloc(4 * c, st);
-    ncoll.alloc(c, st);
-    coll.alloc(9 * c, st);
     ses.alloc(2 * c, st);
     set.alloc(2 * c, st);
     iflag.alloc(c, st);
   }
+  // room for the colleagues of c boxes (contents lost if there was less)
+  void alloc_coll(size_t c) {
+    if (ncoll.n >= c) return;
+    coll.reset();
+    ncoll.alloc(c, ilevel.st);
+    coll.alloc(kMaxColl * c, ilevel.st);
+  }
+  void swap_boxes(Boxes& o) {
+    centers.swap(o.centers);
+    ilevel.swap(o.ilevel);
+    iparent.swap(o.iparent);
+    nchild.swap(o.nchild);
+    ichild.swap(o.ichild);
+    ses.swap(o.ses);
+    set.swap(o.set);
+    iflag.swap(o.iflag);
+    std::swap(cap, o.cap);
+  }
   // capacity for `need` boxes, the first `keep` kept (one copy launch)
-  void grow(size_t need, size_t keep) {
+  void fit(size_t need, size_t keep) {
     if (need <= cap) return;
     const hipStream_t st = ilevel.st;
     Boxes b;
-    b.alloc(std::max(need, cap * 2), st);
+    b.alloc(need, st);
     if (keep > 0) {
       WordCopies c{};
       int k = 0;
@@ -86,16 +106,18 @@ struct Boxes {
       add(iparent.p, b.iparent.p, keep);
       add(nchild.p, b.nchild.p, keep);
       add(ichild.p, b.ichild.p, 4 * keep);
-      add(ncoll.p, b.ncoll.p, keep);
-      add(coll.p, b.coll.p, 9 * keep);
       add(ses.p, b.ses.p, 2 * keep);
       add(set.p, b.set.p, 2 * keep);
       add(iflag.p, b.iflag.p, keep);
-      const unsigned gx = (unsigned)std::min<int64_t>(ceil_div((int64_t)(9 * keep), 256), 1024);
-      hipLaunchKernelGGL(k_copy_words, dim3(gx, 10), dim3(256), 0, st, c);
+      const unsigned gx = (unsigned)std::min<int64_t>(ceil_div((int64_t)(4 * keep), 256), 1024);
+      hipLaunchKernelGGL(k_copy_words, dim3(gx, 8), dim3(256), 0, st, c);
       hip_throw(hipGetLastError(), "box copy");
     }
-    *this = std::move(b);
+    swap_boxes(b);
+  }
+  // the same with twice the capacity there was, for boxes that come level by level
+  void grow(size_t need, size_t keep) {
+    if (need > cap) fit(std::max(need, 2 * cap), keep);
   }
 };
 
@@ -1092,10 +1114,11 @@ __global__ __launch_bounds__(256) void k_ref_make(const double* bounds, int ns, 
 
 // The flag+ passes (k_flag2, finest level first) and the refinement of every
 // flagged box of levels 1 .. nl-2 (refine_segments over the levels in order).
-// cap holds 5 nb boxes.  State: boxes; per level the first and last of its new
-// boxes.
-__global__ __launch_bounds__(kWgThreads) void k_flags_wg(LevelTab T, int nl, int nb, BoxPtrs B,
-                                                         Keys ks, Keys kt, int* st) {
+// State: boxes; per level the first and last of its new boxes; status 1: cap
+// boxes are too few (5 nb never are, each box is refined at most once), and the
+// kernel has to run again with more, which repeats what it has done.
+__global__ __launch_bounds__(kWgThreads) void k_flags_wg(LevelTab T, int nl, int nb, int cap,
+                                                         BoxPtrs B, Keys ks, Keys kt, int* st) {
   __shared__ int list[kWgLevel];
   __shared__ int lds[kWgWaves + 1];
   __shared__ int cnt, per[kMaxLevels + 2];
@@ -1129,6 +1152,7 @@ __global__ __launch_bounds__(kWgThreads) void k_flags_wg(LevelTab T, int nl, int
     }
   }
   const int nb0 = nb;
+  int status = 0;
   if (nl >= 3) {
     const int lo = T.ls[1], n = T.le[nl - 2] - lo;
     for (int r0 = 0; r0 < n; r0 += kWgLevel) {
@@ -1143,6 +1167,10 @@ __global__ __launch_bounds__(kWgThreads) void k_flags_wg(LevelTab T, int nl, int
       int nref;
       int ex = block_exclusive_scan_w<kWgWaves>(c, lds, &nref);
       if (nref == 0) continue;  // uniform
+      if (nb + 4 * nref > cap) {
+        status = 1;
+        break;
+      }
 #pragma unroll
       for (int u = 0; u < 4; ++u)
         if (f[u]) list[ex++] = lo + r0 + 4 * tid + u;
@@ -1165,6 +1193,7 @@ __global__ __launch_bounds__(kWgThreads) void k_flags_wg(LevelTab T, int nl, int
       at += 4 * per[l];
       st[kStLev + 2 * l + 1] = at;
     }
+    st[kStStatus] = status;
     st[kStBoxes] = nb;
   }
 }
@@ -1172,9 +1201,9 @@ __global__ __launch_bounds__(kWgThreads) void k_flags_wg(LevelTab T, int nl, int
 // ------------------------------------------------------------ restriction sweeps
 // A sweep's boxes: n1 boxes from lo1 on, then the tail boxes [ts, te) of the
 // state words.  kLrTile boxes a workgroup of 256 threads, 16 lanes a box where
-// a box looks at its (parent's) colleagues.  Capacity and launch bounds are
-// guesses (cap, tail_ub); a sweep that would pass them sets the status word and
-// makes nothing, and the caller builds again with more room.
+// a box looks at its (parent's) colleagues.  Capacity and launch bounds of the
+// updateflags sweep are guesses (cap, tail_ub); a level that would pass them sets
+// the status word and makes nothing, and the caller builds again with more room.
 constexpr int kLrTile = 64;
 
 struct LrSeq {
@@ -1183,24 +1212,32 @@ struct LrSeq {
   __device__ int box(int i) const { return i < n1 ? lo1 + i : ts + (i - n1); }
 };
 
-// flagged boxes (iflag > 0) of every kLrTile of the n boxes from lo on
-__global__ __launch_bounds__(256) void k_flag_count(int n, int lo, const int* iflag, int* part) {
-  const int i0 = blockIdx.x * 256;
-  const int i = i0 + threadIdx.x;
-  const unsigned long long m = __ballot(i < n && iflag[lo + i] > 0);
+// flagged boxes (iflag > 0) of every kLrTile of the n boxes from lo on, and, by
+// the level of their children, in the state words (zero before)
+__global__ __launch_bounds__(256) void k_flag_count(int n, int lo, const int* iflag,
+                                                    const int* ilevel, int* part, int* st) {
+  __shared__ int per[kMaxLevels + 2];
+  for (int k = threadIdx.x; k < kMaxLevels + 2; k += 256) per[k] = 0;
+  __syncthreads();
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  const bool f = i < n && iflag[lo + i] > 0;
+  const unsigned long long m = __ballot(f);
   if ((threadIdx.x & 63) == 0 && i < n) part[i / kLrTile] = __popcll(m);
+  if (f) atomicAdd(&per[ilevel[lo + i] + 1], 1);
+  __syncthreads();
+  for (int k = threadIdx.x; k < kMaxLevels + 2; k += 256)
+    if (per[k]) atomicAdd(&st[kStLev + 2 * k], per[k]);
 }
 
 // Children of the flagged boxes of a sweep, numbered in sweep order from nb on
 // (make_children_of, mode 1).  SWEEP: level l of the updateflags sweep, nb = te
 // of that level, the new range is level l+1's; else the levels 1 .. nl-2 at
-// once, and st counts the refined boxes by child level.
+// once, which k_flag_count has counted.
 template <int SWEEP>
 __global__ __launch_bounds__(256) void k_flag_children(int n1, int lo1, int l, int nb,
                                                        const int* part, LevelTab T, int cap,
                                                        BoxPtrs B, Keys ks, Keys kt, int* st) {
   __shared__ int lds[kScanWaves + 1];
-  __shared__ int per[kMaxLevels + 2];
   LrSeq q{n1, lo1, 0, 0};
   if (SWEEP) {
     q.ts = st[kStLev + 2 * l];
@@ -1208,7 +1245,6 @@ __global__ __launch_bounds__(256) void k_flag_children(int n1, int lo1, int l, i
   }
   const int n = q.n(), i0 = blockIdx.x * 256, i = i0 + threadIdx.x;
   if (i0 >= n && blockIdx.x > 0) return;
-  for (int k = threadIdx.x; !SWEEP && k < kMaxLevels + 2; k += 256) per[k] = 0;
   const int b = i < n ? q.box(i) : 0;
   const bool f = i < n && B.iflag[b] > 0;
   const int carry = sum_parts(part, min(i0, n) / kLrTile, lds);
@@ -1224,12 +1260,6 @@ __global__ __launch_bounds__(256) void k_flag_children(int n1, int lo1, int l, i
     const int lev = SWEEP ? l + 1 : B.ilevel[b] + 1;
     make_children_of(b, nb + 4 * (carry + ex), 0.5 * T.bs[lev], lev, B.centers, B.ilevel,
                      B.iparent, B.nchild, B.ichild, B.ses, B.set, B.iflag, 1, ks, kt);
-    if (!SWEEP) atomicAdd(&per[lev], 1);
-  }
-  if (!SWEEP) {
-    __syncthreads();
-    for (int k = threadIdx.x; k < kMaxLevels + 2; k += 256)
-      if (per[k]) atomicAdd(&st[kStLev + 2 * k], per[k]);
   }
 }
 
@@ -1465,6 +1495,7 @@ struct Builder {
   }
   void computecoll(const std::vector<int>& ls, const std::vector<int>& le,
                    const std::vector<double>& bs, int nlevels, int* big = nullptr) {
+    B.alloc_coll(nboxes);
     // all levels at once by walking the tree from every box (integer
     // coordinates exact: at most kWalkLevels levels, domain near the origin)
     if (nlevels <= kWalkLevels && walk_ok) {
@@ -1479,9 +1510,10 @@ struct Builder {
       launch1d(k_coll, le[l] - ls[l], st, ls[l], bs[l], B.iparent.p, B.ichild.p, B.centers.p,
                B.ncoll.p, B.coll.p);
   }
-  // pts_tree_reorg: per level >= 2, original boxes then the tail boxes.
+  // pts_tree_reorg: per level >= 2, original boxes then the tail boxes; the
+  // arrays then have room for cap boxes.
   void reorg(std::vector<int>& ls, std::vector<int>& le, const std::vector<int>& ts,
-             const std::vector<int>& te, int nlevels) {
+             const std::vector<int>& te, int nlevels, size_t cap) {
     DBuf<int> map(nboxes, st);
     std::vector<std::pair<int, int>> seg;  // (from, to) of non-empty segments
     for (int l = 0; l <= std::min(1, nlevels); ++l)
@@ -1506,18 +1538,11 @@ struct Builder {
     }
     launch1d(k_map_segments, nboxes, st, T, map.p);
     Boxes N;
-    N.alloc(B.cap, st);
+    N.alloc(cap, st);
     launch1d(k_reorg_apply, nboxes, st, map.p, B.centers.p, B.ilevel.p, B.iparent.p, B.nchild.p,
              B.ichild.p, B.iflag.p, B.ses.p, B.set.p, N.centers.p, N.ilevel.p, N.iparent.p,
              N.nchild.p, N.ichild.p, N.iflag.p, N.ses.p, N.set.p);
-    B.centers.swap(N.centers);
-    B.ilevel.swap(N.ilevel);
-    B.iparent.swap(N.iparent);
-    B.nchild.swap(N.nchild);
-    B.ichild.swap(N.ichild);
-    B.iflag.swap(N.iflag);
-    B.ses.swap(N.ses);
-    B.set.swap(N.set);
+    B.swap_boxes(N);
   }
 };
 
@@ -1601,8 +1626,8 @@ bool tree_prepare_matches(const TreePrep* p, const double* src, int64_t ns, cons
          p->nlmax == nlmax;
 }
 
-// One build with capacity for `room` boxes for each one of the refinement
-// (false: the level restriction needs more).
+// One build with `room` times the usual reserve for the boxes that the
+// updateflags sweep adds (false: it needs more).
 static bool build_try(const TreePrep* P, TreePrep* own, const double* src, int64_t ns,
                       const double* trg, int64_t nt, int ndiv, int idivflag, int nlmax, Tree& t,
                       hipStream_t st, int room) {
@@ -1617,11 +1642,9 @@ static bool build_try(const TreePrep* P, TreePrep* own, const double* src, int64
   bld.ks = pk[0]->view();
   bld.kt = pk[1]->view();
 
-  // room for the level restriction's bound (5 boxes for each one of the
-  // refinement, which makes 2 to 3 for every ndiv points) in small trees
-  size_t cap0 = std::max<size_t>(4096, (size_t)(16 * (ns + nt) / std::max(ndiv, 1)));
-  if (cap0 > 5 * (size_t)kWgBoxes) cap0 /= 2;
-  bld.B.alloc(cap0, st);
+  // the refinement makes 2 to 3 boxes for every ndiv points of an area, 5 on a
+  // curve, and the level restriction as many again on a curve
+  bld.B.alloc(std::max<size_t>(1536, (size_t)(11 * (ns + nt) / std::max(ndiv, 1))), st);
   DBuf<int> state(kStWords, st);
   std::vector<int> hs(kStWords, 0);
 
@@ -1673,13 +1696,15 @@ static bool build_try(const TreePrep* P, TreePrep* own, const double* src, int64
     readback(hs.data(), state.p, sizeof(int) * kStWords, st);
   }
   if (by_keys && hs[kStStatus] == 2) {  // more boxes than expected
-    bld.B.grow((size_t)hs[kStBoxes] + 64, 0);
+    bld.B.fit((size_t)hs[kStBoxes] + 64, 0);
     refine_keys(false);
     hs[kStStatus] = 1;
   } else if (by_keys && hs[kStStatus] == 3) {
     refine_wg(0);
     readback(hs.data(), state.p, sizeof(int) * kStWords, st);
   }
+  kref.reset();
+  kcnt.reset();
   const std::vector<double>& bsall = P->bsall;
   const double* root = P->root;
   bld.walk_ok = P->walk_ok;
@@ -1821,22 +1846,27 @@ static bool build_try(const TreePrep* P, TreePrep* own, const double* src, int64
   int added = 0;
   DBuf<int> part;
   if (nlevels >= 2) {
-    const int64_t nb0 = bld.nboxes;
-    // (large trees, of mostly regular regions, start with less)
-    const int64_t fac = nb0 <= 262144 ? room : std::max(3, room / 3);
-    bld.B.grow((size_t)std::min<int64_t>(fac * nb0 + 4096, INT32_MAX), nb0);
-    const int cap = (int)std::min<size_t>(bld.B.cap, INT32_MAX);
-    part.alloc(bld.B.cap / kLrTile + 1, st);
+    const int nb0 = bld.nboxes;
     {
       LevelReals dist{};
       for (int l = 2; l <= nlevels; ++l) dist.v[l] = 1.05 * (bs[l - 1] + bs[l - 2]) / 2.0;
       launch1d(k_flag1, le[nlevels] - ls[2], st, ls[2], dist, bld.B.ilevel.p, bld.B.iparent.p,
                bld.B.ncoll.p, bld.B.coll.p, bld.B.nchild.p, bld.B.centers.p, bld.B.iflag.p);
     }
-    if (nb0 <= kWgBoxes && cap >= 5 * nb0) {  // (each box is refined at most once)
-      hipLaunchKernelGGL(k_flags_wg, dim3(1), dim3(kWgThreads), 0, st, T, nlevels, bld.nboxes,
-                         ptrs(bld.B), bld.ks, bld.kt, state.p);
-      hip_throw(hipGetLastError(), "level restriction");
+    if (nb0 <= kWgBoxes) {
+      for (;;) {
+        hipLaunchKernelGGL(k_flags_wg, dim3(1), dim3(kWgThreads), 0, st, T, nlevels, nb0,
+                           (int)std::min<size_t>(bld.B.cap, INT32_MAX), ptrs(bld.B), bld.ks,
+                           bld.kt, state.p);
+        hip_throw(hipGetLastError(), "level restriction");
+        readback(hs.data(), state.p, sizeof(int) * kStWords, st);
+        if (hs[kStStatus] == 0) break;
+        bld.B.fit(5 * (size_t)nb0, nb0);
+      }
+      for (int l = 2; l <= nlevels - 1; ++l) {
+        ts[l] = hs[kStLev + 2 * l];
+        te[l] = hs[kStLev + 2 * l + 1];
+      }
     } else {
       for (int k = 0; k < kStWords; ++k)
         if (k != kStBig) hs[k] = 0;
@@ -1847,28 +1877,27 @@ static bool build_try(const TreePrep* P, TreePrep* own, const double* src, int64
         launch1d(k_flag2, le[l] - ls[l], st, ls[l], distest, bld.B.iparent.p, bld.B.ncoll.p,
                  bld.B.coll.p, bld.B.nchild.p, bld.B.centers.p, bld.B.iflag.p);
       }
-      // the flags are fixed now: all levels refine together
+      // the flags are fixed now: all levels refine together, with room for the
+      // boxes that they make
       const int n = nlevels >= 3 ? le[nlevels - 2] - ls[1] : 0;
-      launch1d(k_flag_count, n, st, ls[1], (const int*)bld.B.iflag.p, part.p);
-      if (n > 0) {
+      part.alloc(ceil_div(std::max(n, 1), kLrTile), st);
+      launch1d(k_flag_count, n, st, ls[1], (const int*)bld.B.iflag.p, (const int*)bld.B.ilevel.p,
+               part.p, state.p);
+      readback(hs.data(), state.p, sizeof(int) * kStWords, st);
+      int64_t at = nb0;
+      for (int l = 2; l <= nlevels - 1; ++l) {
+        ts[l] = (int)at;
+        at += 4 * (int64_t)hs[kStLev + 2 * l];
+        if (at > INT32_MAX) throw HipError{hipErrorOutOfMemory, "tree boxes"};
+        te[l] = (int)at;
+      }
+      if (at > nb0) {
+        bld.B.fit((size_t)at, nb0);
         hipLaunchKernelGGL(k_flag_children<0>, dim3(ceil_div(n, 256)), dim3(256), 0, st, n, ls[1],
-                           0, bld.nboxes, (const int*)part.p, T, cap, ptrs(bld.B), bld.ks, bld.kt,
-                           state.p);
+                           0, nb0, (const int*)part.p, T,
+                           (int)std::min<size_t>(bld.B.cap, INT32_MAX), ptrs(bld.B), bld.ks,
+                           bld.kt, state.p);
         hip_throw(hipGetLastError(), "level restriction");
-      }
-    }
-    readback(hs.data(), state.p, sizeof(int) * kStWords, st);
-    if (nb0 <= kWgBoxes && cap >= 5 * nb0) {
-      for (int l = 2; l <= nlevels - 1; ++l) {
-        ts[l] = hs[kStLev + 2 * l];
-        te[l] = hs[kStLev + 2 * l + 1];
-      }
-    } else {
-      if (hs[kStStatus] != 0) return false;  // out of room
-      int at = bld.nboxes;
-      for (int l = 2; l <= nlevels - 1; ++l) {
-        ts[l] = at;
-        te[l] = at += 4 * hs[kStLev + 2 * l];
       }
     }
     for (int l = 2; l <= nlevels - 1; ++l) added += te[l] - ts[l];
@@ -1881,12 +1910,17 @@ static bool build_try(const TreePrep* P, TreePrep* own, const double* src, int64
   // updateflags sweep below refines nothing and both reorganisations are the
   // identity: the tree is already level-restricted.
   if (added > 0) {
-    bld.reorg(ls, le, ts, te, nlevels);
-    bld.computecoll(ls, le, bs, nlevels);
-    level_tab();
     // the sweep over the levels, the new boxes' ranges kept on the device:
     // two launches a level and one round trip in all
-    const int cap = (int)std::min<size_t>(bld.B.cap, INT32_MAX);
+    // (it adds 0.7 to 1.0 times what the flagged refinement added on curves and
+    // clusters, 1.5 around isolated tight clusters, little where that added little)
+    const int cap = (int)std::min<int64_t>(
+        bld.nboxes + (int64_t)room * (13 * (int64_t)added / 8 + 64), INT32_MAX);
+    bld.reorg(ls, le, ts, te, nlevels, (size_t)cap);
+    bld.B.alloc_coll((size_t)cap);
+    part.alloc((size_t)cap / kLrTile + 1, st);
+    bld.computecoll(ls, le, bs, nlevels);
+    level_tab();
     for (int k = 0; k < kStWords; ++k) hs[k] = 0;
     hs[kStLev + 2 * 2] = hs[kStLev + 2 * 2 + 1] = bld.nboxes;
     upload_bytes(state.p, hs.data(), sizeof(int) * kStWords, st);
@@ -1904,7 +1938,7 @@ static bool build_try(const TreePrep* P, TreePrep* own, const double* src, int64
         hip_throw(hipGetLastError(), "level restriction");
       }
       tail_ub = std::min<int64_t>(
-          std::min<int64_t>(4 * (int64_t)n, (int64_t)cap - bld.nboxes), (int64_t)32768 * room);
+          std::min<int64_t>(4 * (int64_t)n, (int64_t)cap - bld.nboxes), (int64_t)262144 * room);
     }
     std::fill(ts.begin(), ts.end(), 0);
     std::fill(te.begin(), te.end(), 0);
@@ -1923,7 +1957,7 @@ static bool build_try(const TreePrep* P, TreePrep* own, const double* src, int64
     // second reorganisation is the identity and the colleagues are those
     // computed above
     if (added2 > 0) {
-      bld.reorg(ls, le, ts, te, nlevels);
+      bld.reorg(ls, le, ts, te, nlevels, (size_t)bld.nboxes);
       bld.computecoll(ls, le, bs, nlevels);
     }
   }
@@ -1987,9 +2021,7 @@ void build_tree(const double* src, int64_t ns, const double* trg, int64_t nt, in
   TreePrep own;
   const bool mine = !tree_prepare_matches(prep, src, ns, trg, nt, nlmax);
   if (mine) prepare_into(own, src, ns, trg, nt, nlmax, st);
-  // The restriction adds about as many boxes as there are on curves and
-  // clusters, up to six times as many around isolated tight clusters.
-  for (int room = 8;; room *= 4) {
+  for (int room = 1;; room *= 4) {
     if (build_try(mine ? &own : prep, mine ? &own : nullptr, src, ns, trg, nt, ndiv, idivflag,
                   nlmax, t, st, room))
       return;
