@@ -193,8 +193,9 @@ template <int IFC, int IFD, int PG, int NDT, bool OOL = false>
 FMM2D_HD void pair_helm(double dx, double dy, cplx zk, const SrcStr<NDT>& s, double thresh,
                         Acc<HELM, PG, NDT>& a) {
   double rr = dx * dx + dy * dy;
-  // 1/r, then r with one correction (a point's own pair: r = 0)
-  const double rinv = fast_rsqrt(fmax(rr, 2.2250738585072014e-308));
+  // 1/r, then r with one correction (a point's own pair: r = 0; the smallest
+  // number keeps 0 out of 1/r and leaves every other rr, subnormals too, as it is)
+  const double rinv = fast_rsqrt(fmax(rr, 4.9406564584124654e-324));
   double r = rr * rinv;
   r = fma(fma(-r, r, rr), 0.5 * rinv, r);
   cplx z = zk * r;

@@ -71,6 +71,18 @@ def test_hankel_edges(zk, dip):
     assert np.all(np.abs(g - wantg) <= 2 * tol * scaleg), np.max(np.abs(g - wantg) / scaleg / tol)
 
 
+@pytest.mark.parametrize("zk", [1e155, 1e155 + 1e154j])
+def test_subnormal_squares(zk):
+    """Distances whose square is subnormal (r < 1.5e-154).  The square's own rounding, half of 4.9e-324, is an error of
+    k r times half of that over r^2 in the argument, more for the singular part of small arguments."""
+    z = np.array([0.3, 1.0, 3.0, 7.0])
+    x = z * 1e-155
+    p, _ = single_source("h", x, zk=zk)
+    h0 = hankel1(0, zk * x)
+    tol = 1e-14 + 4 * ULP * z + 2 * (1 + z) * 4.9406564584124654e-324 / (x * x)
+    assert np.all(np.abs(p - 0.25j * h0) <= tol * 0.25 * np.abs(h0)), np.abs(p / (0.25j * h0) - 1) / tol
+
+
 def test_large_arguments():
     x = np.array([1e7, 2.0 ** 40, 2.0 ** 49, 2.0 ** 50, 2.0 ** 55, 1e30])  # exact squares or far beyond phase accuracy
     p, _ = single_source("h", x, zk=1.0)
