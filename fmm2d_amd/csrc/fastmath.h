@@ -19,11 +19,12 @@
 //   normal (the pair kernels pass |z|^2 of pairs not excluded by the threshold).
 // fast_rcp: 1/x from the hardware approximation and one step of third order,
 //   fast_rsqrt: 1/sqrt(x) likewise; both within one unit in the last place for
-//   normal x.
+//   normal x (fast_rsqrt takes subnormal x too).
 // fast_sincos: x - n pi/2 by two multiply-adds with pi/2 in two parts (the first
 //   product is exact in the multiply-add), then Chebyshev interpolants of
 //   degree 5 of (sin r - r) / r^3 and (cos r - 1 + r^2/2) / r^4 in r^2 on
 //   |r| <= pi/4 (2e-17, 1e-18; mpmath).  |x| < 2^50; the library beyond, out of line.
+// The constants come from gen_fastmath.py.
 //
 // Against the forms before (degree-9 Taylor series, two Newton steps, the
 // library's sincos and square root, constants through moves; and the Helmholtz

@@ -222,7 +222,9 @@ __global__ __launch_bounds__(kPlanT) void k_plan(int64_t nb, int np, PlanLevels 
 // ---------------------------------------------------------- work counters
 // cnt[0] near pairs, [1] list-2 pairs, [2] M2M edges, [3] L2L edges,
 // [4] list-3 (point, box) pairs, [5] list-4 (source, box) pairs; M2M edges
-// count at the parent, L2L edges at the child
+// count at the parent, L2L edges at the child.  These are the edges of the
+// reference's algorithm, whose upward and downward passes reach level 1; the
+// drivers leave the parents of levels 0 and 1 out, whose expansions nothing reads.
 __global__ void k_counts(int64_t n, const int* ilevel, const int* iparent, const int* nchild,
                          const int* ichild, const int* sse, const int* tse, int ifpgh,
                          int ifpght, const int* n1, const int* l1, const int* n2, const int* n3,

@@ -293,7 +293,9 @@ __global__ void k_hp2m_rowlen(int64_t n, const HLev* lev, const int* leaf, const
 // they took 924 us for 678.)  The rows formed in place, of orders from 30 on,
 // keep the limit of five wavefronts a CU that the LDS sets: with as many as fit,
 // more lines are half written at a time (P2M of 5e5 points at order 33 0.53 ->
-// 0.64 ms, of 2e5 at order 39 0.325 -> 0.341).
+// 0.64 ms, of 2e5 at order 39 0.325 -> 0.341).  A smaller cap lets more wavefronts
+// in and more orders out: 23 values take 0.23 ms for 0.25 at orders 8 to 19, but
+// orders 22 to 29 go in place, 0.83 for 0.58 (1e6 points); 39 values 0.63.
 constexpr int kRowCap = 31;  // 31 KB a wavefront: orders up to 29
 
 // The rows of the lanes with w > 0 values at sh + lane * stride to dst (lane's)
@@ -1413,8 +1415,10 @@ void HelmOps::next() {
 // evaluation points (sources / targets), as the planners need.  stage: for the
 // operator tables, kept by the caller until st is done.  mixed: the M2L
 // runs on v_mfma_f32_16x16x4f32 with FP32 copies of the operators (the
-// swizzled A-fragment layout is the same for both element types) and of the
-// multipoles, accumulating in FP32 and adding into the FP64 locals.
+// swizzled A-fragment layout is the same for both element types), adding into the
+// FP64 locals.  Up to kM2LMaxP coefficients the transformed sources are formed in
+// FP64 and rounded, and the sums folded to FP64 twice an orbit (m2l.h); beyond,
+// FP32 copies of the multipoles and FP32 sums (k_translate).
 void helm_box_passes(HelmOps& ops, const Lists& L, int nd, int pg, int pgt, cplx* mpp, cplx* locp,
                      Staging& stage, Timer& tm, hipStream_t st, bool mixed = false) {
   while (!ops.done()) ops.next();

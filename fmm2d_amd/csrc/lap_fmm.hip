@@ -8,18 +8,21 @@
 //
 // Work decomposition (one launch per step, or per level where the reference's
 // loops carry a level dependency):
-//   P2M        one 64-lane wavefront per leaf, lane = coefficient index
-//   M2M / L2L  one wavefront per box, fixed 4 child-offset matrices
-//   M2L        one wavefront per target box, lane = output coefficient; the
-//              translation depends only on the offset (dx,dy) in [-3,3]^2 of
-//              the source box (in box sizes) and is precomputed once
-//              (49 (p+1)x(p+1) matrices; the level enters only through
-//              log(boxsize) M_0 added to L_0)
-//   list 4     one wavefront per box (sources of coarser leaves -> local)
-//   list 3+L2P one thread per evaluation point
+//   P2M        one thread per (leaf, density), all coefficients in registers
+//              (up to kW of them; one wavefront per leaf beyond)
+//   M2M / L2L  shift.h: a thread per row of a parent's operator, one operator
+//              for the four children after a DFT over them
+//   M2L        m2l.h up to kM2LMaxP coefficients: MFMA, 10 operators for the 27
+//              offsets of a child position; translate.h beyond: MFMA, one of 49
+//              operators per offset.  Operators are made once per order (the
+//              level enters only through log(boxsize) M_0 added to L_0)
+//   list 4     wavefronts over the boxes that have it (sources of coarser
+//              leaves -> local)
+//   list 3+L2P one thread per evaluation point and density, list-3 pairs shared
+//              out over a workgroup
 //   near field one thread per evaluation point over its leaf's list 1
-// All kernels read and write the box expansions in place; there are no
-// atomics in the FMM itself (pull form, as the reference's loops).
+// All kernels read and write the box expansions in place; no floating-point
+// atomics (pull form, as the reference's loops).
 #include <algorithm>
 #include <complex>
 #include <map>
@@ -1645,8 +1648,8 @@ int laplace_fmm(int kind, const CauchyArgs& a, hipStream_t st) {
 #undef FMM2D_P2L_W
 #undef FMM2D_P2L_W32
     tm.mark(1);
-    // ---- translation operators as MFMA fragments: 4 M2M, 4 L2L
-    // (levels 0 and 1 have neither M2L nor list-3 or list-4 boxes)
+    // ---- step 3: M2M, finest parents first, on the vector units (levels 0 and 1
+    // have neither M2L nor list-3 or list-4 boxes)
     auto side = [&](cplx* v, int l) { return ShiftSide{v, 0, P, nterms[l] + 1}; };
     for (int l = nl - 1; l >= 2; --l)
       launch_shift<1, 1>(nd, bp.lev_pos[l + 1] - bp.lev_pos[l], bp.list.p + bp.lev_pos[l],

@@ -369,8 +369,20 @@ inline void launch_m2l(int nd, const std::vector<M2LLev>& levels, const int* tli
   hipLaunchKernelGGL((k_m2l<T, RTC, KSC, HB, NW, SGN, LOGT>), dim3((unsigned)(8 * per_xcd)),   \
                      dim3(64 * NW), 0, st, nd, per_xcd, tab, tlist, s2, orb,                   \
                      static_cast<const T*>(A), ilevel, band, logr, src, dst)
-// 8 wavefronts share the operators where their z fits the LDS beside them and
-// 4 would leave one wavefront per SIMD (33 to 40 coefficients, FP64)
+// Row tiles and k steps follow from P; HB, the classes that are transformed at a
+// time, and the wavefronts:
+// HB: with two classes transformed at a time a source row is loaded in two pieces
+// and not four, but their z takes twice the LDS.  Two and three k steps: 2 (M2L
+// of 1e6 points, 10 coefficients 0.37 ms, 0.42 with 1; 19 in FP32 0.32 and 0.38,
+// of 1e7 in FP64 3.83 and 3.91).  Four k steps, where 2 leaves one workgroup a CU,
+// have it too, though 1 is faster in FP64: 1e6 points with 29 coefficients 0.41 ms
+// and 0.31 with 1, hfmm2d of 5e5 with 27 0.35 and 0.25.  From five on 1: 2
+// takes 128 KB at five.
+// Wavefronts: 8 share the operators where their z fits the LDS beside them and 4
+// would leave one wavefront per SIMD, which is FP64 with five k steps alone (33 to
+// 40 coefficients: 5e5 points with 39 0.50 ms, 0.63 with 4; 2e6 points with 17 to
+// 201 4.1 and 5.1).  From six k steps on 8 do not fit the 163840 bytes of LDS
+// (163880 at six) and FP64 stays at one wavefront per SIMD.
 #define FMM2D_M2L_K(T, NW5)                   \
   switch (ksc) {                              \
     case 2: FMM2D_M2L(T, 1, 2, 2, 4); break;  \

@@ -6,11 +6,13 @@
 // 8-bit digits, one launch per digit after one that counts the digits of every
 // pass (k_rs_hist here, or the kernel that makes the keys, rs_count):
 //   k_rs_pass: a workgroup takes the next tile of keys by ticket, ranks its
-//   keys stably (the four waves take contiguous quarters of the tile in rounds
-//   of 64 consecutive keys: rank = keys of the digit in earlier waves + earlier
-//   rounds + lower lanes), publishes its count of each digit, adds the counts
-//   of the tiles before it by looking back over their published words (a
-//   tile's own count, or the sum up to and including it), places its keys in
+//   keys stably (the tile's waves, four or eight, take contiguous parts of it in
+//   rounds of 64 consecutive keys: rank = keys of the digit in earlier waves +
+//   earlier rounds + lower lanes), publishes its count of each digit, adds the
+//   counts of the tiles before it by looking back over their published words (a
+//   tile's own count, or the sum up to and including it: the decoupled look-back
+//   of Merrill and Garland's single-pass scan, used for each digit as in Adinets
+//   and Merrill's one-sweep radix sort), places its keys in
 //   LDS in digit order and writes each digit's run with consecutive threads
 //   on consecutive addresses.
 // A tile waits only for tiles of earlier tickets, whose workgroups are already

@@ -336,7 +336,7 @@ __global__ void k_refine_flags(int64_t n, int lo, const int* ses, const int* set
   flag[i] = nn > ndiv ? 1 : 0;
 }
 
-// flag[i] = iflag[lo+i] > 0 (tree_refine_boxes_flag, tree_routs2d.f:334-388)
+// *total = flags set in flag[0..n), from its exclusive scan offs
 __global__ void k_total(int n, const int* flag, const int* offs, int* total) {
   *total = (n > 0) ? offs[n - 1] + flag[n - 1] : 0;
 }

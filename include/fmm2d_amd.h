@@ -65,7 +65,9 @@ typedef struct {
   /* out (count_work = 1): algorithmic work per stage, same slots as timeinfo: flops for
    * [0..7] (P2P 12+12*nd per Cauchy pair for pot+grad, M2L 8(p+1)^2 nd per
    * list-2 pair, 8(p+1) nd per point for P2M/L2P, 8(p+1)^2 nd per M2M/L2L
-   * edge), bytes for [8] (40 per point + 80 per box); 0 when not counted. */
+   * edge), bytes for [8] (40 per point + 80 per box); 0 when not counted.  M2M
+   * and L2L count the reference algorithm's edges, from parents of level 1 on,
+   * also those of level 1, at most 16 each, which these drivers do not run. */
   double work[16];
   int64_t near_pairs;      /* out: source-target pairs in the near field */
   int64_t m2l_pairs;       /* out: list-2 translations performed */

@@ -1,5 +1,5 @@
 """The GPU quadtree against the C oracle's (oracle/oracle.c), array for array, at the sizes where the
-build changes its ways: the sort's tiles (512, 1024, 2048 keys, by size), one workgroup's scan (16384
+build changes its ways: the sort's tiles (512, 1024, 4096 keys, by size), one workgroup's scan (16384
 boxes) and scan tiles of 4096, room for the level restriction (the last case builds again with more), and
 trees from a single leaf to more than a million boxes."""
 import numpy as np
