@@ -56,20 +56,23 @@ VAL_BLOCKS = 128
 TRAFFIC_KEYS = {"fp64": ("m2l_fp64", "near_fp64"), "mixed": ("m2l_mixed", "near_mixed"),
                 "fp64+learned": ("m2l_fp64_learned", "near_fp64_learned"),
                 "mixed+learned": ("m2l_learned", "near_learned")}
-# HBM bytes per M2L launch measured with rocprofv3 --pmc (FETCH_SIZE, WRITE_SIZE),
-# scaled by the counters' reading for a copy kernel of known size
+# HBM bytes per M2L and near-field launch measured with rocprofv3 --pmc (FETCH_SIZE,
+# WRITE_SIZE), scaled by the counters' reading for a copy kernel of known size
 TRAFFIC_FILE = os.path.join(ROOT, "profiles", "lfmm2d_n1e7_traffic.txt")
 
 
-def read_traffic(precision):
-    """bytes_per_launch recorded for this precision in TRAFFIC_FILE, or None."""
+def read_traffic(pipeline, kernel, nboxes, path=None):
+    """HBM bytes of one launch of `kernel` in `pipeline` as recorded in TRAFFIC_FILE, whose
+    lines read `bytes_per_launch_<pipeline>: <bytes> <kernel> <boxes of its tree>`; None
+    where there is no such line or it is of another kernel or tree."""
     try:
-        with open(TRAFFIC_FILE) as f:
+        with open(path or TRAFFIC_FILE) as f:
             for line in f:
                 key, _, val = line.partition(":")
-                if key.strip() == f"bytes_per_launch_{precision}":
-                    return int(float(val.strip()))
-    except OSError:
+                if key.strip() == f"bytes_per_launch_{pipeline}":
+                    nbytes, name, boxes = val.split()
+                    return int(nbytes) if name == kernel and int(boxes) == nboxes else None
+    except (OSError, ValueError):
         pass
     return None
 
@@ -881,12 +884,12 @@ def main():
         "m2l": {"bound": "mfma", "kernel": "k_m2l (M2L, %s MFMA)" % prec,
                 "achieved": round(a_m2l, 3), "peak": peak, "unit": "TFLOP/s",
                 "frac": round(a_m2l / peak, 4),
-                "traffic": read_traffic(TRAFFIC_KEYS[head][0]),
+                "traffic": read_traffic(TRAFFIC_KEYS[head][0], "k_m2l", R["nboxes"]),
                 "launch_ms": round(t_m2l * 1e3, 4), "flops_per_launch": work[3]},
         "near": {"bound": "valu", "kernel": "k_near (list-1 pairs, %s vector ALU)" % prec,
                  "achieved": round(a_near, 3), "peak": peak, "unit": "TFLOP/s",
                  "frac": round(a_near / peak, 4),
-                 "traffic": read_traffic(TRAFFIC_KEYS[head][1]),
+                 "traffic": read_traffic(TRAFFIC_KEYS[head][1], "k_near", R["nboxes"]),
                  "launch_ms": round(t_near * 1e3, 4), "flops_per_launch": work[7]},
     }
     # the tree stage (build, level restriction, final order, lists) against
