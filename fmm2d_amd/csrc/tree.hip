@@ -1643,8 +1643,11 @@ static bool build_try(const TreePrep* P, TreePrep* own, const double* src, int64
   bld.kt = pk[1]->view();
 
   // the refinement makes 2 to 3 boxes for every ndiv points of an area, 5 on a
-  // curve, and the level restriction as many again on a curve
-  bld.B.alloc(std::max<size_t>(1536, (size_t)(11 * (ns + nt) / std::max(ndiv, 1))), st);
+  // curve, and the level restriction as many again on a curve, twice as many
+  // around a few clusters, for which small trees, whose restriction would run
+  // again, have room
+  const size_t boxes = (size_t)((ns + nt) / std::max(ndiv, 1));
+  bld.B.alloc(std::max<size_t>(2048, boxes <= kWgBoxes / 4 ? 18 * boxes : 11 * boxes), st);
   DBuf<int> state(kStWords, st);
   std::vector<int> hs(kStWords, 0);
 
